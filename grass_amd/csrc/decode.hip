@@ -1,18 +1,20 @@
 // Full decode of the resident compressed graph to CSR (rowptr u64[n+1], col u32[m]).
 //
-// Edge-parallel: each wave64 owns a contiguous range of output slots (a tuning choice, 2048 by
-// default), so writes are coalesced and work is balanced whatever the degree skew.  When 64
-// consecutive slots lie in one list (most slots: the long lists hold most entries) the wave reads
-// that vertex's header once and divides through shared multiply-high reciprocals; otherwise each
-// lane finds its vertex from the 64 row ends after the previous owner (one coalesced load and a
-// register search), parses that vertex's header and decodes its element:
-//   LE: O(1) random access (LE/src/bcg.cuh:196-261);
-//   GT: block heads and checkpoints are absolute and every other body is a gap, so the wave
-//       turns (absolute | gap+1) values into ids with a segmented prefix sum, carrying the
-//       running id from lane 63 into the next 64 slots (the cooperative decode of
-//       GT/src/bcg.cuh:171-345 and GT/src/grass.cu:525-553, without its per-warp cache
-//       limits).  A wave whose range starts between two absolute positions first backs up to
-//       the earlier one.
+// Run-parallel (LE, and GT with a checkpoint interval P <= 4): each wave64 owns a contiguous range
+// of runs, a run being at most 4 consecutive positions that one lane decodes by itself -- LE: of one
+// chunk, from the chunk's rock pair and one contiguous span of seas (LE/src/bcg.cuh:196-261 decodes
+// a position at a time); GT: a block head or checkpoint and the gaps after it.  The outputs of a
+// wave's 64 runs are consecutive, so they are staged in LDS and stored with coalesced writes.
+//
+// Slot-parallel (GT with P > 4): each wave owns a contiguous range of output slots (a tuning choice).
+// When 64 consecutive slots lie in one list the wave reads that vertex's header once and divides
+// through shared multiply-high reciprocals; otherwise each lane finds its vertex from the 64 row
+// ends after the previous owner (one coalesced load and a register search).  Block heads and
+// checkpoints are absolute and every other body is a gap, so the wave turns (absolute | gap+1)
+// values into ids with a segmented prefix sum, carrying the running id from lane 63 into the next
+// 64 slots (the cooperative decode of GT/src/bcg.cuh:171-345 and GT/src/grass.cu:525-553, without
+// its per-warp cache limits).  A wave whose range starts between two absolute positions first backs
+// up to the earlier one.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -129,7 +131,7 @@ __device__ __forceinline__ uint32_t gt_element_src(const Src& w, const Hdr& h, u
 
 // The slots [e0, e1) of one wave: vlo owns e0, vhi bounds the owner of e1 - 1, decoding starts
 // at eb <= e0 (a run's absolute value); GT payload words come from `src`.
-template <int FMT, class Src>
+template <class Src>
 __device__ __forceinline__ void decode_range(const DevGraph& g, const Src& src, const uint64_t* __restrict__ rowptr,
                                              uint32_t* __restrict__ col, uint64_t e0, uint64_t e1, uint64_t eb,
                                              uint32_t vlo, uint32_t vhi, uint32_t span) {
@@ -141,7 +143,6 @@ __device__ __forceinline__ void decode_range(const DevGraph& g, const Src& src, 
     uint64_t rc = rowptr[cur], rn = rowptr[cur + 1];
     uint32_t hv = 0xFFFFFFFFu;  // vertex whose list constants are cached below
     Hdr uh;
-    UDiv d1, d0;
     GtList gl;
     for (uint64_t base = eb; base < e1; base += kWave) {
         const uint64_t e = base + lane;
@@ -153,16 +154,10 @@ __device__ __forceinline__ void decode_range(const DevGraph& g, const Src& src, 
             // the whole wave is inside one list: one header, shared constants, no owner search
             if (cur != hv) {
                 hv = cur;
-                load_hdr<FMT>(g, hv, uh);
-                if (FMT == kGT) {
-                    gl.init(uh, hv, g.cp_shift);
-                } else {
-                    d1.init(uh.q + 1);
-                    d0.init(uh.q);
-                }
+                load_hdr<kGT>(g, hv, uh);
+                gl.init(uh, hv, g.cp_shift);
             }
-            if (FMT == kGT) x = gl.at(src, (uint32_t)(ee - rc), head);
-            else x = element_uniform<FMT>(g, uh, hv, (uint32_t)(ee - rc), d1, d0, head);
+            x = gl.at(src, (uint32_t)(ee - rc), head);
         } else {
             // Owner of slot ee: one coalesced load of the 64 row ends after `cur` (and, beside
             // it, of those 64 vertices' headers), then a 6-step search over them in registers;
@@ -212,112 +207,107 @@ __device__ __forceinline__ void decode_range(const DevGraph& g, const Src& src, 
             }
             const uint32_t k = (uint32_t)(ee - vstart);
             Hdr h;
-            unpack_hdr<FMT>(hv4, h);
-            if (FMT == kLE) {
-                x = le_get(g.w, h, v, k);
-            } else {
-                uint32_t blk, i;
-                gt_locate(h, k, blk, i);
-                x = gt_element_src(src, h, v, blk, i, g.cp_shift, head);
-            }
+            unpack_hdr<kGT>(hv4, h);
+            uint32_t blk, i;
+            gt_locate(h, k, blk, i);
+            x = gt_element_src(src, h, v, blk, i, g.cp_shift, head);
         }
-        if (FMT == kGT) {
-            if (lane == 0 && !head) {
-                x += carry;
-                head = 1;
-            }
-            x = short_segmented_sum(x, head, span);
-            carry = (uint32_t)__builtin_amdgcn_readlane((int)x, kWave - 1);
+        if (lane == 0 && !head) {
+            x += carry;
+            head = 1;
         }
+        x = short_segmented_sum(x, head, span);
+        carry = (uint32_t)__builtin_amdgcn_readlane((int)x, kWave - 1);
         if (act && e >= e0) col[e] = x;
     }
 }
 
+// ---------------------------------------------------------------- runs (LE; GT with P <= 4)
+// A run is at most 4 consecutive positions of a list that decode without any other run.
+//   GT: a block head or a checkpoint and the gap fields after it up to the next one: the absolute
+//       field and its gaps are one contiguous span of the stream.
+//   LE: positions [4j, 4j + 4) of a chunk (the list's last position, rock C, is a chunk of one): the
+//       chunk's rock pair, one division for its slope, and one contiguous span of at most 4 seas.
+// The run kernel gives each lane one run: its slots and stream bits from the run's index in its list
+// (no per-position division), its fields from one 16-byte load (a fifth word when they reach past
+// it; LE: and one for the rock pair), its ids in registers (no cross-lane scan).  The 64 runs of a
+// wave's pass fill consecutive output slots, which are staged in LDS and stored with coalesced
+// writes.  Runs are numbered over the graph (roff = exclusive scan of runs per vertex) and every
+// wave takes a fixed number of them, with its first vertex from a table like the slot-based one.
+// What bounds it is instruction issue: LE_RUNS_FIGURES
 
-// ---------------------------------------------------------------- GT runs (P <= 4)
-// A run is a block head or a checkpoint and the gap fields after it up to the next one: at most P
-// positions, the first absolute, so a run decodes without any other.  The run kernel gives each
-// lane one run: its slots and stream bit from the run's index in its list (no per-position
-// division), its fields from one 16-byte load of the stream (a fifth word when they reach past
-// it), its ids by adding the gaps in registers (no cross-lane scan).  The 64 runs of a wave's pass
-// fill consecutive output slots, which are staged in LDS and stored with coalesced writes.  Runs
-// are numbered over the graph (roff = exclusive scan of runs per vertex) and every wave takes a
-// fixed number of them, with its first vertex from a table like the slot-based one.
+constexpr uint32_t kRunMax = 4;    // positions of a run; the run kernel takes GT checkpoint intervals up to it
+constexpr uint32_t kLeRunShift = 2;  // LE: runs of 1 << 2 positions
 
-constexpr uint32_t kRunMaxP = 4;  // the run kernel takes P <= kRunMaxP (the default P is 4)
-
-// Runs of a GT vertex with d entries: R blocks of q + 1 positions and C - R of q, each
-// ceil(len / P) runs.
-__host__ __device__ __forceinline__ uint64_t gt_runs(uint32_t d, uint32_t C, uint32_t q, uint32_t sh) {
+// Runs of a vertex with d entries in C chunks or blocks: R of q + 1 positions and C - R of q, each
+// ceil(len >> sh) runs, and LE's last rock.
+__host__ __device__ __forceinline__ uint64_t list_runs(int fmt, uint32_t d, uint32_t C, uint32_t q, uint32_t sh) {
     if (!d) return 0;
-    const uint32_t R = d - C * q, P1 = (1u << sh) - 1;
-    return (uint64_t)R * ((q + 1 + P1) >> sh) + (uint64_t)(C - R) * ((q + P1) >> sh);
+    if (fmt == kLE && d == 1) return 1;
+    const uint32_t D = fmt == kLE ? d - 1 : d, R = D - C * q, P1 = (1u << sh) - 1;
+    return (uint64_t)R * ((q + 1 + P1) >> sh) + (uint64_t)(C - R) * ((q + P1) >> sh) + (fmt == kLE ? 1 : 0);
 }
 
 struct RunGen {  // runs of vertex i, from its header
     const uint4* hdr;
+    int fmt;
     uint32_t sh;
     __device__ __forceinline__ uint64_t operator()(uint64_t i) const {
         const uint4 e = hdr[i];
-        return gt_runs(e.z, e.w & 0xFFFFu, e.y >> 16, sh);
+        return list_runs(fmt, e.z, e.w & 0xFFFFu, e.y >> 16, sh);
     }
 };
 
-// One run's place: first output slot, stream bit of its absolute field, positions, whether that
-// field is the block head (else a checkpoint), and its block.
+// One run's place: first output slot, its positions [i0, i0 + cnt) of block (chunk) blk, which has
+// len positions; GT: the stream bit of its absolute field.
 struct RunAt {
     uint64_t slot, bit;
-    uint32_t cnt, blk;
-    bool head;
+    uint32_t cnt, blk, i0, len;
 };
 
-// Run rr (< the vertex's runs) of a vertex: R blocks of nr1 runs, then blocks of nr0.  Div divides
-// by nr1 / nr0 (shared multiply-high reciprocals when the wave is in one list, else per lane).
-template <class Div1, class Div0>
+// Run rr (< the vertex's runs) of a vertex: R blocks of nr1 runs, then blocks of nr0 (LE: then the
+// last rock, block C).  Div divides by nr1 / nr0 (shared multiply-high reciprocals when the wave is
+// in one list, else per lane).
+template <int FMT, class Div1, class Div0>
 __device__ __forceinline__ RunAt run_at(const Hdr& h, uint64_t vstart, uint32_t rr, uint32_t sh, const Div1& div1,
                                         const Div0& div0) {
     const uint32_t P1 = (1u << sh) - 1;
     const uint32_t nr1 = (h.q + 1 + P1) >> sh, nr0 = (h.q + P1) >> sh;
     const uint32_t bigr = h.R * nr1;
-    uint32_t blk, j, len;
-    uint64_t bpos, bbit;
-    if (rr < bigr) {
-        blk = div1(rr, nr1);
-        j = rr - blk * nr1;
-        len = h.q + 1;
-        bpos = (uint64_t)blk * (h.q + 1);
-        bbit = h.pay + (uint64_t)blk * gtx_field(h, h.q + 1, sh);
-    } else {
-        const uint32_t t = rr - bigr, b2 = div0(t, nr0);
-        j = t - b2 * nr0;
-        blk = h.R + b2;
-        len = h.q;
-        bpos = (uint64_t)h.R * (h.q + 1) + (uint64_t)b2 * h.q;
-        bbit = h.pay + (uint64_t)h.R * gtx_field(h, h.q + 1, sh) + (uint64_t)b2 * gtx_field(h, h.q, sh);
-    }
-    const uint32_t i0 = j << sh;
     RunAt a;
-    a.cnt = min(1u << sh, len - i0);
-    a.slot = vstart + bpos + i0;
-    a.bit = bbit + gtx_field(h, i0, sh);
-    a.head = i0 == 0;
-    a.blk = blk;
+    uint32_t j;
+    uint64_t bpos, bbit = 0;
+    if (rr < bigr) {
+        a.blk = div1(rr, nr1);
+        j = rr - a.blk * nr1;
+        a.len = h.q + 1;
+        bpos = (uint64_t)a.blk * (h.q + 1);
+        if (FMT == kGT) bbit = h.pay + (uint64_t)a.blk * gtx_field(h, h.q + 1, sh);
+    } else {
+        // (LE, d = 1: q = 0, one run, whose index 0 divides to 0 by any divisor)
+        const uint32_t t = rr - bigr, b2 = div0(t, FMT == kLE && nr0 == 0 ? 1u : nr0);
+        j = t - b2 * nr0;
+        a.blk = h.R + b2;
+        a.len = FMT == kLE && a.blk == h.C ? 1u : h.q;
+        bpos = (uint64_t)h.R * (h.q + 1) + (uint64_t)b2 * h.q;
+        if (FMT == kGT)
+            bbit = h.pay + (uint64_t)h.R * gtx_field(h, h.q + 1, sh) + (uint64_t)b2 * gtx_field(h, h.q, sh);
+    }
+    a.i0 = j << sh;
+    a.cnt = min(1u << sh, a.len - a.i0);
+    a.slot = vstart + bpos + a.i0;
+    a.bit = FMT == kGT ? bbit + gtx_field(h, a.i0, sh) : 0;
     return a;
 }
 
-// The ids of one run into out[0 .. cnt): the absolute field, then each gap + 1 added on.  One
-// 16-byte load holds the field's offset in its word (< 32), a 32-bit field and three gaps of up to
-// 21 bits; a fifth word is read when they need more (at most 31 + 32 + 3 * 31 < 160 bits).
-__device__ __forceinline__ void run_ids(const uint32_t* __restrict__ w, const Hdr& h, uint32_t v, const RunAt& a,
-                                        uint32_t out[kRunMaxP]) {
-    const uint32_t* p = w + (a.bit >> 5);
-    const Words4 q = *(const Words4*)p;
-    const uint32_t s = (uint32_t)(a.bit & 31);
-    const uint32_t aw = a.head ? h.f1 : 32u, f2 = h.f2;
-    const uint32_t w4 = s + aw + (a.cnt - 1) * f2 > 128 ? p[4] : 0u;
-    uint64_t buf = (((uint64_t)q.x << 32) | q.y) << s;
-    uint32_t avail = 64 - s, n0 = q.z, n1 = q.w, n2 = w4;  // buffered bits, then the words after them
-    auto take = [&](uint32_t wdt) {  // 1 <= wdt <= 32
+// Consecutive fields of 1 to 32 bits from stream bit `bit`: five words from the first field's (the
+// offset in its word and four 32-bit fields take at most 31 + 128 bits).
+struct FieldReader {
+    uint64_t buf;
+    uint32_t avail, n0, n1, n2;  // buffered bits, then the words after them
+    __device__ __forceinline__ FieldReader(const Words4& q, uint32_t w4, uint32_t s)
+        : buf((((uint64_t)q.x << 32) | q.y) << s), avail(64 - s), n0(q.z), n1(q.w), n2(w4) {}
+    __device__ __forceinline__ uint32_t take(uint32_t wdt) {
         if (avail < wdt) {
             buf |= (uint64_t)n0 << (32 - avail);
             avail += 32;
@@ -328,15 +318,71 @@ __device__ __forceinline__ void run_ids(const uint32_t* __restrict__ w, const Hd
         buf <<= wdt;
         avail -= wdt;
         return r;
-    };
-    const uint32_t a0 = take(aw);  // f1 >= 1 for a vertex with entries
-    uint32_t x = a.head ? (a.blk >= h.fp ? v + a0 + 1 : v - a0 - 1) : a0;
+    }
+};
+
+// The ids of one GT run into out[0 .. cnt): the absolute field, then each gap + 1 added on.  One
+// 16-byte load holds the field's offset in its word (< 32), a 32-bit field and three gaps of up to
+// 21 bits; a fifth word is read when they need more.
+__device__ __forceinline__ void gt_run_ids(const uint32_t* __restrict__ w, const Hdr& h, uint32_t v, const RunAt& a,
+                                           uint32_t out[kRunMax]) {
+    const uint32_t* p = w + (a.bit >> 5);
+    const Words4 q = *(const Words4*)p;
+    const uint32_t s = (uint32_t)(a.bit & 31);
+    const bool head = a.i0 == 0;
+    const uint32_t aw = head ? h.f1 : 32u, f2 = h.f2;
+    FieldReader f(q, s + aw + (a.cnt - 1) * f2 > 128 ? p[4] : 0u, s);
+    const uint32_t a0 = f.take(aw);  // f1 >= 1 for a vertex with entries
+    uint32_t x = head ? (a.blk >= h.fp ? v + a0 + 1 : v - a0 - 1) : a0;
     out[0] = x;
 #pragma unroll
-    for (uint32_t k = 1; k < kRunMaxP; ++k) {
+    for (uint32_t k = 1; k < kRunMax; ++k) {
         if (k < a.cnt) {
-            x += (f2 ? take(f2) : 0u) + 1;  // (0-bit gap fields read as 0)
+            x += (f2 ? f.take(f2) : 0u) + 1;  // (0-bit gap fields read as 0)
             out[k] = x;
+        }
+    }
+}
+
+// The ids of one LE run (le_get, codec.h, for each of its positions): rocks c and c + 1 in one
+// window, the interpolation's slope once, and the run's seas, which follow each other.  Both loads
+// are issued before either is used; the rock window of the last rock and the sea span of a run
+// without seas lie at most four words past the record, inside the padded image.
+__device__ __forceinline__ void le_run_ids(const uint32_t* __restrict__ w, const Hdr& h, uint32_t v, const RunAt& a,
+                                           uint32_t out[kRunMax]) {
+    if (h.d == 1) {
+        out[0] = h.f1;
+        return;
+    }
+    const uint32_t c = a.blk, rb = h.f1, sw = h.f2 + 1;
+    const uint32_t i1 = a.i0 ? a.i0 : 1u;        // first sea's position in the chunk
+    const uint32_t skip = a.i0 ? 0u : 1u;        // the run starts with the rock
+    const uint32_t j = (h.q - 1) * c + min(c, h.R) + i1 - 1;
+    const uint64_t rbit = h.pay + (uint64_t)c * rb;
+    const uint64_t sbit = h.pay + (uint64_t)(h.C + 1) * rb + (uint64_t)j * sw;
+    const Words4 rq = *(const Words4*)(w + (rbit >> 5));
+    const uint32_t* sp = w + (sbit >> 5);
+    const Words4 sq = *(const Words4*)sp;
+    const uint32_t ss = (uint32_t)(sbit & 31), rs = (uint32_t)(rbit & 31);
+    const uint32_t w4 = ss + (a.cnt - skip) * sw > 128 ? sp[4] : 0u;
+    uint64_t win = ((uint64_t)rq.x << 32) | rq.y;
+    if (rs) win = (win << rs) | (rq.z >> (32 - rs));
+    const uint32_t r1 = (uint32_t)(win >> (64 - rb)), r2 = (uint32_t)((win << rb) >> (64 - rb));
+    const uint32_t A = c < h.fp ? v - r1 : v + r1;
+    const uint32_t Z = c + 1 < h.fp ? v - r2 : v + r2;
+    const uint32_t step = a.len > 1 ? udiv_chunk(Z - A, a.len) : 0u;
+    FieldReader f(sq, w4, ss);
+    uint32_t x = A + step * a.i0;
+#pragma unroll
+    for (uint32_t k = 0; k < kRunMax; ++k) {
+        if (k < a.cnt) {
+            if (k >= skip) {
+                const uint32_t e = f.take(sw), mag = e >> 1;
+                out[k] = x + ((e & 1) ? 0u - mag : mag);
+            } else {
+                out[k] = A;
+            }
+            x += step;
         }
     }
 }
@@ -352,21 +398,21 @@ struct UDivShared {  // division by the one divisor it was made for
 };
 
 // Wave w decodes runs [w * per_wave, ...) of the graph; rstart[w] is the vertex holding its first.
+template <int FMT>
 __global__ __launch_bounds__(kDecBlock) void decode_runs_kernel(DevGraph g, const uint64_t* __restrict__ rowptr,
                                                                 const uint64_t* __restrict__ roff,
                                                                 const uint32_t* __restrict__ rstart,
                                                                 uint32_t* __restrict__ col, uint64_t nruns,
-                                                                uint32_t per_wave) {
-    __shared__ uint32_t stage_lds[(kDecBlock / kWave) * kWave * kRunMaxP];
+                                                                uint32_t per_wave, uint32_t sh) {
+    __shared__ uint32_t stage_lds[(kDecBlock / kWave) * kWave * kRunMax];
     __shared__ uint32_t owner_lds[kDecBlock];
-    uint32_t* L = stage_lds + (threadIdx.x / kWave) * (kWave * kRunMaxP);
+    uint32_t* L = stage_lds + (threadIdx.x / kWave) * (kWave * kRunMax);
     uint32_t* own = owner_lds + (threadIdx.x & ~(kWave - 1));
     const uint64_t wave = ((uint64_t)blockIdx.x * kDecBlock + threadIdx.x) / kWave;
     const int lane = lane_id();
     const uint64_t r0 = wave * per_wave;
     if (r0 >= nruns) return;  // uniform per wave
     const uint64_t r1 = r0 + per_wave < nruns ? r0 + per_wave : nruns;
-    const uint32_t sh = g.cp_shift;
     // the vertex of the pass's first run and its run bounds, wave-uniform
     uint32_t cur = __builtin_amdgcn_readfirstlane(rstart[wave]);
     uint64_t rc = roff[cur], rn = roff[cur + 1];
@@ -385,7 +431,7 @@ __global__ __launch_bounds__(kDecBlock) void decode_runs_kernel(DevGraph g, cons
             // the whole pass is in one list: one header, shared divisors
             if (cur != hv) {
                 hv = cur;
-                load_hdr<kGT>(g, hv, uh);
+                load_hdr<FMT>(g, hv, uh);
                 uvs = rowptr[hv];
                 const uint32_t P1 = (1u << sh) - 1;
                 u1.u.init((uh.q + 1 + P1) >> sh);
@@ -393,7 +439,7 @@ __global__ __launch_bounds__(kDecBlock) void decode_runs_kernel(DevGraph g, cons
             }
             h = uh;
             v = hv;
-            a = run_at(h, uvs, (uint32_t)(rr - rc), sh, u1, u0);
+            a = run_at<FMT>(h, uvs, (uint32_t)(rr - rc), sh, u1, u0);
         } else {
             // The 64 vertices from `cur`: their run ends (relative to rc), headers and first slots
             // in one coalesced load each.  Vertex cur + j covers the pass's lanes from its first
@@ -452,11 +498,12 @@ __global__ __launch_bounds__(kDecBlock) void decode_runs_kernel(DevGraph g, cons
                 rc = roff[cur];
                 rn = roff[cur + 1];
             }
-            unpack_hdr<kGT>(hv4, h);
-            a = run_at(h, vs, (uint32_t)(rr - rstart_v), sh, UDivBy{}, UDivBy{});
+            unpack_hdr<FMT>(hv4, h);
+            a = run_at<FMT>(h, vs, (uint32_t)(rr - rstart_v), sh, UDivBy{}, UDivBy{});
         }
-        uint32_t ids[kRunMaxP];
-        run_ids(g.w, h, v, a, ids);
+        uint32_t ids[kRunMax];
+        if (FMT == kLE) le_run_ids(g.w, h, v, a, ids);
+        else gt_run_ids(g.w, h, v, a, ids);
         // stage the pass's slots [sb, se) and store them coalesced
         const uint64_t sb = readlane_u64(a.slot, 0);
         const uint32_t lastl = (uint32_t)(r1 - base < (uint64_t)kWave ? r1 - base - 1 : kWave - 1);
@@ -465,7 +512,7 @@ __global__ __launch_bounds__(kDecBlock) void decode_runs_kernel(DevGraph g, cons
         if (act) {
             const uint32_t o = (uint32_t)(a.slot - sb);
 #pragma unroll
-            for (uint32_t k = 0; k < kRunMaxP; ++k)
+            for (uint32_t k = 0; k < kRunMax; ++k)
                 if (k < a.cnt) L[o + k] = ids[k];
         }
         wave_sync();
@@ -480,11 +527,10 @@ __host__ __device__ constexpr uint32_t dec_stage_words(uint32_t per_wave) {
     return (per_wave < kDecStageMax ? per_wave : kDecStageMax) + 64;
 }
 
-// GT with stage != 0: the wave first copies the span of the payload stream its slots use (every
+// The slot-based kernel (GT, P > 4).  With stage != 0 the wave first copies the span of the payload stream its slots use (every
 // field from its first run's absolute value to slot e1) into LDS with coalesced loads, all in
 // flight together, when it fits `stage` words, and then decodes from LDS: no dependent global
 // load per 64 slots.
-template <int FMT>
 __global__ __launch_bounds__(kDecBlock) void decode_csr_kernel(DevGraph g,
                                                                const uint64_t* __restrict__ rowptr,
                                                                const uint32_t* __restrict__ wstart,
@@ -502,53 +548,51 @@ __global__ __launch_bounds__(kDecBlock) void decode_csr_kernel(DevGraph g,
     // GT: an absolute value (block head or checkpoint) starts every run of at most P positions
     const uint32_t span = 1u << g.cp_shift;
     uint64_t eb = e0;
-    if (FMT == kGT) {
-        const uint32_t sh = g.cp_shift;
-        Hdr h;
-        load_hdr<kGT>(g, vlo, h);
-        uint32_t blk, i;
-        gt_locate(h, (uint32_t)(e0 - rowptr[vlo]), blk, i);
-        const uint32_t ib = i & ~(span - 1);
-        eb = e0 - (i - ib);  // back to the block head or checkpoint
-        if (stage) {
-            // bits [B0, B1): from eb's field to slot e1's (the stream's end for the last wave);
-            // a field read touches its word and the next, so words W0 ..= ((B1 - 1) >> 5) + 1
-            const uint64_t B0 = gtx_block_bit(h, blk, sh) + gtx_field(h, ib, sh);
-            Hdr hu;
-            load_hdr<kGT>(g, vhi, hu);
-            uint64_t B1;
-            if (e1 < m) {
-                uint32_t b1, i1;
-                gt_locate(hu, (uint32_t)(e1 - rowptr[vhi]), b1, i1);
-                B1 = gtx_block_bit(hu, b1, sh) + gtx_field(hu, i1, sh);
-            } else {
-                B1 = hu.pay + gtx_payload_bits(hu, sh);
-            }
-            const uint64_t W0 = B0 >> 5;
-            const uint64_t NW = B1 > B0 ? ((B1 - 1) >> 5) + 2 - W0 : 0;
-            if (NW && NW <= stage) {
-                uint32_t* L = dec_lds + (threadIdx.x / kWave) * stage;
-                const uint32_t nw = (uint32_t)NW;
-                for (uint32_t c = 0; c < nw; c += 8 * kWave) {
-                    uint32_t t[8];
+    const uint32_t sh = g.cp_shift;
+    Hdr h;
+    load_hdr<kGT>(g, vlo, h);
+    uint32_t blk, i;
+    gt_locate(h, (uint32_t)(e0 - rowptr[vlo]), blk, i);
+    const uint32_t ib = i & ~(span - 1);
+    eb = e0 - (i - ib);  // back to the block head or checkpoint
+    if (stage) {
+        // bits [B0, B1): from eb's field to slot e1's (the stream's end for the last wave);
+        // a field read touches its word and the next, so words W0 ..= ((B1 - 1) >> 5) + 1
+        const uint64_t B0 = gtx_block_bit(h, blk, sh) + gtx_field(h, ib, sh);
+        Hdr hu;
+        load_hdr<kGT>(g, vhi, hu);
+        uint64_t B1;
+        if (e1 < m) {
+            uint32_t b1, i1;
+            gt_locate(hu, (uint32_t)(e1 - rowptr[vhi]), b1, i1);
+            B1 = gtx_block_bit(hu, b1, sh) + gtx_field(hu, i1, sh);
+        } else {
+            B1 = hu.pay + gtx_payload_bits(hu, sh);
+        }
+        const uint64_t W0 = B0 >> 5;
+        const uint64_t NW = B1 > B0 ? ((B1 - 1) >> 5) + 2 - W0 : 0;
+        if (NW && NW <= stage) {
+            uint32_t* L = dec_lds + (threadIdx.x / kWave) * stage;
+            const uint32_t nw = (uint32_t)NW;
+            for (uint32_t c = 0; c < nw; c += 8 * kWave) {
+                uint32_t t[8];
 #pragma unroll
-                    for (uint32_t u = 0; u < 8; ++u) {
-                        const uint32_t j = c + u * kWave + lane;
-                        t[u] = j < nw ? g.w[W0 + j] : 0u;
-                    }
-#pragma unroll
-                    for (uint32_t u = 0; u < 8; ++u) {
-                        const uint32_t j = c + u * kWave + lane;
-                        if (j < nw) L[j] = t[u];
-                    }
+                for (uint32_t u = 0; u < 8; ++u) {
+                    const uint32_t j = c + u * kWave + lane;
+                    t[u] = j < nw ? g.w[W0 + j] : 0u;
                 }
-                wave_sync();
-                decode_range<FMT>(g, LdsWords{L, W0}, rowptr, col, e0, e1, eb, vlo, vhi, span);
-                return;
+#pragma unroll
+                for (uint32_t u = 0; u < 8; ++u) {
+                    const uint32_t j = c + u * kWave + lane;
+                    if (j < nw) L[j] = t[u];
+                }
             }
+            wave_sync();
+            decode_range(g, LdsWords{L, W0}, rowptr, col, e0, e1, eb, vlo, vhi, span);
+            return;
         }
     }
-    decode_range<FMT>(g, GlobalWords{g.w}, rowptr, col, e0, e1, eb, vlo, vhi, span);
+    decode_range(g, GlobalWords{g.w}, rowptr, col, e0, e1, eb, vlo, vhi, span);
 }
 
 int decode_csr(grass_graph* g, uint64_t* rowptr, uint32_t* col, hipStream_t s) {
@@ -574,10 +618,11 @@ int decode_csr(grass_graph* g, uint64_t* rowptr, uint32_t* col, hipStream_t s) {
     uint32_t slot = 0;
     while ((512u << slot) < per_wave && slot + 1 < kWaveStartSlots) ++slot;
     if ((512u << slot) != per_wave) return GRASS_EINVAL;
-    // GT with P <= 4 decodes by runs: about per_wave slots per wave, per_wave / P runs.  The run
-    // offsets (a scan over the headers) and the total are built once per graph.
-    const bool runs = g->fmt == kGT && (1u << g->cp_shift) <= kRunMaxP;
-    const uint32_t unit = runs ? per_wave >> g->cp_shift : per_wave;
+    // LE, and GT with P <= 4, decode by runs: about per_wave slots per wave, per_wave / P runs.  The
+    // run offsets (a scan over the headers) and the total are built once per graph.
+    const uint32_t sh = g->fmt == kLE ? kLeRunShift : g->cp_shift;
+    const bool runs = (1u << sh) <= kRunMax;
+    const uint32_t unit = runs ? per_wave >> sh : per_wave;
     uint64_t units = m;
     if (runs) {
         std::lock_guard<std::mutex> lock(g->mu);
@@ -590,7 +635,7 @@ int decode_csr(grass_graph* g, uint64_t* rowptr, uint32_t* col, hipStream_t s) {
                 return GRASS_ENOMEM;
             }
             uint64_t total = 0;
-            hipError_t e = exclusive_scan(RunGen{g->d_hdr, g->cp_shift}, Count{n, nullptr}, n, r, part, part + nb, s);
+            hipError_t e = exclusive_scan(RunGen{g->d_hdr, g->fmt, sh}, Count{n, nullptr}, n, r, part, part + nb, s);
             if (e == hipSuccess) e = hipMemcpyAsync(&total, r + n, 8, hipMemcpyDeviceToHost, s);
             if (e == hipSuccess) e = hipStreamSynchronize(s);
             (void)hipFree(part);
@@ -628,15 +673,15 @@ int decode_csr(grass_graph* g, uint64_t* rowptr, uint32_t* col, hipStream_t s) {
         }
         wstart = g->d_wstart[slot];
     }
-    if (runs) {
-        hipLaunchKernelGGL(decode_runs_kernel, dim3((unsigned)blocks), dim3(kDecBlock), 0, s, g->dev(),
-                           (const uint64_t*)rowptr, uoff, wstart, col, units, unit);
-    } else if (g->fmt == kLE) {
-        hipLaunchKernelGGL(decode_csr_kernel<kLE>, dim3((unsigned)blocks), dim3(kDecBlock), 0, s,
-                           g->dev(), (const uint64_t*)rowptr, wstart, col, m, per_wave, 0u);
+    if (runs && g->fmt == kLE) {
+        hipLaunchKernelGGL(decode_runs_kernel<kLE>, dim3((unsigned)blocks), dim3(kDecBlock), 0, s, g->dev(),
+                           (const uint64_t*)rowptr, uoff, wstart, col, units, unit, sh);
+    } else if (runs) {
+        hipLaunchKernelGGL(decode_runs_kernel<kGT>, dim3((unsigned)blocks), dim3(kDecBlock), 0, s, g->dev(),
+                           (const uint64_t*)rowptr, uoff, wstart, col, units, unit, sh);
     } else {
         const uint32_t stage = dec_stage_words(per_wave);
-        hipLaunchKernelGGL(decode_csr_kernel<kGT>, dim3((unsigned)blocks), dim3(kDecBlock),
+        hipLaunchKernelGGL(decode_csr_kernel, dim3((unsigned)blocks), dim3(kDecBlock),
                            (size_t)stage * 4 * (kDecBlock / kWave), s, g->dev(), (const uint64_t*)rowptr, wstart,
                            col, m, per_wave, stage);
     }
