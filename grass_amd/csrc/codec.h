@@ -212,11 +212,12 @@ __device__ __forceinline__ uint32_t udiv_small(uint32_t n, uint32_t d) {
     return q;
 }
 
-// floor(n / d) for any n and 2 <= d < 2^16 (a chunk length): the same estimate, corrected a second
-// time from its remainder.  The first estimate is off by at most 2^-22 of the quotient (and by one
-// for its truncation), so its remainder is within 2^10 + 2 d of zero, which a second estimate
-// turns into a quotient that one signed step fixes.  No branch on the size of n: LE slopes divide
-// differences of neighbour ids, which pass 2^20 in most chunks of a graph of millions of vertices.
+// floor(n / d) for any n and 2 <= d < 2^16 (a chunk length), and for n < 2^31 also d = 1: the same
+// estimate, corrected a second time from its remainder.  The first estimate is off by at most 2^-22
+// of the quotient (and by one for its truncation), so its remainder is within 2^10 + 2 d of zero,
+// which a second estimate turns into a quotient that one signed step fixes.  No branch on the size
+// of n: LE slopes divide differences of neighbour ids, which pass 2^20 in most chunks of a graph of
+// millions of vertices.
 __device__ __forceinline__ uint32_t udiv_chunk(uint32_t n, uint32_t d) {
     const float rc = __builtin_amdgcn_rcpf((float)d);
     uint32_t q = (uint32_t)((float)n * rc);

@@ -234,13 +234,19 @@ __device__ __forceinline__ void decode_range(const DevGraph& g, const Src& src, 
 // wave's pass fill consecutive output slots, which are staged in LDS and stored with coalesced
 // writes.  Runs are numbered over the graph (roff = exclusive scan of runs per vertex) and every
 // wave takes a fixed number of them, with its first vertex from a table like the slot-based one.
-// What bounds it is instruction issue: LE_RUNS_FIGURES
+// Bound by instruction issue, then by the loads a pass waits for, so the geometry avoids branches
+// and 32-bit multiplies, fields come off funnel shifts, a pass's output slots are a wave scan of its
+// counts (no row pointers), and the next pass's run ends and headers are requested before the
+// current pass decodes.  Measured on R-MAT, GT s24 (521 M entries) 1.05 -> 0.94 ms, 3.7 TB/s of the
+// 3.5 GB it needs (a copy reaches 4.85); LE s22 (128 M) 0.62 ms with a lane per position, 0.38 by
+// runs, 0.32 with the above.  Loading each lane's header by itself instead of 64 headers and a
+// shuffle: GT 1.06 ms.
 
 constexpr uint32_t kRunMax = 4;    // positions of a run; the run kernel takes GT checkpoint intervals up to it
 constexpr uint32_t kLeRunShift = 2;  // LE: runs of 1 << 2 positions
 
 // Runs of a vertex with d entries in C chunks or blocks: R of q + 1 positions and C - R of q, each
-// ceil(len >> sh) runs, and LE's last rock.
+// ceil(len / 2^sh) runs, and LE's last rock.
 __host__ __device__ __forceinline__ uint64_t list_runs(int fmt, uint32_t d, uint32_t C, uint32_t q, uint32_t sh) {
     if (!d) return 0;
     if (fmt == kLE && d == 1) return 1;
@@ -258,72 +264,87 @@ struct RunGen {  // runs of vertex i, from its header
     }
 };
 
-// One run's place: first output slot, its positions [i0, i0 + cnt) of block (chunk) blk, which has
-// len positions; GT: the stream bit of its absolute field.
+// One run's place: its positions [i0, i0 + cnt) of block (chunk) blk, which has len positions; GT:
+// the stream bit of its absolute field.
 struct RunAt {
-    uint64_t slot, bit;
+    uint64_t bit;
     uint32_t cnt, blk, i0, len;
+    uint32_t pos;  // position in the list of its first entry
+};
+
+// The list constants of run_at's division by the runs per block (nr1 for blocks of q + 1
+// positions, nr0 for blocks of q): per lane with a float reciprocal, or shared by the wave.
+struct RunDivLane {
+    __device__ __forceinline__ uint32_t operator()(uint32_t n, uint32_t d, bool) const {
+        return udiv_chunk(n, max(d, 1u));  // (LE, d = 1: no runs per chunk, the one run is run 0)
+    }
+};
+struct RunDivShared {
+    UDiv u1, u0;
+    __device__ __forceinline__ uint32_t operator()(uint32_t n, uint32_t d, bool lo) const {
+        UDiv u;
+        u.d = d;
+        u.m = lo ? u1.m : u0.m;
+        return u.div(n);
+    }
 };
 
 // Run rr (< the vertex's runs) of a vertex: R blocks of nr1 runs, then blocks of nr0 (LE: then the
-// last rock, block C).  Div divides by nr1 / nr0 (shared multiply-high reciprocals when the wave is
-// in one list, else per lane).
-template <int FMT, class Div1, class Div0>
-__device__ __forceinline__ RunAt run_at(const Hdr& h, uint64_t vstart, uint32_t rr, uint32_t sh, const Div1& div1,
-                                        const Div0& div0) {
+// last rock, block C).  The block kind is chosen first, so lanes of both kinds share one division.
+// C, q and a block's runs are below 2^16 and the field widths below 2^5, so all products but the
+// bits of whole blocks are 24-bit multiplies (full rate, where 32-bit ones run at a quarter).
+// P = 1 << sh positions per run; in a GT block, run j >= 1 starts f1 - 32 + j K bits after the head's
+// field, K = 32 + (P - 1) f2 (the bits of a whole run), and a block of q positions has the bits of
+// one of q + 1 less one field, which is a checkpoint when q is a multiple of P.
+template <int FMT, class Div>
+__device__ __forceinline__ RunAt run_at(const Hdr& h, uint32_t rr, uint32_t sh, const Div& div) {
     const uint32_t P1 = (1u << sh) - 1;
     const uint32_t nr1 = (h.q + 1 + P1) >> sh, nr0 = (h.q + P1) >> sh;
-    const uint32_t bigr = h.R * nr1;
+    const uint32_t bigr = __umul24(h.R, nr1);
+    const bool lo = rr < bigr;
+    const uint32_t t = lo ? rr : rr - bigr, nr = lo ? nr1 : nr0;
+    const uint32_t b = div(t, nr, lo);
+    const uint32_t j = t - __umul24(b, nr);
     RunAt a;
-    uint32_t j;
-    uint64_t bpos, bbit = 0;
-    if (rr < bigr) {
-        a.blk = div1(rr, nr1);
-        j = rr - a.blk * nr1;
-        a.len = h.q + 1;
-        bpos = (uint64_t)a.blk * (h.q + 1);
-        if (FMT == kGT) bbit = h.pay + (uint64_t)a.blk * gtx_field(h, h.q + 1, sh);
-    } else {
-        // (LE, d = 1: q = 0, one run, whose index 0 divides to 0 by any divisor)
-        const uint32_t t = rr - bigr, b2 = div0(t, FMT == kLE && nr0 == 0 ? 1u : nr0);
-        j = t - b2 * nr0;
-        a.blk = h.R + b2;
-        a.len = FMT == kLE && a.blk == h.C ? 1u : h.q;
-        bpos = (uint64_t)h.R * (h.q + 1) + (uint64_t)b2 * h.q;
-        if (FMT == kGT)
-            bbit = h.pay + (uint64_t)h.R * gtx_field(h, h.q + 1, sh) + (uint64_t)b2 * gtx_field(h, h.q, sh);
-    }
+    a.blk = lo ? b : b + h.R;
+    a.len = lo ? h.q + 1 : h.q;
     a.i0 = j << sh;
-    a.cnt = min(1u << sh, a.len - a.i0);
-    a.slot = vstart + bpos + a.i0;
-    a.bit = FMT == kGT ? bbit + gtx_field(h, a.i0, sh) : 0;
+    a.pos = __umul24(b, a.len) + (lo ? 0u : __umul24(h.R, h.q + 1)) + a.i0;
+    if (FMT == kLE && a.blk == h.C) a.len = 1;
+    a.cnt = min(P1 + 1, a.len - a.i0);
+    a.bit = 0;
+    if (FMT == kGT) {
+        const uint32_t K = 32 + __umul24(P1, h.f2);
+        const uint32_t F1 = h.f1 + __umul24(h.q, h.f2) + __umul24(h.q >> sh, 32 - h.f2);
+        const uint32_t F = lo ? F1 : F1 - ((h.q & P1) ? h.f2 : 32u);
+        a.bit = h.pay + (uint64_t)b * F + (lo ? 0ull : (uint64_t)h.R * F1) + (j ? h.f1 - 32 + __umul24(j, K) : 0u);
+    }
     return a;
 }
 
-// Consecutive fields of 1 to 32 bits from stream bit `bit`: five words from the first field's (the
-// offset in its word and four 32-bit fields take at most 31 + 128 bits).
+// Five words of the stream shifted left by s < 32 bits, the first four of the result kept: fields
+// are taken off the top with 32-bit funnel shifts, without a branch.
 struct FieldReader {
-    uint64_t buf;
-    uint32_t avail, n0, n1, n2;  // buffered bits, then the words after them
+    uint32_t t0, t1, t2, t3;
+    __device__ __forceinline__ static uint32_t shl(uint32_t hi, uint32_t lo, uint32_t n) {  // 1 <= n <= 32
+        return __builtin_amdgcn_alignbit(hi, lo, 32 - n);
+    }
     __device__ __forceinline__ FieldReader(const Words4& q, uint32_t w4, uint32_t s)
-        : buf((((uint64_t)q.x << 32) | q.y) << s), avail(64 - s), n0(q.z), n1(q.w), n2(w4) {}
-    __device__ __forceinline__ uint32_t take(uint32_t wdt) {
-        if (avail < wdt) {
-            buf |= (uint64_t)n0 << (32 - avail);
-            avail += 32;
-            n0 = n1;
-            n1 = n2;
-        }
-        const uint32_t r = (uint32_t)(buf >> (64 - wdt));
-        buf <<= wdt;
-        avail -= wdt;
+        : t0(s ? shl(q.x, q.y, s) : q.x), t1(s ? shl(q.y, q.z, s) : q.y), t2(s ? shl(q.z, q.w, s) : q.z),
+          t3(s ? shl(q.w, w4, s) : q.w) {}
+    __device__ __forceinline__ uint32_t take(uint32_t wdt) {  // 1 <= wdt <= 32
+        const uint32_t r = t0 >> (32 - wdt);
+        t0 = shl(t0, t1, wdt);
+        t1 = shl(t1, t2, wdt);
+        t2 = shl(t2, t3, wdt);
+        t3 = wdt < 32 ? t3 << wdt : 0u;
         return r;
     }
 };
 
 // The ids of one GT run into out[0 .. cnt): the absolute field, then each gap + 1 added on.  One
 // 16-byte load holds the field's offset in its word (< 32), a 32-bit field and three gaps of up to
-// 21 bits; a fifth word is read when they need more.
+// 21 bits; a fifth word is read when they need more.  (Ids past cnt are not meaningful.)
 __device__ __forceinline__ void gt_run_ids(const uint32_t* __restrict__ w, const Hdr& h, uint32_t v, const RunAt& a,
                                            uint32_t out[kRunMax]) {
     const uint32_t* p = w + (a.bit >> 5);
@@ -331,16 +352,18 @@ __device__ __forceinline__ void gt_run_ids(const uint32_t* __restrict__ w, const
     const uint32_t s = (uint32_t)(a.bit & 31);
     const bool head = a.i0 == 0;
     const uint32_t aw = head ? h.f1 : 32u, f2 = h.f2;
-    FieldReader f(q, s + aw + (a.cnt - 1) * f2 > 128 ? p[4] : 0u, s);
+    FieldReader f(q, s + aw + __umul24(a.cnt - 1, f2) > 128 ? p[4] : 0u, s);
     const uint32_t a0 = f.take(aw);  // f1 >= 1 for a vertex with entries
-    uint32_t x = head ? (a.blk >= h.fp ? v + a0 + 1 : v - a0 - 1) : a0;
-    out[0] = x;
-#pragma unroll
-    for (uint32_t k = 1; k < kRunMax; ++k) {
-        if (k < a.cnt) {
-            x += (f2 ? f.take(f2) : 0u) + 1;  // (0-bit gap fields read as 0)
-            out[k] = x;
-        }
+    const uint32_t x0 = head ? (a.blk >= h.fp ? v + a0 + 1 : v - a0 - 1) : a0;
+    out[0] = x0;
+    if (f2) {
+        out[1] = x0 + f.take(f2) + 1;
+        out[2] = out[1] + f.take(f2) + 1;
+        out[3] = out[2] + f.take(f2) + 1;
+    } else {  // (0-bit gap fields read as 0)
+        out[1] = x0 + 1;
+        out[2] = x0 + 2;
+        out[3] = x0 + 3;
     }
 }
 
@@ -351,51 +374,39 @@ __device__ __forceinline__ void gt_run_ids(const uint32_t* __restrict__ w, const
 __device__ __forceinline__ void le_run_ids(const uint32_t* __restrict__ w, const Hdr& h, uint32_t v, const RunAt& a,
                                            uint32_t out[kRunMax]) {
     if (h.d == 1) {
-        out[0] = h.f1;
+        out[0] = out[1] = out[2] = out[3] = h.f1;
         return;
     }
     const uint32_t c = a.blk, rb = h.f1, sw = h.f2 + 1;
-    const uint32_t i1 = a.i0 ? a.i0 : 1u;        // first sea's position in the chunk
-    const uint32_t skip = a.i0 ? 0u : 1u;        // the run starts with the rock
-    const uint32_t j = (h.q - 1) * c + min(c, h.R) + i1 - 1;
-    const uint64_t rbit = h.pay + (uint64_t)c * rb;
-    const uint64_t sbit = h.pay + (uint64_t)(h.C + 1) * rb + (uint64_t)j * sw;
+    const uint32_t i1 = a.i0 ? a.i0 : 1u;  // first sea's position in the chunk
+    const bool rock = a.i0 == 0;           // the run starts with the rock
+    const uint32_t j = __umul24(h.q - 1, c) + min(c, h.R) + i1 - 1;
+    const uint64_t rbit = h.pay + __umul24(c, rb);
+    const uint64_t sbit = h.pay + __umul24(h.C + 1, rb) + (uint64_t)j * sw;
     const Words4 rq = *(const Words4*)(w + (rbit >> 5));
     const uint32_t* sp = w + (sbit >> 5);
     const Words4 sq = *(const Words4*)sp;
     const uint32_t ss = (uint32_t)(sbit & 31), rs = (uint32_t)(rbit & 31);
-    const uint32_t w4 = ss + (a.cnt - skip) * sw > 128 ? sp[4] : 0u;
-    uint64_t win = ((uint64_t)rq.x << 32) | rq.y;
-    if (rs) win = (win << rs) | (rq.z >> (32 - rs));
-    const uint32_t r1 = (uint32_t)(win >> (64 - rb)), r2 = (uint32_t)((win << rb) >> (64 - rb));
+    const uint32_t w4 = ss + __umul24(a.cnt, sw) > 128 ? sp[4] : 0u;
+    const uint32_t u0 = rs ? FieldReader::shl(rq.x, rq.y, rs) : rq.x;
+    const uint32_t u1 = rs ? FieldReader::shl(rq.y, rq.z, rs) : rq.y;
+    const uint32_t r1 = u0 >> (32 - rb), r2 = FieldReader::shl(u0, u1, rb) >> (32 - rb);
     const uint32_t A = c < h.fp ? v - r1 : v + r1;
     const uint32_t Z = c + 1 < h.fp ? v - r2 : v + r2;
     const uint32_t step = a.len > 1 ? udiv_chunk(Z - A, a.len) : 0u;
     FieldReader f(sq, w4, ss);
-    uint32_t x = A + step * a.i0;
+    uint32_t x = A + step * i1, e[kRunMax];
 #pragma unroll
-    for (uint32_t k = 0; k < kRunMax; ++k) {
-        if (k < a.cnt) {
-            if (k >= skip) {
-                const uint32_t e = f.take(sw), mag = e >> 1;
-                out[k] = x + ((e & 1) ? 0u - mag : mag);
-            } else {
-                out[k] = A;
-            }
-            x += step;
-        }
+    for (uint32_t k = 0; k < kRunMax; ++k) {  // seas i1, i1 + 1, ...
+        const uint32_t r = f.take(sw), mag = r >> 1;
+        e[k] = x + ((r & 1) ? 0u - mag : mag);
+        x += step;
     }
+    out[0] = rock ? A : e[0];
+    out[1] = rock ? e[0] : e[1];
+    out[2] = rock ? e[1] : e[2];
+    out[3] = rock ? e[2] : e[3];
 }
-
-struct UDivBy {  // per-lane division by a list constant (float reciprocal, corrected)
-    __device__ __forceinline__ uint32_t operator()(uint32_t n, uint32_t d) const {
-        return d == 1 ? n : udiv_small(n, d);  // short lists: one run per block
-    }
-};
-struct UDivShared {  // division by the one divisor it was made for
-    UDiv u;
-    __device__ __forceinline__ uint32_t operator()(uint32_t n, uint32_t) const { return u.div(n); }
-};
 
 // Wave w decodes runs [w * per_wave, ...) of the graph; rstart[w] is the vertex holding its first.
 template <int FMT>
@@ -418,8 +429,23 @@ __global__ __launch_bounds__(kDecBlock) void decode_runs_kernel(DevGraph g, cons
     uint64_t rc = roff[cur], rn = roff[cur + 1];
     uint32_t hv = 0xFFFFFFFFu;  // vertex whose list constants are cached below
     Hdr uh;
-    uint64_t uvs = 0;
-    UDivShared u1, u0;
+    RunDivShared ud;
+    // the pass's first output slot: from the row pointer here, then carried from pass to pass
+    uint64_t sb;
+    {
+        Hdr h;
+        load_hdr<FMT>(g, cur, h);
+        sb = rowptr[cur] + run_at<FMT>(h, (uint32_t)(r0 - rc), sh, RunDivLane{}).pos;
+    }
+    // run ends and headers of the 64 vertices from `cur`, requested a pass ahead
+    uint64_t bj = 0;
+    uint4 hj = make_uint4(0u, 0u, 0u, 0u);
+    auto request = [&]() {
+        bj = (uint64_t)cur + 1 + lane <= g.n ? roff[cur + 1 + lane] : ~0ull;
+        if (cur + (uint32_t)lane < g.n) hj = g.hdr[cur + lane];
+    };
+    auto in_list = [&](uint64_t base) { return base >= rc && base + (kWave - 1) < rn; };
+    if (!in_list(r0)) request();
     for (uint64_t base = r0; base < r1; base += kWave) {
         const uint64_t rho = base + lane;
         const bool act = rho < r1;
@@ -427,97 +453,76 @@ __global__ __launch_bounds__(kDecBlock) void decode_runs_kernel(DevGraph g, cons
         RunAt a;
         Hdr h;
         uint32_t v;
-        if (base >= rc && base + (kWave - 1) < rn) {
+        if (in_list(base)) {
             // the whole pass is in one list: one header, shared divisors
             if (cur != hv) {
                 hv = cur;
                 load_hdr<FMT>(g, hv, uh);
-                uvs = rowptr[hv];
                 const uint32_t P1 = (1u << sh) - 1;
-                u1.u.init((uh.q + 1 + P1) >> sh);
-                u0.u.init((uh.q + P1) >> sh);
+                ud.u1.init((uh.q + 1 + P1) >> sh);
+                ud.u0.init((uh.q + P1) >> sh);
             }
             h = uh;
             v = hv;
-            a = run_at<FMT>(h, uvs, (uint32_t)(rr - rc), sh, u1, u0);
+            a = run_at<FMT>(h, (uint32_t)(rr - rc), sh, ud);
         } else {
-            // The 64 vertices from `cur`: their run ends (relative to rc), headers and first slots
-            // in one coalesced load each.  Vertex cur + j covers the pass's lanes from its first
-            // run on; each vertex that starts a lane of the pass (or holds its first run) writes
-            // j + 1 into that lane's LDS slot, and an inclusive max over the slots gives every
-            // lane its vertex (no search).  When those vertices end before the pass does (only
-            // across vertices without entries), each lane searches the run offsets instead.
-            const uint64_t bj = (uint64_t)cur + 1 + lane <= g.n ? roff[cur + 1 + lane] : ~0ull;
-            uint4 hj = make_uint4(0u, 0u, 0u, 0u);
-            uint64_t sj = 0;
-            if (cur + (uint32_t)lane < g.n) {
-                hj = g.hdr[cur + lane];
-                sj = rowptr[cur + lane];
-            }
+            // Vertex cur + j covers the pass's lanes from its first run on; each vertex that starts
+            // a lane of the pass (or holds its first run) writes j + 1 into that lane's LDS slot,
+            // and an inclusive max over the slots gives every lane its vertex (no search).  When
+            // the 64 vertices end before the pass does (only across vertices without entries), each
+            // lane searches the run offsets instead.
             const uint32_t rj = bj - rc > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)(bj - rc);
             const uint32_t pj = dpp_move<0x138>(rj);  // start of vertex cur + lane (lane 0: 0)
             const uint32_t e0 = (uint32_t)(base - rc);
             const uint32_t lastl = (uint32_t)(r1 - base < (uint64_t)kWave ? r1 - base - 1 : kWave - 1);
             const uint32_t elast = e0 + lastl;
-            int jo;
-            uint64_t rstart_v;
+            uint32_t ro;  // the lane's run in its vertex's list
             if ((uint32_t)__builtin_amdgcn_readlane((int)rj, kWave - 1) > elast) {
                 const bool cand = rj > pj && rj > e0 && pj <= elast;
                 own[lane] = 0;
                 wave_sync();
                 if (cand) own[pj > e0 ? pj - e0 : 0u] = lane + 1;
                 wave_sync();
-                jo = (int)wave_inclusive_max(own[lane]) - 1;  // lane 0 always has a vertex
+                int jo = (int)wave_inclusive_max(own[lane]) - 1;  // lane 0 always has a vertex
                 wave_sync();
-                jo = act ? jo : __builtin_amdgcn_readlane(jo, (int)lastl);
+                const int jl = __builtin_amdgcn_readlane(jo, (int)lastl);
+                jo = act ? jo : jl;
                 v = cur + jo;
-                rstart_v = rc + __shfl(pj, jo, kWave);
-            } else {
-                v = owner_of(roff, cur, g.n - 1, rr);
-                jo = (int)(v - cur < (uint32_t)kWave ? v - cur : 0u);
-                rstart_v = roff[v];
-            }
-            uint4 hv4 = make_uint4(__shfl(hj.x, jo, kWave), __shfl(hj.y, jo, kWave), __shfl(hj.z, jo, kWave),
-                                   __shfl(hj.w, jo, kWave));
-            uint64_t vs = ((uint64_t)__shfl((uint32_t)(sj >> 32), jo, kWave) << 32) | __shfl((uint32_t)sj, jo, kWave);
-            if (v - cur >= (uint32_t)kWave) {
-                hv4 = g.hdr[v];
-                vs = rowptr[v];
-            }
-            // the next pass starts at or after the last active lane's vertex
-            const uint32_t vl = (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lastl);
-            if (vl - cur < (uint32_t)kWave) {
-                const int jl = (int)(vl - cur);
+                ro = (uint32_t)(rr - rc) - __shfl(pj, jo, kWave);
+                unpack_hdr<FMT>(make_uint4(__shfl(hj.x, jo, kWave), __shfl(hj.y, jo, kWave), __shfl(hj.z, jo, kWave),
+                                           __shfl(hj.w, jo, kWave)), h);
+                // the next pass starts at or after the last active lane's vertex
                 if (jl) {
-                    cur = vl;
+                    cur += jl;
                     rc = readlane_u64(bj, jl - 1);
                     rn = readlane_u64(bj, jl);
                 }
             } else {
-                cur = vl;
+                v = owner_of(roff, cur, g.n - 1, rr);
+                ro = (uint32_t)(rr - roff[v]);
+                cur = (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lastl);
                 rc = roff[cur];
                 rn = roff[cur + 1];
+                load_hdr<FMT>(g, v, h);
             }
-            unpack_hdr<FMT>(hv4, h);
-            a = run_at<FMT>(h, vs, (uint32_t)(rr - rstart_v), sh, UDivBy{}, UDivBy{});
+            a = run_at<FMT>(h, ro, sh, RunDivLane{});
         }
+        if (base + kWave < r1 && !in_list(base + kWave)) request();
         uint32_t ids[kRunMax];
         if (FMT == kLE) le_run_ids(g.w, h, v, a, ids);
         else gt_run_ids(g.w, h, v, a, ids);
-        // stage the pass's slots [sb, se) and store them coalesced
-        const uint64_t sb = readlane_u64(a.slot, 0);
-        const uint32_t lastl = (uint32_t)(r1 - base < (uint64_t)kWave ? r1 - base - 1 : kWave - 1);
-        const uint32_t count = (uint32_t)(readlane_u64(a.slot, (int)lastl) - sb) +
-                               (uint32_t)__builtin_amdgcn_readlane((int)a.cnt, (int)lastl);
-        if (act) {
-            const uint32_t o = (uint32_t)(a.slot - sb);
+        // the runs' slots follow each other: staged in LDS at the sum of the counts before, and
+        // stored coalesced
+        const uint32_t cnt = act ? a.cnt : 0u;
+        const uint32_t inc = wave_inclusive_sum(cnt);
+        const uint32_t o = inc - cnt, count = (uint32_t)__builtin_amdgcn_readlane((int)inc, kWave - 1);
 #pragma unroll
-            for (uint32_t k = 0; k < kRunMax; ++k)
-                if (k < a.cnt) L[o + k] = ids[k];
-        }
+        for (uint32_t k = 0; k < kRunMax; ++k)
+            if (k < cnt) L[o + k] = ids[k];
         wave_sync();
         for (uint32_t k = lane; k < count; k += kWave) col[sb + k] = L[k];
         wave_sync();  // the stage is read before the next pass writes it
+        sb += count;
     }
 }
 
