@@ -111,9 +111,18 @@ __device__ __forceinline__ uint32_t header_bits(const Hdr& h) {
 
 // The payload bit of a GT entry points into the device's GT payload stream once the loader
 // has built it (into .graph before that).
+//
+// The entry is loaded as one vector: loaded as four words, the compiler puts off the payload word
+// until a vertex without neighbours has been ruled out, and a step waits for memory once more.
+__device__ __forceinline__ uint4 load_hdr_words(const DevGraph& g, uint32_t v) {
+    typedef uint32_t V4 __attribute__((ext_vector_type(4)));
+    const V4 e = *(const V4*)(g.hdr + v);
+    return make_uint4(e.x, e.y, e.z, e.w);
+}
+
 template <int FMT>
 __device__ __forceinline__ void load_hdr(const DevGraph& g, uint32_t v, Hdr& h) {
-    unpack_hdr<FMT>(g.hdr[v], h);
+    unpack_hdr<FMT>(load_hdr_words(g, v), h);
 }
 
 __host__ __device__ __forceinline__ uint32_t isqrt_u32(uint32_t x) {
@@ -230,44 +239,70 @@ __device__ __forceinline__ uint32_t udiv_chunk(uint32_t n, uint32_t d) {
     return q;
 }
 
-// Position k of an LE record -> (chunk c, index i in chunk, chunk length len).
-__device__ __forceinline__ void le_locate(const Hdr& h, uint32_t k, uint32_t& c, uint32_t& i,
-                                          uint32_t& len) {
-    const uint32_t big = h.R * (h.q + 1);
-    const bool lo = k < big;
-    len = lo ? h.q + 1 : h.q;
-    const uint32_t kk = lo ? k : k - big;
-    c = udiv_small(kk, len);
-    i = kk - c * len;
-    if (!lo) c += h.R;
-}
+// Four words from any word address in one load.
+struct __attribute__((packed, aligned(4))) Words4 {
+    uint32_t x, y, z, w;
+};
 
-// Neighbour k of vertex v, LE (LE/src/bcg.cuh:196-261); 0 <= k < d.
+// Five words of the stream shifted left by s < 32 bits, the first four of the result kept: fields
+// are taken off the top with 32-bit funnel shifts, without a branch.
+struct FieldReader {
+    uint32_t t0, t1, t2, t3;
+    __device__ __forceinline__ static uint32_t shl(uint32_t hi, uint32_t lo, uint32_t n) {  // 1 <= n <= 32
+        return __builtin_amdgcn_alignbit(hi, lo, 32 - n);
+    }
+    // the same for 0 <= n < 32; the shift is made first so that the choice is a select, not a branch
+    __device__ __forceinline__ static uint32_t shl0(uint32_t hi, uint32_t lo, uint32_t n) {
+        const uint32_t x = shl(hi, lo, n);
+        return n ? x : hi;
+    }
+    __device__ __forceinline__ FieldReader(const Words4& q, uint32_t w4, uint32_t s)
+        : t0(shl0(q.x, q.y, s)), t1(shl0(q.y, q.z, s)), t2(shl0(q.z, q.w, s)), t3(shl0(q.w, w4, s)) {}
+    __device__ __forceinline__ uint32_t take(uint32_t wdt) {  // 1 <= wdt <= 32
+        const uint32_t r = t0 >> (32 - wdt);
+        t0 = shl(t0, t1, wdt);
+        t1 = shl(t1, t2, wdt);
+        t2 = shl(t2, t3, wdt);
+        t3 = wdt < 32 ? t3 << wdt : 0u;
+        return r;
+    }
+};
+
+// Neighbour k of vertex v, LE (LE/src/bcg.cuh:196-261); 0 <= k < d.  The rock pair and the sea lie
+// apart; both loads are issued before either is used (one after the other, a walk step waited for
+// memory three times: R-MAT s22, 2^20 walks of 80 steps 4.15 -> 3.74 ms, 22.4 G steps/s).
 __device__ __forceinline__ uint32_t le_get(const uint32_t* __restrict__ w, const Hdr& h,
                                            uint32_t v, uint32_t k, uint32_t* fbits = nullptr) {
     if (h.d == 1) {
         if (fbits) *fbits = 0;
         return h.f1;
     }
-    uint32_t c, i, len;
-    le_locate(h, k, c, i, len);
-    const uint32_t rb = h.f1;
-    // rocks c and c+1 are adjacent fields of rb <= 31 bits: one 64-bit window holds both
-    const uint64_t win = peek64(w, h.pay + (uint64_t)c * rb);
-    uint32_t r1 = (uint32_t)(win >> (64 - rb));
-    uint32_t a = c < h.fp ? v - r1 : v + r1;
-    if (i == 0) {
-        if (fbits) *fbits = rb;
-        return a;
+    const uint32_t big = __umul24(h.R, h.q + 1);
+    const bool lo = k < big;
+    const uint32_t len = lo ? h.q + 1 : h.q, kk = lo ? k : k - big;
+    const uint32_t b = udiv_chunk(kk, len), i = kk - __umul24(b, len), c = lo ? b : b + h.R;
+    const uint32_t rb = h.f1, sw = h.f2 + 1;
+    // rocks c and c + 1 are adjacent fields of rb <= 31 bits; rock c alone ends within two words
+    const uint64_t rbit = h.pay + __umul24(c, rb);
+    const uint32_t* rp = w + (rbit >> 5);
+    const uint32_t rs = (uint32_t)(rbit & 31);
+    const uint32_t w0 = rp[0], w1 = rp[1];
+    uint32_t w2 = 0, s0 = 0, s1 = 0, ss = 0;
+    if (i) {
+        const uint32_t j = __umul24(h.q - 1, c) + (c < h.R ? c : h.R) + i - 1;
+        const uint64_t sbit = h.pay + __umul24(h.C + 1, rb) + (uint64_t)j * sw;
+        const uint32_t* sp = w + (sbit >> 5);
+        ss = (uint32_t)(sbit & 31);
+        s0 = sp[0];
+        s1 = sp[1];
+        if (rs + 2 * rb > 64) w2 = rp[2];
     }
-    uint32_t r2 = (uint32_t)((win << rb) >> (64 - rb));
-    uint32_t z = c + 1 < h.fp ? v - r2 : v + r2;
-    uint32_t j = (h.q - 1) * c + (c < h.R ? c : h.R) + i - 1;
-    uint64_t so = h.pay + (uint64_t)(h.C + 1) * rb + (uint64_t)j * (h.f2 + 1);
-    uint32_t x = read_bits(w, so, h.f2 + 1);
-    uint32_t mag = x >> 1;
-    if (fbits) *fbits = 2 * rb + h.f2 + 1;
-    return udiv_small(z - a, len) * i + a + ((x & 1) ? 0u - mag : mag);
+    const uint32_t u0 = FieldReader::shl0(w0, w1, rs), u1 = FieldReader::shl0(w1, w2, rs);
+    const uint32_t r1 = u0 >> (32 - rb), r2 = FieldReader::shl(u0, u1, rb) >> (32 - rb);
+    const uint32_t a = c < h.fp ? v - r1 : v + r1, z = c + 1 < h.fp ? v - r2 : v + r2;
+    const uint32_t x = FieldReader::shl0(s0, s1, ss) >> (32 - sw), mag = x >> 1;
+    if (fbits) *fbits = i ? 2 * rb + sw : rb;
+    return i ? udiv_chunk(z - a, max(len, 2u)) * i + a + ((x & 1) ? 0u - mag : mag) : a;
 }
 
 // Position k of a GT record -> (block, index i in block).
@@ -341,44 +376,56 @@ __device__ __forceinline__ uint32_t sum_fields(const uint32_t* __restrict__ w, u
 // The absolute field and the gaps after it are read with one 16-byte load (four words from the
 // field's first word; the stream is padded, so the words past its end exist): 128 bits hold the
 // field's offset in its word (< 32), the field and `rem` gaps when they add up to 128 or less --
-// a checkpoint and three gaps of up to 21 bits.  Longer spans read the gaps word by word.
-struct __attribute__((packed, aligned(4))) Words4 {
-    uint32_t x, y, z, w;
-};
-
+// a checkpoint and three gaps of up to 21 bits.  With P <= 4 a fifth word completes any span, and the
+// fields are taken without a branch; longer spans of a larger P read the gaps word by word.
+// The block kind is chosen before the division, and all products but the bits of whole blocks are
+// 24-bit ones (C, q < 2^16, widths < 2^5).  In a block, the absolute field of run j >= 1 (positions
+// [jP, jP + P)) starts f1 - 32 + j K bits after the head's, K = 32 + (P - 1) f2, and a block of q
+// positions is one of q + 1 less its last field, a checkpoint when q is a multiple of P.
 __device__ __forceinline__ uint32_t gt_get_cp(const DevGraph& g, const Hdr& h, uint32_t v, uint32_t k,
                                               uint32_t* fbits = nullptr) {
-    uint32_t blk, i;
-    gt_locate(h, k, blk, i);
-    const uint32_t sh = g.cp_shift;
-    const uint64_t bo = gtx_block_bit(h, blk, sh);
-    const uint32_t b = (i >> sh) << sh;  // 0 when the vertex has no checkpoints (q < P)
-    const uint32_t rem = i - b;
-    const uint64_t at = b ? bo + gtx_field(h, b, sh) : bo;  // the checkpoint, or the block head
-    const uint32_t aw = b ? 32u : h.f1;
-    const Words4 q = *(const Words4*)(g.w + (at >> 5));
-    uint64_t hi = ((uint64_t)q.x << 32) | q.y, lo = ((uint64_t)q.z << 32) | q.w;
-    const uint32_t s = (uint32_t)(at & 31);
+    const uint32_t sh = g.cp_shift, P1 = (1u << sh) - 1, f2 = h.f2;
+    const uint32_t big = __umul24(h.R, h.q + 1);
+    const bool lo = k < big;
+    const uint32_t len = lo ? h.q + 1 : h.q, kk = lo ? k : k - big;
+    const uint32_t b = udiv_chunk(kk, len), i = kk - __umul24(b, len), blk = lo ? b : b + h.R;
+    const uint32_t j = i >> sh, rem = i & P1;
+    const uint32_t F1 = h.f1 + __umul24(h.q, f2) + __umul24(h.q >> sh, 32 - f2);
+    const uint32_t F = lo ? F1 : F1 - ((h.q & P1) ? f2 : 32u);
+    const uint64_t at = h.pay + (uint64_t)b * F + (lo ? 0ull : (uint64_t)h.R * F1) +
+                        (j ? h.f1 - 32 + __umul24(j, 32 + __umul24(P1, f2)) : 0u);
+    const uint32_t aw = j ? 32u : h.f1, s = (uint32_t)(at & 31);
+    const uint32_t* p = g.w + (at >> 5);
+    const Words4 q = *(const Words4*)p;
+    if (fbits) *fbits = aw + rem * f2;
+    if (sh <= 2) {
+        FieldReader f(q, s + aw + __umul24(rem, f2) > 128 ? p[4] : 0u, s);
+        const uint32_t a = f.take(aw);
+        const uint32_t val = j ? a : (blk >= h.fp ? v + a + 1 : v - a - 1);
+        const uint32_t wd = max(f2, 1u), g1 = f.take(wd), g2 = f.take(wd), g3 = f.take(wd);
+        const uint32_t gaps = (rem > 0 ? g1 : 0u) + (rem > 1 ? g2 : 0u) + (rem > 2 ? g3 : 0u);
+        return val + rem + (f2 ? gaps : 0u);  // (0-bit gap fields read as 0)
+    }
+    uint64_t hi = ((uint64_t)q.x << 32) | q.y, low = ((uint64_t)q.z << 32) | q.w;
     const uint32_t a = (uint32_t)((hi << s) >> (64 - aw));
-    uint32_t val = b ? a : (blk >= h.fp ? v + a + 1 : v - a - 1);
+    uint32_t val = j ? a : (blk >= h.fp ? v + a + 1 : v - a - 1);
     if (rem) {
-        const uint32_t f2 = h.f2, sft = s + aw;  // 1 <= sft <= 63
+        const uint32_t sft = s + aw;  // 1 <= sft <= 63
         if (sft + rem * f2 <= 128) {
-            hi = (hi << sft) | (lo >> (64 - sft));
-            lo <<= sft;
+            hi = (hi << sft) | (low >> (64 - sft));
+            low <<= sft;
             uint32_t sum = rem;
             if (f2)  // (a well-formed block with gaps has f2 >= 1; 0-bit fields read as 0)
                 for (uint32_t t = 0; t < rem; ++t) {
                     sum += (uint32_t)(hi >> (64 - f2));
-                    hi = (hi << f2) | (lo >> (64 - f2));
-                    lo <<= f2;
+                    hi = (hi << f2) | (low >> (64 - f2));
+                    low <<= f2;
                 }
             val += sum;
         } else {
             val += sum_fields(g.w, at + aw, rem, f2) + rem;
         }
     }
-    if (fbits) *fbits = aw + rem * h.f2;
     return val;
 }
 

@@ -322,26 +322,6 @@ __device__ __forceinline__ RunAt run_at(const Hdr& h, uint32_t rr, uint32_t sh, 
     return a;
 }
 
-// Five words of the stream shifted left by s < 32 bits, the first four of the result kept: fields
-// are taken off the top with 32-bit funnel shifts, without a branch.
-struct FieldReader {
-    uint32_t t0, t1, t2, t3;
-    __device__ __forceinline__ static uint32_t shl(uint32_t hi, uint32_t lo, uint32_t n) {  // 1 <= n <= 32
-        return __builtin_amdgcn_alignbit(hi, lo, 32 - n);
-    }
-    __device__ __forceinline__ FieldReader(const Words4& q, uint32_t w4, uint32_t s)
-        : t0(s ? shl(q.x, q.y, s) : q.x), t1(s ? shl(q.y, q.z, s) : q.y), t2(s ? shl(q.z, q.w, s) : q.z),
-          t3(s ? shl(q.w, w4, s) : q.w) {}
-    __device__ __forceinline__ uint32_t take(uint32_t wdt) {  // 1 <= wdt <= 32
-        const uint32_t r = t0 >> (32 - wdt);
-        t0 = shl(t0, t1, wdt);
-        t1 = shl(t1, t2, wdt);
-        t2 = shl(t2, t3, wdt);
-        t3 = wdt < 32 ? t3 << wdt : 0u;
-        return r;
-    }
-};
-
 // The ids of one GT run into out[0 .. cnt): the absolute field, then each gap + 1 added on.  One
 // 16-byte load holds the field's offset in its word (< 32), a 32-bit field and three gaps of up to
 // 21 bits; a fifth word is read when they need more.  (Ids past cnt are not meaningful.)
@@ -388,8 +368,8 @@ __device__ __forceinline__ void le_run_ids(const uint32_t* __restrict__ w, const
     const Words4 sq = *(const Words4*)sp;
     const uint32_t ss = (uint32_t)(sbit & 31), rs = (uint32_t)(rbit & 31);
     const uint32_t w4 = ss + __umul24(a.cnt, sw) > 128 ? sp[4] : 0u;
-    const uint32_t u0 = rs ? FieldReader::shl(rq.x, rq.y, rs) : rq.x;
-    const uint32_t u1 = rs ? FieldReader::shl(rq.y, rq.z, rs) : rq.y;
+    const uint32_t u0 = FieldReader::shl0(rq.x, rq.y, rs);
+    const uint32_t u1 = FieldReader::shl0(rq.y, rq.z, rs);
     const uint32_t r1 = u0 >> (32 - rb), r2 = FieldReader::shl(u0, u1, rb) >> (32 - rb);
     const uint32_t A = c < h.fp ? v - r1 : v + r1;
     const uint32_t Z = c + 1 < h.fp ? v - r2 : v + r2;

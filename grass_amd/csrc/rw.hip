@@ -75,13 +75,17 @@ __device__ __forceinline__ uint64_t walk_wave(const DevGraph& g, bool active, ui
     for (uint32_t s = 0; s < L; ++s) {
         uint32_t nv = 0;
         if (live) {
+            // The draw does not need the header: it is made while the header is on its way (left to
+            // itself the compiler makes it after the degree check, on the step's dependent chain).
+            const uint4 hw = load_hdr_words(g, v);
+            U4 r = philox4x32_10(inst, w, s, 0, seed);
+            asm volatile("" : "+v"(r.x), "+v"(r.y));
             Hdr h;
-            load_hdr<FMT>(g, v, h);
+            unpack_hdr<FMT>(hw, h);
             if (COUNT) acc += 8 + bytes_of_bits(header_bits<FMT>(h));
             if (h.d == 0) {
                 live = false;
             } else {
-                U4 r = philox4x32_10(inst, w, s, 0, seed);
                 const uint32_t k = (uint32_t)uniform_index(r.x, r.y, h.d);
                 uint32_t fb = 0;
                 nv = get_neighbor<FMT>(g, h, v, k, COUNT ? &fb : nullptr);
