@@ -7,11 +7,10 @@
 // induced edge list of that set.
 //
 // 1. mdrw_walk_kernel: persistent, one wave per instance taken from a device queue.  The
-//    frontier ids and degrees sit in LDS.  Lane L owns the contiguous block [L*B, L*B + B) of
-//    entries (B = ceil(m / 64)) and keeps its degree sum in a register, so the degree-
-//    proportional pick is two wave scans: one over the 64 block sums to find the block, one over
-//    that block's degrees to find the entry.  A step is then one header load, one neighbour
-//    decode and one degree load, all wave-uniform.
+//    frontier and a three-level prefix sum of its degrees sit in LDS.  The wave works in rounds:
+//    its lanes guess the picks of the next five steps and read their neighbours together, then
+//    the steps are checked and taken one after the other as long as a guess was the exact pick.
+//    (mdrw_walk_plain_kernel, one step at a time, takes frontiers and degrees that do not fit.)
 // 2. mdrw_verts_kernel: one workgroup per instance sorts frontier + step destinations in LDS
 //    (bitonic) and keeps the first of each run of equal ids.
 // 3. Induced edges, per slice of up to 512 instances: a bit mask row per distinct vertex of the
@@ -38,7 +37,7 @@
 namespace grass {
 
 constexpr uint32_t kIndChunk = 2048;  // adjacency entries per chunk (32 wave iterations)
-constexpr uint32_t kMdrwHdrLdsMax = 4096;  // largest frontier whose headers the walk keeps in LDS
+constexpr uint32_t kMdrwRoundMax = 4096;  // largest frontier mdrw_walk_kernel takes (16 x 16 x 16 entries)
 constexpr int kSortBlock = 1024;
 
 struct MdDesc {
@@ -50,43 +49,228 @@ struct MdDesc {
 
 // ---------------------------------------------------------------------------- 1. walks
 
-// HDR: the frontier entries' header-cache words sit in LDS next to their ids and degrees (20 bytes
-// per entry instead of 8), so a step's chain is two dependent loads (the picked entry's neighbour,
-// then that neighbour's header) instead of three (header, neighbour, degree).
-template <int FMT, bool HDR>
-__global__ __launch_bounds__(kWave) void mdrw_walk_kernel(DevGraph g, const MdDesc* __restrict__ desc,
+// A frontier in LDS: entry e is {vertex, header words x, y, w} (word z, the degree, is the
+// difference of two prefix sums).  The degrees' prefix sums have three levels of 16, inclusive
+// within each 16: over the entries of a block, over the 16 blocks of a group, and over the groups.
+// Changing one degree adds the difference to at most 16 words of each level.
+constexpr uint32_t kRadix = 16;
+constexpr uint32_t kSumsBlocks = kRadix;                          // word offsets of the levels
+constexpr uint32_t kSumsEntries = kSumsBlocks + kRadix * kRadix;  // (groups at 0)
+constexpr uint32_t kRoundsWMax = 1u << 30;  // degree sums the rounds take: a round adds at most 5 * 2^24
+__host__ __device__ constexpr uint32_t mdrw_round_up(uint32_t m) { return (m + kRadix - 1) / kRadix * kRadix; }
+// LDS bytes of a frontier of mp entries (whole blocks)
+__host__ __device__ constexpr size_t mdrw_round_lds(uint32_t mp) { return (size_t)mp * 20 + kSumsEntries * 4; }
+
+// Entries of a 16-word inclusive prefix row that are <= y (the row's last valid word exceeds y).
+// Four counts side by side: a lone wave waits for every dependent instruction.
+__device__ __forceinline__ uint32_t row_count(const uint32_t* row, uint32_t y) {
+    const uint4* q = (const uint4*)row;
+    const uint4 a = q[0], b = q[1], c = q[2], d = q[3];
+    const uint32_t ca = (a.x <= y) + (a.y <= y) + (a.z <= y) + (a.w <= y);
+    const uint32_t cb = (b.x <= y) + (b.y <= y) + (b.z <= y) + (b.w <= y);
+    const uint32_t cc = (c.x <= y) + (c.y <= y) + (c.z <= y) + (c.w <= y);
+    const uint32_t cd = (d.x <= y) + (d.y <= y) + (d.z <= y) + (d.w <= y);
+    return (ca + cb) + (cc + cd);
+}
+
+// floor(r * b / 2^64) for b < 2^32: uniform_index with a 32-bit bound.
+__device__ __forceinline__ uint32_t index32(uint32_t lo, uint32_t hi, uint32_t b) {
+    return (uint32_t)(((uint64_t)hi * b + __umulhi(lo, b)) >> 32);
+}
+
+// The step a lane guesses for: lane 0 makes the round's first step (its pick is exact), lanes 1-15
+// guess the second, and each further 16 lanes one more.
+constexpr uint32_t kAhead = 1 + kWave / 16;
+
+// Rounds.  A step is a chain of two dependent loads (the picked entry's neighbour, then that
+// neighbour's header, whose degree enters the frontier) and some hundred dependent instructions, all
+// of one instance and so of one wave.  A round makes one such chain for up to kAhead steps: the draws
+// of the coming steps are known, and a step moves the degree sums only a little, so the entry a
+// later step picks is guessed from the frontier as it is.  The 16 lanes of a later step try
+// positions around the one its draw has now, at distances of up to the recent degrees' running
+// average (times the root of the steps between), denser near zero.  Every lane then reads its
+// entry's neighbour and the neighbour's header.  The steps are taken in order: a lane of the step
+// whose entry is unchanged and whose degree range, moved by the changes so far, holds the step's exact
+// pick has the exact neighbour.  The first step always has one (lane 0); where a later one has none
+// the round ends and the next starts there, so the result never depends on the guesses.
+// What bounds it is the latency of a lone wave: a round takes about 5600 cycles on R-MAT s22 (GT), of
+// which the two loads are 1400, the search 1300, the rest of the neighbour's decode 1000 and each
+// step taken 400, and makes 2.2 steps (3.3 on a milder skew, 4.8 without); one step at a time took
+// 3700 cycles a step.  64 instances of 16384, s22: the batch 28.7 -> 21.7 ms; 5 of 3000 on the
+// milder s18 (LE): 4.7 -> 2.6 ms.
+// An instance whose degree sum reaches wmax (<= kRoundsWMax) is left to mdrw_walk_plain_kernel (scnt = kRedo).
+constexpr uint32_t kRedo = 0xFFFFFFFFu;
+template <int FMT>
+__global__ __launch_bounds__(kWave) void mdrw_walk_kernel(DevGraph g, const MdDesc* __restrict__ desc, uint32_t I,
+                                                          unsigned long long* queue, uint64_t seed,
+                                                          uint32_t* __restrict__ init, uint32_t* __restrict__ ssrc,
+                                                          uint32_t* __restrict__ sdst, uint32_t* __restrict__ scnt,
+                                                          uint32_t mp, uint32_t wmax, uint32_t* __restrict__ err) {
+    extern __shared__ __align__(16) uint32_t lds[];
+    uint32_t* const S = lds;                      // prefix sums: groups, blocks, entries
+    uint4* const E = (uint4*)(lds + kSumsEntries + mp);
+    const uint32_t lane = lane_id();
+    const uint32_t mystep = lane ? 1 + lane / 16 : 0;
+    float reach;  // distance of this lane's guess, in running averages: sign(c) c^2 sqrt(steps between)
+    {
+        const float c = ((float)(int)(lane & 15) - 8.0f) * 0.125f;
+        reach = mystep ? c * fabsf(c) * sqrtf((float)mystep) : 0.0f;
+    }
+    // lanes 0-15 add to the entries' sums, 16-31 to the blocks', 32-47 to the groups'
+    const uint32_t lev = lane / 16, o16 = lane & 15;
+    const uint32_t lshift = lev * 4, lbase = lev == 0 ? kSumsEntries : lev == 1 ? kSumsBlocks : 0;
+    for (;;) {
+        unsigned long long gi = 0;
+        if (lane == 0) gi = atomicAdd(queue, 1ull);
+        gi = readlane_u64(gi, 0);
+        if (gi >= I) break;  // every wave exits once the queue is drained
+        const MdDesc q = desc[gi];
+        const uint32_t m = q.m, nb = (m + kRadix - 1) / kRadix, ns = (nb + kRadix - 1) / kRadix;
+        const uint32_t llim = lev == 0 ? m : lev == 1 ? nb : lev == 2 ? ns : 0;
+        // the frontier, with its degrees in the entries' sums until those replace them
+        uint64_t W64 = 0;
+        for (uint32_t j = lane; j < nb * kRadix; j += kWave) {
+            uint32_t d = 0;
+            if (j < m) {
+                const uint32_t v = (uint32_t)uniform(seed, q.inst, j, kTagStart, 0, g.n);
+                const uint4 e = load_hdr_words(g, v);
+                E[j] = make_uint4(v, e.x, e.y, e.w);
+                d = e.z;
+                init[q.init_base + j] = v;
+            }
+            S[kSumsEntries + j] = d;
+            W64 += d;
+        }
+        W64 = wave_sum(W64);
+        wave_sync();
+        // words past the last entry, block or group never count as <= a position
+        for (uint32_t b = lane; b < ns * kRadix; b += kWave) {
+            uint32_t acc = 0;
+            if (b < nb)
+                for (uint32_t i = b * kRadix; i < (b + 1) * kRadix; ++i) {
+                    acc += S[kSumsEntries + i];
+                    S[kSumsEntries + i] = i < m ? acc : 0xFFFFFFFFu;
+                }
+            S[kSumsBlocks + b] = acc;
+        }
+        wave_sync();
+        {
+            uint32_t acc = 0;
+            if (lane < ns)
+                for (uint32_t i = lane * kRadix; i < (lane + 1) * kRadix; ++i) {
+                    acc += S[kSumsBlocks + i];
+                    S[kSumsBlocks + i] = i < nb ? acc : 0xFFFFFFFFu;
+                }
+            const uint32_t inc = wave_inclusive_sum(acc);
+            if (lane < kRadix) S[lane] = lane < ns ? inc : 0xFFFFFFFFu;
+        }
+        wave_sync();
+        bool wide = (__builtin_amdgcn_readfirstlane((uint32_t)(W64 >> 32)) != 0);
+        uint32_t W = __builtin_amdgcn_readfirstlane((uint32_t)W64);
+        float avg = (float)W / (float)m;  // of recent degrees (guesses only)
+        uint32_t t = 0;
+        bool bad = false;
+        U4 ahead{0, 0, 0, 0};  // lane l: the draws of step t0 + l of the current 64
+        while (t < q.steps && W > 0 && !bad) {
+            wide = wide || W >= wmax;
+            if (wide) break;
+            const uint32_t t64 = t & (kWave - 1);
+            if (t64 == 0) ahead = philox4x32_10(q.inst, t + lane, kTagMdrwStep, 0, seed);
+            // steps of this round: not past the walk's end, nor the 64 whose draws are here
+            const uint32_t K = min(min(kAhead, q.steps - t), kWave - t64);
+            const int from = (int)min(t64 + mystep, (uint32_t)kWave - 1);
+            const uint32_t rp0 = __shfl(ahead.x, from, kWave), rp1 = __shfl(ahead.y, from, kWave);
+            const uint32_t rk0 = __shfl(ahead.z, from, kWave), rk1 = __shfl(ahead.w, from, kWave);
+            // the position this lane tries, in the frontier as it is (lane 0: exact)
+            const int32_t yg = (int32_t)index32(rp0, rp1, W) + (int32_t)(reach * avg);  // < 2^30 + 2^25
+            const uint32_t y = (uint32_t)min(max(yg, 0), (int32_t)W - 1);
+            // its entry e, the entry's first position and degree
+            const uint32_t c1 = row_count(S, y);
+            const uint32_t b1 = c1 ? S[c1 - 1] : 0u;
+            const uint32_t* row2 = S + kSumsBlocks + c1 * kRadix;
+            const uint32_t y2 = y - b1, c2 = row_count(row2, y2);
+            const uint32_t b2 = c2 ? row2[c2 - 1] : 0u;
+            const uint32_t blk = c1 * kRadix + c2;
+            const uint32_t* row3 = S + kSumsEntries + blk * kRadix;
+            const uint32_t y3 = y2 - b2, c3 = row_count(row3, y3);
+            const uint32_t b3 = c3 ? row3[c3 - 1] : 0u;
+            const uint32_t e = blk * kRadix + c3, du = row3[c3] - b3;
+            uint32_t start = b1 + b2 + b3;
+            // its neighbour and the neighbour's header
+            const uint4 ew = E[e];
+            Hdr h;
+            unpack_hdr<FMT>(make_uint4(ew.y, ew.z, du, ew.w), h);
+            const uint32_t v = get_neighbor<FMT>(g, h, ew.x, index32(rk0, rk1, du), nullptr);
+            const uint4 hv = load_hdr_words(g, v < g.n ? v : 0u);
+            const uint32_t diff = hv.z - du;
+            uint32_t range = mystep < K ? du : 0u;  // 0: no guess, or its entry has changed
+            // the round's steps, in order
+            uint32_t done = 0;
+            unsigned long long won = 0;
+            while (done < K && W > 0) {
+                const uint32_t x = index32(rp0, rp1, W);  // (of the lane's own step)
+                const unsigned long long hits = __ballot(mystep == done && x - start < range);
+                if (!hits) break;  // the first step always has lane 0
+                const int w = __builtin_ctzll(hits);
+                won |= 1ull << w;
+                const uint32_t we = lane_get(e, w), wd = lane_get(diff, w);
+                W += wd;
+                start += e > we ? wd : 0u;
+                range = e == we ? 0u : range;
+                const uint32_t pos = we >> lshift, idx = (pos & ~15u) + o16;
+                if (idx >= pos && idx < llim) atomicAdd(&S[lbase + idx], wd);
+                ++done;
+            }
+            // the lanes that made a step write it, and their entry
+            const bool mine = (won >> lane) & 1;
+            if (mine) {
+                ssrc[q.step_base + t + mystep] = ew.x;
+                sdst[q.step_base + t + mystep] = v;
+                E[e] = make_uint4(v, hv.x, hv.y, hv.w);
+            }
+            if (__any(mine && v >= g.n)) {  // the graph decodes to garbage: stop this instance
+                if (lane == 0) atomicCAS(err, kErrNone, kErrBadNeighbor);
+                bad = true;
+            }
+            avg += ((float)lane_get(hv.z, 63 - __builtin_clzll(won)) - avg) * 0.25f;
+            t += done;
+            wave_sync();
+        }
+        if (lane == 0) scnt[gi] = bad ? 0u : wide ? kRedo : t;
+        wave_sync();  // the frontier is rewritten by the next instance
+    }
+}
+
+// One step at a time, for frontiers above kMdrwRoundMax or degrees whose 32-bit partial sums could
+// overflow: ids and degrees in LDS (8 bytes per entry), the picked entry's header from memory.
+// Lane L owns the contiguous block [L*B, L*B + B) of entries (B = ceil(m / 64)) and keeps its degree
+// sum in a register, so the pick is two wave scans: one over the 64 block sums to find the block,
+// one over that block's degrees to find the entry.  redo: only the instances the rounds left
+// (scnt = kRedo).
+template <int FMT>
+__global__ __launch_bounds__(kWave) void mdrw_walk_plain_kernel(DevGraph g, const MdDesc* __restrict__ desc,
                                                           uint32_t I, unsigned long long* queue,
                                                           uint64_t seed, uint32_t* __restrict__ init,
                                                           uint32_t* __restrict__ ssrc,
                                                           uint32_t* __restrict__ sdst,
                                                           uint32_t* __restrict__ scnt,
-                                                          uint32_t mmax, uint32_t* __restrict__ err) {
+                                                          uint32_t mmax, uint32_t* __restrict__ err, bool redo) {
     extern __shared__ uint32_t lds[];
     uint32_t* F = lds;         // frontier ids
     uint32_t* D = lds + mmax;  // their degrees
-    uint32_t* Hx = lds + 2 * mmax;  // HDR: their header words x, y, w (z is the degree)
-    uint32_t* Hy = lds + 3 * mmax;
-    uint32_t* Hw = lds + 4 * mmax;
     const int lane = lane_id();
     for (;;) {
         unsigned long long gi = 0;
         if (lane == 0) gi = atomicAdd(queue, 1ull);
         gi = __shfl(gi, 0, kWave);
         if (gi >= I) break;  // every wave exits once the queue is drained
+        if (redo && scnt[gi] != kRedo) continue;  // (wave-uniform)
         const MdDesc q = desc[gi];
         const uint32_t m = q.m;
         for (uint32_t j = lane; j < m; j += kWave) {
             const uint32_t v = (uint32_t)uniform(seed, q.inst, j, kTagStart, 0, g.n);
             F[j] = v;
-            if (HDR) {
-                const uint4 e = g.hdr[v];
-                D[j] = e.z;
-                Hx[j] = e.x;
-                Hy[j] = e.y;
-                Hw[j] = e.w;
-            } else {
-                D[j] = g.deg[v];
-            }
+            D[j] = g.deg[v];
             init[q.init_base + j] = v;
         }
         __syncthreads();
@@ -149,8 +333,7 @@ __global__ __launch_bounds__(kWave) void mdrw_walk_kernel(DevGraph g, const MdDe
             }
             const uint32_t u = F[j], du = D[j];
             Hdr h;
-            if (HDR) unpack_hdr<FMT>(make_uint4(Hx[j], Hy[j], du, Hw[j]), h);
-            else load_hdr<FMT>(g, u, h);
+            load_hdr<FMT>(g, u, h);
             const uint32_t k = (uint32_t)mulhi64(((uint64_t)r.w << 32) | r.z, du);
             const uint32_t v = get_neighbor<FMT>(g, h, u, k, nullptr);
             if (v >= g.n) {  // the graph decodes to garbage: stop this instance
@@ -158,20 +341,13 @@ __global__ __launch_bounds__(kWave) void mdrw_walk_kernel(DevGraph g, const MdDe
                 bad = true;
                 break;
             }
-            uint4 ev = make_uint4(0, 0, 0, 0);
-            if (HDR) ev = g.hdr[v];
-            const uint32_t dv = HDR ? ev.z : g.deg[v];
-            __syncthreads();  // every lane has read F[j], D[j] (and the header words)
+            const uint32_t dv = g.deg[v];
+            __syncthreads();  // every lane has read F[j], D[j]
             if (lane == 0) {
                 ssrc[q.step_base + t] = u;
                 sdst[q.step_base + t] = v;
                 F[j] = v;
                 D[j] = dv;
-                if (HDR) {
-                    Hx[j] = ev.x;
-                    Hy[j] = ev.y;
-                    Hw[j] = ev.w;
-                }
             }
             if (lane == L) bs = bs - du + dv;
             if (lane >= L) incl = incl - du + dv;
@@ -751,25 +927,41 @@ static int mdrw_run(grass_graph* g, MdrwState& st, hipStream_t s, bool replay) {
     if (e != hipSuccess) return status_of(e);
     hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3(1), dim3(64), 0, s, d_queue, (uint64_t)1, 0ull);
     {
-        // headers in LDS while two instances still fit a CU (20 bytes per frontier entry)
-        const bool hdr = st.mmax <= kMdrwHdrLdsMax;
-        const size_t lds = (hdr ? 5ull : 2ull) * st.mmax * 4;
-        const void* kfn = le ? (hdr ? (const void*)mdrw_walk_kernel<kLE, true> : (const void*)mdrw_walk_kernel<kLE, false>)
-                             : (hdr ? (const void*)mdrw_walk_kernel<kGT, true> : (const void*)mdrw_walk_kernel<kGT, false>);
-        allow_lds(kfn, lds);
-        int dev = 0, cus = 0, per = 0;
+        // Rounds for frontiers whose sums fit three levels of 16 and steps that add less than 2^24;
+        // 20 bytes of LDS per entry, so that two instances of up to 4032 share a CU.  One step at a
+        // time otherwise, and for instances whose degree sum grows past kRoundsWMax (only launched
+        // where the largest degree allows that; GRASS_MDRW_WMAX lowers the limit, for tests).
+        const bool rounds = st.mmax <= kMdrwRoundMax && g->max_degree < (1ull << 24);
+        uint32_t wmax = kRoundsWMax;
+        if (const char* ev = getenv("GRASS_MDRW_WMAX")) {
+            const unsigned long x = strtoul(ev, nullptr, 10);
+            if (x && x < wmax) wmax = (uint32_t)x;
+        }
+        const bool may_redo = rounds && (uint64_t)st.mmax * g->max_degree >= wmax;
+        int dev = 0, cus = 0;
         (void)hipGetDevice(&dev);
         (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kfn, kWave, lds);
-        const unsigned grid = (unsigned)std::min<uint64_t>(I, (uint64_t)std::max(cus, 1) * std::max(per, 1));
-#define GRASS_MDRW_WALK(F, H)                                                                                   \
-    hipLaunchKernelGGL((mdrw_walk_kernel<F, H>), dim3(grid), dim3(kWave), lds, s, dg, d_desc, I, d_queue, seed, \
-                       d_init, d_ssrc, d_sdst, d_scnt, st.mmax, g->d_err)
-        if (le && hdr) GRASS_MDRW_WALK(kLE, true);
-        else if (le) GRASS_MDRW_WALK(kLE, false);
-        else if (hdr) GRASS_MDRW_WALK(kGT, true);
-        else GRASS_MDRW_WALK(kGT, false);
-#undef GRASS_MDRW_WALK
+        auto grid_of = [&](const void* kfn, size_t lds) {
+            int per = 0;
+            allow_lds(kfn, lds);
+            (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kfn, kWave, lds);
+            return (unsigned)std::min<uint64_t>(I, (uint64_t)std::max(cus, 1) * std::max(per, 1));
+        };
+        if (rounds) {
+            const uint32_t mp = mdrw_round_up(st.mmax);
+            const size_t lds = mdrw_round_lds(mp);
+            auto kern = le ? mdrw_walk_kernel<kLE> : mdrw_walk_kernel<kGT>;
+            hipLaunchKernelGGL(kern, dim3(grid_of((const void*)kern, lds)), dim3(kWave), lds, s, dg, d_desc, I, d_queue,
+                               seed, d_init, d_ssrc, d_sdst, d_scnt, mp, wmax, g->d_err);
+        }
+        if (!rounds || may_redo) {
+            if (rounds)
+                hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3(1), dim3(64), 0, s, d_queue, (uint64_t)1, 0ull);
+            const size_t lds = 8ull * st.mmax;
+            auto kern = le ? mdrw_walk_plain_kernel<kLE> : mdrw_walk_plain_kernel<kGT>;
+            hipLaunchKernelGGL(kern, dim3(grid_of((const void*)kern, lds)), dim3(kWave), lds, s, dg, d_desc, I, d_queue,
+                               seed, d_init, d_ssrc, d_sdst, d_scnt, st.mmax, g->d_err, rounds);
+        }
     }
     const uint32_t cap = next_pow2(st.vmax);
     hipLaunchKernelGGL(mdrw_verts_kernel, dim3(I), dim3(kSortBlock), (size_t)cap * 4, s, d_desc, d_init,
