@@ -613,17 +613,14 @@ int decode_csr(grass_graph* g, uint64_t* rowptr, uint32_t* col, hipStream_t s) {
         std::lock_guard<std::mutex> lock(g->mu);
         if (!g->d_roff) {
             uint64_t* r = nullptr;
-            uint64_t* part = nullptr;
-            if (hipMalloc(&r, (n + 1) * 8) != hipSuccess) return GRASS_ENOMEM;
-            if (hipMalloc(&part, (nb + 4) * 8) != hipSuccess) {
-                (void)hipFree(r);
-                return GRASS_ENOMEM;
-            }
+            WorkMem m_part;
+            if (m_part.alloc((nb + 4) * 8, s) != hipSuccess) return GRASS_ENOMEM;
+            uint64_t* part = m_part.as<uint64_t>();
+            if (device_malloc((void**)&r, (n + 1) * 8) != hipSuccess) return GRASS_ENOMEM;
             uint64_t total = 0;
             hipError_t e = exclusive_scan(RunGen{g->d_hdr, g->fmt, sh}, Count{n, nullptr}, n, r, part, part + nb, s);
             if (e == hipSuccess) e = hipMemcpyAsync(&total, r + n, 8, hipMemcpyDeviceToHost, s);
             if (e == hipSuccess) e = hipStreamSynchronize(s);
-            (void)hipFree(part);
             if (e != hipSuccess) {
                 (void)hipFree(r);
                 return status_of(e);
@@ -645,7 +642,7 @@ int decode_csr(grass_graph* g, uint64_t* rowptr, uint32_t* col, hipStream_t s) {
         std::lock_guard<std::mutex> lock(g->mu);
         if (!g->d_wstart[slot]) {
             uint32_t* t = nullptr;
-            if (hipMalloc(&t, (waves + 1) * 4) != hipSuccess) return GRASS_ENOMEM;
+            if (device_malloc((void**)&t, (waves + 1) * 4) != hipSuccess) return GRASS_ENOMEM;
             const unsigned grid = (unsigned)std::min<uint64_t>((n + 255) / 256, 16384);
             hipLaunchKernelGGL(wave_start_kernel, dim3(grid), dim3(256), 0, s, uoff, (uint32_t)n, unit, waves, t);
             hipError_t e = hipGetLastError();

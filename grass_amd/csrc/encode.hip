@@ -342,12 +342,14 @@ __global__ void bswap64_kernel(unsigned long long* w, uint64_t count) {
 int fetch_to_host(uint8_t* dst, const void* src, uint64_t len, hipStream_t s) {
     if (len == 0) return GRASS_OK;
     const uint64_t chunk = std::min<uint64_t>(64ull << 20, len);
+    PinnedWork pinned[2];
     void* pin[2] = {nullptr, nullptr};
     hipEvent_t ev[2] = {nullptr, nullptr};
     int rc = GRASS_OK;
     for (int i = 0; i < 2 && !rc; ++i) {
-        if (hipHostMalloc(&pin[i], chunk, hipHostMallocDefault) != hipSuccess) rc = GRASS_ENOMEM;
-        else if (hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) != hipSuccess) rc = GRASS_EDEVICE;
+        if (pinned[i].alloc(chunk) != hipSuccess) rc = GRASS_ENOMEM;
+        pin[i] = pinned[i].p;
+        if (!rc && hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) != hipSuccess) rc = GRASS_EDEVICE;
     }
     const unsigned threads = load_threads();
     const uint64_t nch = (len + chunk - 1) / chunk;
@@ -370,16 +372,14 @@ int fetch_to_host(uint8_t* dst, const void* src, uint64_t len, hipStream_t s) {
         parallel_copy(dst + off, (const uint8_t*)pin[c & 1], std::min(chunk, len - off), threads);
     }
     if (hipStreamSynchronize(s) != hipSuccess && !rc) rc = GRASS_EDEVICE;
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < 2; ++i)
         if (ev[i]) (void)hipEventDestroy(ev[i]);
-        if (pin[i]) (void)hipHostFree(pin[i]);
-    }
     return rc;
 }
 
 // The .graph and .offset images in device memory (the files' bytes), complete when this returns.
 struct Images {
-    DevMem g, o;
+    WorkMem g, o;
     uint64_t gbytes = 0, obytes = 0;
 };
 
@@ -387,7 +387,7 @@ int encode_images(const uint64_t* rowptr, const uint32_t* col, uint64_t n, int f
                   Images& im) {
     const bool le = format == GRASS_FMT_LE;
     const uint64_t nb = scan_blocks(n);
-    DevMem tmp;  // len[n], start[n + 1], widths[n], partials, total, maxlen
+    WorkMem tmp;  // len[n], start[n + 1], widths[n], partials, total, maxlen
     Carve need(nullptr);
     auto plan = [&](Carve& c, uint64_t** len, uint64_t** start, uint2** widths, uint64_t** part,
                     unsigned long long** most) {
@@ -401,7 +401,7 @@ int encode_images(const uint64_t* rowptr, const uint32_t* col, uint64_t n, int f
     uint2* d_w;
     unsigned long long* d_max;
     plan(need, &d_len, &d_start, &d_w, &d_part, &d_max);
-    if (tmp.alloc(need.off + 256) != hipSuccess) return GRASS_ENOMEM;
+    if (tmp.alloc(need.off + 256, s) != hipSuccess) return GRASS_ENOMEM;
     Carve c(tmp.p);
     plan(c, &d_len, &d_start, &d_w, &d_part, &d_max);
     int dev = 0, cus = 0;
@@ -423,8 +423,8 @@ int encode_images(const uint64_t* rowptr, const uint32_t* col, uint64_t n, int f
     if (total >= (1ull << 40)) return GRASS_EINVAL;  // past what a reader's 40-bit offsets address
     // .graph
     const uint64_t gwords = (total + 31) / 32 + 2;
-    DevMem& gbuf = im.g;
-    if (gbuf.alloc(gwords * 4) != hipSuccess) return GRASS_ENOMEM;
+    WorkMem& gbuf = im.g;
+    if (gbuf.alloc(gwords * 4, s) != hipSuccess) return GRASS_ENOMEM;
     uint32_t* d_g = (uint32_t*)gbuf.p;
     e = hipMemsetAsync(d_g, 0, gwords * 4, s);
     if (e != hipSuccess) return status_of(e);
@@ -439,8 +439,8 @@ int encode_images(const uint64_t* rowptr, const uint32_t* col, uint64_t n, int f
     while (ubl < 64 && (maxlen >> ubl)) ++ubl;
     const uint64_t obits = 8 + n * (uint64_t)ubl;
     const uint64_t owords = (obits + 63) / 64 + 1;
-    DevMem& obuf = im.o;
-    if (obuf.alloc(owords * 8) != hipSuccess) return GRASS_ENOMEM;
+    WorkMem& obuf = im.o;
+    if (obuf.alloc(owords * 8, s) != hipSuccess) return GRASS_ENOMEM;
     unsigned long long* d_o = (unsigned long long*)obuf.p;
     e = hipMemsetAsync(d_o, 0, owords * 8, s);
     if (e != hipSuccess) return status_of(e);

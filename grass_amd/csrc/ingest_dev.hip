@@ -152,8 +152,8 @@ int graph_sort_device(const uint32_t* src, const uint32_t* dst, uint64_t m, int 
                       uint64_t* m_out) {
     const int per = directed ? 1 : 2;
     const uint64_t P = (uint64_t)per * m;
-    DevMem small;
-    if (small.alloc(64) != hipSuccess) return GRASS_ENOMEM;
+    WorkMem small;
+    if (small.alloc(64, s) != hipSuccess) return GRASS_ENOMEM;
     unsigned int* d_max = small.as<unsigned int>();
     uint64_t* d_tot = (uint64_t*)(small.as<char>() + 8);
     hipLaunchKernelGGL(fill_kernel<unsigned int>, dim3(1), dim3(64), 0, s, d_max, (uint64_t)1, 0u);
@@ -167,11 +167,11 @@ int graph_sort_device(const uint32_t* src, const uint32_t* dst, uint64_t m, int 
     const uint64_t nid = m ? (uint64_t)maxid + 1 : 0;
 
     // 1-2: first positions, the ids that appear, their new ids
-    DevMem d_first, d_rank, d_fkey, d_fid, d_newid, d_part;
+    WorkMem d_first, d_rank, d_fkey, d_fid, d_newid, d_part;
     const uint64_t nbI = scan_blocks(std::max<uint64_t>(nid, 1)), nbP = scan_blocks(std::max<uint64_t>(P, 1));
-    if (d_first.alloc(std::max<uint64_t>(nid, 1) * 8) != hipSuccess ||
-        d_rank.alloc((nid + 1) * 8) != hipSuccess ||
-        d_part.alloc((std::max(nbI, nbP) + 2) * 8) != hipSuccess)
+    if (d_first.alloc(std::max<uint64_t>(nid, 1) * 8, s) != hipSuccess ||
+        d_rank.alloc((nid + 1) * 8, s) != hipSuccess ||
+        d_part.alloc((std::max(nbI, nbP) + 2) * 8, s) != hipSuccess)
         return GRASS_ENOMEM;
     unsigned long long* first = d_first.as<unsigned long long>();
     uint64_t* rank = d_rank.as<uint64_t>();
@@ -185,9 +185,9 @@ int graph_sort_device(const uint32_t* src, const uint32_t* dst, uint64_t m, int 
     if (e != hipSuccess) return status_of(e);
     *n_out = n;
     if (rowptr_cap < n + 1) return GRASS_ECAPACITY;
-    if (d_fkey.alloc(std::max<uint64_t>(n, 1) * 16) != hipSuccess ||
-        d_fid.alloc(std::max<uint64_t>(n, 1) * 8) != hipSuccess ||
-        d_newid.alloc(std::max<uint64_t>(nid, 1) * 4) != hipSuccess)
+    if (d_fkey.alloc(std::max<uint64_t>(n, 1) * 16, s) != hipSuccess ||
+        d_fid.alloc(std::max<uint64_t>(n, 1) * 8, s) != hipSuccess ||
+        d_newid.alloc(std::max<uint64_t>(nid, 1) * 4, s) != hipSuccess)
         return GRASS_ENOMEM;
     unsigned long long* fk = d_fkey.as<unsigned long long>();
     uint32_t* fid = d_fid.as<uint32_t>();
@@ -199,8 +199,8 @@ int graph_sort_device(const uint32_t* src, const uint32_t* dst, uint64_t m, int 
         size_t tb = 0;
         const unsigned eb = (unsigned)std::max(1, bits_for(2 * m));
         e = rocprim::radix_sort_pairs(nullptr, tb, kb, vb, (size_t)n, 0u, eb, s);
-        DevMem tmp;
-        if (e == hipSuccess && tmp.alloc(tb) != hipSuccess) return GRASS_ENOMEM;
+        WorkMem tmp;
+        if (e == hipSuccess && tmp.alloc(tb, s) != hipSuccess) return GRASS_ENOMEM;
         if (e == hipSuccess && n) e = rocprim::radix_sort_pairs(tmp.p, tb, kb, vb, (size_t)n, 0u, eb, s);
         if (e != hipSuccess) return status_of(e);
         const unsigned gn = (unsigned)std::min<uint64_t>((n + kIgBlock - 1) / kIgBlock + 1, kIgGrid);
@@ -217,8 +217,8 @@ int graph_sort_device(const uint32_t* src, const uint32_t* dst, uint64_t m, int 
     // 3-4: keys, sorted over the bits a key of the renumbered ids can set (~0 still sorts last)
     // two buffers of P + 1 keys: the sort's double buffer, and after it the free one holds the
     // ranks of the distinct keys (P + 1 entries)
-    DevMem d_keys;
-    if (d_keys.alloc((P + 1) * 16) != hipSuccess) return GRASS_ENOMEM;
+    WorkMem d_keys;
+    if (d_keys.alloc((P + 1) * 16, s) != hipSuccess) return GRASS_ENOMEM;
     unsigned long long* keys = d_keys.as<unsigned long long>();
     if (m) hipLaunchKernelGGL(edge_keys_kernel, dim3(gm), dim3(kIgBlock), 0, s, src, dst, m,
                               (const uint32_t*)d_newid.as<uint32_t>(), per, keys);
@@ -227,8 +227,8 @@ int graph_sort_device(const uint32_t* src, const uint32_t* dst, uint64_t m, int 
         size_t tb = 0;
         const unsigned eb = 32u + (unsigned)std::max(1, bits_for(n ? n - 1 : 0));
         e = rocprim::radix_sort_keys(nullptr, tb, kb, (size_t)P, 0u, eb, s);
-        DevMem tmp;
-        if (e == hipSuccess && tmp.alloc(tb) != hipSuccess) return GRASS_ENOMEM;
+        WorkMem tmp;
+        if (e == hipSuccess && tmp.alloc(tb, s) != hipSuccess) return GRASS_ENOMEM;
         if (e == hipSuccess && P) e = rocprim::radix_sort_keys(tmp.p, tb, kb, (size_t)P, 0u, eb, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) return status_of(e);
@@ -294,8 +294,8 @@ int grass_compress_on_device(const grass_csr* csr, int format, int device, grass
     if (!grass::enter_device(device)) return GRASS_EDEVICE;
     int rc = GRASS_OK;
     {
-        grass::DevMem rp, cl;
-        if (rp.alloc((csr->n + 1) * 8) != hipSuccess || cl.alloc(std::max<uint64_t>(csr->m, 1) * 4) != hipSuccess)
+        grass::WorkMem rp, cl;
+        if (rp.alloc((csr->n + 1) * 8, nullptr) != hipSuccess || cl.alloc(std::max<uint64_t>(csr->m, 1) * 4, nullptr) != hipSuccess)
             rc = GRASS_ENOMEM;
         hipError_t e = hipSuccess;
         if (!rc) e = hipMemcpy(rp.p, csr->rowptr.data(), (csr->n + 1) * 8, hipMemcpyHostToDevice);
@@ -324,10 +324,10 @@ int grass_graph_sort_on_device(const uint32_t* src, const uint32_t* dst, uint64_
     grass_csr* csr = new (std::nothrow) grass_csr();
     if (!csr) rc = GRASS_ENOMEM;
     {
-        grass::DevMem ds, dd, rp, cl;
-        if (!rc && (ds.alloc(std::max<uint64_t>(m, 1) * 4) != hipSuccess ||
-                    dd.alloc(std::max<uint64_t>(m, 1) * 4) != hipSuccess || rp.alloc(rcap * 8) != hipSuccess ||
-                    cl.alloc(ccap * 4) != hipSuccess))
+        grass::WorkMem ds, dd, rp, cl;
+        if (!rc && (ds.alloc(std::max<uint64_t>(m, 1) * 4, nullptr) != hipSuccess ||
+                    dd.alloc(std::max<uint64_t>(m, 1) * 4, nullptr) != hipSuccess || rp.alloc(rcap * 8, nullptr) != hipSuccess ||
+                    cl.alloc(ccap * 4, nullptr) != hipSuccess))
             rc = GRASS_ENOMEM;
         hipError_t e = hipSuccess;
         if (!rc && m) e = hipMemcpy(ds.p, src, m * 4, hipMemcpyHostToDevice);

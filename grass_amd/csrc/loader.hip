@@ -252,13 +252,15 @@ int stage_to_device(ByteSource& src, char* dst, hipStream_t stream, uint64_t* ta
         return e == hipSuccess ? GRASS_OK : GRASS_EDEVICE;
     }
     const uint64_t chunk = std::min<uint64_t>(kChunk, total);
+    PinnedWork pinned[2];
     void* pin[2] = {nullptr, nullptr};
     hipEvent_t ev[2] = {nullptr, nullptr};
     int rc = GRASS_OK;
     for (int i = 0; i < 2 && rc == GRASS_OK; ++i) {
-        if (hipHostMalloc(&pin[i], chunk, hipHostMallocDefault) != hipSuccess) rc = GRASS_ENOMEM;
+        if (pinned[i].alloc(chunk) != hipSuccess) rc = GRASS_ENOMEM;
         else if (hipEventCreateWithFlags(&ev[i], hipEventDisableTiming) != hipSuccess)
             rc = GRASS_EDEVICE;
+        pin[i] = pinned[i].p;
     }
     uint64_t off = 0;
     int slot = 0;
@@ -287,10 +289,8 @@ int stage_to_device(ByteSource& src, char* dst, hipStream_t stream, uint64_t* ta
     }
     if (tail) *tail = std::min<uint64_t>(tail_len, total);
     if (hipStreamSynchronize(stream) != hipSuccess && rc == GRASS_OK) rc = GRASS_EDEVICE;
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < 2; ++i)
         if (ev[i]) (void)hipEventDestroy(ev[i]);
-        if (pin[i]) (void)hipHostFree(pin[i]);
-    }
     return rc;
 }
 
@@ -319,29 +319,41 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
     hipStream_t s = g->stream;
     const uint64_t gwords = (gbytes + 3) / 4 + kPadWords;
     const uint64_t owords = (obytes + 3) / 4 + kPadWords;
-    uint32_t* d_off = nullptr;
-    if (hipMalloc(&g->d_words, gwords * 4) != hipSuccess) return GRASS_ENOMEM;
-    if (hipMalloc(&d_off, owords * 4) != hipSuccess) return GRASS_ENOMEM;
+    // The GT .graph words, the .offset words, the record starts and the scan's and the validator's
+    // totals are used here only; the graph points at the first and third while it is being built.
+    WorkMem m_words, m_off, m_start, m_tmp;
+    struct Detach {
+        grass_graph* g;
+        ~Detach() {
+            if (g->fmt == kGT) g->d_words = nullptr;
+            g->d_start = nullptr;
+        }
+    } detach{g};
+    if (g->fmt == kGT) {
+        if (m_words.alloc(gwords * 4, s) != hipSuccess) return GRASS_ENOMEM;
+        g->d_words = m_words.as<uint32_t>();
+    } else if (device_malloc((void**)&g->d_words, gwords * 4) != hipSuccess) {
+        return GRASS_ENOMEM;
+    }
+    if (m_off.alloc(owords * 4, s) != hipSuccess) return GRASS_ENOMEM;
+    uint32_t* d_off = m_off.as<uint32_t>();
     int rc = GRASS_OK;
-    auto fail = [&](int code) {
-        (void)hipFree(d_off);
-        return code;
-    };
-    if (hipMemsetAsync(g->d_words, 0, gwords * 4, s) != hipSuccess ||
-        hipMemsetAsync(d_off, 0, owords * 4, s) != hipSuccess)
-        return fail(GRASS_EDEVICE);
+    // zero from the files' last partial words on (the images are copied over the start of them)
+    if (hipMemsetAsync(g->d_words + gbytes / 4, 0, (gwords - gbytes / 4) * 4, s) != hipSuccess ||
+        hipMemsetAsync(d_off + obytes / 4, 0, (owords - obytes / 4) * 4, s) != hipSuccess)
+        return GRASS_EDEVICE;
     rc = stage_to_device(gsrc, (char*)g->d_words, s, nullptr, 0, nullptr);
-    if (rc) return fail(rc);
+    if (rc) return rc;
     uint8_t tailb[64];
     uint64_t tlen = 0;
     rc = stage_to_device(osrc, (char*)d_off, s, &tlen, sizeof(tailb), tailb);
-    if (rc) return fail(rc);
+    if (rc) return rc;
 
     // ubl = byte 0 of .offset; n = floor(8 (bytes - 1) / ubl) (LE/src/grass.cu:1071,1088),
     // minus trailing zero-length fields, which can only be padding (a record is >= 1 bit).
     uint8_t ubl = 0;
-    if (hipMemcpy(&ubl, d_off, 1, hipMemcpyDeviceToHost) != hipSuccess) return fail(GRASS_EDEVICE);
-    if (ubl == 0 || ubl > 64) return fail(GRASS_EFORMAT);
+    if (hipMemcpy(&ubl, d_off, 1, hipMemcpyDeviceToHost) != hipSuccess) return GRASS_EDEVICE;
+    if (ubl == 0 || ubl > 64) return GRASS_EFORMAT;
     uint64_t n = ((obytes - 1) * 8) / ubl;
     uint64_t tail_fields_max = std::min<uint64_t>(n, 7);
     for (uint64_t t = 0; t < tail_fields_max && n > 0; ++t) {
@@ -349,7 +361,7 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
         if (host_field(tailb, tlen, obytes, n - 1, ubl) != 0) break;
         --n;
     }
-    if (n == 0 || n >= 0x80000000ull) return fail(GRASS_EFORMAT);
+    if (n == 0 || n >= 0x80000000ull) return GRASS_EFORMAT;
     g->n = n;
     g->ubl = ubl;
     g->graph_bytes = gbytes;
@@ -359,13 +371,14 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
     hipLaunchKernelGGL(bswap_words_kernel, dim3(bsg), dim3(256), 0, s, g->d_words, gwords);
     hipLaunchKernelGGL(bswap_words_kernel, dim3(bsg), dim3(256), 0, s, d_off, owords);
 
-    if (hipMalloc(&g->d_start, (n + 1) * 8) != hipSuccess) return fail(GRASS_ENOMEM);
-    if (hipMalloc(&g->d_deg, n * 4) != hipSuccess) return fail(GRASS_ENOMEM);
+    if (m_start.alloc((n + 1) * 8, s) != hipSuccess) return GRASS_ENOMEM;
+    g->d_start = m_start.as<uint64_t>();
+    if (device_malloc((void**)&g->d_deg, n * 4) != hipSuccess) return GRASS_ENOMEM;
     const uint64_t hdr_bytes = n * 16;
-    if (hipMalloc(&g->d_hdr, hdr_bytes) != hipSuccess) return fail(GRASS_ENOMEM);
+    if (device_malloc((void**)&g->d_hdr, hdr_bytes) != hipSuccess) return GRASS_ENOMEM;
     const uint64_t nb = scan_blocks(n);
-    uint64_t* d_tmp = nullptr;  // partials[nb], total, stats[4]
-    if (hipMalloc(&d_tmp, (nb + 8) * 8) != hipSuccess) return fail(GRASS_ENOMEM);
+    if (m_tmp.alloc((nb + 8) * 8, s) != hipSuccess) return GRASS_ENOMEM;
+    uint64_t* d_tmp = m_tmp.as<uint64_t>();  // partials[nb], total, stats[4]
     uint64_t* d_total = d_tmp + nb;
     unsigned long long* d_stats = (unsigned long long*)(d_tmp + nb + 2);
     unsigned long long init[4] = {0, 0, 0, ~0ull};
@@ -388,8 +401,6 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
     if (e == hipSuccess) e = hipMemcpyAsync(&total, d_total, 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipMemcpyAsync(stats, d_stats, sizeof(stats), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(d_tmp);
-    (void)hipFree(d_off);
     if (e != hipSuccess) return status_of(e);
     // records must cover the .graph bits up to < 8 bits of final padding
     if (total > 8 * gbytes || 8 * gbytes - total >= 8) return GRASS_EFORMAT;
@@ -405,12 +416,6 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
     // What stays resident is what the kernels read: the payload words (LE: the .graph image; GT:
     // the payload stream, which replaces the image), the header cache and the degrees.  The record
     // starts are folded into the header cache.
-    (void)hipFree(g->d_start);
-    g->d_start = nullptr;
-    if (g->fmt == kGT) {
-        (void)hipFree(g->d_words);
-        g->d_words = nullptr;
-    }
     g->device_bytes = (g->fmt == kGT ? xwords : gwords) * 4 + n * 4 + hdr_bytes;
     return GRASS_OK;
 }
@@ -419,8 +424,9 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
 int build_gt_stream(grass_graph* g, uint64_t* words) {
     hipStream_t s = g->stream;
     const uint64_t n = g->n, nb = scan_blocks(n);
-    uint64_t* d_woff = nullptr;  // n + 1 word offsets, partials, total
-    if (hipMalloc(&d_woff, (n + 1 + nb + 2) * 8) != hipSuccess) return GRASS_ENOMEM;
+    WorkMem m_woff;  // n + 1 word offsets, partials, total
+    if (m_woff.alloc((n + 1 + nb + 2) * 8, s) != hipSuccess) return GRASS_ENOMEM;
+    uint64_t* d_woff = m_woff.as<uint64_t>();
     hipError_t e = exclusive_scan(GtxWordsGen{g->d_hdr, g->cp_shift}, Count{n, nullptr}, n, d_woff,
                                   d_woff + n + 1, d_woff + n + 1 + nb, s);
     uint64_t total = 0;
@@ -430,9 +436,9 @@ int build_gt_stream(grass_graph* g, uint64_t* words) {
     int rc = status_of(e);
     // payload bits must fit the header cache
     if (!rc && 32 * total >= kMaxPayloadBits) rc = GRASS_EFORMAT;
-    if (!rc && hipMalloc(&out, (total + kPadWords) * 4) != hipSuccess) rc = GRASS_ENOMEM;
+    if (!rc && device_malloc((void**)&out, (total + kPadWords) * 4) != hipSuccess) rc = GRASS_ENOMEM;
     if (!rc) {
-        e = hipMemsetAsync(out, 0, (total + kPadWords) * 4, s);
+        e = hipMemsetAsync(out + total, 0, kPadWords * 4, s);  // every word before is stored below
         if (e == hipSuccess) {
             // g->dev() still decodes .graph here: d_gtx is set once the stream is complete
             hipLaunchKernelGGL(gt_expand_kernel, dim3(4096), dim3(kExpBlock), 0, s, g->dev(),
@@ -442,7 +448,6 @@ int build_gt_stream(grass_graph* g, uint64_t* words) {
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         rc = status_of(e);
     }
-    (void)hipFree(d_woff);
     if (rc) {
         if (out) (void)hipFree(out);
         return rc;

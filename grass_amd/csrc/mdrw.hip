@@ -836,7 +836,7 @@ struct MdrwState {
     uint64_t tot_steps = 0, tot_init = 0, tot_vb = 0;
     uint32_t mmax = 1, vmax = 1;
     uint64_t NS = 0, NV = 0, NC = 0, NI = 0;  // steps, sampled vertices, list chunks, induced edges
-    DevMem tmp, tmp2, tmp3;
+    WorkMem tmp, tmp2, tmp3;
     grass_mdrw_result* res = nullptr;
     ~MdrwState() {
         if (res) res->release();
@@ -908,7 +908,7 @@ static int mdrw_run(grass_graph* g, MdrwState& st, hipStream_t s, bool replay) {
     if (!replay) {
         Carve need(nullptr);
         plan1(need);
-        if (st.tmp.alloc(need.off + 256) != hipSuccess) return GRASS_ENOMEM;
+        if (st.tmp.alloc(need.off + 256, s) != hipSuccess) return GRASS_ENOMEM;
     }
     Carve c(st.tmp.p);
     MdDesc* d_desc = c.take<MdDesc>(I);
@@ -1000,7 +1000,7 @@ static int mdrw_run(grass_graph* g, MdrwState& st, hipStream_t s, bool replay) {
 
     // phase 2: chunks of the sampled vertices' lists
     const uint64_t nbV = scan_blocks(NV);
-    if (!replay && st.tmp2.alloc((NV + 1) * 8 + (nbV + 2) * 8 + 512) != hipSuccess) return GRASS_ENOMEM;
+    if (!replay && st.tmp2.alloc((NV + 1) * 8 + (nbV + 2) * 8 + 512, s) != hipSuccess) return GRASS_ENOMEM;
     Carve c2(st.tmp2.p);
     uint64_t* d_coff = c2.take<uint64_t>(NV + 1);
     uint64_t* d_part2 = c2.take<uint64_t>(nbV + 2);
@@ -1045,7 +1045,7 @@ static int mdrw_run(grass_graph* g, MdrwState& st, hipStream_t s, bool replay) {
     if (!replay) {
         Carve need3(nullptr);
         plan3(need3);
-        if (st.tmp3.alloc(need3.off + 256) != hipSuccess) return GRASS_ENOMEM;
+        if (st.tmp3.alloc(need3.off + 256, s) != hipSuccess) return GRASS_ENOMEM;
     }
     Carve c3(st.tmp3.p);
     plan3(c3);
@@ -1158,6 +1158,8 @@ int mdrw_capture_prepare(grass_graph* g, const grass_mdrw_request* reqs, uint32_
     int rc = mdrw_prepare(reqs, I, target, seed, c->st);
     if (!rc) rc = mdrw_run(g, c->st, s, false);
     if (rc) return rc;
+    // the plan is replayed on any stream, and its own streams go before this state does
+    c->st.tmp.whole_device = c->st.tmp2.whole_device = c->st.tmp3.whole_device = true;
     *out = c.release();
     return GRASS_OK;
 }

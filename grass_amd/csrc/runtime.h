@@ -12,6 +12,9 @@
 
 namespace grass {
 
+// hipMalloc that frees the idle working memory kept between calls (pool.cpp) before it fails.
+hipError_t device_malloc(void** p, size_t bytes);
+
 // Device scratch that grows on demand and is reused across calls (no per-call hipMalloc in
 // steady state).  Guarded by the owning graph's mutex.
 struct Scratch {
@@ -26,7 +29,7 @@ struct Scratch {
             bytes = 0;
         }
         size_t cap = need + need / 4 + (1u << 20);
-        hipError_t e = hipMalloc(&ptr, cap);
+        hipError_t e = device_malloc(&ptr, cap);
         if (e == hipSuccess) bytes = cap;
         return e;
     }
@@ -60,6 +63,36 @@ struct PinnedBuf {
     }
 };
 
+// A call's device working memory on the current device, used on one stream: taken from, and returned
+// to, the blocks kept between calls.  Returning it waits for that stream.
+struct WorkMem {
+    void* p = nullptr;
+    size_t bytes = 0;
+    int dev = 0;
+    hipStream_t s = nullptr;
+    bool whole_device = false;  // used on streams that may be gone by then: wait for the device instead
+    WorkMem() = default;
+    WorkMem(const WorkMem&) = delete;
+    WorkMem& operator=(const WorkMem&) = delete;
+    ~WorkMem() { reset(); }
+    hipError_t alloc(size_t need, hipStream_t stream);
+    void reset();
+    template <typename T>
+    T* as() const { return (T*)p; }
+};
+
+// The same for pinned host memory: return it only when no copy to or from it is in flight.
+struct PinnedWork {
+    void* p = nullptr;
+    size_t bytes = 0;
+    PinnedWork() = default;
+    PinnedWork(const PinnedWork&) = delete;
+    PinnedWork& operator=(const PinnedWork&) = delete;
+    ~PinnedWork() { reset(); }
+    hipError_t alloc(size_t need);
+    void reset();
+};
+
 // An owned device allocation, freed with its owner.
 struct DevMem {
     void* p = nullptr;
@@ -69,7 +102,7 @@ struct DevMem {
     ~DevMem() {
         if (p) (void)hipFree(p);
     }
-    hipError_t alloc(size_t bytes) { return hipMalloc(&p, bytes > 256 ? bytes : 256); }
+    hipError_t alloc(size_t bytes) { return device_malloc(&p, bytes > 256 ? bytes : 256); }
     void reset() {
         if (p) (void)hipFree(p);
         p = nullptr;
