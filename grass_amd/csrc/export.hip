@@ -4,14 +4,16 @@
 // k-hop blocks.  Request r's sequence is its seeds, then its hop-0 destinations, its hop-1
 // destinations, ...; the sequences of all requests are laid end to end (request-major, starts
 // Q[r]) so that one position space covers the batch.
-//   1. rel_len_kernel + scan: Q.
-//   2. rel_insert_kernel: every position p inserts the key (r, vertex) into a hash table and
-//      atomicMins p into the key's slot -- the slot ends up holding the first appearance.
-//   3. rel_mark_kernel: flag[p] = p is its key's first appearance; a scan of the flags gives F,
-//      and the local id of the vertex at p is F[first(p)] - F[Q[r]].
-//   4. rel_emit_kernel: writes each first appearance to nodes[F[p]] and the local ids of every
+//   1. rel_prepare_kernel (or, for very many requests, a few kernels and a scan): checks the batch's
+//      offsets and fills Q, while other workgroups clear the table.
+//   2. rel_insert_kernel: every position p inserts the key (r, vertex) into a hash table that keeps
+//      the key's smallest position, and p stays on the list of first appearances (firsts.h) or takes
+//      a larger one off it.  A scan of the list's words numbers the first appearances: the local id
+//      of the vertex whose first position is f is rank(f) - rank(Q[r]).
+//   3. rel_emit_kernel: writes each first appearance to nodes[rank(p)] and the local ids of every
 //      batch edge (its destination is a position, its source a key looked up in the table).
 // Every step is a data-parallel pass over the positions; the result does not depend on timing.
+// Bound by the table's random atomics and loads.  REL_FIGURES
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -21,6 +23,7 @@
 
 #include "../../include/grass_export.h"
 #include "devutil.h"
+#include "firsts.h"
 #include "runtime.h"
 #include "scan.h"
 
@@ -36,17 +39,6 @@ struct RelReq {
     uint64_t num;
     uint32_t hops;
 };
-
-// Largest r in [0, R) with Q[r] <= p (Q ascending).
-__device__ __forceinline__ uint32_t req_of(const uint64_t* __restrict__ Q, uint32_t R, uint64_t p) {
-    uint32_t lo = 0, hi = R - 1;
-    while (lo < hi) {
-        const uint32_t mid = lo + (hi - lo + 1) / 2;
-        if (Q[mid] <= p) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
 
 // Open-addressing tables from (request r, vertex v) to the first position of v in r's sequence.
 // Both have the same interface; the kernels below take either.  Linear probing from a
@@ -69,7 +61,8 @@ struct RelTab16 {
     __device__ __forceinline__ void clear(uint64_t i) const {
         reinterpret_cast<ulonglong2*>(slot)[i] = make_ulonglong2(0ull, ~0ull);
     }
-    __device__ __forceinline__ void insert(uint32_t r, uint32_t v, uint64_t p, uint32_t* err) const {
+    // Whether p is its key's smallest position so far; the position it displaces is taken off `words`.
+    __device__ __forceinline__ bool insert(uint32_t r, uint32_t v, uint64_t p, FirstWord* words, uint32_t* err) const {
         const unsigned long long k = key(r, v);
         uint64_t h = home(k);
         for (uint64_t probes = 0; probes <= mask; ++probes) {
@@ -80,12 +73,16 @@ struct RelTab16 {
             }
             if (cur == k) {
                 // read first: a repeat after the first occurrence needs no atomic
-                if (__atomic_load_n(kp(h) + 1, __ATOMIC_RELAXED) > p) atomicMin(kp(h) + 1, (unsigned long long)p);
-                return;
+                if (__atomic_load_n(kp(h) + 1, __ATOMIC_RELAXED) < p) return false;
+                const unsigned long long old = atomicMin(kp(h) + 1, (unsigned long long)p);
+                if (old < p) return false;
+                if (old != ~0ull) not_first(words, old);
+                return true;
             }
             h = (h + 1) & mask;
         }
         atomicOr(err, 1u);  // cannot happen: slots > positions
+        return false;
     }
     // First position of v in request r; ~0 when absent.
     __device__ __forceinline__ uint64_t first(uint32_t r, uint32_t v) const {
@@ -113,10 +110,10 @@ struct RelTab8 {
         return (((k + 1) * 0x9E3779B97F4A7C15ull) >> shift) & mask;
     }
     __device__ __forceinline__ void clear(uint64_t i) const { slot[i] = ~0ull; }
-    __device__ __forceinline__ void insert(uint32_t r, uint32_t v, uint64_t p, uint32_t* err) const {
+    __device__ __forceinline__ bool insert(uint32_t r, uint32_t v, uint64_t p, FirstWord* words, uint32_t* err) const {
         if (vb < 32 && (v >> vb) != 0) {  // not a vertex of the graph
             atomicOr(err, 1u);
-            return;
+            return false;
         }
         const unsigned long long k = ((unsigned long long)r << vb) | v;
         const unsigned long long w = (k << pb) | p;
@@ -125,15 +122,19 @@ struct RelTab8 {
             unsigned long long cur = __atomic_load_n(slot + h, __ATOMIC_RELAXED);
             if (cur == ~0ull) {
                 cur = atomicCAS(slot + h, ~0ull, w);
-                if (cur == ~0ull) return;
+                if (cur == ~0ull) return true;
             }
             if ((cur >> pb) == k) {
-                if (cur > w) atomicMin(slot + h, w);
-                return;
+                if (cur < w) return false;
+                const unsigned long long old = atomicMin(slot + h, w);
+                if (old < w) return false;
+                not_first(words, old & ((1ull << pb) - 1));
+                return true;
             }
             h = (h + 1) & mask;
         }
         atomicOr(err, 1u);  // cannot happen: slots > positions
+        return false;
     }
     __device__ __forceinline__ uint64_t first(uint32_t r, uint32_t v) const {
         if (vb < 32 && (v >> vb) != 0) return ~0ull;
@@ -149,13 +150,6 @@ struct RelTab8 {
     }
 };
 
-template <class Tab>
-__global__ void rel_clear_kernel(Tab t) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i <= t.mask;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        t.clear(i);
-}
-
 // The batch as one position space.  Every offset row has been checked (rel_check_kernel) to be
 // ascending and to end at or below the batch total before any pass reads through it, so every
 // edge index e below is < total.
@@ -167,9 +161,8 @@ struct RelSeq {
     const uint64_t* Q;  // R + 1 request starts
     uint32_t R, H;
     uint32_t n;  // vertices of the graph: an id >= n is not a vertex
-    // Vertex at position p < Q[R]; r = its request, e = its batch edge (~0 for a seed).
-    __device__ __forceinline__ uint32_t at(uint64_t p, uint32_t& r, uint64_t& e) const {
-        r = req_of(Q, R, p);
+    // Vertex at position p of request r; e = its batch edge (~0 for a seed).
+    __device__ __forceinline__ uint32_t at(uint64_t p, uint32_t r, uint64_t& e) const {
         uint64_t j = p - Q[r];
         const RelReq q = req[r];
         e = ~0ull;
@@ -192,32 +185,42 @@ struct RelSeq {
 // ascending and ending at or below `total`, no edges of request r at hops >= its hop count, and
 // the sequence lengths summing to P.  Any failure sets *invalid, and the passes then touch
 // nothing.
-__global__ void rel_check_kernel(const uint64_t* __restrict__ off, const RelReq* __restrict__ req,
-                                 uint32_t R, uint32_t H, uint64_t total, uint32_t* invalid) {
+__device__ __forceinline__ bool rel_check(const uint64_t* __restrict__ off, const RelReq* __restrict__ req, uint32_t R,
+                                          uint32_t H, uint64_t total, uint64_t t, uint64_t threads) {
     const uint64_t cells = (uint64_t)H * (R + 1);
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cells;
-         i += (uint64_t)gridDim.x * blockDim.x) {
+    bool ok = true;
+    for (uint64_t i = t; i < cells; i += threads) {
         const uint32_t h = (uint32_t)(i / (R + 1)), r = (uint32_t)(i % (R + 1));
         const uint64_t a = off[i];
-        bool ok = a <= total;
+        ok = ok && a <= total;
         if (r < R) {
             const uint64_t b = off[i + 1];
             ok = ok && a <= b && (h < req[r].hops || a == b);
         }
-        if (!ok) atomicOr(invalid, 1u);
     }
+    return ok;
 }
 
-// Sequence lengths: seeds plus the request's edges at every hop (only after rel_check_kernel).
+// Length of request r's sequence: its seeds and its edges at every hop (only after the check).
+__device__ __forceinline__ uint64_t rel_length(const RelReq* __restrict__ req, const uint64_t* __restrict__ off,
+                                               uint32_t R, uint32_t H, uint32_t r) {
+    uint64_t L = req[r].num;
+    for (uint32_t h = 0; h < H; ++h) L += off[(uint64_t)h * (R + 1) + r + 1] - off[(uint64_t)h * (R + 1) + r];
+    return L;
+}
+
+__global__ void rel_check_kernel(const uint64_t* __restrict__ off, const RelReq* __restrict__ req,
+                                 uint32_t R, uint32_t H, uint64_t total, uint32_t* invalid) {
+    if (!rel_check(off, req, R, H, total, (uint64_t)blockIdx.x * blockDim.x + threadIdx.x,
+                   (uint64_t)gridDim.x * blockDim.x))
+        atomicOr(invalid, 1u);
+}
+
 __global__ void rel_len_kernel(const RelReq* __restrict__ req, const uint64_t* __restrict__ off, uint32_t R,
                                uint32_t H, const uint32_t* __restrict__ invalid, uint64_t* __restrict__ len) {
-    const bool bad = *invalid != 0;
-    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < R; r += gridDim.x * blockDim.x) {
-        uint64_t L = req[r].num;
-        if (!bad)
-            for (uint32_t h = 0; h < H; ++h) L += off[(uint64_t)h * (R + 1) + r + 1] - off[(uint64_t)h * (R + 1) + r];
-        len[r] = L;
-    }
+    const uint32_t hops = *invalid ? 0 : H;
+    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < R; r += gridDim.x * blockDim.x)
+        len[r] = rel_length(req, off, R, hops, r);
 }
 
 // The sequence total must be the seeds plus the batch's edges: rows of different hops that
@@ -231,94 +234,145 @@ struct LenGen {
     __device__ __forceinline__ uint64_t operator()(uint64_t i) const { return len[i]; }
 };
 
+// The table's slots emptied and every position a first appearance.
 template <class Tab>
-__global__ __launch_bounds__(kExBlock) void rel_insert_kernel(RelSeq q, uint64_t P, Tab t,
+__device__ __forceinline__ void rel_clear(const Tab& t, FirstWord* words, uint64_t nwords, uint64_t i0, uint64_t threads) {
+    for (uint64_t i = i0; i < nwords; i += threads) words[i] = make_ulonglong2(~0ull, 0ull);
+    for (uint64_t i = i0; i <= t.mask; i += threads) t.clear(i);
+}
+
+template <class Tab>
+__global__ __launch_bounds__(1024) void rel_clear_kernel(Tab t, FirstWord* words, uint64_t nwords) {
+    rel_clear(t, words, nwords, (uint64_t)blockIdx.x * 1024 + threadIdx.x, (uint64_t)gridDim.x * 1024);
+}
+
+// Up to kPrepRequests requests: workgroup 0 checks the offsets, scans the lengths into Q and checks their
+// total, while the others clear the table (with one workgroup, it does both): one launch where the
+// steps by themselves are seven.
+constexpr uint32_t kPrepRequests = 8192;
+template <class Tab>
+__global__ __launch_bounds__(1024) void rel_prepare_kernel(Tab t, FirstWord* words, uint64_t nwords,
+                                                           const uint64_t* __restrict__ off,
+                                                           const RelReq* __restrict__ req, uint32_t R, uint32_t H,
+                                                           uint64_t total, uint64_t P, uint64_t* __restrict__ Q,
+                                                           uint32_t* bad, uint32_t* invalid) {
+    if (blockIdx.x || gridDim.x == 1)
+        rel_clear(t, words, nwords, (uint64_t)(gridDim.x == 1 ? 0 : blockIdx.x - 1) * 1024 + threadIdx.x,
+                  (uint64_t)(gridDim.x == 1 ? 1 : gridDim.x - 1) * 1024);
+    if (blockIdx.x) return;
+    __shared__ uint64_t lds[1024 / kWave];
+    const bool mine = H == 0 || rel_check(off, req, R, H, total, threadIdx.x, 1024);
+    const bool ok = block_sum<uint64_t, 1024>(mine ? 0 : 1, lds) == 0;
+    constexpr uint32_t kPer = kPrepRequests / 1024;
+    const uint32_t per = (R + 1023) / 1024, r0 = threadIdx.x * per;
+    uint64_t len[kPer], s = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+        len[i] = i < per && r0 + i < R ? rel_length(req, off, R, ok ? H : 0, r0 + i) : 0;
+        s += len[i];
+    }
+    uint64_t sum;
+    uint64_t pre = block_exclusive_sum<uint64_t, 1024>(s, sum, lds);
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+        if (i < per && r0 + i < R) Q[r0 + i] = pre;
+        pre += len[i];
+    }
+    if (threadIdx.x == 0) {
+        Q[R] = sum;
+        *bad = 0;
+        *invalid = ok && sum == P ? 0 : 1;
+    }
+}
+
+// One wave per 64 positions (a word of `words`).
+template <class Tab>
+__global__ __launch_bounds__(kExBlock) void rel_insert_kernel(RelSeq q, uint64_t P, Tab t, FirstWord* words,
                                                               const uint32_t* __restrict__ invalid, uint32_t* err) {
     if (*invalid) return;
-    for (uint64_t p = (uint64_t)blockIdx.x * kExBlock + threadIdx.x; p < P; p += (uint64_t)gridDim.x * kExBlock) {
-        uint32_t r;
-        uint64_t e;
-        const uint32_t v = q.at(p, r, e);
-        if (v >= q.n) {  // a seed or destination that is not a vertex of the graph
-            atomicOr(err, 1u);
-            continue;
+    const uint64_t nw = (uint64_t)gridDim.x * (kExBlock / kWave);
+    for (uint64_t w = readfirstlane_u64(((uint64_t)blockIdx.x * kExBlock + threadIdx.x) / kWave); w * kWave < P; w += nw) {
+        const uint64_t p = w * kWave + lane_id();
+        const uint32_t r = segment_of_lane(q.Q, q.R, w, P);
+        bool first = false;
+        if (p < P) {
+            uint64_t e;
+            const uint32_t v = q.at(p, r, e);
+            if (v < q.n) first = t.insert(r, v, p, words, err);
+            else atomicOr(err, 1u);  // a seed or destination that is not a vertex of the graph
         }
-        t.insert(r, v, p, err);
+        const unsigned long long keep = __ballot(first);
+        if (lane_id() == 0 && keep != ~0ull) atomicAnd(&words[w].x, keep);
     }
 }
-
-template <class Tab>
-__global__ __launch_bounds__(kExBlock) void rel_mark_kernel(RelSeq q, uint64_t P, Tab t,
-                                                            const uint32_t* __restrict__ invalid,
-                                                            uint32_t* __restrict__ flag) {
-    const bool bad = *invalid != 0;
-    for (uint64_t p = (uint64_t)blockIdx.x * kExBlock + threadIdx.x; p < P; p += (uint64_t)gridDim.x * kExBlock) {
-        uint32_t r;
-        uint64_t e;
-        if (bad) {
-            flag[p] = 0;
-            continue;
-        }
-        const uint32_t v = q.at(p, r, e);
-        flag[p] = v < q.n && t.first(r, v) == p;
-    }
-}
-
-struct FlagGen {
-    const uint32_t* flag;
-    __device__ __forceinline__ uint64_t operator()(uint64_t i) const { return flag[i]; }
-};
 
 template <class Tab>
 __global__ __launch_bounds__(kExBlock) void rel_emit_kernel(RelSeq q, uint64_t P, Tab t,
-                                                            const uint32_t* __restrict__ flag,
-                                                            const uint64_t* __restrict__ F,
+                                                            const FirstWord* __restrict__ words,
+                                                            const uint64_t* __restrict__ node_off,
                                                             uint32_t* __restrict__ nodes, uint64_t cap,
-                                                            uint32_t* __restrict__ lsrc,
-                                                            uint32_t* __restrict__ ldst,
+                                                            uint32_t* __restrict__ lsrc, uint32_t* __restrict__ ldst,
                                                             const uint32_t* __restrict__ invalid, uint32_t* err) {
     if (*invalid) return;
-    for (uint64_t p = (uint64_t)blockIdx.x * kExBlock + threadIdx.x; p < P; p += (uint64_t)gridDim.x * kExBlock) {
-        uint32_t r;
+    const uint64_t nw = (uint64_t)gridDim.x * (kExBlock / kWave);
+    for (uint64_t w = readfirstlane_u64(((uint64_t)blockIdx.x * kExBlock + threadIdx.x) / kWave); w * kWave < P; w += nw) {
+        const FirstWord fw = words[w];
+        const uint64_t p = w * kWave + lane_id();
+        const uint32_t r = segment_of_lane(q.Q, q.R, w, P);
+        if (p >= P) continue;
         uint64_t e;
         const uint32_t v = q.at(p, r, e);
-        if (flag[p] && F[p] < cap) nodes[F[p]] = v;
+        const bool first = (fw.x >> lane_id()) & 1;
+        const uint64_t mine = fw.y + lanes_below(fw.x);
+        if (first && mine < cap) nodes[mine] = v;
         if (e == ~0ull) continue;
-        const uint64_t base = F[q.Q[r]];
-        const uint64_t fd = flag[p] ? p : v < q.n ? t.first(r, v) : ~0ull;
+        const uint64_t base = node_off[r];
+        const uint64_t fd = first ? p : v < q.n ? t.first(r, v) : ~0ull;
         const uint64_t fs = t.first(r, q.src[e]);
         if (fd >= P || fs >= P) {  // a source that is neither a seed nor an earlier destination
             atomicOr(err, 1u);
             ldst[e] = lsrc[e] = kNoId;
             continue;
         }
-        ldst[e] = (uint32_t)(F[fd] - base);
-        lsrc[e] = (uint32_t)(F[fs] - base);
+        ldst[e] = (uint32_t)((first ? mine : first_rank(words, fd)) - base);
+        lsrc[e] = (uint32_t)(first_rank(words, fs) - base);
     }
 }
 
-__global__ void rel_node_off_kernel(const uint64_t* __restrict__ Q, const uint64_t* __restrict__ F, uint32_t R,
-                                    uint64_t* __restrict__ node_off) {
-    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r <= R; r += gridDim.x * blockDim.x) node_off[r] = F[Q[r]];
-}
-
-// Clears the table, inserts every position, marks the first appearances, numbers them (scan) and
+// Fills Q and clears the table, inserts every position, numbers the first appearances (scan) and
 // writes the sampled vertices and the local ids of every edge.
 template <class Tab>
-hipError_t rel_build(const Tab& t, const RelSeq& q, uint64_t P, uint32_t* d_flag, uint64_t* d_F, uint64_t* d_part,
-                     uint64_t* d_total, const uint32_t* d_invalid, uint32_t* d_bad, grass_khop_blocks* out,
+hipError_t rel_build(const Tab& t, const RelSeq& q, uint64_t P, uint64_t* d_len, FirstWord* d_words, uint64_t* d_part,
+                     uint64_t* d_sc, uint32_t* d_bad, const grass_khop_output* b, grass_khop_blocks* out,
                      hipStream_t s) {
-    const unsigned gP = (unsigned)std::min<uint64_t>((P + kExBlock - 1) / kExBlock + 1, kExGrid);
-    hipLaunchKernelGGL(rel_clear_kernel<Tab>, dim3(kExGrid), dim3(256), 0, s, t);
-    if (P) {
-        hipLaunchKernelGGL(rel_insert_kernel<Tab>, dim3(gP), dim3(kExBlock), 0, s, q, P, t, d_invalid, d_bad);
-        hipLaunchKernelGGL(rel_mark_kernel<Tab>, dim3(gP), dim3(kExBlock), 0, s, q, P, t, d_invalid, d_flag);
+    uint32_t* d_invalid = d_bad + 1;
+    uint64_t* Q = const_cast<uint64_t*>(q.Q);
+    const uint64_t nwords = firsts_words(P);
+    const unsigned gC = 1 + (unsigned)std::min<uint64_t>((t.mask + 1) / 2048, 2048);
+    if (q.R <= kPrepRequests) {
+        hipLaunchKernelGGL(rel_prepare_kernel<Tab>, dim3(gC), dim3(1024), 0, s, t, d_words, nwords, q.off, q.req, q.R,
+                           q.H, b->total, P, Q, d_bad, d_invalid);
+    } else {
+        hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(1), dim3(64), 0, s, d_bad, (uint64_t)2, 0u);
+        const unsigned gR = (unsigned)std::min<uint64_t>((q.R + 255) / 256 + 1, 1024);
+        if (q.H) hipLaunchKernelGGL(rel_check_kernel, dim3(1024), dim3(256), 0, s, q.off, q.req, q.R, q.H, b->total, d_invalid);
+        hipLaunchKernelGGL(rel_len_kernel, dim3(gR), dim3(256), 0, s, q.req, q.off, q.R, q.H, (const uint32_t*)d_invalid,
+                           d_len);
+        hipError_t e = exclusive_scan(LenGen{d_len}, Count{q.R, nullptr}, q.R, Q, d_part, d_sc, s);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(rel_total_kernel, dim3(1), dim3(64), 0, s, q.Q, q.R, P, d_invalid);
+        hipLaunchKernelGGL(rel_clear_kernel<Tab>, dim3(gC), dim3(1024), 0, s, t, d_words, nwords);
     }
-    hipError_t e = exclusive_scan(FlagGen{d_flag}, Count{P, nullptr}, P, d_F, d_part, d_total, s);
+    const unsigned gP = (unsigned)std::min<uint64_t>((P + kExBlock - 1) / kExBlock + 1, kExGrid);
+    if (P)
+        hipLaunchKernelGGL(rel_insert_kernel<Tab>, dim3(gP), dim3(kExBlock), 0, s, q, P, t, d_words,
+                           (const uint32_t*)d_invalid, d_bad);
+    // node_off[r] = first appearances before request r; their total beside the other results
+    hipError_t e = scan_firsts(d_words, Count{P, nullptr}, P, q.Q, q.R, out->node_off_dev, d_sc + 1, d_part, d_sc, s);
     if (e != hipSuccess || !P) return e;
-    hipLaunchKernelGGL(rel_emit_kernel<Tab>, dim3(gP), dim3(kExBlock), 0, s, q, P, t, (const uint32_t*)d_flag,
-                       (const uint64_t*)d_F, out->nodes_dev, out->node_capacity, out->lsrc_dev, out->ldst_dev,
-                       d_invalid, d_bad);
+    hipLaunchKernelGGL(rel_emit_kernel<Tab>, dim3(gP), dim3(kExBlock), 0, s, q, P, t, (const FirstWord*)d_words,
+                       (const uint64_t*)out->node_off_dev, out->nodes_dev, out->node_capacity, out->lsrc_dev,
+                       out->ldst_dev, (const uint32_t*)d_invalid, d_bad);
     return hipGetLastError();
 }
 
@@ -343,9 +397,9 @@ int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, cons
     if (P && (!out->nodes_dev && out->node_capacity)) return GRASS_EINVAL;
     uint64_t slots = 1024;
     while (slots < P + P / 2 + 2) slots <<= 1;  // load <= 2/3: distinct keys <= positions
-    const uint64_t nb = scan_blocks(std::max<uint64_t>(std::max<uint64_t>(P, R), 1));
+    const uint64_t nb = scan_blocks(std::max<uint64_t>(firsts_words(P), R));
     const size_t need = Carve::need(R * sizeof(RelReq)) + Carve::need(R * 8) + Carve::need((R + 1) * 8) +
-                        Carve::need(P * 4 + 4) + Carve::need((P + 1) * 8) + Carve::need((nb + 2) * 8) +
+                        Carve::need(firsts_words(P) * sizeof(FirstWord)) + Carve::need((nb + 2) * 8) +
                         Carve::need(64);
     // Packed 8-byte slots when the request, vertex and position bits fit one word; 16-byte slots
     // otherwise, or when GRASS_EXPORT_SLOT=16 asks for them.
@@ -366,53 +420,35 @@ int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, cons
     RelReq* d_req = cv.take<RelReq>(R);
     uint64_t* d_len = cv.take<uint64_t>(R);
     uint64_t* d_Q = cv.take<uint64_t>(R + 1);
-    uint32_t* d_flag = cv.take<uint32_t>(P + 1);
-    uint64_t* d_F = cv.take<uint64_t>(P + 1);
+    FirstWord* d_words = cv.take<FirstWord>(firsts_words(P));
     uint64_t* d_part = cv.take<uint64_t>(nb + 2);
-    uint64_t* d_sc = cv.take<uint64_t>(8);  // [0] sequence total, [1] node total, [2] error flags
+    uint64_t* d_sc = cv.take<uint64_t>(8);  // [0] scratch total, [1] node total, [2] error flags
     const uint32_t lg = (uint32_t)__builtin_ctzll(slots);
 
-    hipError_t e = hipMemcpyAsync(d_req, hreq, R * sizeof(RelReq), hipMemcpyHostToDevice, s);
+    hipError_t e = hipSuccess;
+    if (R) e = hipMemcpyAsync(d_req, hreq, R * sizeof(RelReq), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return status_of(e);
-    // the two halves of d_sc[2]: read back together below
-    uint32_t* d_bad = (uint32_t*)(d_sc + 2);  // an id that is not a vertex, or an unknown source
-    uint32_t* d_invalid = d_bad + 1;          // offsets that do not fit the requests
-    hipLaunchKernelGGL(fill_kernel<uint32_t>, dim3(1), dim3(64), 0, s, d_bad, (uint64_t)2, 0u);
-    const unsigned gR = (unsigned)std::min<uint64_t>((R + 255) / 256 + 1, 1024);
-    if (H) {
-        const uint64_t cells = (uint64_t)H * (R + 1);
-        const unsigned gC = (unsigned)std::min<uint64_t>((cells + 255) / 256, 1024);
-        hipLaunchKernelGGL(rel_check_kernel, dim3(gC), dim3(256), 0, s, (const uint64_t*)b->offsets_dev,
-                           (const RelReq*)d_req, R, H, b->total, d_invalid);
-    }
-    hipLaunchKernelGGL(rel_len_kernel, dim3(gR), dim3(256), 0, s, (const RelReq*)d_req,
-                       (const uint64_t*)b->offsets_dev, R, H, (const uint32_t*)d_invalid, d_len);
-    e = exclusive_scan(LenGen{d_len}, Count{R, nullptr}, R, d_Q, d_part, d_sc, s);
-    if (e != hipSuccess) return status_of(e);
-    hipLaunchKernelGGL(rel_total_kernel, dim3(1), dim3(64), 0, s, (const uint64_t*)d_Q, R, P, d_invalid);
+    // the two halves of d_sc[2]: an id that is not a vertex, or an unknown source; and offsets that
+    // do not fit the requests
+    uint32_t* d_bad = (uint32_t*)(d_sc + 2);
     RelSeq q{d_req, b->offsets_dev, b->src_dev, b->dst_dev, d_Q, R, H, (uint32_t)g->n};
     if (wide) {
         RelTab16 t{(unsigned long long*)ws.ht.ptr, slots - 1, 64 - lg};
-        e = rel_build(t, q, P, d_flag, d_F, d_part, d_sc + 1, d_invalid, d_bad, out, s);
+        e = rel_build(t, q, P, d_len, d_words, d_part, d_sc, d_bad, b, out, s);
     } else {
         RelTab8 t{(unsigned long long*)ws.ht.ptr, slots - 1, 64 - lg, vb, pb};
-        e = rel_build(t, q, P, d_flag, d_F, d_part, d_sc + 1, d_invalid, d_bad, out, s);
+        e = rel_build(t, q, P, d_len, d_words, d_part, d_sc, d_bad, b, out, s);
     }
     if (e != hipSuccess) return status_of(e);
-    hipLaunchKernelGGL(rel_node_off_kernel, dim3(gR), dim3(256), 0, s, (const uint64_t*)d_Q, (const uint64_t*)d_F, R,
-                       out->node_off_dev);
     uint64_t* hres = ws.result_slot();
-    hres[2] = 0;
-    e = hipMemcpyAsync(hres, d_Q + R, 8, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(hres + 1, d_F + P, 8, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(hres + 2, d_bad, 8, hipMemcpyDeviceToHost, s);
+    e = hipMemcpyAsync(hres, d_sc + 1, 16, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return status_of(e);
     // the offsets are not the batch of these requests (rows out of order or past the total, edges
     // at hops a request does not have, sizes that differ), an id is not a vertex, or an edge's
     // source is not among the request's earlier vertices
-    if (hres[0] != P || hres[2] != 0) return GRASS_EINVAL;
-    out->nodes = hres[1];
+    if (hres[1] != 0) return GRASS_EINVAL;
+    out->nodes = hres[0];
     return out->nodes > out->node_capacity ? GRASS_ECAPACITY : GRASS_OK;
 }
 
@@ -437,7 +473,7 @@ __global__ __launch_bounds__(kExBlock) void mdrw_local_kernel(const uint64_t* __
                                                               uint32_t* __restrict__ lsrc,
                                                               uint32_t* __restrict__ ldst) {
     for (uint64_t e = (uint64_t)blockIdx.x * kExBlock + threadIdx.x; e < E; e += (uint64_t)gridDim.x * kExBlock) {
-        const uint32_t i = req_of(eoff, I, e);
+        const uint32_t i = segment_in(eoff, 0, I - 1, e);
         const uint32_t* V = verts + voff[i];
         const uint64_t nv = voff[i + 1] - voff[i];
         lsrc[e] = rank_in(V, nv, esrc[e]);

@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "devutil.h"
+#include "firsts.h"
 #include "philox.h"
 #include "runtime.h"
 #include "scan.h"
@@ -41,17 +42,6 @@ struct KhReq {
     uint32_t hops;
     uint32_t fan[GRASS_KHOP_MAX_HOPS];
 };
-
-// Largest r in [0, R-1] with off[r] <= p.
-__device__ __forceinline__ uint32_t seg_of(const uint64_t* __restrict__ off, uint32_t R, uint64_t p) {
-    uint32_t lo = 0, hi = R - 1;
-    while (lo < hi) {
-        uint32_t mid = lo + (hi - lo + 1) / 2;
-        if (off[mid] <= p) lo = mid;
-        else hi = mid - 1;
-    }
-    return lo;
-}
 
 // ------------------------------------------------------------------ hash table (dedup)
 // Slot h = {key, val} in one aligned 16-byte pair, so that a probe, its insert and its atomicMin
@@ -78,13 +68,25 @@ __global__ void ht_clear_kernel(HashTab t) {
     }
 }
 
-// Value of the p-th entry of a dedup input, kInvalid when absent or past the output capacity.
-struct DedupIn {
+// Entry p (of request r) of a dedup input, kInvalid when it is none.
+struct SeedIn {  // the requests' seeds; one that is not a vertex is reported and dropped
+    const KhReq* reqs;
+    const uint64_t* sbeg;
+    uint32_t n;
+    uint32_t* err;
+    __device__ __forceinline__ uint32_t at(uint64_t p, uint32_t r) const {
+        const uint32_t v = reqs[r].seeds[p - sbeg[r]];
+        if (v < n) return v;
+        atomicCAS(err, kErrNone, kErrBadStart);
+        return kInvalid;
+    }
+};
+struct EdgeIn {  // the destinations of a hop's edges; past the output capacity there are none
     const uint32_t* arr;
-    const uint64_t* base;  // device offset added to p (hop base); nullptr = 0
+    const uint64_t* base;  // device offset of the hop
     uint64_t cap;          // entries of arr that exist
-    __device__ __forceinline__ uint32_t at(uint64_t p) const {
-        uint64_t q = (base ? *base : 0) + p;
+    __device__ __forceinline__ uint32_t at(uint64_t p, uint32_t) const {
+        const uint64_t q = *base + p;
         return q < cap ? arr[q] : kInvalid;
     }
 };
@@ -93,7 +95,8 @@ struct DedupIn {
 struct GenTab {
     HashTab t;
     uint32_t gen;
-    __device__ __forceinline__ void insert(uint32_t r, uint32_t v, uint64_t p, uint32_t* err) const {
+    // Whether p is its key's smallest position so far; the position it displaces is taken off `words`.
+    __device__ __forceinline__ bool insert(uint32_t r, uint32_t v, uint64_t p, FirstWord* words, uint32_t* err) const {
         const uint64_t key48 = ((uint64_t)r << 31) | v;
         const unsigned long long full = ((unsigned long long)gen << 48) | key48;
         uint64_t h = ht_home(t, key48);
@@ -109,24 +112,17 @@ struct GenTab {
             h = (h + 1) & t.mask;
             if (++probes > t.mask) {  // cannot happen while slots > entries; never spin
                 atomicCAS(err, kErrNone, kErrBadNeighbor);
-                return;
+                return false;
             }
         }
         // min of (generation, position): read first, since most repeats come after the first
         // occurrence and then need no atomic (an atomic costs a write to memory)
         const unsigned long long mine = ((unsigned long long)(0xFFFFu - gen) << 32) | (uint32_t)p;
-        if (__atomic_load_n(t.val(h), __ATOMIC_RELAXED) > mine) atomicMin(t.val(h), mine);
-    }
-    __device__ __forceinline__ bool first_is(uint32_t r, uint32_t v, uint64_t p) const {
-        const uint64_t key48 = ((uint64_t)r << 31) | v;
-        const unsigned long long full = ((unsigned long long)gen << 48) | key48;
-        uint64_t h = ht_home(t, key48);
-        for (uint64_t probes = 0; probes <= t.mask; ++probes) {
-            const ulonglong2 kv = *(const ulonglong2*)t.key(h);  // key and val in one load
-            if (kv.x == full) return (uint32_t)kv.y == (uint32_t)p;
-            h = (h + 1) & t.mask;
-        }
-        return false;
+        if (__atomic_load_n(t.val(h), __ATOMIC_RELAXED) < mine) return false;
+        const unsigned long long old = atomicMin(t.val(h), mine);
+        if (old < mine) return false;
+        if ((old >> 32) == (mine >> 32)) not_first(words, (uint32_t)old);
+        return true;
     }
 };
 
@@ -142,142 +138,138 @@ struct PackTab {
     __device__ __forceinline__ uint64_t home(unsigned long long k) const {
         return (((k + 1) * 0x9E3779B97F4A7C15ull) >> shift) & mask;
     }
-    __device__ __forceinline__ void insert(uint32_t r, uint32_t v, uint64_t p, uint32_t* err) const {
+    __device__ __forceinline__ bool insert(uint32_t r, uint32_t v, uint64_t p, FirstWord* words, uint32_t* err) const {
         const unsigned long long k = ((unsigned long long)r << vb) | v;
         const unsigned long long w = (k << pb) | p;
         uint64_t h = home(k);
         for (uint64_t probes = 0; probes <= mask; ++probes) {
             // the CAS claims an empty slot, or returns what the slot holds
             const unsigned long long cur = atomicCAS(slot + h, ~0ull, w);
-            if (cur == ~0ull) return;
+            if (cur == ~0ull) return true;
             if ((cur >> pb) == k) {
-                if (cur > w) atomicMin(slot + h, w);
-                return;
+                if (cur < w) return false;
+                const unsigned long long old = atomicMin(slot + h, w);
+                if (old < w) return false;
+                not_first(words, old & ((1ull << pb) - 1));
+                return true;
             }
             h = (h + 1) & mask;
         }
         atomicCAS(err, kErrNone, kErrBadNeighbor);  // cannot happen: slots > entries
-    }
-    __device__ __forceinline__ bool first_is(uint32_t r, uint32_t v, uint64_t p) const {
-        const unsigned long long k = ((unsigned long long)r << vb) | v;
-        uint64_t h = home(k);
-        for (uint64_t probes = 0; probes <= mask; ++probes) {
-            const unsigned long long cur = slot[h];
-            if (cur == ~0ull) break;
-            if ((cur >> pb) == k) return (cur & ((1ull << pb) - 1)) == p;
-            h = (h + 1) & mask;
-        }
         return false;
     }
 };
 
-template <class Tab>
-__global__ __launch_bounds__(kKhBlock) void dedup_insert_kernel(DedupIn in, Count E,
-                                                                const uint64_t* __restrict__ eoff_r,
-                                                                uint32_t R, Tab t, uint32_t* err) {
+// One wave per 64 positions (a word of `words`, all ones at first): every entry goes into the table,
+// and the word keeps the bits of those that are, so far, their key's first.
+template <class Tab, class In>
+__global__ __launch_bounds__(kKhBlock) void dedup_insert_kernel(In in, Count E, const uint64_t* __restrict__ off_r,
+                                                                uint32_t R, Tab t, FirstWord* words, uint32_t* err) {
     const uint64_t n = E.get();
-    for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n;
-         p += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t v = in.at(p);
-        if (v == kInvalid) continue;
-        t.insert(seg_of(eoff_r, R, p), v, p, err);
+    const int lane = lane_id();
+    const uint64_t nw = (uint64_t)gridDim.x * (kKhBlock / kWave);
+    for (uint64_t w = readfirstlane_u64(((uint64_t)blockIdx.x * kKhBlock + threadIdx.x) / kWave); w * kWave < n; w += nw) {
+        const uint64_t p = w * kWave + lane;
+        const uint32_t r = segment_of_lane(off_r, R, w, n);
+        const uint32_t v = p < n ? in.at(p, r) : kInvalid;
+        const bool first = v != kInvalid && t.insert(r, v, p, words, err);
+        const unsigned long long keep = __ballot(first);
+        if (lane == 0 && keep != ~0ull) atomicAnd(&words[w].x, keep);
     }
 }
 
-// flag[p] = 1 when entry p is the first occurrence of its (request, vertex) key.
-template <class Tab>
-__global__ __launch_bounds__(kKhBlock) void dedup_mark_kernel(DedupIn in, Count E,
-                                                              const uint64_t* __restrict__ eoff_r,
-                                                              uint32_t R, Tab t,
-                                                              uint32_t* __restrict__ flag) {
-    const uint64_t n = E.get();
-    for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n;
-         p += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t v = in.at(p);
-        flag[p] = v != kInvalid && t.first_is(seg_of(eoff_r, R, p), v, p);
-    }
-}
-
-struct FlagGen {
-    const uint32_t* flag;
-    __device__ __forceinline__ uint64_t operator()(uint64_t i) const { return flag[i]; }
-};
-
-__global__ __launch_bounds__(kKhBlock) void compact_kernel(DedupIn in, Count E,
-                                                           const uint64_t* __restrict__ eoff_r,
-                                                           uint32_t R,
-                                                           const uint32_t* __restrict__ flag,
-                                                           const uint64_t* __restrict__ fpos,
+// The first appearances become the next frontier, in order: vertex, request, degree and draws at
+// hop h of each.
+template <class In>
+__global__ __launch_bounds__(kKhBlock) void compact_kernel(In in, Count E, const uint64_t* __restrict__ off_r,
+                                                           uint32_t R, const FirstWord* __restrict__ words,
                                                            const uint32_t* __restrict__ deg,
-                                                           uint32_t* __restrict__ fv,
-                                                           uint32_t* __restrict__ fr,
-                                                           uint32_t* __restrict__ fd) {
+                                                           const KhReq* __restrict__ reqs, uint32_t h,
+                                                           uint32_t* __restrict__ fv, uint32_t* __restrict__ fr,
+                                                           uint32_t* __restrict__ fd, uint32_t* __restrict__ fc) {
     const uint64_t n = E.get();
-    for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < n;
-         p += (uint64_t)gridDim.x * blockDim.x) {
-        if (!flag[p]) continue;
-        uint64_t q = fpos[p];
-        const uint32_t v = in.at(p);
+    const int lane = lane_id();
+    const uint64_t nw = (uint64_t)gridDim.x * (kKhBlock / kWave);
+    for (uint64_t w = readfirstlane_u64(((uint64_t)blockIdx.x * kKhBlock + threadIdx.x) / kWave); w * kWave < n; w += nw) {
+        const FirstWord fw = words[w];
+        const uint32_t r = segment_of_lane(off_r, R, w, n);
+        if (!((fw.x >> lane) & 1)) continue;
+        const uint64_t q = fw.y + lanes_below(fw.x);
+        const uint32_t v = in.at(w * kWave + lane, r);
+        const uint32_t d = deg[v];  // read here once; the sampler reads it in order
+        const KhReq& k = reqs[r];
         fv[q] = v;
-        fr[q] = seg_of(eoff_r, R, p);
-        fd[q] = deg[v];  // read here once; the count scan and the sampler read it in order
-    }
-}
-
-// foff[r] = first frontier item of request r; icount = frontier size.
-__global__ void front_offsets_kernel(const uint64_t* __restrict__ eoff_r, uint32_t R,
-                                     const uint64_t* __restrict__ fpos, uint64_t* __restrict__ foff,
-                                     uint64_t* icount) {
-    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r <= R; r += gridDim.x * blockDim.x) {
-        uint64_t x = fpos[eoff_r[r]];
-        foff[r] = x;
-        if (r == R) *icount = x;
-    }
-}
-
-// ------------------------------------------------------------------ seeds -> virtual edges
-__global__ __launch_bounds__(kKhBlock) void seed_gather_kernel(const KhReq* __restrict__ reqs,
-                                                               const uint64_t* __restrict__ sbeg,
-                                                               uint32_t R, uint64_t S, uint32_t n,
-                                                               uint32_t* __restrict__ out,
-                                                               uint32_t* err) {
-    for (uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; p < S;
-         p += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t r = seg_of(sbeg, R, p);
-        uint32_t v = reqs[r].seeds[p - sbeg[r]];
-        if (v >= n) {
-            atomicCAS(err, kErrNone, kErrBadStart);
-            v = kInvalid;
-        }
-        out[p] = v;
+        fr[q] = r;
+        fd[q] = d;
+        fc[q] = min(d, h < k.hops ? k.fan[h] : 0u);
     }
 }
 
 // ------------------------------------------------------------------ per hop
-struct CountGen {  // draws of frontier item i at hop h: min(fanout, degree)
-    const uint32_t* fd;
-    const uint32_t* fr;
-    const KhReq* reqs;
-    uint32_t h;
-    __device__ __forceinline__ uint64_t operator()(uint64_t i) const {
-        const KhReq& q = reqs[fr[i]];
-        uint32_t f = h < q.hops ? q.fan[h] : 0u;
-        uint32_t d = fd[i];
-        return d < f ? d : f;
-    }
+struct DrawsGen {  // draws of frontier item i
+    const uint32_t* fc;
+    __device__ __forceinline__ uint64_t operator()(uint64_t i) const { return fc[i]; }
 };
 
 // eoff_r[r] = first edge (within hop h) of request r; out_off[h][r] = hop base + eoff_r[r];
 // hb[h+1] = hb[h] + edges of hop h.
-__global__ void hop_offsets_kernel(const uint64_t* __restrict__ foff, uint32_t R,
-                                   const uint64_t* __restrict__ eoff, uint64_t* __restrict__ eoff_r,
-                                   uint64_t* hb, uint32_t h, uint64_t* __restrict__ out_off) {
-    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r <= R; r += gridDim.x * blockDim.x) {
-        uint64_t e = eoff[foff[r]];
+__device__ __forceinline__ void hop_offsets(const uint64_t* __restrict__ foff, uint32_t R, const uint64_t* eoff,
+                                            uint64_t* __restrict__ eoff_r, uint64_t* hb, uint32_t h,
+                                            uint64_t* __restrict__ out_off, uint32_t t, uint32_t threads) {
+    for (uint32_t r = t; r <= R; r += threads) {
+        const uint64_t e = eoff[foff[r]];
         eoff_r[r] = e;
         out_off[(uint64_t)h * (R + 1) + r] = hb[h] + e;
         if (r == R) hb[h + 1] = hb[h] + e;
     }
+}
+
+__global__ void hop_offsets_kernel(const uint64_t* __restrict__ foff, uint32_t R, const uint64_t* eoff,
+                                   uint64_t* __restrict__ eoff_r, uint64_t* hb, uint32_t h,
+                                   uint64_t* __restrict__ out_off) {
+    hop_offsets(foff, R, eoff, eoff_r, hb, h, out_off, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+}
+
+// A frontier of at most kOneWgItems items: the scan of its draws and the hop's offsets in one launch of
+// one workgroup (where the scan's launches, not its work, are the time).
+constexpr uint32_t kOneWgItems = 16384;
+__global__ __launch_bounds__(1024) void small_offsets_kernel(const uint32_t* __restrict__ fc,
+                                                             const uint64_t* __restrict__ icount, uint64_t* eoff,
+                                                             uint64_t* etot, const uint64_t* __restrict__ foff,
+                                                             uint32_t R, uint64_t* __restrict__ eoff_r, uint64_t* hb,
+                                                             uint32_t h, uint64_t* __restrict__ out_off) {
+    __shared__ uint32_t lds[1024 / kWave];
+    constexpr uint32_t kPer = kOneWgItems / 1024;
+    const uint32_t I = (uint32_t)*icount, per = (I + 1023) / 1024, i0 = threadIdx.x * per;
+    uint32_t c[kPer], s = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        c[k] = k < per && i0 + k < I ? fc[i0 + k] : 0u;
+        s += c[k];
+    }
+    uint32_t total;  // (at most 16384 * 64)
+    uint32_t pre = block_exclusive_sum<uint32_t, 1024>(s, total, lds);
+#pragma unroll
+    for (uint32_t k = 0; k < kPer; ++k) {
+        if (k < per && i0 + k < I) eoff[i0 + k] = pre;
+        pre += c[k];
+    }
+    if (threadIdx.x == 0) {
+        eoff[I] = total;
+        *etot = total;
+    }
+    __syncthreads();  // the offsets are read across the workgroup
+    hop_offsets(foff, R, eoff, eoff_r, hb, h, out_off, threadIdx.x, 1024);
+}
+
+// Start of a batch: zeroed scalars, all-one first words, empty table slots.
+__global__ __launch_bounds__(256) void khop_init_kernel(uint64_t* sc, uint32_t nsc, FirstWord* words, uint64_t nwords,
+                                                        unsigned long long* slots, uint64_t nslots) {
+    const uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x, all = (uint64_t)gridDim.x * 256;
+    if (t < nsc) sc[t] = 0;
+    for (uint64_t i = t; i < nwords; i += all) words[i] = make_ulonglong2(~0ull, 0ull);
+    ulonglong2* s2 = (ulonglong2*)slots;
+    for (uint64_t i = t; i < nslots / 2; i += all) s2[i] = make_ulonglong2(~0ull, ~0ull);
 }
 
 // Lane layouts of the sampling kernel.
@@ -602,12 +594,27 @@ static bool kh_packed_table(const grass_graph* g, uint32_t R, uint64_t S, uint64
     return bit_width(R - 1) + vb + pb <= 64 && !(force16 && strcmp(force16, "16") == 0);
 }
 
-// Device scratch of a batch of R requests, S seeds, frontier bound Imax and dedup bound Dmax.
-static size_t kh_scratch_need(uint64_t R, uint64_t S, uint64_t Imax, uint64_t Dmax) {
-    const uint64_t nb = std::max(scan_blocks(Imax), scan_blocks(Dmax));
-    return Carve::need(R * sizeof(KhReq)) + Carve::need((R + 1) * 8) * 4 + Carve::need(S * 4 + 4) +
-           Carve::need(Imax * 4) * 6 + Carve::need((Imax + 1) * 8) + Carve::need(Dmax * 4) +
-           Carve::need((Dmax + 1) * 8) + Carve::need(nb * 8) + Carve::need(64 * 8);
+// A batch's packed dedup tables: one per pass (the seeds, then every hop's destinations but the
+// last's), all cleared at its start, while they fit kTablesAtOnce; one shared by the passes and
+// cleared before each otherwise.
+constexpr uint64_t kTablesAtOnce = 64ull << 20;
+struct Tables {
+    bool at_once;
+    uint64_t slots;  // of all tables, or of the shared one
+};
+static Tables plan_tables(uint64_t S, uint64_t Dmax, uint32_t H) {
+    const uint64_t all = pack_slots(S) + (H - 1) * pack_slots(Dmax);
+    if (all * 8 <= kTablesAtOnce) return Tables{true, all};
+    return Tables{false, pack_slots(std::max(S, Dmax))};
+}
+static uint64_t kh_words(uint64_t S, uint64_t Dmax, uint32_t H) { return firsts_words(S) + (H - 1) * firsts_words(Dmax); }
+
+// Device scratch of a batch of R requests, S seeds, frontier bound Imax, dedup bound Dmax and H hops.
+static size_t kh_scratch_need(uint64_t R, uint64_t S, uint64_t Imax, uint64_t Dmax, uint32_t H) {
+    const uint64_t nb = std::max(scan_blocks(Imax), scan_blocks(firsts_words(std::max(S, Dmax))));
+    return Carve::need(R * sizeof(KhReq) + (R + 1) * 8) + Carve::need((R + 1) * 8) * 3 + Carve::need(Imax * 4) * 8 +
+           Carve::need((Imax + 1) * 8) + Carve::need(kh_words(S, Dmax, H) * sizeof(FirstWord)) + Carve::need(nb * 8) +
+           Carve::need(64 * 8);
 }
 
 static hipError_t ensure_table(Workspace& ws, uint64_t entries, HashTab& t) {
@@ -650,10 +657,13 @@ int khop_reserve(const grass_graph* g, Workspace& ws, uint32_t R, uint64_t S, ui
     if (!R) return GRASS_OK;
     const uint64_t Imax = std::max<uint64_t>(I, 1), Dmax = std::max<uint64_t>(D, 1);
     if (ws.reserve_stage(R * sizeof(KhReq) + (R + 1) * 8 + 64) != hipSuccess ||
-        ws.scratch.reserve(kh_scratch_need(R, S, Imax, Dmax)) != hipSuccess)
+        ws.scratch.reserve(kh_scratch_need(R, S, Imax, Dmax, GRASS_KHOP_MAX_HOPS)) != hipSuccess)
         return GRASS_ENOMEM;
     if (kh_packed_table(g, R, S, Dmax)) {
-        if (ws.ht.reserve(pack_slots(std::max(S, Dmax)) * 8) != hipSuccess) return GRASS_ENOMEM;
+        // (a smaller batch of more hops may take several tables at once, up to kTablesAtOnce)
+        uint64_t bytes = pack_slots(std::max(S, Dmax)) * 8;
+        bytes = std::max(bytes, std::min(kTablesAtOnce, bytes * GRASS_KHOP_MAX_HOPS));
+        if (ws.ht.reserve(bytes) != hipSuccess) return GRASS_ENOMEM;
         ws.ht_gen = 0xFFFF;
     } else {
         HashTab t{};
@@ -695,23 +705,23 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     }
     const uint64_t S = sbeg[R];
     const uint64_t Imax = std::max<uint64_t>(Ibound, 1), Dmax = std::max<uint64_t>(Dbound, 1);
-    const uint64_t nbI = scan_blocks(Imax), nbD = scan_blocks(Dmax);
-    hipError_t e = ws.scratch.reserve(kh_scratch_need(R, S, Imax, Dmax));
+    const uint64_t nbI = scan_blocks(Imax), nbD = scan_blocks(firsts_words(std::max(S, Dmax)));
+    hipError_t e = ws.scratch.reserve(kh_scratch_need(R, S, Imax, Dmax, H));
     if (e != hipSuccess) return GRASS_ENOMEM;
     Carve cv(ws.scratch.ptr);
-    KhReq* d_req = cv.take<KhReq>(R);
-    uint64_t* d_sbeg = cv.take<uint64_t>(R + 1);
+    KhReq* d_req = (KhReq*)cv.take<char>(R * sizeof(KhReq) + (R + 1) * 8);  // the requests, then their seed starts
+    uint64_t* d_sbeg = (uint64_t*)(d_req + R);
     uint64_t* d_foff[2] = {cv.take<uint64_t>(R + 1), cv.take<uint64_t>(R + 1)};
     uint64_t* d_eoff_r = cv.take<uint64_t>(R + 1);
-    uint32_t* d_seedv = cv.take<uint32_t>(S + 1);
     uint32_t* d_fv[2] = {cv.take<uint32_t>(Imax), cv.take<uint32_t>(Imax)};
     uint32_t* d_fr[2] = {cv.take<uint32_t>(Imax), cv.take<uint32_t>(Imax)};
     uint32_t* d_fd[2] = {cv.take<uint32_t>(Imax), cv.take<uint32_t>(Imax)};  // frontier degrees
+    uint32_t* d_fc[2] = {cv.take<uint32_t>(Imax), cv.take<uint32_t>(Imax)};  // and draws
     uint64_t* d_eoff = cv.take<uint64_t>(Imax + 1);
-    uint32_t* d_flag = cv.take<uint32_t>(Dmax);
-    uint64_t* d_fpos = cv.take<uint64_t>(Dmax + 1);
+    const uint64_t nwords = kh_words(S, Dmax, H);
+    FirstWord* d_words = cv.take<FirstWord>(nwords);
     uint64_t* d_part = cv.take<uint64_t>(std::max(nbI, nbD));
-    uint64_t* d_sc = cv.take<uint64_t>(64);  // [0..1] item counts, [2] edges total, [3] flags total,
+    uint64_t* d_sc = cv.take<uint64_t>(64);  // [0..1] item counts, [2] edges total, [3] firsts total,
                                              // [8..8+H] hop bases
     uint64_t* d_icount[2] = {d_sc + 0, d_sc + 1};
     uint64_t* d_etot = d_sc + 2;
@@ -723,59 +733,64 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     const uint32_t vb = std::max<uint32_t>(bit_width(g->n ? g->n - 1 : 0), 1u);
     const uint32_t pb = std::max<uint32_t>(bit_width(std::max(S, Dmax)), 1u);  // positions < 2^pb - 1
     const bool packed = kh_packed_table(g, R, S, Dmax);
+    const Tables tables = plan_tables(S, Dmax, H);
     HashTab ht{};
     if (packed) {
-        if (ws.ht.reserve(pack_slots(std::max(S, Dmax)) * 8) != hipSuccess) return GRASS_ENOMEM;
+        if (ws.ht.reserve(tables.slots * 8) != hipSuccess) return GRASS_ENOMEM;
         ws.ht_gen = 0xFFFF;  // the 16-byte table's next use starts from a clear
     } else {
         e = ensure_table(ws, Dmax, ht);
         if (e != hipSuccess) return GRASS_ENOMEM;
     }
-    // the table for `entries` positions: packed (cleared now, only the slots it uses) or the next
-    // generation of the 16-byte one
-    auto pack_tab = [&](uint64_t entries) {
-        const uint64_t slots = pack_slots(entries);
-        const unsigned grid = (unsigned)std::min<uint64_t>((slots + 255) / 256, 4096);
-        hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3(grid), dim3(256), 0, s,
-                           (unsigned long long*)ws.ht.ptr, slots, ~0ull);
-        return PackTab{(unsigned long long*)ws.ht.ptr, slots - 1, (uint32_t)(64 - __builtin_ctzll(slots)), vb, pb};
-    };
-    auto dedup = [&](const DedupIn& in, Count E, const uint64_t* off_r, uint64_t entries) {
+    uint32_t* err = err_word(g, ws);
+    // Inserts pass `pass`'s entries (0: the seeds, h + 1: hop h's destinations): packed table of the
+    // pass or the shared one, or the next generation of the 16-byte one.
+    auto words_of = [&](uint32_t pass) { return pass ? d_words + firsts_words(S) + (pass - 1) * firsts_words(Dmax) : d_words; };
+    auto insert = [&](auto in, Count E, const uint64_t* off_r, uint32_t pass) {
+        const uint64_t entries = pass ? Dmax : S;
+        const unsigned grid = (unsigned)std::min<uint64_t>((entries + kKhBlock - 1) / kKhBlock, 2048);
         if (packed) {
-            const PackTab t = pack_tab(entries);
-            hipLaunchKernelGGL(dedup_insert_kernel<PackTab>, dim3(2048), dim3(kKhBlock), 0, s, in, E, off_r, R, t,
-                               err_word(g, ws));
-            hipLaunchKernelGGL(dedup_mark_kernel<PackTab>, dim3(2048), dim3(kKhBlock), 0, s, in, E, off_r, R, t,
-                               d_flag);
+            const uint64_t slots = pack_slots(entries);
+            unsigned long long* p = (unsigned long long*)ws.ht.ptr;
+            if (tables.at_once) {
+                if (pass) p += pack_slots(S) + (pass - 1) * slots;
+            } else {
+                hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3((unsigned)std::min<uint64_t>((slots + 255) / 256, 4096)),
+                                   dim3(256), 0, s, p, slots, ~0ull);
+            }
+            const PackTab t{p, slots - 1, (uint32_t)(64 - __builtin_ctzll(slots)), vb, pb};
+            hipLaunchKernelGGL((dedup_insert_kernel<PackTab, decltype(in)>), dim3(grid), dim3(kKhBlock), 0, s, in, E, off_r,
+                               R, t, words_of(pass), err);
         } else {
             const GenTab t{ht, next_gen(ws, ht, s)};
-            hipLaunchKernelGGL(dedup_insert_kernel<GenTab>, dim3(2048), dim3(kKhBlock), 0, s, in, E, off_r, R, t,
-                               err_word(g, ws));
-            hipLaunchKernelGGL(dedup_mark_kernel<GenTab>, dim3(2048), dim3(kKhBlock), 0, s, in, E, off_r, R, t,
-                               d_flag);
+            hipLaunchKernelGGL((dedup_insert_kernel<GenTab, decltype(in)>), dim3(grid), dim3(kKhBlock), 0, s, in, E, off_r, R,
+                               t, words_of(pass), err);
         }
     };
+    // The pass's first appearances, numbered and written as the frontier of hop h into buffer k.
+    auto next_frontier = [&](auto in, Count E, const uint64_t* off_r, uint32_t pass, uint32_t h, int k) -> hipError_t {
+        const uint64_t entries = pass ? Dmax : S;
+        hipError_t e = scan_firsts(words_of(pass), E, entries, off_r, R, d_foff[k], d_icount[k], d_part, d_ftot, s);
+        if (e != hipSuccess) return e;
+        const unsigned grid = (unsigned)std::min<uint64_t>(std::max<uint64_t>((entries + kKhBlock - 1) / kKhBlock, 1), 4096);
+        hipLaunchKernelGGL((compact_kernel<decltype(in)>), dim3(grid), dim3(kKhBlock), 0, s, in, E, off_r, R,
+                           (const FirstWord*)words_of(pass), (const uint32_t*)g->d_deg, (const KhReq*)d_req, h, d_fv[k],
+                           d_fr[k], d_fd[k], d_fc[k]);
+        return hipGetLastError();
+    };
 
-    e = hipMemcpyAsync(d_req, hreq, R * sizeof(KhReq), hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(d_sbeg, sbeg, (R + 1) * 8, hipMemcpyHostToDevice, s);
+    e = hipMemcpyAsync(d_req, hreq, R * sizeof(KhReq) + (R + 1) * 8, hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return status_of(e);
-    hipLaunchKernelGGL(fill_kernel<uint64_t>, dim3(1), dim3(64), 0, s, d_sc, (uint64_t)64, (uint64_t)0);
+    const uint64_t clear = packed && tables.at_once ? tables.slots : 0;
+    hipLaunchKernelGGL(khop_init_kernel, dim3((unsigned)std::min<uint64_t>((std::max(clear / 2, nwords) + 255) / 256, 4096)),
+                       dim3(256), 0, s, d_sc, 64u, d_words, nwords, (unsigned long long*)ws.ht.ptr, clear);
 
-    const unsigned gridE = 2048;
-    uint32_t* err = err_word(g, ws);
     // frontier 0: seeds, deduplicated
-    const uint32_t n32 = (uint32_t)g->n;
-    if (S) hipLaunchKernelGGL(seed_gather_kernel, dim3(gridE), dim3(kKhBlock), 0, s, d_req, d_sbeg, R, S, n32,
-                              d_seedv, err);
     {
-        DedupIn in{d_seedv, nullptr, S};
-        dedup(in, Count{S, nullptr}, d_sbeg, S);
-        e = exclusive_scan(FlagGen{d_flag}, Count{S, nullptr}, Dmax, d_fpos, d_part, d_ftot, s);
+        const SeedIn in{d_req, d_sbeg, (uint32_t)g->n, err};
+        if (S) insert(in, Count{S, nullptr}, d_sbeg, 0);
+        e = next_frontier(in, Count{S, nullptr}, d_sbeg, 0, 0, 0);
         if (e != hipSuccess) return status_of(e);
-        hipLaunchKernelGGL(compact_kernel, dim3(gridE), dim3(kKhBlock), 0, s, in, Count{S, nullptr}, d_sbeg, R,
-                           d_flag, d_fpos, (const uint32_t*)g->d_deg, d_fv[0], d_fr[0], d_fd[0]);
-        hipLaunchKernelGGL(front_offsets_kernel, dim3((R + 256) / 256), dim3(256), 0, s, d_sbeg, R, d_fpos,
-                           d_foff[0], d_icount[0]);
     }
     // group width of each hop and the hop's largest fanout; the tuned scale picks the layout:
     // 0 packed lanes, 1 packed or groups as the hop's draws fill the groups, 2 groups of twice
@@ -799,11 +814,16 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     }
     for (uint32_t h = 0; h < H; ++h) {
         const int cur = h & 1, nxt = cur ^ 1;
-        CountGen cg{d_fd[cur], d_fr[cur], d_req, h};
-        e = exclusive_scan(cg, Count{0, d_icount[cur]}, Imax, d_eoff, d_part, d_etot, s);
-        if (e != hipSuccess) return status_of(e);
-        hipLaunchKernelGGL(hop_offsets_kernel, dim3((R + 256) / 256), dim3(256), 0, s, d_foff[cur], R, d_eoff,
-                           d_eoff_r, d_hb, h, out->offsets_dev);
+        if (Imax <= kOneWgItems) {
+            hipLaunchKernelGGL(small_offsets_kernel, dim3(1), dim3(1024), 0, s, (const uint32_t*)d_fc[cur],
+                               (const uint64_t*)d_icount[cur], d_eoff, d_etot, (const uint64_t*)d_foff[cur], R, d_eoff_r,
+                               d_hb, h, out->offsets_dev);
+        } else {
+            e = exclusive_scan(DrawsGen{d_fc[cur]}, Count{0, d_icount[cur]}, Imax, d_eoff, d_part, d_etot, s);
+            if (e != hipSuccess) return status_of(e);
+            hipLaunchKernelGGL(hop_offsets_kernel, dim3((R + 256) / 256), dim3(256), 0, s, d_foff[cur], R, d_eoff,
+                               d_eoff_r, d_hb, h, out->offsets_dev);
+        }
         if (g->fmt == kLE)
             launch_sample<kLE>(g, lanes[h], fmax[h], layout, s, d_fv[cur], d_fr[cur], d_fd[cur], d_icount[cur],
                                d_req, h, seed, d_eoff, d_hb, out->src_dev, out->dst_dev, out->capacity, err);
@@ -811,15 +831,10 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
             launch_sample<kGT>(g, lanes[h], fmax[h], layout, s, d_fv[cur], d_fr[cur], d_fd[cur], d_icount[cur],
                                d_req, h, seed, d_eoff, d_hb, out->src_dev, out->dst_dev, out->capacity, err);
         if (h + 1 == H) break;
-        DedupIn in{out->dst_dev, d_hb + h, out->capacity};
-        Count E{0, d_etot};
-        dedup(in, E, d_eoff_r, Dmax);
-        e = exclusive_scan(FlagGen{d_flag}, E, Dmax, d_fpos, d_part, d_ftot, s);
+        const EdgeIn in{out->dst_dev, d_hb + h, out->capacity};
+        insert(in, Count{0, d_etot}, d_eoff_r, h + 1);
+        e = next_frontier(in, Count{0, d_etot}, d_eoff_r, h + 1, h + 1, nxt);
         if (e != hipSuccess) return status_of(e);
-        hipLaunchKernelGGL(compact_kernel, dim3(gridE), dim3(kKhBlock), 0, s, in, E, d_eoff_r, R, d_flag, d_fpos,
-                           (const uint32_t*)g->d_deg, d_fv[nxt], d_fr[nxt], d_fd[nxt]);
-        hipLaunchKernelGGL(front_offsets_kernel, dim3((R + 256) / 256), dim3(256), 0, s, d_eoff_r, R, d_fpos,
-                           d_foff[nxt], d_icount[nxt]);
     }
     e = hipGetLastError();
     if (e == hipSuccess)

@@ -24,7 +24,10 @@ constexpr uint64_t kScanFoldMax = 2048;  // tiles whose start each tile sums its
 struct Count {
     uint64_t imm;
     const uint64_t* dev;  // when non-null the count is *dev
-    __device__ __forceinline__ uint64_t get() const { return dev ? *dev : imm; }
+    uint32_t shift = 0;   // in units of 2^shift, rounded up
+    __device__ __forceinline__ uint64_t get() const {
+        return ((dev ? *dev : imm) + ((1ull << shift) - 1)) >> shift;
+    }
 };
 
 template <class Gen>
@@ -84,8 +87,8 @@ __device__ __forceinline__ uint64_t wave_inclusive_sum_u64(uint64_t x) {
 // and each round is one DPP wave scan carried into the next (no workgroup scan per round).
 // FOLD: partials[] are the tile sums themselves (at most kScanFoldMax of them): each tile adds up
 // those before it, and the tile holding item n - 1 also writes *total; otherwise partials[] are
-// the tiles' exclusive prefixes and *total was written with them.
-template <class Gen, bool FOLD>
+// the tiles' exclusive prefixes and *total was written with them.  Outputs lie STRIDE words apart.
+template <class Gen, bool FOLD, int STRIDE>
 __global__ __launch_bounds__(kScanBlock) void scan_write_kernel(Gen gen, Count cnt,
                                                                 const uint64_t* partials,
                                                                 uint64_t* total,
@@ -128,17 +131,17 @@ __global__ __launch_bounds__(kScanBlock) void scan_write_kernel(Gen gen, Count c
     for (int j = 0; j < kScanItems; ++j) {
         const uint64_t i = wb + (uint64_t)j * kWave;
         const uint64_t inc = wave_inclusive_sum_u64(x[j]);
-        if (i < n) out[i] = carry + inc - x[j];
+        if (i < n) out[i * STRIDE] = carry + inc - x[j];
         carry += readlane_u64(inc, kWave - 1);
     }
     if (threadIdx.x == 0 && base + kScanTile >= n) {
         if (FOLD) {
             uint64_t t = start;
             for (int w = 0; w < kScanBlock / kWave; ++w) t += wsum[w];
-            out[n] = t;
+            out[n * STRIDE] = t;
             if (total) *total = t;
         } else {
-            out[n] = *total;
+            out[n * STRIDE] = *total;
         }
     }
 }
@@ -146,18 +149,18 @@ __global__ __launch_bounds__(kScanBlock) void scan_write_kernel(Gen gen, Count c
 inline uint64_t scan_blocks(uint64_t n_max) { return n_max ? (n_max + kScanTile - 1) / kScanTile : 1; }
 
 // Scratch: partials[scan_blocks(n_max)] and total[1].
-template <class Gen>
+template <int STRIDE = 1, class Gen>
 hipError_t exclusive_scan(Gen gen, Count cnt, uint64_t n_max, uint64_t* out, uint64_t* partials,
                           uint64_t* total, hipStream_t stream) {
     const uint64_t nb = scan_blocks(n_max);
     hipLaunchKernelGGL(scan_reduce_kernel<Gen>, dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
                        gen, cnt, partials);
     if (nb <= kScanFoldMax) {
-        hipLaunchKernelGGL((scan_write_kernel<Gen, true>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
+        hipLaunchKernelGGL((scan_write_kernel<Gen, true, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
                            gen, cnt, (const uint64_t*)partials, total, out);
     } else {
         hipLaunchKernelGGL(scan_partials_kernel<uint64_t>, dim3(1), dim3(1024), 0, stream, partials, nb, total);
-        hipLaunchKernelGGL((scan_write_kernel<Gen, false>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
+        hipLaunchKernelGGL((scan_write_kernel<Gen, false, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
                            gen, cnt, (const uint64_t*)partials, total, out);
     }
     return hipGetLastError();
