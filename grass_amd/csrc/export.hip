@@ -13,7 +13,11 @@
 //   3. rel_emit_kernel: writes each first appearance to nodes[rank(p)] and the local ids of every
 //      batch edge (its destination is a position, its source a key looked up in the table).
 // Every step is a data-parallel pass over the positions; the result does not depend on timing.
-// Bound by the table's random atomics and loads.  REL_FIGURES
+// A batch of few positions is one launch of one workgroup (rel_small_kernel).  A large one is bound by
+// the random atomics of the inserts, which the chip takes at 22 to 27 G/s whatever the table's size
+// (a load of a slot and a CAS on it: 25.7 G/s), so a position touches the table once: 16 x 8192 seeds
+// [25, 10] on R-MAT s24, 10.7 M positions, insert 435 us; a second pass that looked every key up again
+// took 196 us more.  The emit is 223 us, most of it waiting on the source's lookup.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -285,19 +289,55 @@ __global__ __launch_bounds__(1024) void rel_prepare_kernel(Tab t, FirstWord* wor
     }
 }
 
+// Where a wave that goes through consecutive words is: the stretch of positions (a request's seeds,
+// or its edges of one hop) it found last, whose vertices follow each other in one array.
+struct RelCursor {
+    uint64_t beg = 1, end = 0;  // positions of the stretch
+    uint32_t r = 0;             // its request
+    uint64_t e0 = 0;            // its first batch edge, ~0 for seeds
+    const uint32_t* arr = nullptr;
+    __device__ __forceinline__ void find(const RelSeq& q, uint64_t p) {
+        r = segment_in(q.Q, 0, q.R - 1, p);
+        const RelReq k = q.req[r];
+        beg = q.Q[r];
+        end = beg + k.num;
+        arr = k.seeds;
+        e0 = ~0ull;
+        for (uint32_t h = 0; h < q.H && p >= end; ++h) {
+            e0 = q.off[(uint64_t)h * (q.R + 1) + r];
+            beg = end;
+            end += q.off[(uint64_t)h * (q.R + 1) + r + 1] - e0;
+            arr = q.dst + e0;
+        }
+    }
+    // The vertex, request and batch edge (~0 for a seed) at the lane's position p <= last of word w.
+    __device__ __forceinline__ uint32_t at(const RelSeq& q, uint64_t w, uint64_t p, uint64_t last, uint32_t& rr, uint64_t& e) {
+        const uint64_t p0 = w * kWave;
+        if (p0 < beg || p0 >= end) find(q, p0);
+        if (last < end) {  // the whole word
+            rr = r;
+            e = e0 == ~0ull ? ~0ull : e0 + (p - beg);
+            return arr[p - beg];
+        }
+        rr = segment_in(q.Q, r, q.R - 1, p);
+        return q.at(p, rr, e);
+    }
+};
+
 // One wave per 64 positions (a word of `words`).
 template <class Tab>
 __global__ __launch_bounds__(kExBlock) void rel_insert_kernel(RelSeq q, uint64_t P, Tab t, FirstWord* words,
                                                               const uint32_t* __restrict__ invalid, uint32_t* err) {
     if (*invalid) return;
-    const uint64_t nw = (uint64_t)gridDim.x * (kExBlock / kWave);
-    for (uint64_t w = readfirstlane_u64(((uint64_t)blockIdx.x * kExBlock + threadIdx.x) / kWave); w * kWave < P; w += nw) {
-        const uint64_t p = w * kWave + lane_id();
-        const uint32_t r = segment_of_lane(q.Q, q.R, w, P);
+    const WordChunk wc = wave_words<kExBlock>(P);
+    RelCursor cur;
+    for (uint64_t w = wc.w; w < wc.end; ++w) {
+        const uint64_t p = w * kWave + lane_id(), last = min(w * kWave + kWave - 1, P - 1);
+        uint32_t r;
+        uint64_t e;
+        const uint32_t v = cur.at(q, w, min(p, last), last, r, e);
         bool first = false;
         if (p < P) {
-            uint64_t e;
-            const uint32_t v = q.at(p, r, e);
             if (v < q.n) first = t.insert(r, v, p, words, err);
             else atomicOr(err, 1u);  // a seed or destination that is not a vertex of the graph
         }
@@ -314,14 +354,15 @@ __global__ __launch_bounds__(kExBlock) void rel_emit_kernel(RelSeq q, uint64_t P
                                                             uint32_t* __restrict__ lsrc, uint32_t* __restrict__ ldst,
                                                             const uint32_t* __restrict__ invalid, uint32_t* err) {
     if (*invalid) return;
-    const uint64_t nw = (uint64_t)gridDim.x * (kExBlock / kWave);
-    for (uint64_t w = readfirstlane_u64(((uint64_t)blockIdx.x * kExBlock + threadIdx.x) / kWave); w * kWave < P; w += nw) {
+    const WordChunk wc = wave_words<kExBlock>(P);
+    RelCursor cur;
+    for (uint64_t w = wc.w; w < wc.end; ++w) {
         const FirstWord fw = words[w];
-        const uint64_t p = w * kWave + lane_id();
-        const uint32_t r = segment_of_lane(q.Q, q.R, w, P);
-        if (p >= P) continue;
+        const uint64_t p = w * kWave + lane_id(), last = min(w * kWave + kWave - 1, P - 1);
+        uint32_t r;
         uint64_t e;
-        const uint32_t v = q.at(p, r, e);
+        const uint32_t v = cur.at(q, w, min(p, last), last, r, e);
+        if (p >= P) continue;
         const bool first = (fw.x >> lane_id()) & 1;
         const uint64_t mine = fw.y + lanes_below(fw.x);
         if (first && mine < cap) nodes[mine] = v;
@@ -376,6 +417,77 @@ hipError_t rel_build(const Tab& t, const RelSeq& q, uint64_t P, uint64_t* d_len,
     return hipGetLastError();
 }
 
+// At most kOneWgEntries positions and 1024 requests: the whole build in one launch of one workgroup, the
+// table in LDS.  reqs and result lie in host memory; result[0] = nodes, result[1] = 0 or 1 (the
+// offsets are not the batch of these requests, an id is not a vertex, or a source is unknown).
+__global__ __launch_bounds__(kOneWgThreads) void rel_small_kernel(RelSeq q, const RelReq* __restrict__ hreq,
+                                                                  RelReq* dreq, uint64_t* Q, uint32_t P, uint64_t total,
+                                                                  uint32_t vb, uint64_t* node_off,
+                                                                  uint32_t* __restrict__ nodes, uint64_t cap,
+                                                                  uint32_t* __restrict__ lsrc,
+                                                                  uint32_t* __restrict__ ldst, uint64_t* result) {
+    extern __shared__ unsigned long long rel_lds[];
+    __shared__ OneWgFirsts f;
+    __shared__ uint64_t lds[kOneWgThreads / kWave];
+    const uint32_t t = threadIdx.x;
+    if (t < q.R) dreq[t] = hreq[t];
+    __syncthreads();
+    const bool mine_ok = q.H == 0 || rel_check(q.off, q.req, q.R, q.H, total, t, kOneWgThreads);
+    bool ok = block_sum<uint64_t, kOneWgThreads>(mine_ok ? 0 : 1, lds) == 0;
+    uint64_t sum;
+    const uint64_t len = t < q.R ? rel_length(q.req, q.off, q.R, ok ? q.H : 0, t) : 0;
+    const uint64_t pre = block_exclusive_sum<uint64_t, kOneWgThreads>(len, sum, lds);
+    ok = ok && sum == P;
+    if (t < q.R) Q[t] = pre;
+    if (t == 0) Q[q.R] = sum;
+    if (!ok) {  // uniform: nothing below reads through the offsets
+        if (t == 0) {
+            result[0] = 0;
+            result[1] = 1;
+        }
+        return;
+    }
+    one_wg_begin(f, rel_lds, P, vb);  // (its barrier also orders Q)
+    uint32_t slot[kOneWgPer], rr[kOneWgPer], vv[kOneWgPer];
+    uint64_t ee[kOneWgPer];
+    bool bad = false;
+#pragma unroll
+    for (uint32_t i = 0; i < kOneWgPer; ++i) {
+        const uint32_t p = i * kOneWgThreads + t;
+        slot[i] = ~0u;
+        if (p < P) {
+            rr[i] = segment_in(q.Q, 0, q.R - 1, p);
+            vv[i] = q.at(p, rr[i], ee[i]);
+            if (vv[i] < q.n) slot[i] = f.insert(rr[i], vv[i], p);
+            else bad = true;
+        }
+    }
+    const uint32_t mine = one_wg_rank(f, P, slot);
+#pragma unroll
+    for (uint32_t i = 0; i < kOneWgPer; ++i) {
+        const uint32_t p = i * kOneWgThreads + t;
+        if (p >= P || slot[i] == ~0u) continue;
+        const uint32_t first = (uint32_t)f.tab[slot[i]] & (kOneWgEntries - 1), id = f.rank(first);
+        if (((mine >> i) & 1) && id < cap) nodes[id] = vv[i];
+        if (ee[i] == ~0ull) continue;
+        const uint32_t base = f.rank((uint32_t)q.Q[rr[i]]);
+        const uint32_t src = q.src[ee[i]];
+        const uint32_t fs = src < q.n ? f.first(rr[i], src) : ~0u;
+        bad = bad || fs == ~0u;
+        ldst[ee[i]] = id - base;
+        lsrc[ee[i]] = fs == ~0u ? kNoId : f.rank(fs) - base;
+    }
+    for (uint32_t r = t; r <= q.R; r += kOneWgThreads) {
+        const uint32_t p = (uint32_t)q.Q[r];
+        node_off[r] = p < P ? f.rank(p) : f.total;
+    }
+    const uint64_t nbad = block_sum<uint64_t, kOneWgThreads>(bad ? 1 : 0, lds);
+    if (t == 0) {
+        result[0] = f.total;
+        result[1] = nbad ? 1 : 0;
+    }
+}
+
 int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, const grass_khop_output* b,
                 grass_khop_blocks* out, hipStream_t s) {
     std::lock_guard<std::mutex> lock(g->mu);
@@ -426,6 +538,25 @@ int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, cons
     const uint32_t lg = (uint32_t)__builtin_ctzll(slots);
 
     hipError_t e = hipSuccess;
+    uint64_t* hres = ws.result_slot();
+    // (GRASS_EXPORT_SLOT asks for a table in memory)
+    if (P && P <= kOneWgEntries && R && R <= kOneWgThreads && !force) {
+        const size_t lds = (size_t)one_wg_slots((uint32_t)P) * 8;
+        if (lds > 65536) {
+            (void)hipFuncSetAttribute((const void*)rel_small_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            (void)hipGetLastError();
+        }
+        const RelSeq q{d_req, b->offsets_dev, b->src_dev, b->dst_dev, d_Q, R, H, (uint32_t)g->n};
+        hipLaunchKernelGGL(rel_small_kernel, dim3(1), dim3(kOneWgThreads), lds, s, q, (const RelReq*)hreq, d_req, d_Q,
+                           (uint32_t)P, b->total, vb, out->node_off_dev, out->nodes_dev, out->node_capacity, out->lsrc_dev,
+                           out->ldst_dev, hres);
+        e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return status_of(e);
+        if (hres[1] != 0) return GRASS_EINVAL;
+        out->nodes = hres[0];
+        return out->nodes > out->node_capacity ? GRASS_ECAPACITY : GRASS_OK;
+    }
     if (R) e = hipMemcpyAsync(d_req, hreq, R * sizeof(RelReq), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return status_of(e);
     // the two halves of d_sc[2]: an id that is not a vertex, or an unknown source; and offsets that
@@ -440,7 +571,6 @@ int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, cons
         e = rel_build(t, q, P, d_len, d_words, d_part, d_sc, d_bad, b, out, s);
     }
     if (e != hipSuccess) return status_of(e);
-    uint64_t* hres = ws.result_slot();
     e = hipMemcpyAsync(hres, d_sc + 1, 16, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return status_of(e);

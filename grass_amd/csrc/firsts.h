@@ -39,15 +39,35 @@ __device__ __forceinline__ uint32_t segment_in(const uint64_t* __restrict__ off,
     return lo;
 }
 
-// Segments of the 64 positions from 64 w (n in all, R segments): one search for the wave, and one
-// per lane only where a segment ends inside the word.
-__device__ __forceinline__ uint32_t segment_of_lane(const uint64_t* __restrict__ off, uint32_t R, uint64_t w, uint64_t n) {
-    const uint64_t p0 = w * kWave;
-    const uint32_t r0 = segment_in(off, 0, R - 1, p0);
-    const uint64_t last = min(p0 + kWave - 1, n - 1);
-    if (r0 + 1 == R || off[r0 + 1] > last) return r0;
-    return segment_in(off, r0, R - 1, min(p0 + (uint64_t)lane_id(), last));
+// The words a wave takes, one after the other: consecutive ones, so that the segment it is in (and the
+// loads that find it, each waiting for the one before) serves many words.
+struct WordChunk {
+    uint64_t w, end;
+};
+template <int BLOCK>
+__device__ __forceinline__ WordChunk wave_words(uint64_t n) {
+    const uint64_t nwords = (n + kWave - 1) / kWave, waves = (uint64_t)gridDim.x * (BLOCK / kWave);
+    const uint64_t wave = (uint64_t)blockIdx.x * (BLOCK / kWave) + threadIdx.x / kWave;
+    const uint64_t per = (nwords + waves - 1) / waves, w = readfirstlane_u64(wave * per);
+    return WordChunk{w, min(w + per, nwords)};
 }
+
+// The segment of each lane's position, for a wave that goes through consecutive words of 64 positions
+// (n in all, R segments starting at off[]): the last segment found serves every word inside it.
+struct SegmentCursor {
+    uint32_t r = 0;
+    uint64_t beg = 1, end = 0;  // positions of segment r
+    __device__ __forceinline__ uint32_t of_lane(const uint64_t* __restrict__ off, uint32_t R, uint64_t w, uint64_t n) {
+        const uint64_t p0 = w * kWave, last = min(p0 + kWave - 1, n - 1);
+        if (p0 < beg || p0 >= end) {
+            r = segment_in(off, 0, R - 1, p0);
+            beg = off[r];
+            end = r + 1 < R ? off[r + 1] : n;
+        }
+        if (last < end) return r;
+        return segment_in(off, r, R - 1, min(p0 + (uint64_t)lane_id(), last));
+    }
+};
 
 struct FirstsGen {
     const FirstWord* words;
@@ -99,6 +119,101 @@ static __global__ __launch_bounds__(256) void firsts_segments_kernel(const First
     const uint64_t n = cnt.get();
     const uint64_t total = words[(n + kWave - 1) / kWave].y;  // (the scan's total follows the last word)
     segment_firsts(words, n, total, off, R, foff, count, blockIdx.x * 256 + threadIdx.x, gridDim.x * 256);
+}
+
+// One workgroup's dedup of up to kOneWgEntries positions: table, firsts and ranks in LDS.  A slot is
+// ((request << vb | vertex) << kOneWgPosBits) | position, all ones when empty (requests < 2^17, vertices <
+// 2^31).  The table's memory is the caller's again once the ranks are made.
+constexpr uint32_t kOneWgThreads = 1024;
+constexpr uint32_t kOneWgPer = 8;  // positions of a thread: tid, tid + 1024, ...
+constexpr uint32_t kOneWgEntries = kOneWgThreads * kOneWgPer;
+constexpr uint32_t kOneWgPosBits = 13;
+constexpr uint32_t kOneWgWords = kOneWgEntries / kWave;
+
+// Slots for n entries (load <= 2/3), a power of two.
+__host__ __device__ inline uint32_t one_wg_slots(uint32_t n) {
+    uint32_t slots = 1024;
+    while (slots < n + n / 2 + 2) slots <<= 1;
+    return slots;
+}
+
+struct OneWgFirsts {
+    unsigned long long* tab;            // one_wg_slots(n) slots
+    unsigned long long bits[kOneWgWords];  // firsts of 64 positions each
+    uint32_t pre[kOneWgWords];          // firsts before them
+    uint32_t total;
+    uint32_t mask, shift, vb;
+
+    __device__ __forceinline__ uint32_t home(unsigned long long k) const {
+        return (uint32_t)(((k + 1) * 0x9E3779B97F4A7C15ull) >> shift);
+    }
+    __device__ __forceinline__ uint32_t rank(uint32_t p) const {
+        return pre[p / kWave] + (uint32_t)__popcll(bits[p / kWave] & ((1ull << (p & (kWave - 1))) - 1));
+    }
+    // Slot of (r, v), which position p enters.
+    __device__ __forceinline__ uint32_t insert(uint32_t r, uint32_t v, uint32_t p) {
+        const unsigned long long k = ((unsigned long long)r << vb) | v, w = (k << kOneWgPosBits) | p;
+        uint32_t h = home(k);
+        for (;;) {  // ends: more slots than entries
+            const unsigned long long cur = atomicCAS(tab + h, ~0ull, w);
+            if (cur == ~0ull) return h;
+            if ((cur >> kOneWgPosBits) == k) {
+                if (cur > w) atomicMin(tab + h, w);
+                return h;
+            }
+            h = (h + 1) & mask;
+        }
+    }
+    // First position of (r, v), or ~0 where it was never entered (after the inserts).
+    __device__ __forceinline__ uint32_t first(uint32_t r, uint32_t v) const {
+        const unsigned long long k = ((unsigned long long)r << vb) | v;
+        uint32_t h = home(k);
+        for (;;) {
+            const unsigned long long cur = tab[h];
+            if (cur == ~0ull) return ~0u;
+            if ((cur >> kOneWgPosBits) == k) return (uint32_t)cur & (kOneWgEntries - 1);
+            h = (h + 1) & mask;
+        }
+    }
+};
+
+// Empties the table for n positions.  Every function below is called by the whole workgroup.
+__device__ __forceinline__ void one_wg_begin(OneWgFirsts& f, unsigned long long* tab, uint32_t n, uint32_t vb) {
+    const uint32_t slots = one_wg_slots(n);
+    for (uint32_t i = threadIdx.x; i < slots; i += kOneWgThreads) tab[i] = ~0ull;
+    if (threadIdx.x == 0) {
+        f.tab = tab;
+        f.mask = slots - 1;
+        f.shift = 64 - (31 - __clz(slots));
+        f.vb = vb;
+    }
+    __syncthreads();
+}
+
+// After the inserts (slot[i] of position i * 1024 + tid, ~0 for none): which of the thread's positions are
+// firsts (bit i), and the ranks of all.
+__device__ __forceinline__ uint32_t one_wg_rank(OneWgFirsts& f, uint32_t n, const uint32_t* slot) {
+    __syncthreads();
+    uint32_t mine = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kOneWgPer; ++i) {
+        const uint32_t p = i * kOneWgThreads + threadIdx.x;
+        const bool first = p < n && slot[i] != ~0u && ((uint32_t)f.tab[slot[i]] & (kOneWgEntries - 1)) == p;
+        mine |= (first ? 1u : 0u) << i;
+        const unsigned long long b = __ballot(first);
+        if (lane_id() == 0) f.bits[p / kWave] = b;
+    }
+    __syncthreads();
+    static_assert(kOneWgWords == 2 * kWave, "one wave scans two words a lane");
+    if (threadIdx.x < kWave) {
+        const uint32_t a = (uint32_t)__popcll(f.bits[2 * threadIdx.x]), b = (uint32_t)__popcll(f.bits[2 * threadIdx.x + 1]);
+        const uint32_t inc = wave_inclusive_sum(a + b);
+        f.pre[2 * threadIdx.x] = inc - a - b;
+        f.pre[2 * threadIdx.x + 1] = inc - b;
+        if (threadIdx.x == kWave - 1) f.total = inc;
+    }
+    __syncthreads();
+    return mine;
 }
 
 // Words of a sequence of at most n_max positions, the entry after the last included.

@@ -167,10 +167,11 @@ __global__ __launch_bounds__(kKhBlock) void dedup_insert_kernel(In in, Count E, 
                                                                 uint32_t R, Tab t, FirstWord* words, uint32_t* err) {
     const uint64_t n = E.get();
     const int lane = lane_id();
-    const uint64_t nw = (uint64_t)gridDim.x * (kKhBlock / kWave);
-    for (uint64_t w = readfirstlane_u64(((uint64_t)blockIdx.x * kKhBlock + threadIdx.x) / kWave); w * kWave < n; w += nw) {
+    const WordChunk wc = wave_words<kKhBlock>(n);
+    SegmentCursor seg;
+    for (uint64_t w = wc.w; w < wc.end; ++w) {
         const uint64_t p = w * kWave + lane;
-        const uint32_t r = segment_of_lane(off_r, R, w, n);
+        const uint32_t r = seg.of_lane(off_r, R, w, n);
         const uint32_t v = p < n ? in.at(p, r) : kInvalid;
         const bool first = v != kInvalid && t.insert(r, v, p, words, err);
         const unsigned long long keep = __ballot(first);
@@ -189,10 +190,11 @@ __global__ __launch_bounds__(kKhBlock) void compact_kernel(In in, Count E, const
                                                            uint32_t* __restrict__ fd, uint32_t* __restrict__ fc) {
     const uint64_t n = E.get();
     const int lane = lane_id();
-    const uint64_t nw = (uint64_t)gridDim.x * (kKhBlock / kWave);
-    for (uint64_t w = readfirstlane_u64(((uint64_t)blockIdx.x * kKhBlock + threadIdx.x) / kWave); w * kWave < n; w += nw) {
+    const WordChunk wc = wave_words<kKhBlock>(n);
+    SegmentCursor seg;
+    for (uint64_t w = wc.w; w < wc.end; ++w) {
         const FirstWord fw = words[w];
-        const uint32_t r = segment_of_lane(off_r, R, w, n);
+        const uint32_t r = seg.of_lane(off_r, R, w, n);
         if (!((fw.x >> lane) & 1)) continue;
         const uint64_t q = fw.y + lanes_below(fw.x);
         const uint32_t v = in.at(w * kWave + lane, r);
@@ -261,6 +263,101 @@ __global__ __launch_bounds__(1024) void small_offsets_kernel(const uint32_t* __r
     __syncthreads();  // the offsets are read across the workgroup
     hop_offsets(foff, R, eoff, eoff_r, hb, h, out_off, threadIdx.x, 1024);
 }
+
+// A small pass in one launch of one workgroup, where launches are the time: the next frontier from at most
+// kOneWgEntries entries (dedup, ranks, compaction) and its draws' offsets, with everything the
+// separate kernels write.  desc: the batch's descriptors in host memory, copied to the device first
+// (the pass of the seeds).  The last hop's pass writes the edge total to *result (host memory).
+// The line: it took 6 us for 48 seeds and 41 us for 6400, where the four launches it replaces took 9
+// and 33 us one after the other (and about 5 us more each where the host submits them).
+constexpr uint32_t kSmallFront = 4096;
+static_assert(kSmallFront <= kOneWgEntries, "one workgroup holds a small pass");
+struct FrontOut {
+    uint32_t *fv, *fr, *fd, *fc;
+    uint64_t *eoff, *etot, *foff, *icount, *eoff_r, *hb, *out_off;
+    uint64_t* result;
+};
+template <class In>
+__global__ __launch_bounds__(kOneWgThreads) void small_front_kernel(In in, Count E, const uint64_t* off_r, uint32_t R,
+                                                                    uint32_t vb, const uint32_t* __restrict__ deg,
+                                                                    const KhReq* reqs, uint32_t h, FrontOut o,
+                                                                    const uint64_t* desc, uint64_t* desc_dev,
+                                                                    uint32_t desc_words) {
+    extern __shared__ unsigned long long front_lds[];
+    __shared__ OneWgFirsts f;
+    __shared__ uint32_t sums[kOneWgThreads / kWave];
+    if (desc) {
+        for (uint32_t i = threadIdx.x; i < desc_words; i += kOneWgThreads) desc_dev[i] = desc[i];
+        __syncthreads();
+    }
+    const uint32_t n = (uint32_t)E.get();
+    const uint64_t hbase = h ? o.hb[h] : 0;
+    one_wg_begin(f, front_lds, n, vb);
+    uint32_t slot[kOneWgPer], rr[kOneWgPer], vv[kOneWgPer];
+#pragma unroll
+    for (uint32_t i = 0; i < kOneWgPer; ++i) {
+        const uint32_t p = i * kOneWgThreads + threadIdx.x;
+        slot[i] = ~0u;
+        if (p < n) {
+            rr[i] = segment_in(off_r, 0, R - 1, p);
+            vv[i] = in.at(p, rr[i]);
+            if (vv[i] != kInvalid) slot[i] = f.insert(rr[i], vv[i], p);
+        }
+    }
+    const uint32_t mine = one_wg_rank(f, n, slot);
+    // the frontier, its draws kept in the table's memory for their scan
+    uint32_t* draws = (uint32_t*)front_lds;
+#pragma unroll
+    for (uint32_t i = 0; i < kOneWgPer; ++i) {
+        if (!((mine >> i) & 1)) continue;
+        const uint32_t q = f.rank(i * kOneWgThreads + threadIdx.x), d = deg[vv[i]];
+        const KhReq& k = reqs[rr[i]];
+        const uint32_t c = min(d, h < k.hops ? k.fan[h] : 0u);
+        o.fv[q] = vv[i];
+        o.fr[q] = rr[i];
+        o.fd[q] = d;
+        o.fc[q] = c;
+        draws[q] = c;
+    }
+    __syncthreads();
+    const uint32_t I = f.total, per = (I + kOneWgThreads - 1) / kOneWgThreads, i0 = threadIdx.x * per;
+    uint32_t c[kOneWgPer], s = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kOneWgPer; ++k) {
+        c[k] = k < per && i0 + k < I ? draws[i0 + k] : 0u;
+        s += c[k];
+    }
+    uint32_t total;
+    uint32_t pre = block_exclusive_sum<uint32_t, kOneWgThreads>(s, total, sums);
+#pragma unroll
+    for (uint32_t k = 0; k < kOneWgPer; ++k) {
+        if (k < per && i0 + k < I) {
+            draws[i0 + k] = pre;
+            o.eoff[i0 + k] = pre;
+        }
+        pre += c[k];
+    }
+    if (threadIdx.x == 0) {
+        o.eoff[I] = total;
+        *o.etot = total;
+        *o.icount = I;
+        if (h == 0) o.hb[0] = 0;
+        o.hb[h + 1] = hbase + total;
+        if (o.result) *o.result = hbase + total;
+    }
+    __syncthreads();
+    for (uint32_t r = threadIdx.x; r <= R; r += kOneWgThreads) {
+        const uint32_t p = (uint32_t)off_r[r];
+        const uint32_t fo = p < n ? f.rank(p) : I;
+        const uint64_t e = fo < I ? draws[fo] : total;
+        o.foff[r] = fo;
+        o.eoff_r[r] = e;
+        o.out_off[(uint64_t)h * (R + 1) + r] = hbase + e;
+    }
+}
+
+// LDS of small_front_kernel for at most n entries.
+static size_t small_front_lds(uint32_t n) { return (size_t)one_wg_slots(n) * 8; }
 
 // Start of a batch: zeroed scalars, all-one first words, empty table slots.
 __global__ __launch_bounds__(256) void khop_init_kernel(uint64_t* sc, uint32_t nsc, FirstWord* words, uint64_t nwords,
@@ -541,15 +638,20 @@ static unsigned sample_grid() {
     return grid;
 }
 
+constexpr uint64_t kGroupLanes = 1u << 18;  // half the chip's lanes
+
 // Hop h in `lanes` layout (SampleLanes) with groups of G lanes: the smallest of 4, 6, 8, 10, 12,
 // 16, 21, 32, 64 that covers the hop's largest fanout (twice that with the tuned scale 2), so that
 // a fanout-10 hop runs six vertices per wave instead of four in 16-lane groups.  kLanesAuto
-// launches both kernels and the one the hop does not take returns at once.
+// launches both kernels and the one the hop does not take returns at once; a frontier of so few items
+// (`items` at most) that every one gets its group in the first pass takes groups without asking, since
+// the second launch (4.7 us) would cost more than idle lanes.
 template <int FMT>
-static void launch_sample(grass_graph* g, uint32_t G, uint32_t fmax, int lanes, hipStream_t s,
+static void launch_sample(grass_graph* g, uint32_t G, uint32_t fmax, int lanes, uint64_t items, hipStream_t s,
                           const uint32_t* fv, const uint32_t* fr, const uint32_t* fd, const uint64_t* ic,
                           const KhReq* reqs, uint32_t h, uint64_t seed, const uint64_t* eoff, const uint64_t* hb,
                           uint32_t* osrc, uint32_t* odst, uint64_t cap, uint32_t* err) {
+    if (lanes == kLanesAuto && items * G <= kGroupLanes) lanes = kLanesGroups;
     if (lanes != kLanesGroups) {
         static unsigned grid = 0;
         if (!grid) grid = persistent_grid((const void*)sample_packed_kernel<FMT>, kKhBlock);
@@ -779,18 +881,44 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
         return hipGetLastError();
     };
 
-    e = hipMemcpyAsync(d_req, hreq, R * sizeof(KhReq) + (R + 1) * 8, hipMemcpyHostToDevice, s);
-    if (e != hipSuccess) return status_of(e);
+    // A pass of at most kSmallFront entries (and requests) is one launch of one workgroup; the
+    // pass of the seeds then also brings the descriptors over.  (GRASS_KHOP_SLOT=16 asks for a table in
+    // memory.)
+    const bool small_seeds = packed && S <= kSmallFront && R <= kSmallFront,
+               small_hops = Dmax <= kSmallFront && small_seeds;
+    auto small_front = [&](auto in, Count E, const uint64_t* off_r, uint32_t pass, uint32_t h, int k) {
+        using In = decltype(in);
+        const size_t lds = small_front_lds((uint32_t)(pass ? Dmax : S));
+        if (lds > 65536) {
+            (void)hipFuncSetAttribute((const void*)small_front_kernel<In>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            (void)hipGetLastError();
+        }
+        const FrontOut o{d_fv[k], d_fr[k], d_fd[k], d_fc[k], d_eoff, d_etot, d_foff[k], d_icount[k], d_eoff_r, d_hb,
+                         out->offsets_dev, h + 1 == H ? ws.result_slot() : nullptr};
+        const uint64_t desc_words = (R * sizeof(KhReq) + (R + 1) * 8) / 8;
+        hipLaunchKernelGGL(small_front_kernel<In>, dim3(1), dim3(kOneWgThreads), lds, s, in, E, off_r, R, vb, (const uint32_t*)g->d_deg, (const KhReq*)d_req, h, o,
+                           pass ? nullptr : (const uint64_t*)hreq, (uint64_t*)d_req, (uint32_t)desc_words);
+    };
+    if (!small_seeds) {
+        e = hipMemcpyAsync(d_req, hreq, R * sizeof(KhReq) + (R + 1) * 8, hipMemcpyHostToDevice, s);
+        if (e != hipSuccess) return status_of(e);
+    }
     const uint64_t clear = packed && tables.at_once ? tables.slots : 0;
-    hipLaunchKernelGGL(khop_init_kernel, dim3((unsigned)std::min<uint64_t>((std::max(clear / 2, nwords) + 255) / 256, 4096)),
-                       dim3(256), 0, s, d_sc, 64u, d_words, nwords, (unsigned long long*)ws.ht.ptr, clear);
+    if (!small_seeds || (H > 1 && !small_hops))
+        hipLaunchKernelGGL(khop_init_kernel,
+                           dim3((unsigned)std::min<uint64_t>((std::max(clear / 2, nwords) + 255) / 256, 4096)), dim3(256), 0,
+                           s, d_sc, 64u, d_words, nwords, (unsigned long long*)ws.ht.ptr, clear);
 
     // frontier 0: seeds, deduplicated
     {
         const SeedIn in{d_req, d_sbeg, (uint32_t)g->n, err};
-        if (S) insert(in, Count{S, nullptr}, d_sbeg, 0);
-        e = next_frontier(in, Count{S, nullptr}, d_sbeg, 0, 0, 0);
-        if (e != hipSuccess) return status_of(e);
+        if (small_seeds) {
+            small_front(in, Count{S, nullptr}, d_sbeg, 0, 0, 0);
+        } else {
+            insert(in, Count{S, nullptr}, d_sbeg, 0);
+            e = next_frontier(in, Count{S, nullptr}, d_sbeg, 0, 0, 0);
+            if (e != hipSuccess) return status_of(e);
+        }
     }
     // group width of each hop and the hop's largest fanout; the tuned scale picks the layout:
     // 0 packed lanes, 1 packed or groups as the hop's draws fill the groups, 2 groups of twice
@@ -814,7 +942,9 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     }
     for (uint32_t h = 0; h < H; ++h) {
         const int cur = h & 1, nxt = cur ^ 1;
-        if (Imax <= kOneWgItems) {
+        const bool small_pass = h ? small_hops : small_seeds;  // the frontier came with its offsets
+        if (small_pass) {
+        } else if (Imax <= kOneWgItems) {
             hipLaunchKernelGGL(small_offsets_kernel, dim3(1), dim3(1024), 0, s, (const uint32_t*)d_fc[cur],
                                (const uint64_t*)d_icount[cur], d_eoff, d_etot, (const uint64_t*)d_foff[cur], R, d_eoff_r,
                                d_hb, h, out->offsets_dev);
@@ -825,19 +955,23 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
                                d_eoff_r, d_hb, h, out->offsets_dev);
         }
         if (g->fmt == kLE)
-            launch_sample<kLE>(g, lanes[h], fmax[h], layout, s, d_fv[cur], d_fr[cur], d_fd[cur], d_icount[cur],
+            launch_sample<kLE>(g, lanes[h], fmax[h], layout, h ? Imax : S, s, d_fv[cur], d_fr[cur], d_fd[cur], d_icount[cur],
                                d_req, h, seed, d_eoff, d_hb, out->src_dev, out->dst_dev, out->capacity, err);
         else
-            launch_sample<kGT>(g, lanes[h], fmax[h], layout, s, d_fv[cur], d_fr[cur], d_fd[cur], d_icount[cur],
+            launch_sample<kGT>(g, lanes[h], fmax[h], layout, h ? Imax : S, s, d_fv[cur], d_fr[cur], d_fd[cur], d_icount[cur],
                                d_req, h, seed, d_eoff, d_hb, out->src_dev, out->dst_dev, out->capacity, err);
         if (h + 1 == H) break;
         const EdgeIn in{out->dst_dev, d_hb + h, out->capacity};
+        if (small_hops) {
+            small_front(in, Count{0, d_etot}, d_eoff_r, h + 1, h + 1, nxt);
+            continue;
+        }
         insert(in, Count{0, d_etot}, d_eoff_r, h + 1);
         e = next_frontier(in, Count{0, d_etot}, d_eoff_r, h + 1, h + 1, nxt);
         if (e != hipSuccess) return status_of(e);
     }
     e = hipGetLastError();
-    if (e == hipSuccess)
+    if (e == hipSuccess && !(H == 1 ? small_seeds : small_hops))
         e = hipMemcpyAsync(ws.result_slot(), d_hb + H, 8, hipMemcpyDeviceToHost, s);
     return status_of(e);
 }

@@ -5,9 +5,9 @@
 // into the same device buffers) pays the ~30 kernel launches of a 2-hop pipeline plus the walk
 // launch every step.  A plan runs the batch once eagerly (which sizes every workspace, so that
 // nothing allocates while capturing), then captures it with the walks and the k-hop pipeline on
-// two branches forked from the launch stream and joined back into it, and instantiates the graph.  Each replay starts with a clear of the k-hop
-// dedup table (the captured pipeline uses the table's first generations), so replays are
-// independent of each other and of any eager call.
+// two branches forked from the launch stream and joined back into it, and instantiates the graph.
+// Each replay starts with a clear of the k-hop dedup tables (the captured pipeline uses the 16-byte
+// table's first generations), so replays are independent of each other and of any eager call.
 #include <hip/hip_runtime.h>
 #include <string.h>
 
@@ -46,13 +46,11 @@ struct grass_plan {
     }
 
     // The batch: walks on s_main, the k-hop pipeline on s_side forked from and joined back into
-    // s_main, so that in the graph the two run side by side.
+    // s_main, so that in the graph the two run side by side.  The fork comes before the walks are
+    // enqueued: recorded behind them, the k-hop pipeline waited for the walks to end (a replay of 16
+    // walk requests, 178 us, and 16 k-hop requests, 95 us, took 273 us).
     int enqueue() {
         if (md) return mdrw_capture_enqueue(g, md, s_main);
-        if (!rw.empty()) {
-            int rc = rw_batch_enqueue(g, rw.data(), (uint32_t)rw.size(), seed, s_main, ws_rw, nullptr);
-            if (rc) return rc;
-        }
         if (!kh.empty()) {
             if (hipEventRecord(fork, s_main) != hipSuccess || hipStreamWaitEvent(s_side, fork, 0) != hipSuccess)
                 return GRASS_EDEVICE;
@@ -60,9 +58,14 @@ struct grass_plan {
             grass_khop_output o = kout;
             int rc = khop_enqueue(g, kh.data(), (uint32_t)kh.size(), seed, &o, s_side, ws_kh);
             if (rc) return rc;
-            if (hipEventRecord(join, s_side) != hipSuccess || hipStreamWaitEvent(s_main, join, 0) != hipSuccess)
-                return GRASS_EDEVICE;
         }
+        if (!rw.empty()) {
+            int rc = rw_batch_enqueue(g, rw.data(), (uint32_t)rw.size(), seed, s_main, ws_rw, nullptr);
+            if (rc) return rc;
+        }
+        if (!kh.empty() &&
+            (hipEventRecord(join, s_side) != hipSuccess || hipStreamWaitEvent(s_main, join, 0) != hipSuccess))
+            return GRASS_EDEVICE;
         return GRASS_OK;
     }
 };
