@@ -443,6 +443,22 @@ __device__ __forceinline__ uint32_t gt_element(const DevGraph& g, const Hdr& h, 
     return hd ? (blk >= h.fp ? v + raw + 1 : v - raw - 1) : abs ? raw : raw + 1;
 }
 
+// Runs (decode.hip): at most 4 consecutive positions of a list that decode without any other.
+constexpr uint32_t kRunMax = 4;    // positions of a run; the run kernel takes GT checkpoint intervals up to it
+constexpr uint32_t kLeRunShift = 2;  // LE: runs of 1 << 2 positions
+__host__ __device__ __forceinline__ uint32_t run_shift(int fmt, uint32_t cp_shift) {
+    return fmt == kLE ? kLeRunShift : cp_shift;
+}
+
+// Runs of a vertex with d entries in C chunks or blocks: R of q + 1 positions and C - R of q, each
+// ceil(len / 2^sh) runs, and LE's last rock.
+__host__ __device__ __forceinline__ uint64_t list_runs(int fmt, uint32_t d, uint32_t C, uint32_t q, uint32_t sh) {
+    if (!d) return 0;
+    if (fmt == kLE && d == 1) return 1;
+    const uint32_t D = fmt == kLE ? d - 1 : d, R = D - C * q, P1 = (1u << sh) - 1;
+    return (uint64_t)R * ((q + 1 + P1) >> sh) + (uint64_t)(C - R) * ((q + P1) >> sh) + (fmt == kLE ? 1 : 0);
+}
+
 // Division by a divisor every lane shares, as a multiply-high and one correction: with
 // m = floor(2^32 / d) the estimate floor(n * m / 2^32) is floor(n / d) or one less, n < 2^32.
 struct UDiv {

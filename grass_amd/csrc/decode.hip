@@ -242,18 +242,6 @@ __device__ __forceinline__ void decode_range(const DevGraph& g, const Src& src, 
 // runs, 0.32 with the above.  Loading each lane's header by itself instead of 64 headers and a
 // shuffle: GT 1.06 ms.
 
-constexpr uint32_t kRunMax = 4;    // positions of a run; the run kernel takes GT checkpoint intervals up to it
-constexpr uint32_t kLeRunShift = 2;  // LE: runs of 1 << 2 positions
-
-// Runs of a vertex with d entries in C chunks or blocks: R of q + 1 positions and C - R of q, each
-// ceil(len / 2^sh) runs, and LE's last rock.
-__host__ __device__ __forceinline__ uint64_t list_runs(int fmt, uint32_t d, uint32_t C, uint32_t q, uint32_t sh) {
-    if (!d) return 0;
-    if (fmt == kLE && d == 1) return 1;
-    const uint32_t D = fmt == kLE ? d - 1 : d, R = D - C * q, P1 = (1u << sh) - 1;
-    return (uint64_t)R * ((q + 1 + P1) >> sh) + (uint64_t)(C - R) * ((q + P1) >> sh) + (fmt == kLE ? 1 : 0);
-}
-
 struct RunGen {  // runs of vertex i, from its header
     const uint4* hdr;
     int fmt;
@@ -583,7 +571,10 @@ __global__ __launch_bounds__(kDecBlock) void decode_csr_kernel(DevGraph g,
 int decode_csr(grass_graph* g, uint64_t* rowptr, uint32_t* col, hipStream_t s) {
     const uint64_t n = g->n, m = g->m;
     const uint64_t nb = scan_blocks(n);
-    {
+    if (nb <= kScanDirectMax) {  // one launch, no partials
+        const hipError_t e = exclusive_scan(DegGen{g->d_deg}, Count{n, nullptr}, n, rowptr, nullptr, nullptr, s);
+        if (e != hipSuccess) return status_of(e);
+    } else {
         // The scan's partials have a buffer of their own, ordered between calls on the device:
         // each call's stream waits for the previous call's scan (on whatever stream) before its
         // own scan reuses the buffer, so no call waits on the host.
@@ -604,55 +595,54 @@ int decode_csr(grass_graph* g, uint64_t* rowptr, uint32_t* col, hipStream_t s) {
     while ((512u << slot) < per_wave && slot + 1 < kWaveStartSlots) ++slot;
     if ((512u << slot) != per_wave) return GRASS_EINVAL;
     // LE, and GT with P <= 4, decode by runs: about per_wave slots per wave, per_wave / P runs.  The
-    // run offsets (a scan over the headers) and the total are built once per graph.
-    const uint32_t sh = g->fmt == kLE ? kLeRunShift : g->cp_shift;
+    // run offsets (a scan over the headers) are built once per graph; their total is known since load.
+    const uint32_t sh = run_shift(g->fmt, g->cp_shift);
     const bool runs = (1u << sh) <= kRunMax;
     const uint32_t unit = runs ? per_wave >> sh : per_wave;
-    uint64_t units = m;
-    if (runs) {
-        std::lock_guard<std::mutex> lock(g->mu);
-        if (!g->d_roff) {
-            uint64_t* r = nullptr;
-            WorkMem m_part;
-            if (m_part.alloc((nb + 4) * 8, s) != hipSuccess) return GRASS_ENOMEM;
-            uint64_t* part = m_part.as<uint64_t>();
-            if (device_malloc((void**)&r, (n + 1) * 8) != hipSuccess) return GRASS_ENOMEM;
-            uint64_t total = 0;
-            hipError_t e = exclusive_scan(RunGen{g->d_hdr, g->fmt, sh}, Count{n, nullptr}, n, r, part, part + nb, s);
-            if (e == hipSuccess) e = hipMemcpyAsync(&total, r + n, 8, hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipStreamSynchronize(s);
-            if (e != hipSuccess) {
-                (void)hipFree(r);
-                return status_of(e);
-            }
-            g->d_roff = r;
-            g->dec_runs = total;
-        }
-        units = g->dec_runs;
-    }
-    const uint64_t* uoff = runs ? (const uint64_t*)g->d_roff : (const uint64_t*)rowptr;
+    const uint64_t units = runs ? g->dec_runs : m;
     const uint64_t waves = (units + unit - 1) / unit;
     const uint64_t blocks = (waves + kDecBlock / kWave - 1) / (kDecBlock / kWave);
     if (blocks > 0x7fffffffull) return GRASS_EINVAL;
     // The waves' first vertices depend only on the graph and per_wave: built once per per_wave
     // value from the row pointers (or the run offsets), complete before it is published, never
     // changed after.
+    const uint64_t* uoff;
     const uint32_t* wstart;
     {
         std::lock_guard<std::mutex> lock(g->mu);
-        if (!g->d_wstart[slot]) {
-            uint32_t* t = nullptr;
-            if (device_malloc((void**)&t, (waves + 1) * 4) != hipSuccess) return GRASS_ENOMEM;
-            const unsigned grid = (unsigned)std::min<uint64_t>((n + 255) / 256, 16384);
-            hipLaunchKernelGGL(wave_start_kernel, dim3(grid), dim3(256), 0, s, uoff, (uint32_t)n, unit, waves, t);
-            hipError_t e = hipGetLastError();
-            if (e == hipSuccess) e = hipStreamSynchronize(s);
-            if (e != hipSuccess) {
-                (void)hipFree(t);
-                return status_of(e);
+        uint64_t* r = g->d_roff;
+        uint32_t* t = g->d_wstart[slot];
+        const bool new_r = runs && !r, new_t = !t;
+        if (new_r || new_t) {
+            WorkMem m_part;
+            hipError_t e = hipSuccess;
+            if (new_r) {
+                if (m_part.alloc((nb + 4) * 8, s) != hipSuccess) return GRASS_ENOMEM;
+                if (device_malloc((void**)&r, (n + 1) * 8) != hipSuccess) return GRASS_ENOMEM;
+                uint64_t* part = m_part.as<uint64_t>();
+                e = exclusive_scan(RunGen{g->d_hdr, g->fmt, sh}, Count{n, nullptr}, n, r, part, part + nb, s);
             }
+            if (e == hipSuccess && new_t && device_malloc((void**)&t, (waves + 1) * 4) != hipSuccess) {
+                t = nullptr;
+                e = hipErrorOutOfMemory;
+            }
+            if (e == hipSuccess && new_t) {
+                const unsigned grid = (unsigned)std::min<uint64_t>((n + 255) / 256, 16384);
+                hipLaunchKernelGGL(wave_start_kernel, dim3(grid), dim3(256), 0, s, runs ? (const uint64_t*)r : (const uint64_t*)rowptr,
+                                   (uint32_t)n, unit, waves, t);
+                e = hipGetLastError();
+            }
+            const hipError_t done = hipStreamSynchronize(s);
+            if (e == hipSuccess) e = done;
+            if (e != hipSuccess) {
+                if (new_r && r) (void)hipFree(r);
+                if (new_t && t) (void)hipFree(t);
+                return e == hipErrorOutOfMemory ? GRASS_ENOMEM : status_of(e);
+            }
+            g->d_roff = r;
             g->d_wstart[slot] = t;
         }
+        uoff = runs ? (const uint64_t*)g->d_roff : (const uint64_t*)rowptr;
         wstart = g->d_wstart[slot];
     }
     if (runs && g->fmt == kLE) {

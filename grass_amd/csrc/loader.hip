@@ -43,16 +43,17 @@ struct OffsetFieldGen {
 
 constexpr int kValBlock = 256;
 
-// stats: [0] sum of degrees, [1] max degree, [2] malformed records, [3] first malformed vertex
+// stats: [0] sum of degrees, [1] max degree, [2] malformed records, [3] first malformed vertex,
+// [4] decode runs of 1 << run_sh positions
 template <int FMT>
 __global__ __launch_bounds__(kValBlock) void validate_kernel(const uint32_t* __restrict__ w,
                                                              const uint64_t* __restrict__ start,
                                                              uint32_t n, uint64_t gbits,
                                                              uint32_t* __restrict__ deg,
-                                                             uint4* __restrict__ hdr,
+                                                             uint4* __restrict__ hdr, uint32_t run_sh,
                                                              unsigned long long* stats) {
     __shared__ unsigned long long lds[kValBlock / kWave];
-    unsigned long long sum = 0, mx = 0, bad = 0;
+    unsigned long long sum = 0, mx = 0, bad = 0, runs = 0;
     for (uint32_t v = blockIdx.x * kValBlock + threadIdx.x; v < n; v += gridDim.x * kValBlock) {
         const uint64_t b0 = start[v], end = start[v + 1];
         uint64_t b = b0;
@@ -94,15 +95,18 @@ __global__ __launch_bounds__(kValBlock) void validate_kernel(const uint32_t* __r
         deg[v] = h.d;
         hdr[v] = pack_hdr(h, FMT);
         sum += h.d;
+        runs += list_runs(FMT, h.d, h.C, h.q, run_sh);
         mx = h.d > mx ? h.d : mx;
     }
     sum = block_sum<unsigned long long, kValBlock>(sum, lds);
     mx = block_max<unsigned long long, kValBlock>(mx, lds);
     bad = block_sum<unsigned long long, kValBlock>(bad, lds);
+    runs = block_sum<unsigned long long, kValBlock>(runs, lds);
     if (threadIdx.x == 0) {
         atomicAdd(&stats[0], sum);
         atomicMax(&stats[1], mx);
         if (bad) atomicAdd(&stats[2], bad);
+        atomicAdd(&stats[4], runs);
     }
 }
 
@@ -378,10 +382,10 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
     if (device_malloc((void**)&g->d_hdr, hdr_bytes) != hipSuccess) return GRASS_ENOMEM;
     const uint64_t nb = scan_blocks(n);
     if (m_tmp.alloc((nb + 8) * 8, s) != hipSuccess) return GRASS_ENOMEM;
-    uint64_t* d_tmp = m_tmp.as<uint64_t>();  // partials[nb], total, stats[4]
+    uint64_t* d_tmp = m_tmp.as<uint64_t>();  // partials[nb], total, stats[5]
     uint64_t* d_total = d_tmp + nb;
     unsigned long long* d_stats = (unsigned long long*)(d_tmp + nb + 2);
-    unsigned long long init[4] = {0, 0, 0, ~0ull};
+    unsigned long long init[5] = {0, 0, 0, ~0ull, 0};
     hipError_t e = hipMemcpyAsync(d_stats, init, sizeof(init), hipMemcpyHostToDevice, s);
     if (e == hipSuccess)
         e = exclusive_scan(OffsetFieldGen{d_off, ubl}, Count{n, nullptr}, n, g->d_start, d_tmp,
@@ -390,14 +394,16 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
         unsigned grid = (unsigned)std::min<uint64_t>((n + kValBlock - 1) / kValBlock, 16384);
         if (g->fmt == kLE)
             hipLaunchKernelGGL(validate_kernel<kLE>, dim3(grid), dim3(kValBlock), 0, s, g->d_words,
-                               g->d_start, (uint32_t)n, 8 * gbytes, g->d_deg, g->d_hdr, d_stats);
+                               g->d_start, (uint32_t)n, 8 * gbytes, g->d_deg, g->d_hdr,
+                               run_shift(g->fmt, g->cp_shift), d_stats);
         else
             hipLaunchKernelGGL(validate_kernel<kGT>, dim3(grid), dim3(kValBlock), 0, s, g->d_words,
-                               g->d_start, (uint32_t)n, 8 * gbytes, g->d_deg, g->d_hdr, d_stats);
+                               g->d_start, (uint32_t)n, 8 * gbytes, g->d_deg, g->d_hdr,
+                               run_shift(g->fmt, g->cp_shift), d_stats);
         e = hipGetLastError();
     }
     uint64_t total = 0;
-    unsigned long long stats[4] = {0, 0, 0, 0};
+    unsigned long long stats[5] = {0, 0, 0, 0, 0};
     if (e == hipSuccess) e = hipMemcpyAsync(&total, d_total, 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipMemcpyAsync(stats, d_stats, sizeof(stats), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -408,6 +414,7 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
     g->total_bits = total;
     g->m = stats[0];
     g->max_degree = stats[1];
+    g->dec_runs = stats[4];
     uint64_t xwords = 0;
     if (g->fmt == kGT) {
         int rc2 = build_gt_stream(g, &xwords);

@@ -192,7 +192,7 @@ struct grass_graph {
     // GT with P <= 4: of every wave's first run, the waves taking (512 << i) / P runs each)
     uint32_t* d_wstart[grass::kWaveStartSlots] = {};
     uint64_t* d_roff = nullptr;  // full decode by runs: runs before each vertex (n + 1)
-    uint64_t dec_runs = 0;       // and their total
+    uint64_t dec_runs = 0;       // and their total (set at load)
     grass::Scratch dec_part;     // full decode: the row-pointer scan's partials (under mu)
     hipEvent_t dec_ev = nullptr;  // recorded after each full decode's scan
     hipStream_t stream = nullptr;

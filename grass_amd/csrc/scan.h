@@ -3,7 +3,8 @@
 // Launches with no inter-workgroup waiting: per-tile sums, then each tile re-generates its values
 // and writes prefixes.  A sequence of at most kScanFoldMax tiles has each tile add up the tile sums
 // before it itself (a few thousand cached values); a longer one scans the tile sums in one
-// workgroup in between (a third launch).  The length can be
+// workgroup in between (a third launch).  Of at most kScanDirectMax tiles each generates the values
+// before it itself and one launch does it all.  The length can be
 // a host value or a device-resident count (so a sequence whose size a previous kernel
 // produced needs no host round trip); the grid is sized for the host-side upper bound.
 // Used for the record-length scan at load (replacing cub::DeviceScan::ExclusiveSum,
@@ -20,6 +21,11 @@ constexpr int kScanBlock = 256;
 constexpr int kScanItems = 16;
 constexpr uint64_t kScanTile = (uint64_t)kScanBlock * kScanItems;
 constexpr uint64_t kScanFoldMax = 2048;  // tiles whose start each tile sums itself
+// Tiles whose start each tile sums from the values (the generator must not read what is written): a
+// launch saved against up to 48 more values per thread.  A full decode of R-MAT s14 (16 k rows, 148 k
+// entries), whose calls the host's launches bound, went from 14.4 to 10.2 us with the one launch.
+constexpr uint64_t kScanDirectMax = 4;
+enum ScanMode { kScanDirect, kScanFold, kScanThree };
 
 struct Count {
     uint64_t imm;
@@ -85,14 +91,16 @@ __device__ __forceinline__ uint64_t wave_inclusive_sum_u64(uint64_t x) {
 // kWave * kScanItems consecutive items in kScanItems rounds of kWave consecutive ones (coalesced
 // loads and stores): its lanes' sums and one exchange of the wave sums give each wave its start,
 // and each round is one DPP wave scan carried into the next (no workgroup scan per round).
-// FOLD: partials[] are the tile sums themselves (at most kScanFoldMax of them): each tile adds up
-// those before it, and the tile holding item n - 1 also writes *total; otherwise partials[] are
+// kScanFold: partials[] are the tile sums themselves (at most kScanFoldMax of them): each tile adds up
+// those before it, and the tile holding item n - 1 also writes *total; kScanDirect: the same from the
+// values themselves, partials[] unread; kScanThree: partials[] are
 // the tiles' exclusive prefixes and *total was written with them.  Outputs lie STRIDE words apart.
-template <class Gen, bool FOLD, int STRIDE>
+template <class Gen, ScanMode MODE, int STRIDE>
 __global__ __launch_bounds__(kScanBlock) void scan_write_kernel(Gen gen, Count cnt,
                                                                 const uint64_t* partials,
                                                                 uint64_t* total,
                                                                 uint64_t* out) {
+    constexpr bool FOLD = MODE != kScanThree;
     __shared__ uint64_t wsum[kScanBlock / kWave];
     __shared__ uint64_t fold_lds[kScanBlock / kWave];
     const uint64_t n = cnt.get();
@@ -107,7 +115,12 @@ __global__ __launch_bounds__(kScanBlock) void scan_write_kernel(Gen gen, Count c
     uint64_t start;
     if (FOLD) {
         uint64_t p = 0;
-        for (uint64_t k = threadIdx.x; k < blockIdx.x; k += kScanBlock) p += partials[k];
+        if (MODE == kScanDirect) {
+#pragma unroll 8
+            for (uint64_t k = threadIdx.x; k < base; k += kScanBlock) p += gen(k);
+        } else {
+            for (uint64_t k = threadIdx.x; k < blockIdx.x; k += kScanBlock) p += partials[k];
+        }
         start = block_sum<uint64_t, kScanBlock>(p, fold_lds);
     } else {
         start = partials[blockIdx.x];
@@ -153,14 +166,19 @@ template <int STRIDE = 1, class Gen>
 hipError_t exclusive_scan(Gen gen, Count cnt, uint64_t n_max, uint64_t* out, uint64_t* partials,
                           uint64_t* total, hipStream_t stream) {
     const uint64_t nb = scan_blocks(n_max);
+    if (nb <= kScanDirectMax) {
+        hipLaunchKernelGGL((scan_write_kernel<Gen, kScanDirect, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
+                           gen, cnt, (const uint64_t*)nullptr, total, out);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(scan_reduce_kernel<Gen>, dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
                        gen, cnt, partials);
     if (nb <= kScanFoldMax) {
-        hipLaunchKernelGGL((scan_write_kernel<Gen, true, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
+        hipLaunchKernelGGL((scan_write_kernel<Gen, kScanFold, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
                            gen, cnt, (const uint64_t*)partials, total, out);
     } else {
         hipLaunchKernelGGL(scan_partials_kernel<uint64_t>, dim3(1), dim3(1024), 0, stream, partials, nb, total);
-        hipLaunchKernelGGL((scan_write_kernel<Gen, false, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
+        hipLaunchKernelGGL((scan_write_kernel<Gen, kScanThree, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
                            gen, cnt, (const uint64_t*)partials, total, out);
     }
     return hipGetLastError();
