@@ -92,6 +92,10 @@ struct DeviceGuard {
     }
 };
 
+hipStream_t pick(grass_graph* g, void* stream) { return stream ? (hipStream_t)stream : g->stream; }
+
+}  // namespace
+
 void free_graph(grass_graph* g) {
     if (!g) return;
     if (g->d_words) (void)hipFree(g->d_words);
@@ -111,15 +115,8 @@ void free_graph(grass_graph* g) {
     delete g;
 }
 
-
-hipStream_t pick(grass_graph* g, void* stream) { return stream ? (hipStream_t)stream : g->stream; }
-
-}  // namespace
-
-int open_sources(ByteSource& gs, ByteSource& os, int format, int device, grass_graph** out) {
-    if (!out) return GRASS_EINVAL;
+int new_graph(int format, int device, grass_graph** out) {
     *out = nullptr;
-    if (format != GRASS_FMT_LE && format != GRASS_FMT_GT) return GRASS_EINVAL;
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return GRASS_EDEVICE;
     if (device < 0 || device >= ndev) return GRASS_EINVAL;
@@ -139,7 +136,23 @@ int open_sources(ByteSource& gs, ByteSource& os, int format, int device, grass_g
     if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess) rc = GRASS_EDEVICE;
     if (!rc && hipMalloc(&g->d_err, 64) != hipSuccess) rc = GRASS_ENOMEM;
     if (!rc && hipMemset(g->d_err, 0, 64) != hipSuccess) rc = GRASS_EDEVICE;
-    if (!rc) rc = load_graph(g, gs, os);
+    if (rc) {
+        free_graph(g);
+        return rc;
+    }
+    *out = g;
+    return GRASS_OK;
+}
+
+int open_sources(ByteSource& gs, ByteSource& os, int format, int device, grass_graph** out) {
+    if (!out) return GRASS_EINVAL;
+    *out = nullptr;
+    if (format != GRASS_FMT_LE && format != GRASS_FMT_GT) return GRASS_EINVAL;
+    grass_graph* g = nullptr;
+    int rc = new_graph(format, device, &g);
+    if (rc) return rc;
+    DeviceGuard guard(device);
+    rc = guard.ok ? load_graph(g, gs, os) : GRASS_EDEVICE;
     if (rc) {
         free_graph(g);
         return rc;

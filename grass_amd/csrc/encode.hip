@@ -2,6 +2,9 @@
 // (the reference's "normal" compressors, LE/chunk_compress/compressor.hpp:49-71,288-403 and
 // GT/chunk_compress/compressor.hpp:49-62,245-349), computed from a CSR resident in device memory.
 //
+// Rows that are strictly ascending, ids below 2^31 (encode_flat.h): by slots, 64 fields of any records a
+// pass, into the images or, for a graph that is opened right away, into the words, headers and degrees
+// it keeps resident, without the images.  Other rows:
 // 1. enc_plan_kernel, one wave per vertex: the record's field widths (LE rock_bit, sea_bit,
 //    first_pos; GT head_bit, body_bit, first_pos) as maxima over the list, and its length.
 // 2. An exclusive scan of the lengths: the bit where each record starts.
@@ -9,7 +12,7 @@
 //    (LE: rocks, then signed seas; GT: per block the head, then the bodies), so the header's gamma
 //    codes and 64 fields at a time are assembled in LDS and stored; only the words a record shares
 //    with its neighbours are ORed into memory.
-// 4. enc_offset_kernel: the .offset image, byte 0 = ubl then n length fields of ubl bits.
+// Then enc_offset_kernel: the .offset image, byte 0 = ubl then n length fields of ubl bits.
 // The stream is MSB-first in big-endian-bit words; .graph words are stored byte-swapped, so that
 // memory holds the file's bytes, and the .offset words are swapped after assembly.
 #include <hip/hip_runtime.h>
@@ -20,6 +23,7 @@
 #include "../../include/grass_ingest.h"
 #include "blob.h"
 #include "devutil.h"
+#include "encode_flat.h"
 #include "runtime.h"
 #include "scan.h"
 
@@ -29,17 +33,6 @@ namespace {
 constexpr int kEncBlock = 256;
 constexpr int kEncWaves = kEncBlock / kWave;
 constexpr uint32_t kEncWords = kWave + 2;  // words one pass of 64 fields of <= 32 bits can touch
-
-// get_bit_num (compressor.hpp:16-22): bit length of |x|, 1 for 0.
-__device__ __forceinline__ uint32_t bit_num(int64_t x) {
-    if (x < 0) x = -x;
-    return x == 0 ? 1u : 64u - (uint32_t)__clzll((unsigned long long)x);
-}
-
-// Length of the Elias-gamma code of x + 1 (compressor.hpp:411-417).
-__device__ __forceinline__ uint32_t gamma_bits(uint64_t x) {
-    return 2u * (63u - (uint32_t)__clzll((unsigned long long)(x + 1))) + 1u;
-}
 
 // GT head field as the reference writes it: |N - v| - 1, a self loop (-1) coming out as 1
 // (GT/chunk_compress/compressor.hpp:407-419 keeps the low bit of -1).
@@ -162,15 +155,6 @@ struct RecState {   // wave-uniform
     uint64_t pend_w;  // its index, ~0 when nothing is carried
     bool pend_first;  // it is the record's first word
 };
-
-// Elias-gamma code of x + 1 (x + 1 < 2^32) at stream bit `at` of the pass buffer: L zero bits,
-// then x + 1 in L + 1 bits.
-__device__ __forceinline__ void put_gamma(uint32_t* B, uint64_t w0, uint64_t& at, uint32_t x) {
-    const uint32_t y = x + 1;
-    const uint32_t L = 31u - (uint32_t)__clz(y);
-    put_field(B, w0, at + L, L + 1, y);
-    at += 2 * L + 1;
-}
 
 // One pass over stream bits [from, ...): the header codes hv[0..nh) at `from` (first pass only,
 // written by lane 0), then up to 64 fields, lane l holding field l at `at` (act: the lane has one,
@@ -383,60 +367,132 @@ struct Images {
     uint64_t gbytes = 0, obytes = 0;
 };
 
-int encode_images(const uint64_t* rowptr, const uint32_t* col, uint64_t n, int format, hipStream_t s,
-                  Images& im) {
-    const bool le = format == GRASS_FMT_LE;
+// A plan over the slots of a CSR: every record's widths, and where it starts (bits, or words of the GT
+// stream).
+struct FlatPlan {
+    WorkMem mem;
+    uint64_t* len = nullptr;
+    uint64_t* start = nullptr;
+    uint2* widths = nullptr;
+    FlatStats st{};
+    unsigned grid = 0;
+};
+
+template <int FMT, bool STREAM>
+int flat_plan(const uint64_t* rowptr, const uint32_t* col, uint64_t n, uint32_t sh, hipStream_t s, FlatPlan& p) {
     const uint64_t nb = scan_blocks(n);
-    WorkMem tmp;  // len[n], start[n + 1], widths[n], partials, total, maxlen
-    Carve need(nullptr);
-    auto plan = [&](Carve& c, uint64_t** len, uint64_t** start, uint2** widths, uint64_t** part,
-                    unsigned long long** most) {
-        *len = c.take<uint64_t>(n);
-        *start = c.take<uint64_t>(n + 1);
-        *widths = c.take<uint2>(n);
-        *part = c.take<uint64_t>(nb + 2);
-        *most = c.take<unsigned long long>(1);
+    uint32_t* fps = nullptr;
+    uint64_t* part = nullptr;
+    FlatStats* d_st = nullptr;
+    auto layout = [&](Carve& c) {
+        p.len = c.take<uint64_t>(n);
+        p.start = c.take<uint64_t>(n + 1);
+        p.widths = c.take<uint2>(n);
+        fps = c.take<uint32_t>(n);
+        part = c.take<uint64_t>(nb + 2);
+        d_st = c.take<FlatStats>(1);
     };
-    uint64_t *d_len, *d_start, *d_part;
-    uint2* d_w;
-    unsigned long long* d_max;
-    plan(need, &d_len, &d_start, &d_w, &d_part, &d_max);
-    if (tmp.alloc(need.off + 256, s) != hipSuccess) return GRASS_ENOMEM;
-    Carve c(tmp.p);
-    plan(c, &d_len, &d_start, &d_w, &d_part, &d_max);
+    Carve need(nullptr);
+    layout(need);
+    if (p.mem.alloc(need.off + 256, s) != hipSuccess) return GRASS_ENOMEM;
+    Carve c(p.mem.p);
+    layout(c);
+    uint2* ors = (uint2*)p.start;  // until the scan
     int dev = 0, cus = 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    const unsigned grid = (unsigned)std::max(cus, 1) * 16;
-    hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3(1), dim3(64), 0, s, d_max, (uint64_t)1, 0ull);
-    if (le)
-        hipLaunchKernelGGL(enc_plan_kernel<kLE>, dim3(grid), dim3(kEncBlock), 0, s, rowptr, col, n, d_len, d_w, d_max);
-    else
-        hipLaunchKernelGGL(enc_plan_kernel<kGT>, dim3(grid), dim3(kEncBlock), 0, s, rowptr, col, n, d_len, d_w, d_max);
-    hipError_t e = exclusive_scan(LenGen{d_len}, Count{n, nullptr}, n, d_start, d_part, d_part + nb + 1, s);
-    uint64_t hv[2] = {0, 0};  // total bits, longest record
-    if (e == hipSuccess) e = hipMemcpyAsync(&hv[0], d_start + n, 8, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(&hv[1], d_max, 8, hipMemcpyDeviceToHost, s);
+    p.grid = (unsigned)std::max(cus, 1) * 8;
+    const unsigned gn = (unsigned)std::min<uint64_t>((n + kFlatBlock - 1) / kFlatBlock, p.grid);
+    hipLaunchKernelGGL(fill_kernel<uint64_t>, dim3(gn), dim3(256), 0, s, (uint64_t*)ors, n, 0ull);
+    hipLaunchKernelGGL(fill_kernel<uint64_t>, dim3(1), dim3(64), 0, s, (uint64_t*)d_st, (uint64_t)(sizeof(FlatStats) / 8), 0ull);
+    hipLaunchKernelGGL(flat_plan_kernel<FMT>, dim3(p.grid), dim3(kFlatBlock), 0, s, rowptr, col, n, ors, fps, d_st);
+    // (each workgroup adds to the same few totals, one after another: 2048 workgroups took
+    // 133 us, 512 take 51)
+    hipLaunchKernelGGL((flat_vertex_kernel<FMT, STREAM>), dim3(std::min(gn, (unsigned)std::max(cus, 1) * 2)), dim3(kFlatBlock), 0, s, rowptr, col, n, (const uint2*)ors,
+                       (const uint32_t*)fps, sh, p.len, p.widths, d_st);
+    hipError_t e = exclusive_scan(LenGen{p.len}, Count{n, nullptr}, n, p.start, part, part + nb + 1, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(&p.st, d_st, sizeof(FlatStats), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) return status_of(e);
-    const uint64_t total = hv[0], maxlen = hv[1];
+    return status_of(e);
+}
+
+template <int FMT, FlatOut OUT>
+void flat_write(const FlatPlan& p, const uint64_t* rowptr, const uint32_t* col, uint64_t n, uint32_t sh, uint32_t* out,
+                hipStream_t s) {
+    hipLaunchKernelGGL((flat_write_kernel<FMT, OUT>), dim3(p.grid), dim3(kFlatBlock), 0, s, rowptr, col, n,
+                       (const uint64_t*)p.start, (const uint2*)p.widths, sh, out);
+}
+
+// A plan by enc_plan_kernel, for rows that the slots' kernels do not take.
+int general_plan(const uint64_t* rowptr, const uint32_t* col, uint64_t n, bool le, hipStream_t s, FlatPlan& p) {
+    const uint64_t nb = scan_blocks(n);
+    uint64_t* part = nullptr;
+    unsigned long long* most = nullptr;
+    auto layout = [&](Carve& c) {
+        p.len = c.take<uint64_t>(n);
+        p.start = c.take<uint64_t>(n + 1);
+        p.widths = c.take<uint2>(n);
+        part = c.take<uint64_t>(nb + 2);
+        most = c.take<unsigned long long>(1);
+    };
+    Carve need(nullptr);
+    layout(need);
+    p.mem.reset();
+    if (p.mem.alloc(need.off + 256, s) != hipSuccess) return GRASS_ENOMEM;
+    Carve c(p.mem.p);
+    layout(c);
+    p.grid *= 2;
+    hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3(1), dim3(64), 0, s, most, (uint64_t)1, 0ull);
+    if (le)
+        hipLaunchKernelGGL(enc_plan_kernel<kLE>, dim3(p.grid), dim3(kEncBlock), 0, s, rowptr, col, n, p.len, p.widths, most);
+    else
+        hipLaunchKernelGGL(enc_plan_kernel<kGT>, dim3(p.grid), dim3(kEncBlock), 0, s, rowptr, col, n, p.len, p.widths, most);
+    hipError_t e = exclusive_scan(LenGen{p.len}, Count{n, nullptr}, n, p.start, part, part + nb + 1, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(&p.st.bits, p.start + n, 8, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipMemcpyAsync(&p.st.longest, most, 8, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    return status_of(e);
+}
+
+// ubl = get_bit_num(longest record)
+uint32_t offset_width(uint64_t longest) {
+    uint32_t ubl = 1;
+    while (ubl < 64 && (longest >> ubl)) ++ubl;
+    return ubl;
+}
+
+int encode_images(const uint64_t* rowptr, const uint32_t* col, uint64_t n, int format, hipStream_t s,
+                  Images& im) {
+    const bool le = format == GRASS_FMT_LE;
+    FlatPlan p;
+    int rc = le ? flat_plan<kLE, false>(rowptr, col, n, 0, s, p) : flat_plan<kGT, false>(rowptr, col, n, 0, s, p);
+    const bool general = p.st.flags & kFlatGeneral;
+    if (!rc && general) rc = general_plan(rowptr, col, n, le, s, p);
+    if (rc) return rc;
+    const uint64_t total = p.st.bits;
     if (total >= (1ull << 40)) return GRASS_EINVAL;  // past what a reader's 40-bit offsets address
     // .graph
     const uint64_t gwords = (total + 31) / 32 + 2;
     WorkMem& gbuf = im.g;
     if (gbuf.alloc(gwords * 4, s) != hipSuccess) return GRASS_ENOMEM;
     uint32_t* d_g = (uint32_t*)gbuf.p;
-    e = hipMemsetAsync(d_g, 0, gwords * 4, s);
-    if (e != hipSuccess) return status_of(e);
-    if (le)
-        hipLaunchKernelGGL(enc_write_kernel<kLE>, dim3(grid), dim3(kEncBlock), 0, s, rowptr, col, n,
-                           (const uint64_t*)d_start, (const uint2*)d_w, d_g);
-    else
-        hipLaunchKernelGGL(enc_write_kernel<kGT>, dim3(grid), dim3(kEncBlock), 0, s, rowptr, col, n,
-                           (const uint64_t*)d_start, (const uint2*)d_w, d_g);
-    // .offset: ubl = get_bit_num(longest record), then the n lengths
-    uint32_t ubl = 1;
-    while (ubl < 64 && (maxlen >> ubl)) ++ubl;
+    hipError_t e = hipSuccess;
+    if (general) {
+        e = hipMemsetAsync(d_g, 0, gwords * 4, s);
+        if (e != hipSuccess) return status_of(e);
+        if (le)
+            hipLaunchKernelGGL(enc_write_kernel<kLE>, dim3(p.grid), dim3(kEncBlock), 0, s, rowptr, col, n,
+                               (const uint64_t*)p.start, (const uint2*)p.widths, d_g);
+        else
+            hipLaunchKernelGGL(enc_write_kernel<kGT>, dim3(p.grid), dim3(kEncBlock), 0, s, rowptr, col, n,
+                               (const uint64_t*)p.start, (const uint2*)p.widths, d_g);
+    } else if (le) {
+        flat_write<kLE, kFlatImage>(p, rowptr, col, n, 0, d_g, s);
+    } else {
+        flat_write<kGT, kFlatImage>(p, rowptr, col, n, 0, d_g, s);
+    }
+    // .offset: ubl, then the n lengths
+    const uint32_t ubl = offset_width(p.st.longest);
     const uint64_t obits = 8 + n * (uint64_t)ubl;
     const uint64_t owords = (obits + 63) / 64 + 1;
     WorkMem& obuf = im.o;
@@ -447,13 +503,55 @@ int encode_images(const uint64_t* rowptr, const uint32_t* col, uint64_t n, int f
     hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3(1), dim3(64), 0, s, d_o, (uint64_t)1,
                        (unsigned long long)ubl << 56);
     hipLaunchKernelGGL(enc_offset_kernel, dim3((unsigned)std::min<uint64_t>((n + 255) / 256, 16384)), dim3(256), 0, s,
-                       (const uint64_t*)d_len, n, ubl, d_o);
+                       (const uint64_t*)p.len, n, ubl, d_o);
     hipLaunchKernelGGL(bswap64_kernel, dim3(256), dim3(256), 0, s, d_o, owords);
     e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return status_of(e);
     im.gbytes = (total + 7) / 8;
     im.obytes = (obits + 7) / 8;
+    return GRASS_OK;
+}
+
+// Fills a new graph from a CSR without its images: the payload words (LE: .graph's; GT: the stream),
+// headers and degrees the loader makes from them, and the same figures.  *images: the rows need the
+// images instead, nothing was built.
+template <int FMT>
+int build_resident(grass_graph* g, const uint64_t* rowptr, const uint32_t* col, uint64_t n, hipStream_t s, bool* images) {
+    constexpr bool STREAM = FMT == kGT;
+    FlatPlan p;
+    int rc = flat_plan<FMT, STREAM>(rowptr, col, n, g->cp_shift, s, p);
+    if (rc) return rc;
+    *images = p.st.flags != 0;
+    if (*images) return GRASS_OK;
+    const uint64_t bits = p.st.bits, gbytes = (bits + 7) / 8;
+    if (bits >= (1ull << 40)) return GRASS_EINVAL;
+    // payload bits must fit the header cache
+    if (8 * gbytes >= kMaxPayloadBits || (STREAM && 32 * p.st.words >= kMaxPayloadBits)) return GRASS_EFORMAT;
+    const uint64_t used = STREAM ? p.st.words : (bits + 31) / 32, words = used + kPadWords;
+    uint32_t** out = STREAM ? &g->d_gtx : &g->d_words;
+    if (device_malloc((void**)out, words * 4) != hipSuccess || device_malloc((void**)&g->d_deg, n * 4) != hipSuccess ||
+        device_malloc((void**)&g->d_hdr, n * 16) != hipSuccess)
+        return GRASS_ENOMEM;
+    hipError_t e = hipMemsetAsync(*out + used, 0, kPadWords * 4, s);  // every word before is stored below
+    if (e != hipSuccess) return status_of(e);
+    flat_write<FMT, kFlatResident>(p, rowptr, col, n, g->cp_shift, *out, s);
+    hipLaunchKernelGGL(flat_header_kernel<FMT>, dim3((unsigned)std::min<uint64_t>((n + kFlatBlock - 1) / kFlatBlock, p.grid)),
+                       dim3(kFlatBlock), 0, s, rowptr, col, n, (const uint64_t*)p.start, (const uint2*)p.widths, g->d_hdr,
+                       g->d_deg);
+    e = hipGetLastError();
+    const hipError_t done = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = done;
+    if (e != hipSuccess) return status_of(e);
+    g->n = n;
+    g->m = p.st.m;
+    g->max_degree = p.st.max_degree;
+    g->dec_runs = p.st.runs;
+    g->total_bits = bits;
+    g->ubl = offset_width(p.st.longest);
+    g->graph_bytes = gbytes;
+    g->offset_bytes = (8 + n * (uint64_t)g->ubl + 7) / 8;
+    g->device_bytes = words * 4 + n * 4 + n * 16;
     return GRASS_OK;
 }
 
@@ -504,15 +602,26 @@ int grass_compress_device_open(const uint64_t* rowptr_dev, const uint32_t* col_d
     int prev = 0;
     (void)hipGetDevice(&prev);
     if (!grass::enter_device(device)) return GRASS_EDEVICE;
-    int rc;
-    {
+    bool images = false;
+    grass_graph* g = nullptr;
+    int rc = grass::new_graph(format, device, &g);
+    if (!rc)
+        rc = format == GRASS_FMT_LE
+                 ? grass::build_resident<grass::kLE>(g, rowptr_dev, col_dev, n, (hipStream_t)stream, &images)
+                 : grass::build_resident<grass::kGT>(g, rowptr_dev, col_dev, n, (hipStream_t)stream, &images);
+    if (rc || images) {
+        grass::free_graph(g);
+        g = nullptr;
+    }
+    if (!rc && images) {
         grass::Images im;
         rc = grass::encode_images(rowptr_dev, col_dev, n, format, (hipStream_t)stream, im);
         if (!rc) {
             grass::DeviceSource gs(im.g.p, im.gbytes), os(im.o.p, im.obytes);
-            rc = grass::open_sources(gs, os, format, device, out);
+            rc = grass::open_sources(gs, os, format, device, &g);
         }
     }
+    *out = g;
     (void)hipSetDevice(prev);
     return rc;
 }

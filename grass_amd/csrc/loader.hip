@@ -391,7 +391,9 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
         e = exclusive_scan(OffsetFieldGen{d_off, ubl}, Count{n, nullptr}, n, g->d_start, d_tmp,
                            d_total, s);
     if (e == hipSuccess) {
-        unsigned grid = (unsigned)std::min<uint64_t>((n + kValBlock - 1) / kValBlock, 16384);
+        // (every workgroup adds to the same totals, one after another: 2.4 M vertices took 250 us with 9360
+        // workgroups, 78 with 1024)
+        unsigned grid = (unsigned)std::min<uint64_t>((n + kValBlock - 1) / kValBlock, 1024);
         if (g->fmt == kLE)
             hipLaunchKernelGGL(validate_kernel<kLE>, dim3(grid), dim3(kValBlock), 0, s, g->d_words,
                                g->d_start, (uint32_t)n, 8 * gbytes, g->d_deg, g->d_hdr,

@@ -271,7 +271,9 @@ struct ByteSource {
     virtual bool read(void* dst, uint64_t len) = 0;
 };
 int load_graph(grass_graph* g, ByteSource& graph_src, ByteSource& offset_src);
-// capi.cpp: a graph on `device` from two sources (grass_open and its variants)
+// capi.cpp: an empty graph on `device`, and its end; a graph from two sources (grass_open and its variants)
+int new_graph(int format, int device, grass_graph** out);
+void free_graph(grass_graph* g);
 int open_sources(ByteSource& graph_src, ByteSource& offset_src, int format, int device, grass_graph** out);
 // Images already in device memory.
 struct DeviceSource : ByteSource {

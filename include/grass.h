@@ -75,8 +75,10 @@ int grass_open_device_images(const void *graph_dev, uint64_t graph_bytes, const 
                              uint64_t offset_bytes, int format, int device, grass_graph **out);
 
 /* Encodes a CSR in device memory with the LE or GT compressor (as grass_compress_device in
- * grass_ingest.h) and loads the images it made as grass_open would load their files, without
- * either leaving the GPU.  No reference counterpart; for a graph built on the GPU. */
+ * grass_ingest.h) into the graph that grass_open would load from those images, on the GPU; the images
+ * themselves are only made for rows whose resident form depends on them (a GT self loop at a block
+ * head, ids >= n, rows that are not strictly ascending).  No reference counterpart; for a graph built
+ * on the GPU. */
 int grass_compress_device_open(const uint64_t *rowptr_dev, const uint32_t *col_dev, uint64_t n,
                                int format, int device, void *stream, grass_graph **out);
 
