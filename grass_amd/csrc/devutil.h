@@ -131,21 +131,6 @@ __device__ __forceinline__ T wave_max(T x) {
     return x;
 }
 
-// Segmented inclusive sum over the wave: a lane with head != 0 starts a new segment.
-__device__ __forceinline__ uint32_t wave_segmented_sum(uint32_t x, int head) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        uint32_t px = __shfl_up(x, off, kWave);
-        int ph = __shfl_up(head, off, kWave);
-        if (lane >= off && !head) {
-            x += px;
-            head = ph;
-        }
-    }
-    return x;
-}
-
 // Segmented inclusive sum over runs of at most `span` lanes (a lane with head != 0 starts a
 // run): log2(span) shuffle steps instead of six.
 __device__ __forceinline__ uint32_t short_segmented_sum(uint32_t x, int head, uint32_t span) {

@@ -147,10 +147,11 @@ struct SlotWalk {
     }
 };
 
-// Inclusive OR over the lanes head .. lane (a lane's head is its segment's first lane).
-struct SegmentOr {
+// Inclusive OR (or sum) over the lanes head .. lane (a lane's head is its segment's first lane), the DPP
+// tree of wave_inclusive_sum with the moves that would cross a segment's start left out.
+struct SegmentScan {
     bool c1, c2, c4, c8, c16, c32;
-    __device__ __forceinline__ explicit SegmentOr(uint32_t head) {
+    __device__ __forceinline__ explicit SegmentScan(uint32_t head) {
         const uint32_t lane = lane_id(), back = lane - head, row = lane & 15;
         c1 = back >= 1 && row >= 1;
         c2 = back >= 2 && row >= 2;
@@ -159,7 +160,7 @@ struct SegmentOr {
         c16 = (lane & 16) && head <= (lane & ~15u) - 1;
         c32 = lane >= 32 && head <= 31;
     }
-    __device__ __forceinline__ uint32_t operator()(uint32_t x) const {
+    __device__ __forceinline__ uint32_t any(uint32_t x) const {
         uint32_t t = dpp_move<0x111>(x);
         x |= c1 ? t : 0u;
         t = dpp_move<0x112>(x);
@@ -172,6 +173,21 @@ struct SegmentOr {
         x |= c16 ? t : 0u;
         t = dpp_move<0x143, 0xc>(x);
         x |= c32 ? t : 0u;
+        return x;
+    }
+    __device__ __forceinline__ uint32_t sum(uint32_t x) const {
+        uint32_t t = dpp_move<0x111>(x);
+        x += c1 ? t : 0u;
+        t = dpp_move<0x112>(x);
+        x += c2 ? t : 0u;
+        t = dpp_move<0x114>(x);
+        x += c4 ? t : 0u;
+        t = dpp_move<0x118>(x);
+        x += c8 ? t : 0u;
+        t = dpp_move<0x142, 0xa>(x);
+        x += c16 ? t : 0u;
+        t = dpp_move<0x143, 0xc>(x);
+        x += c32 ? t : 0u;
         return x;
     }
 };
@@ -255,9 +271,9 @@ __global__ __launch_bounds__(kFlatBlock) void flat_plan_kernel(const uint64_t* _
                 }
                 if (x < v ? end : !k || prev < v) fps[v] = x < v ? (FMT == kLE ? C + 1 : C) : c + (i != 0);
             }
-            const SegmentOr seg(head);
-            a = seg(a) | (j ? 0u : ca);
-            b = seg(b) | (j ? 0u : cb);
+            const SegmentScan seg(head);
+            a = seg.any(a) | (j ? 0u : ca);
+            b = seg.any(b) | (j ? 0u : cb);
             if (act && end) {
                 if (v == before) {
                     atomicOr(&ors[v].x, a);
@@ -360,13 +376,62 @@ __global__ __launch_bounds__(kFlatBlock) void flat_header_kernel(const uint64_t*
     }
 }
 
+// The words of a chunk's passes.  A chunk owns the words whose first bit its slots hold; its last pass
+// reaches kFlatLook slots past them (a slot or the one after it has at least two bits, and the stream's
+// padding ends a word) to complete the last of these: every word is stored once and nothing is ORed into
+// memory.  A pass assembles its words in LDS; its partial last word is carried into the next.
+template <bool SWAP>  // stored byte-swapped
+struct FlatWindow {
+    uint32_t* B;
+    uint32_t* __restrict__ out;
+    uint64_t from0, w0;  // bit of the chunk's first slot; word of the pass's first bit
+    uint64_t pend_w;     // the carried word's index, ~0 when there is none
+    uint32_t pend, nwords;
+
+    __device__ __forceinline__ void store(uint64_t w, uint32_t x) const { out[w] = SWAP ? __builtin_bswap32(x) : x; }
+
+    // Bits [from, to) are put next (put_field at B, w0).
+    __device__ __forceinline__ void begin(bool first, uint64_t from, uint64_t to) {
+        const uint32_t lane = lane_id();
+        w0 = from >> 5;
+        if (first) {
+            from0 = from;
+            pend_w = ~0ull;
+        }
+        if (pend_w != ~0ull && pend_w != w0) {  // completed by padding
+            if (lane == 0 && pend_w << 5 >= from0) store(pend_w, pend);
+            pend_w = ~0ull;
+        }
+        nwords = to > from ? (uint32_t)(((to - 1) >> 5) - w0 + 1) : pend_w == w0 ? 1u : 0u;
+        for (uint32_t x = lane; x < nwords; x += kWave) B[x] = x == 0 && pend_w == w0 ? pend : 0u;
+        wave_sync();
+    }
+    // The chunk's last pass stores the words that start before bit `end`.
+    __device__ __forceinline__ void finish(bool last, uint64_t to, uint64_t end) {
+        wave_sync();
+        if (!last) end = to & ~31ull;
+        for (uint32_t x = lane_id(); x < nwords; x += kWave) {
+            const uint64_t bit = (w0 + x) << 5;
+            if (bit >= from0 && bit < end) store(w0 + x, B[x]);
+        }
+        const bool part = !last && nwords && (to & 31);
+        pend = part ? B[nwords - 1] : 0u;
+        pend_w = part ? w0 + nwords - 1 : ~0ull;
+        wave_sync();
+    }
+};
+
+// GT stream: fields of a list's checkpoint positions before position i of block b (each takes 32 bits in
+// place of f2).
+__device__ __forceinline__ uint32_t flat_checkpoints(uint32_t b, uint32_t i, uint32_t q, uint32_t R, uint32_t sh) {
+    const uint32_t lo = min(b, R);
+    return __umul24(lo, q >> sh) + __umul24(b - lo, (q - 1) >> sh) + (i ? (i - 1) >> sh : 0u);
+}
+
 enum FlatOut { kFlatImage, kFlatResident };
 
 // The words of the .graph image (kFlatImage: stored byte-swapped, as the file's bytes), or of the
 // resident graph: LE the same words, GT the checkpointed payload stream (no headers; start[] in words).
-// A chunk owns the words whose first bit its slots hold, its last pass reaches kFlatLook slots past
-// them (a slot or the one after it has at least two bits, and the stream's padding ends a word) to
-// complete the last of these: every word is stored once and nothing is ORed into memory.
 template <int FMT, FlatOut OUT>
 __global__ __launch_bounds__(kFlatBlock) void flat_write_kernel(const uint64_t* __restrict__ rowptr,
                                                                 const uint32_t* __restrict__ col, uint64_t n,
@@ -377,7 +442,7 @@ __global__ __launch_bounds__(kFlatBlock) void flat_write_kernel(const uint64_t* 
     __shared__ uint32_t own_lds[kFlatBlock];
     __shared__ uint32_t buf[kFlatWaves][kFlatWords + 1];
     uint32_t* own = own_lds + (threadIdx.x & ~(kWave - 1));
-    uint32_t* B = buf[threadIdx.x / kWave];
+    FlatWindow<OUT == kFlatImage> win{buf[threadIdx.x / kWave], out};
     const uint32_t lane = lane_id();
     const uint64_t waves = (uint64_t)gridDim.x * kFlatWaves;
     const uint64_t slots = rowptr[n] + n;
@@ -396,9 +461,6 @@ __global__ __launch_bounds__(kFlatBlock) void flat_write_kernel(const uint64_t* 
         };
         request();
         uint32_t px = FMT == kGT && s0 - walk.sc >= 2 ? col[s0 - walk.cur - 2] : 0u;
-        uint32_t pend = 0;        // the partial last word of the previous pass
-        uint64_t pend_w = ~0ull;  // its index, ~0 when there is none
-        uint64_t from0 = 0;       // bit of the chunk's first slot
         for (uint32_t t = 0; t < passes; ++t) {
             const uint64_t base = s0 + (uint64_t)t * kWave;
             if (base >= slots) break;
@@ -438,9 +500,7 @@ __global__ __launch_bounds__(kFlatBlock) void flat_write_kernel(const uint64_t* 
                     val = i ? x - prev - 1 : diff ? diff - 1 : 1u;
                     wdt = i ? f2 : f1;
                     if (STREAM) {
-                        const uint32_t lo = min(b, R);
-                        const uint32_t cps = __umul24(lo, q >> sh) + __umul24(b - lo, (q - 1) >> sh) + (i ? (i - 1) >> sh : 0u);
-                        at += (uint64_t)cps * (32 - f2);
+                        at += (uint64_t)flat_checkpoints(b, i, q, R, sh) * (32 - f2);
                         if (i && !(i & ((1u << sh) - 1))) {
                             val = x;
                             wdt = 32;
@@ -472,36 +532,20 @@ __global__ __launch_bounds__(kFlatBlock) void flat_write_kernel(const uint64_t* 
                 wdt = hb;
             }
             const uint64_t from = readlane_u64(at, 0), to = readlane_u64(at + wdt, (int)last);
-            const uint64_t w0 = from >> 5;
-            const uint64_t end = !fin ? to & ~31ull : s0 + W < slots ? readlane_u64(at, kWave - kFlatLook) : ~0ull;
-            if (t == 0) from0 = from;
-            if (pend_w != ~0ull && pend_w != w0) {  // completed by padding
-                if (lane == 0 && pend_w << 5 >= from0) out[pend_w] = OUT == kFlatImage ? __builtin_bswap32(pend) : pend;
-                pend_w = ~0ull;
-            }
-            const uint32_t nwords = to > from ? (uint32_t)(((to - 1) >> 5) - w0 + 1) : pend_w == w0 ? 1u : 0u;
-            for (uint32_t x = lane; x < nwords; x += kWave) B[x] = x == 0 && pend_w == w0 ? pend : 0u;
-            wave_sync();
-            if (field) put_field(B, w0, at, wdt, wdt < 32 ? val & ((1u << wdt) - 1) : val);
+            const uint64_t end = s0 + W < slots ? readlane_u64(at, kWave - kFlatLook) : ~0ull;  // (last pass)
+            win.begin(t == 0, from, to);
+            if (field) put_field(win.B, win.w0, at, wdt, wdt < 32 ? val & ((1u << wdt) - 1) : val);
             if (!STREAM && act && k < 0) {
-                put_gamma(B, w0, at, d);
+                put_gamma(win.B, win.w0, at, d);
                 if (FMT == kGT || d > 1) {
-                    put_gamma(B, w0, at, f1);
-                    put_gamma(B, w0, at, f2);
-                    put_gamma(B, w0, at, fp);
+                    put_gamma(win.B, win.w0, at, f1);
+                    put_gamma(win.B, win.w0, at, f2);
+                    put_gamma(win.B, win.w0, at, fp);
                 } else if (d) {
-                    put_gamma(B, w0, at, col[row]);
+                    put_gamma(win.B, win.w0, at, col[row]);
                 }
             }
-            wave_sync();
-            for (uint32_t x = lane; x < nwords; x += kWave) {
-                const uint64_t bit = (w0 + x) << 5;
-                if (bit >= from0 && bit < end) out[w0 + x] = OUT == kFlatImage ? __builtin_bswap32(B[x]) : B[x];
-            }
-            const bool part = !fin && nwords && (to & 31);
-            pend = part ? B[nwords - 1] : 0u;
-            pend_w = part ? w0 + nwords - 1 : ~0ull;
-            wave_sync();
+            win.finish(fin, to, end);
         }
     }
 }

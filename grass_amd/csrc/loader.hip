@@ -3,7 +3,7 @@
 //   2. record-length extraction from .offset fused into a reduce-then-scan (bit starts),
 //   3. a validator that parses every record header, checks header + payload == record
 //      length, and writes the degree array and the decoded-header cache,
-//   4. GT: the checkpointed payload stream the samplers decode (gt_expand_kernel).
+//   4. GT: the checkpointed payload stream the samplers decode (flat_expand_kernel).
 // Replaces loadGraph (LE/src/grass.cu:1015-1095), copyPartitionToGPU (LE/src/utils.hpp:328-353)
 // with its decode_offset kernel (LE/src/bcg.cuh:284-329) and CUB scan.
 #include <hip/hip_runtime.h>
@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "devutil.h"
+#include "encode_flat.h"
 #include "runtime.h"
 #include "scan.h"
 
@@ -123,84 +124,113 @@ struct GtxWordsGen {
     }
 };
 
-constexpr int kExpBlock = 256;
-constexpr uint32_t kExpWords = kWave + 2;  // words that one pass of 64 fields (<= 32 bits) can touch
-
-// One wave per GT vertex: decodes the .graph record 64 positions at a time (heads absolute,
-// bodies as gaps, a segmented prefix sum carrying the running id from pass to pass) and writes
-// the vertex's payload in the device stream at word woff[v]: heads and bodies copied, the 32-bit
-// id at every checkpoint position.  A pass assembles its fields in LDS and stores its complete
-// words; a last word that the pass leaves partial is carried into the next pass.  A vertex's
-// stream words are its own (its payload starts on a word), so every word is stored once and
-// nothing is ORed into memory.  Finally the header's payload bit is moved to the stream.
-__global__ __launch_bounds__(kExpBlock) void gt_expand_kernel(DevGraph g, const uint64_t* __restrict__ woff,
-                                                              uint4* __restrict__ hdr, uint32_t* __restrict__ out) {
-    __shared__ uint32_t buf[kExpBlock / kWave][kExpWords];
-    const int lane = lane_id();
-    uint32_t* B = buf[threadIdx.x / kWave];
-    const uint32_t sh = g.cp_shift, P = 1u << sh;
-    const uint64_t nw = (uint64_t)gridDim.x * kExpBlock / kWave;
-    for (uint64_t v = ((uint64_t)blockIdx.x * kExpBlock + threadIdx.x) / kWave; v < g.n; v += nw) {
-        uint4 e = hdr[v];
-        Hdr h;
-        unpack_hdr<kGT>(e, h);  // payload bit in .graph
-        Hdr hx = h;
-        hx.pay = woff[v] << 5;  // payload bit in the stream
-        uint32_t carry = 0;
-        uint32_t pend = 0;        // the partial last word of the previous pass
-        uint64_t pend_w = ~0ull;  // its index, ~0 when that pass ended on a word boundary
-        for (uint32_t base = 0; base < h.d; base += kWave) {
-            const uint32_t k = base + lane;
-            const bool act = k < h.d;
-            uint32_t blk, i;
-            gt_locate(h, act ? k : h.d - 1, blk, i);
-            const uint64_t bo = gt_file_block_bit(h, blk);
-            uint32_t raw, x, wdt;
-            int head;
-            if (i == 0) {
-                raw = read_bits(g.w, bo, h.f1);
-                x = blk >= h.fp ? (uint32_t)v + raw + 1 : (uint32_t)v - raw - 1;
-                wdt = h.f1;
-                head = 1;
-            } else {
-                raw = read_bits0(g.w, bo + h.f1 + (uint64_t)(i - 1) * h.f2, h.f2);
-                x = raw + 1;
-                wdt = h.f2;
-                head = 0;
+// The GT payload stream from a .graph image: the same words as flat_write_kernel's from the rows.  `hdr`
+// are the image's headers (payload bits in `w`), woff[] the payloads' first words in the stream,
+// rowptr[] the degrees' prefix sums.  Heads and gaps are copied; a checkpoint's id is the sum over its
+// block so far, a segmented sum over the lanes carried from pass to pass, which a chunk that starts
+// inside a block begins with the fields before its own.  R-MAT s22 (128 M entries): 3.24 ms with a wave
+// per vertex, 1.14 by slots.
+__global__ __launch_bounds__(kFlatBlock) void flat_expand_kernel(const uint32_t* __restrict__ w,
+                                                                 const uint64_t* __restrict__ rowptr,
+                                                                 const uint4* __restrict__ hdr, uint64_t n,
+                                                                 const uint64_t* __restrict__ woff, uint32_t sh,
+                                                                 uint32_t* __restrict__ out) {
+    __shared__ uint32_t own_lds[kFlatBlock];
+    __shared__ uint32_t buf[kFlatWaves][kFlatWords + 1];
+    uint32_t* own = own_lds + (threadIdx.x & ~(kWave - 1));
+    FlatWindow<false> win{buf[threadIdx.x / kWave], out};
+    const uint32_t lane = lane_id();
+    const uint64_t waves = (uint64_t)gridDim.x * kFlatWaves;
+    const uint64_t slots = rowptr[n] + n;
+    const uint32_t passes = flat_passes(slots, waves);
+    const uint64_t W = (uint64_t)passes * kWave - kFlatLook;
+    for (uint64_t s0 = ((uint64_t)blockIdx.x * kFlatBlock + threadIdx.x) / kWave * W; s0 < slots; s0 += waves * W) {
+        SlotWalk walk{rowptr, n};
+        walk.seek(s0);
+        uint64_t st = 0;
+        uint4 hj = make_uint4(0u, 0u, 0u, 0u);
+        auto request = [&]() {
+            if (walk.cur + (uint64_t)lane < n) {
+                st = woff[walk.cur + lane];
+                hj = hdr[walk.cur + lane];
             }
-            if (lane == 0 && !head) {
-                x += carry;
-                head = 1;
+        };
+        request();
+        uint32_t carry = 0;  // the id at the slot before the pass's first
+        if (s0 - walk.sc >= 2) {
+            Hdr h;
+            unpack_hdr<kGT>(hdr[walk.cur], h);
+            uint32_t b, i;
+            flat_pos((uint32_t)(s0 - walk.sc) - 2, h.q, h.R, b, i);  // the field before the chunk's first
+            const uint64_t bo = gt_file_block_bit(h, b);
+            uint32_t sum = 0;
+            for (uint32_t g = 1 + lane; g <= i; g += kWave) sum += read_bits0(w, bo + h.f1 + (uint64_t)(g - 1) * h.f2, h.f2) + 1;
+            const uint32_t raw = read_bits(w, bo, h.f1);
+            carry = wave_sum(sum) + (b >= h.fp ? walk.cur + raw + 1 : walk.cur - raw - 1);
+        }
+        for (uint32_t t = 0; t < passes; ++t) {
+            const uint64_t base = s0 + (uint64_t)t * kWave;
+            if (base >= slots) break;
+            const bool fin = t + 1 == passes || base + kWave >= slots;
+            const uint32_t last = (uint32_t)(slots - base < (uint64_t)kWave ? slots - base - 1 : kWave - 1);
+            uint32_t j, d, head;
+            int32_t k;
+            walk.place(base, last, own, j, k, d, head);
+            const uint32_t v = walk.cur + j;
+            Hdr h;
+            unpack_hdr<kGT>(make_uint4(__shfl(hj.x, (int)j, kWave), __shfl(hj.y, (int)j, kWave), d, __shfl(hj.w, (int)j, kWave)), h);
+            const uint64_t sv = ((uint64_t)__shfl((uint32_t)(st >> 32), (int)j, kWave) << 32) | __shfl((uint32_t)st, (int)j, kWave);
+            walk.advance((uint32_t)__builtin_amdgcn_readlane((int)j, (int)last),
+                         __builtin_amdgcn_readlane((int)(k + 1 == (int32_t)d), (int)last));
+            if (!fin) {
+                walk.request();
+                request();
             }
-            x = wave_segmented_sum(x, head);
-            carry = __shfl(x, kWave - 1, kWave);
-            if (i && (i & (P - 1)) == 0) {
+            const bool act = lane <= last, field = act && k >= 0;
+            uint32_t b, i;
+            flat_pos(k < 0 ? 0u : (uint32_t)k, h.q, h.R, b, i);
+            const uint32_t heads = b + (i != 0), wf = i ? h.f2 : h.f1;
+            const uint64_t off = __umul24(heads, h.f1) + (uint64_t)((uint32_t)k - heads) * h.f2;
+            uint32_t raw = 0, x = 0;
+            uint64_t at = sv << 5;
+            uint32_t wdt = 0;
+            if (field) {
+                raw = read_bits(w, h.pay + off, wf);
+                x = i ? raw + 1 : b >= h.fp ? v + raw + 1 : v - raw - 1;
+                at += off + (uint64_t)flat_checkpoints(b, i, h.q, h.R, sh) * (32 - h.f2);
+                wdt = wf;
+            }
+            // the ids: sums from the block's head, or from the carry where that lies in an earlier pass
+            if (lane == 0 && field && i) x += carry;
+            x = SegmentScan(!field ? lane : i <= lane ? lane - i : 0u).sum(x);
+            carry = (uint32_t)__builtin_amdgcn_readlane((int)x, kWave - 1);
+            if (i && !(i & ((1u << sh) - 1))) {
                 raw = x;
-                wdt = 32;
+                if (field) wdt = 32;
             }
-            const uint64_t at = gtx_block_bit(hx, blk, sh) + gtx_field(hx, i, sh);
-            // words [w0, w0 + nwords) hold this pass's fields; the last active lane ends them
-            const uint32_t la = min((uint32_t)kWave - 1, h.d - 1 - base);
-            const uint64_t w0 = __shfl(at, 0, kWave) >> 5;
-            const uint64_t end = __shfl(at + wdt, (int)la, kWave);
-            const uint32_t nwords = (uint32_t)(((end - 1) >> 5) - w0 + 1);
-            for (uint32_t j = lane; j < kExpWords; j += kWave) B[j] = (j == 0 && pend_w == w0) ? pend : 0u;
-            wave_sync();
-            if (act) put_field(B, w0, at, wdt, raw);
-            wave_sync();
-            const bool open = (end & 31) != 0;
-            const uint32_t full = open ? nwords - 1 : nwords;
-            for (uint32_t j = lane; j < full; j += kWave) out[w0 + j] = B[j];
-            pend = B[nwords - 1];
-            pend_w = open ? w0 + nwords - 1 : ~0ull;
-            wave_sync();
+            const uint64_t from = readlane_u64(at, 0), to = readlane_u64(at + wdt, (int)last);
+            const uint64_t end = s0 + W < slots ? readlane_u64(at, kWave - kFlatLook) : ~0ull;  // (last pass)
+            win.begin(t == 0, from, to);
+            if (field) put_field(win.B, win.w0, at, wdt, raw);
+            win.finish(fin, to, end);
         }
-        if (pend_w != ~0ull && lane == 0) out[pend_w] = pend;
-        if (lane == 0) {
-            e.x = (uint32_t)hx.pay;
-            e.y = (e.y & ~63u) | (uint32_t)(hx.pay >> 32);
-            hdr[v] = e;
-        }
+    }
+}
+
+struct DegreeGen {
+    const uint32_t* deg;
+    __device__ __forceinline__ uint64_t operator()(uint64_t v) const { return deg[v]; }
+};
+
+// The headers' payload bits moved from .graph to the stream.
+__global__ __launch_bounds__(256) void gt_headers_kernel(const uint64_t* __restrict__ woff, uint64_t n,
+                                                         uint4* __restrict__ hdr) {
+    for (uint64_t v = (uint64_t)blockIdx.x * 256 + threadIdx.x; v < n; v += (uint64_t)gridDim.x * 256) {
+        uint4 e = hdr[v];
+        const uint64_t pay = woff[v] << 5;
+        e.x = (uint32_t)pay;
+        e.y = (e.y & ~63u) | (uint32_t)(pay >> 32);
+        hdr[v] = e;
     }
 }
 
@@ -433,11 +463,14 @@ int load_graph(grass_graph* g, ByteSource& gsrc, ByteSource& osrc) {
 int build_gt_stream(grass_graph* g, uint64_t* words) {
     hipStream_t s = g->stream;
     const uint64_t n = g->n, nb = scan_blocks(n);
-    WorkMem m_woff;  // n + 1 word offsets, partials, total
-    if (m_woff.alloc((n + 1 + nb + 2) * 8, s) != hipSuccess) return GRASS_ENOMEM;
+    WorkMem m_woff;  // n + 1 word offsets, n + 1 row starts, partials, total
+    if (m_woff.alloc((2 * (n + 1) + nb + 2) * 8, s) != hipSuccess) return GRASS_ENOMEM;
     uint64_t* d_woff = m_woff.as<uint64_t>();
+    uint64_t* d_row = d_woff + n + 1;
+    uint64_t* d_part = d_row + n + 1;
     hipError_t e = exclusive_scan(GtxWordsGen{g->d_hdr, g->cp_shift}, Count{n, nullptr}, n, d_woff,
-                                  d_woff + n + 1, d_woff + n + 1 + nb, s);
+                                  d_part, d_part + nb, s);
+    if (e == hipSuccess) e = exclusive_scan(DegreeGen{g->d_deg}, Count{n, nullptr}, n, d_row, d_part, d_part + nb, s);
     uint64_t total = 0;
     if (e == hipSuccess) e = hipMemcpyAsync(&total, d_woff + n, 8, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -449,9 +482,14 @@ int build_gt_stream(grass_graph* g, uint64_t* words) {
     if (!rc) {
         e = hipMemsetAsync(out + total, 0, kPadWords * 4, s);  // every word before is stored below
         if (e == hipSuccess) {
-            // g->dev() still decodes .graph here: d_gtx is set once the stream is complete
-            hipLaunchKernelGGL(gt_expand_kernel, dim3(4096), dim3(kExpBlock), 0, s, g->dev(),
-                               (const uint64_t*)d_woff, g->d_hdr, out);
+            int dev = 0, cus = 0;
+            (void)hipGetDevice(&dev);
+            (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+            hipLaunchKernelGGL(flat_expand_kernel, dim3((unsigned)std::max(cus, 1) * 8), dim3(kFlatBlock), 0, s,
+                               (const uint32_t*)g->d_words, (const uint64_t*)d_row, (const uint4*)g->d_hdr, n,
+                               (const uint64_t*)d_woff, g->cp_shift, out);
+            hipLaunchKernelGGL(gt_headers_kernel, dim3((unsigned)std::min<uint64_t>((n + 255) / 256, 4096)), dim3(256), 0, s,
+                               (const uint64_t*)d_woff, n, g->d_hdr);
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = hipStreamSynchronize(s);
