@@ -13,11 +13,12 @@
 //   3. rel_emit_kernel: writes each first appearance to nodes[rank(p)] and the local ids of every
 //      batch edge (its destination is a position, its source a key looked up in the table).
 // Every step is a data-parallel pass over the positions; the result does not depend on timing.
-// A batch of few positions is one launch of one workgroup (rel_small_kernel).  A large one is bound by
+// A batch of few positions is one launch of one workgroup (rel_small_kernel).  A larger one is bound by
 // the random atomics of the inserts, which the chip takes at 22 to 27 G/s whatever the table's size
 // (a load of a slot and a CAS on it: 25.7 G/s), so a position touches the table once: 16 x 8192 seeds
 // [25, 10] on R-MAT s24, 10.7 M positions, insert 435 us; a second pass that looked every key up again
-// took 196 us more.  The emit is 223 us, most of it waiting on the source's lookup.
+// took 196 us more.  A large one therefore makes step 2 by partition (rel_part_*): 241 us with all its
+// passes.  The emit, by lookups of the sources and loads a word ahead, is 150 us (229 without either).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -88,6 +89,9 @@ struct RelTab16 {
         atomicOr(err, 1u);  // cannot happen: slots > positions
         return false;
     }
+    // First position of v in request r, where hint(p) was loaded for a position p that holds it.
+    __device__ __forceinline__ uint32_t hint(uint64_t) const { return 0; }
+    __device__ __forceinline__ uint64_t first_of(uint32_t, uint32_t r, uint32_t v) const { return first(r, v); }
     // First position of v in request r; ~0 when absent.
     __device__ __forceinline__ uint64_t first(uint32_t r, uint32_t v) const {
         const unsigned long long k = key(r, v);
@@ -140,6 +144,8 @@ struct RelTab8 {
         atomicOr(err, 1u);  // cannot happen: slots > positions
         return false;
     }
+    __device__ __forceinline__ uint32_t hint(uint64_t) const { return 0; }
+    __device__ __forceinline__ uint64_t first_of(uint32_t, uint32_t r, uint32_t v) const { return first(r, v); }
     __device__ __forceinline__ uint64_t first(uint32_t r, uint32_t v) const {
         if (vb < 32 && (v >> vb) != 0) return ~0ull;
         const unsigned long long k = ((unsigned long long)r << vb) | v;
@@ -250,10 +256,64 @@ __global__ __launch_bounds__(1024) void rel_clear_kernel(Tab t, FirstWord* words
     rel_clear(t, words, nwords, (uint64_t)blockIdx.x * 1024 + threadIdx.x, (uint64_t)gridDim.x * 1024);
 }
 
+constexpr uint32_t kPrepRequests = 8192;
+
+// Partitions (rel_part_*): a request's sequence is cut into tiles of kPartTile positions, and its keys go
+// by their hash into buckets of about kPartKeys, whose distinct ones fit a table of kPartSlots.
+constexpr uint32_t kPartTile = 8192, kPartKeys = 2560, kPartSlots = 4096, kPartBuckets = 8192;
+__host__ __device__ inline uint32_t part_buckets(uint64_t len) {
+    const uint64_t b = (len + kPartKeys - 1) / kPartKeys;
+    return (uint32_t)(b < kPartBuckets ? b : kPartBuckets);
+}
+
+// One workgroup of 1024: the offsets' check, the requests' starts Q, their total's check; tile0 and bkt0
+// (or null): their first tiles and buckets.
+__device__ __forceinline__ void rel_starts(const uint64_t* __restrict__ off, const RelReq* __restrict__ req, uint32_t R,
+                                           uint32_t H, uint64_t total, uint64_t P, uint64_t* __restrict__ Q,
+                                           uint32_t* __restrict__ tile0, uint32_t* __restrict__ bkt0, uint32_t* bad,
+                                           uint32_t* invalid) {
+    __shared__ uint64_t lds[1024 / kWave];
+    const bool mine = H == 0 || rel_check(off, req, R, H, total, threadIdx.x, 1024);
+    const bool ok = block_sum<uint64_t, 1024>(mine ? 0 : 1, lds) == 0;
+    constexpr uint32_t kPer = kPrepRequests / 1024;
+    const uint32_t per = (R + 1023) / 1024, r0 = threadIdx.x * per;
+    uint64_t len[kPer], s = 0, parts = 0;  // parts: tiles << 32 | buckets
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+        len[i] = i < per && r0 + i < R ? rel_length(req, off, R, ok ? H : 0, r0 + i) : 0;
+        s += len[i];
+        parts += ((len[i] + kPartTile - 1) / kPartTile << 32) | part_buckets(len[i]);
+    }
+    uint64_t sum, all = 0;
+    uint64_t pre = block_exclusive_sum<uint64_t, 1024>(s, sum, lds);
+    if (tile0) parts = block_exclusive_sum<uint64_t, 1024>(parts, all, lds);
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; ++i) {
+        if (i < per && r0 + i < R) {
+            Q[r0 + i] = pre;
+            if (tile0) {
+                tile0[r0 + i] = (uint32_t)(parts >> 32);
+                bkt0[r0 + i] = (uint32_t)parts;
+            }
+        }
+        pre += len[i];
+        parts += ((len[i] + kPartTile - 1) / kPartTile << 32) | part_buckets(len[i]);
+    }
+    if (threadIdx.x == 0) {
+        Q[R] = sum;
+        *bad = 0;
+        const bool fits = ok && sum == P;
+        *invalid = fits ? 0 : 1;
+        if (tile0) {
+            tile0[R] = fits ? (uint32_t)(all >> 32) : 0u;
+            bkt0[R] = fits ? (uint32_t)all : 0u;
+        }
+    }
+}
+
 // Up to kPrepRequests requests: workgroup 0 checks the offsets, scans the lengths into Q and checks their
 // total, while the others clear the table (with one workgroup, it does both): one launch where the
 // steps by themselves are seven.
-constexpr uint32_t kPrepRequests = 8192;
 template <class Tab>
 __global__ __launch_bounds__(1024) void rel_prepare_kernel(Tab t, FirstWord* words, uint64_t nwords,
                                                            const uint64_t* __restrict__ off,
@@ -264,29 +324,7 @@ __global__ __launch_bounds__(1024) void rel_prepare_kernel(Tab t, FirstWord* wor
         rel_clear(t, words, nwords, (uint64_t)(gridDim.x == 1 ? 0 : blockIdx.x - 1) * 1024 + threadIdx.x,
                   (uint64_t)(gridDim.x == 1 ? 1 : gridDim.x - 1) * 1024);
     if (blockIdx.x) return;
-    __shared__ uint64_t lds[1024 / kWave];
-    const bool mine = H == 0 || rel_check(off, req, R, H, total, threadIdx.x, 1024);
-    const bool ok = block_sum<uint64_t, 1024>(mine ? 0 : 1, lds) == 0;
-    constexpr uint32_t kPer = kPrepRequests / 1024;
-    const uint32_t per = (R + 1023) / 1024, r0 = threadIdx.x * per;
-    uint64_t len[kPer], s = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < kPer; ++i) {
-        len[i] = i < per && r0 + i < R ? rel_length(req, off, R, ok ? H : 0, r0 + i) : 0;
-        s += len[i];
-    }
-    uint64_t sum;
-    uint64_t pre = block_exclusive_sum<uint64_t, 1024>(s, sum, lds);
-#pragma unroll
-    for (uint32_t i = 0; i < kPer; ++i) {
-        if (i < per && r0 + i < R) Q[r0 + i] = pre;
-        pre += len[i];
-    }
-    if (threadIdx.x == 0) {
-        Q[R] = sum;
-        *bad = 0;
-        *invalid = ok && sum == P ? 0 : 1;
-    }
+    rel_starts(off, req, R, H, total, P, Q, nullptr, nullptr, bad, invalid);
 }
 
 // Where a wave that goes through consecutive words is: the stretch of positions (a request's seeds,
@@ -356,28 +394,57 @@ __global__ __launch_bounds__(kExBlock) void rel_emit_kernel(RelSeq q, uint64_t P
     if (*invalid) return;
     const WordChunk wc = wave_words<kExBlock>(P);
     RelCursor cur;
-    for (uint64_t w = wc.w; w < wc.end; ++w) {
-        const FirstWord fw = words[w];
+    // what a word's positions need that no lookup tells, loaded a word ahead
+    struct Item {
+        FirstWord fw;
+        uint64_t e;  // ~0: a seed, or past the end
+        uint32_t v, r, src, hint;
+    };
+    auto fetch = [&](uint64_t w) {
+        Item it;
+        it.fw = words[w];
         const uint64_t p = w * kWave + lane_id(), last = min(w * kWave + kWave - 1, P - 1);
-        uint32_t r;
-        uint64_t e;
-        const uint32_t v = cur.at(q, w, min(p, last), last, r, e);
-        if (p >= P) continue;
-        const bool first = (fw.x >> lane_id()) & 1;
-        const uint64_t mine = fw.y + lanes_below(fw.x);
-        if (first && mine < cap) nodes[mine] = v;
-        if (e == ~0ull) continue;
-        const uint64_t base = node_off[r];
-        const uint64_t fd = first ? p : v < q.n ? t.first(r, v) : ~0ull;
-        const uint64_t fs = t.first(r, q.src[e]);
+        it.v = cur.at(q, w, min(p, last), last, it.r, it.e);
+        if (p >= P) it.e = ~0ull;
+        it.src = it.e != ~0ull ? q.src[it.e] : 0u;
+        it.hint = t.hint(min(p, last));
+        return it;
+    };
+    if (wc.w >= wc.end) return;
+    Item next = fetch(wc.w);
+    for (uint64_t w = wc.w; w < wc.end; ++w) {
+        const Item it = next;
+        if (w + 1 < wc.end) next = fetch(w + 1);
+        const uint64_t p = w * kWave + lane_id();
+        const bool first = (it.fw.x >> lane_id()) & 1;  // (not past the end)
+        const uint64_t mine = it.fw.y + lanes_below(it.fw.x);
+        if (first && mine < cap) nodes[mine] = it.v;
+        if (it.e == ~0ull) continue;
+        const uint64_t base = node_off[it.r];
+        const uint64_t fd = first ? p : it.v < q.n ? t.first_of(it.hint, it.r, it.v) : ~0ull;
+        const uint64_t fs = t.first(it.r, it.src);
         if (fd >= P || fs >= P) {  // a source that is neither a seed nor an earlier destination
             atomicOr(err, 1u);
-            ldst[e] = lsrc[e] = kNoId;
+            ldst[it.e] = lsrc[it.e] = kNoId;
             continue;
         }
-        ldst[e] = (uint32_t)((first ? mine : first_rank(words, fd)) - base);
-        lsrc[e] = (uint32_t)(first_rank(words, fs) - base);
+        ldst[it.e] = (uint32_t)((first ? mine : first_rank(words, fd)) - base);
+        lsrc[it.e] = (uint32_t)(first_rank(words, fs) - base);
     }
+}
+
+// The first appearances numbered, then the sampled vertices and the local ids of every edge.
+template <class Tab>
+hipError_t rel_number(const Tab& t, const RelSeq& q, uint64_t P, FirstWord* d_words, uint64_t* d_part, uint64_t* d_sc,
+                      uint32_t* d_bad, grass_khop_blocks* out, hipStream_t s) {
+    // node_off[r] = first appearances before request r; their total beside the other results
+    hipError_t e = scan_firsts(d_words, Count{P, nullptr}, P, q.Q, q.R, out->node_off_dev, d_sc + 1, d_part, d_sc, s);
+    if (e != hipSuccess || !P) return e;
+    const unsigned gP = (unsigned)std::min<uint64_t>((P + kExBlock - 1) / kExBlock + 1, kExGrid);
+    hipLaunchKernelGGL(rel_emit_kernel<Tab>, dim3(gP), dim3(kExBlock), 0, s, q, P, t, (const FirstWord*)d_words,
+                       (const uint64_t*)out->node_off_dev, out->nodes_dev, out->node_capacity, out->lsrc_dev,
+                       out->ldst_dev, (const uint32_t*)(d_bad + 1), d_bad);
+    return hipGetLastError();
 }
 
 // Fills Q and clears the table, inserts every position, numbers the first appearances (scan) and
@@ -408,13 +475,208 @@ hipError_t rel_build(const Tab& t, const RelSeq& q, uint64_t P, uint64_t* d_len,
     if (P)
         hipLaunchKernelGGL(rel_insert_kernel<Tab>, dim3(gP), dim3(kExBlock), 0, s, q, P, t, d_words,
                            (const uint32_t*)d_invalid, d_bad);
-    // node_off[r] = first appearances before request r; their total beside the other results
-    hipError_t e = scan_firsts(d_words, Count{P, nullptr}, P, q.Q, q.R, out->node_off_dev, d_sc + 1, d_part, d_sc, s);
-    if (e != hipSuccess || !P) return e;
-    hipLaunchKernelGGL(rel_emit_kernel<Tab>, dim3(gP), dim3(kExBlock), 0, s, q, P, t, (const FirstWord*)d_words,
-                       (const uint64_t*)out->node_off_dev, out->nodes_dev, out->node_capacity, out->lsrc_dev,
-                       out->ldst_dev, (const uint32_t*)d_invalid, d_bad);
-    return hipGetLastError();
+    return rel_number(t, q, P, d_words, d_part, d_sc, d_bad, out, s);
+}
+
+// ------------------------------------------------------------------ blocks by partition
+// Random atomics on a table in memory bound the insert above, so where most keys are distinct and the
+// table is far larger than the L2 the keys are first brought together: the positions of every bucket
+// (a request's keys of one hash range) are written next to each other as {vertex, position}, and one
+// workgroup deduplicates a bucket in LDS.  fpos[p] becomes the first position of p's key where that is
+// not p; the bucket's table goes to memory for the lookups of the edges' sources.  10.7 M positions, R-MAT
+// s24: prepare 12 us, count 30, scatter 69, dedup 110, words 15.
+
+struct RelParts {
+    const uint32_t* tile0;  // R + 1: first tile, first bucket of each request
+    const uint32_t* bkt0;
+    uint32_t* bend;              // per bucket: count, then start, then (scattered) end of its positions
+    unsigned long long* rec;     // (vertex << 32 | position), by bucket
+    unsigned long long* tab;     // kPartSlots per bucket: such words, all ones = empty
+    uint32_t* fpos;
+    // Stands for the table in rel_emit_kernel.
+    __device__ __forceinline__ uint32_t hint(uint64_t p) const { return fpos[p]; }
+    __device__ __forceinline__ uint64_t first_of(uint32_t hint, uint32_t, uint32_t) const { return hint; }
+    __device__ __forceinline__ uint64_t first(uint32_t r, uint32_t v) const;
+};
+
+__device__ __forceinline__ uint32_t part_hash(uint32_t v) {
+    uint32_t h = v * 0x9E3779B1u;
+    h ^= h >> 15;
+    h *= 0x85EBCA77u;
+    return h ^ (h >> 13);
+}
+// The bucket takes the hash's high bits, the first slot its low ones: one of every four, so that a
+// lookup reads the four in one go (a wave waits for the longest of its lanes' probes).
+__device__ __forceinline__ uint32_t part_slot(uint32_t h) { return h & (kPartSlots - 4); }
+__device__ __forceinline__ uint32_t part_bucket(uint32_t h, uint32_t buckets) { return __umulhi(h, buckets); }
+
+__device__ __forceinline__ uint64_t RelParts::first(uint32_t r, uint32_t v) const {
+    const uint32_t b0 = bkt0[r], nb = bkt0[r + 1] - b0, h = part_hash(v);
+    if (!nb || v == 0xFFFFFFFFu) return ~0ull;  // (no vertex; an empty slot's)
+    const ulonglong2* t = (const ulonglong2*)(tab + (uint64_t)(b0 + part_bucket(h, nb)) * kPartSlots);
+    for (uint32_t i = 0, s = part_slot(h); i < kPartSlots; i += 4, s = (s + 4) & (kPartSlots - 1)) {
+        const ulonglong2 a = t[s / 2], b = t[s / 2 + 1];
+        if ((uint32_t)(a.x >> 32) == v) return (uint32_t)a.x;
+        if ((uint32_t)(a.y >> 32) == v) return (uint32_t)a.y;
+        if ((uint32_t)(b.x >> 32) == v) return (uint32_t)b.x;
+        if ((uint32_t)(b.y >> 32) == v) return (uint32_t)b.y;
+        if (b.y == ~0ull) break;  // (a group fills in order)
+    }
+    return ~0ull;
+}
+
+__global__ __launch_bounds__(1024) void rel_part_prepare_kernel(RelParts t, uint32_t maxb, const uint64_t* __restrict__ off,
+                                                                const RelReq* __restrict__ req, uint32_t R, uint32_t H,
+                                                                uint64_t total, uint64_t P, uint64_t* __restrict__ Q,
+                                                                uint32_t* bad, uint32_t* invalid) {
+    if (blockIdx.x) {
+        const uint64_t i0 = (uint64_t)(blockIdx.x - 1) * 1024 + threadIdx.x, threads = (uint64_t)(gridDim.x - 1) * 1024;
+        for (uint64_t i = i0; i < P; i += threads) t.fpos[i] = ~0u;
+        for (uint64_t i = i0; i < maxb; i += threads) t.bend[i] = 0;
+        return;
+    }
+    rel_starts(off, req, R, H, total, P, Q, const_cast<uint32_t*>(t.tile0), const_cast<uint32_t*>(t.bkt0), bad, invalid);
+}
+
+// Batches that go by partition: kPartMin positions and a tile per request on average (GRASS_EXPORT_SLOT asks
+// for a table in memory).  Whole mini-batch by table / by partition, us: R-MAT s24 [25, 10] one request
+// of 365 k positions 158 / 187, of 677 k 204 / 223, four together 1.45 M 278 / 276, sixteen 1.6 M 314 / 288;
+// s22 uniform 21 M 2088 / 1329; s16, most positions repeats, 3.7 M 540 / 451; 120 requests of 9.6 k 257 / 225.
+constexpr uint64_t kPartMin = 1ull << 20;
+constexpr int kPartBlock = 512;
+constexpr int kPartPer = kPartTile / kPartBlock;
+
+// One workgroup per tile: counts its buckets' positions (SCATTER: takes room for them in each bucket,
+// and writes them there).
+template <bool SCATTER>
+__global__ __launch_bounds__(kPartBlock) void rel_part_kernel(RelSeq q, RelParts t, uint32_t* err) {
+    __shared__ uint32_t hist[kPartBuckets];
+    __shared__ uint64_t beg[GRASS_KHOP_MAX_HOPS + 1];
+    __shared__ const uint32_t* arr[GRASS_KHOP_MAX_HOPS + 1];
+    if (blockIdx.x >= t.tile0[q.R]) return;
+    uint32_t r = 0;
+    for (uint32_t hi = q.R - 1; r < hi;) {  // the last request whose first tile is not after this one
+        const uint32_t mid = r + (hi - r + 1) / 2;
+        if (t.tile0[mid] <= blockIdx.x) r = mid;
+        else hi = mid - 1;
+    }
+    const uint32_t b0 = t.bkt0[r], nb = t.bkt0[r + 1] - b0;
+    const uint64_t p0 = q.Q[r] + (uint64_t)(blockIdx.x - t.tile0[r]) * kPartTile, p1 = min(p0 + kPartTile, q.Q[r + 1]);
+    for (uint32_t i = threadIdx.x; i < nb; i += kPartBlock) hist[i] = 0;
+    if (threadIdx.x == 0) {  // the stretches of the request's positions: its seeds, and its edges of each hop
+        const RelReq k = q.req[r];
+        beg[0] = q.Q[r];
+        arr[0] = k.seeds;
+        uint64_t at = q.Q[r] + k.num;
+        for (uint32_t h = 0; h < q.H; ++h) {
+            const uint64_t e0 = q.off[(uint64_t)h * (q.R + 1) + r];
+            beg[h + 1] = at;
+            arr[h + 1] = q.dst + e0;
+            at += q.off[(uint64_t)h * (q.R + 1) + r + 1] - e0;
+        }
+    }
+    __syncthreads();
+    uint32_t v[kPartPer], at[kPartPer];
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kPartPer; ++i) {
+        const uint64_t p = p0 + (uint64_t)i * kPartBlock + threadIdx.x;
+        v[i] = 0xFFFFFFFFu;
+        if (p < p1) {
+            uint32_t s = 0;
+            for (uint32_t h = 1; h <= q.H; ++h) s = p >= beg[h] ? h : s;
+            v[i] = arr[s][p - beg[s]];
+            if (v[i] >= q.n) {  // a seed or destination that is not a vertex of the graph
+                bad = true;
+                v[i] = 0xFFFFFFFFu;
+            }
+        }
+    }
+    if (bad) atomicOr(err, 1u);
+#pragma unroll
+    for (int i = 0; i < kPartPer; ++i)
+        if (v[i] != 0xFFFFFFFFu) at[i] = atomicAdd(&hist[part_bucket(part_hash(v[i]), nb)], 1u);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < nb; i += kPartBlock) {
+        const uint32_t c = hist[i];
+        if (c) {
+            const uint32_t base = atomicAdd(&t.bend[b0 + i], c);
+            if (SCATTER) hist[i] = base;
+        }
+    }
+    if (!SCATTER) return;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kPartPer; ++i) {
+        const uint32_t p = (uint32_t)(p0 + (uint64_t)i * kPartBlock + threadIdx.x);
+        if (v[i] != 0xFFFFFFFFu)
+            t.rec[hist[part_bucket(part_hash(v[i]), nb)] + at[i]] = ((unsigned long long)v[i] << 32) | p;
+    }
+}
+
+// One workgroup per bucket.  *bad |= 2: more distinct keys than slots.
+__global__ __launch_bounds__(kPartBlock) void rel_part_dedup_kernel(RelSeq q, RelParts t, uint32_t* bad) {
+    __shared__ unsigned long long tab[kPartSlots];
+    const uint32_t k = blockIdx.x;
+    if (k >= t.bkt0[q.R]) return;
+    for (uint32_t i = threadIdx.x; i < kPartSlots; i += kPartBlock) tab[i] = ~0ull;
+    __syncthreads();
+    const uint32_t lo = k ? t.bend[k - 1] : 0u, hi = t.bend[k];
+    bool full = false;
+    for (uint32_t i = lo + threadIdx.x; i < hi; i += kPartBlock) {
+        const unsigned long long w = t.rec[i];
+        uint32_t s = part_slot(part_hash((uint32_t)(w >> 32))), probes = 0;
+        for (;; ++s) {
+            unsigned long long* slot = &tab[s & (kPartSlots - 1)];
+            unsigned long long cur = *(volatile unsigned long long*)slot;
+            if (cur == ~0ull) cur = atomicCAS(slot, ~0ull, w);
+            if (cur == ~0ull) break;
+            if (((cur ^ w) >> 32) == 0) {
+                if (cur > w) atomicMin(slot, w);
+                break;
+            }
+            if (++probes == kPartSlots) {
+                full = true;
+                break;
+            }
+        }
+    }
+    if (full) atomicOr(bad, 2u);
+    __syncthreads();
+    for (uint32_t i = lo + threadIdx.x; i < hi; i += kPartBlock) {
+        const unsigned long long w = t.rec[i];
+        uint32_t s = part_slot(part_hash((uint32_t)(w >> 32))), probes = 0;
+        unsigned long long cur = tab[s & (kPartSlots - 1)];
+        while (((cur ^ w) >> 32) && ++probes < kPartSlots) cur = tab[++s & (kPartSlots - 1)];
+        if (cur < w) t.fpos[(uint32_t)w] = (uint32_t)cur;
+    }
+    unsigned long long* out = t.tab + (uint64_t)k * kPartSlots;
+    for (uint32_t i = threadIdx.x; i < kPartSlots; i += kPartBlock) out[i] = tab[i];
+}
+
+__global__ __launch_bounds__(kExBlock) void rel_part_words_kernel(const uint32_t* __restrict__ fpos, uint64_t P,
+                                                                  FirstWord* __restrict__ words) {
+    const uint64_t nwords = (P + kWave - 1) / kWave, waves = (uint64_t)gridDim.x * (kExBlock / kWave);
+    for (uint64_t w = ((uint64_t)blockIdx.x * kExBlock + threadIdx.x) / kWave; w < nwords; w += waves) {
+        const uint64_t p = w * kWave + lane_id();
+        const unsigned long long bits = __ballot(p < P && fpos[p] == ~0u);
+        if (lane_id() == 0) words[w] = make_ulonglong2(bits, 0ull);
+    }
+}
+
+hipError_t rel_build_parts(const RelParts& t, uint32_t maxb, const RelSeq& q, uint64_t P, FirstWord* d_words,
+                           uint64_t* d_part, uint64_t* d_sc, uint32_t* d_bad, const grass_khop_output* b,
+                           grass_khop_blocks* out, hipStream_t s) {
+    const unsigned tiles = (unsigned)(P / kPartTile + q.R);
+    hipLaunchKernelGGL(rel_part_prepare_kernel, dim3(1 + (unsigned)std::min<uint64_t>(P / 16384 + 1, 512)), dim3(1024), 0, s, t,
+                       maxb, q.off, q.req, q.R, q.H, b->total, P, const_cast<uint64_t*>(q.Q), d_bad, d_bad + 1);
+    hipLaunchKernelGGL(rel_part_kernel<false>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad);
+    hipLaunchKernelGGL(scan_partials_kernel<uint32_t>, dim3(1), dim3(1024), 0, s, t.bend, (uint64_t)maxb, (uint32_t*)nullptr);
+    hipLaunchKernelGGL(rel_part_kernel<true>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad);
+    hipLaunchKernelGGL(rel_part_dedup_kernel, dim3(maxb), dim3(kPartBlock), 0, s, q, t, d_bad);
+    const unsigned gP = (unsigned)std::min<uint64_t>((P + kExBlock - 1) / kExBlock + 1, kExGrid);
+    hipLaunchKernelGGL(rel_part_words_kernel, dim3(gP), dim3(kExBlock), 0, s, (const uint32_t*)t.fpos, P, d_words);
+    return rel_number(t, q, P, d_words, d_part, d_sc, d_bad, out, s);
 }
 
 // At most kOneWgEntries positions and 1024 requests: the whole build in one launch of one workgroup, the
@@ -524,8 +786,24 @@ int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, cons
                    pb = std::max<uint32_t>(bits(P), 1u);  // positions < 2^pb - 1
     const char* force = getenv("GRASS_EXPORT_SLOT");
     const bool wide = rb + vb + pb > 64 || (force && strcmp(force, "16") == 0);
-    if (ws.scratch.reserve(need) != hipSuccess || ws.ht.reserve(slots * (wide ? 16 : 8)) != hipSuccess)
-        return GRASS_ENOMEM;
+    if (ws.scratch.reserve(need) != hipSuccess) return GRASS_ENOMEM;
+    const uint32_t maxb = (uint32_t)std::min<uint64_t>(P / kPartKeys + R, 0xFFFFFFFFull);
+    auto carve_parts = [&](Carve& c, RelParts& t) {
+        t.tile0 = c.take<uint32_t>(R + 1);
+        t.bkt0 = c.take<uint32_t>(R + 1);
+        t.bend = c.take<uint32_t>(maxb + 1);
+        t.rec = c.take<unsigned long long>(P);
+        t.tab = c.take<unsigned long long>((uint64_t)maxb * kPartSlots);
+        t.fpos = c.take<uint32_t>(P);
+    };
+    bool parts = P >= kPartMin && P < 0xFFFFFFFFull && R && R <= kPrepRequests && P / R >= kPartTile && !force;
+    if (parts) {
+        Carve size(nullptr);
+        RelParts t{};
+        carve_parts(size, t);
+        parts = ws.ht.reserve(size.off + 256) == hipSuccess;
+    }
+    if (!parts && ws.ht.reserve(slots * (wide ? 16 : 8)) != hipSuccess) return GRASS_ENOMEM;
     // this overwrites the k-hop dedup table's memory: the next k-hop batch clears it first
     ws.ht_gen = 0xFFFF;
     Carve cv(ws.scratch.ptr);
@@ -563,6 +841,22 @@ int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, cons
     // do not fit the requests
     uint32_t* d_bad = (uint32_t*)(d_sc + 2);
     RelSeq q{d_req, b->offsets_dev, b->src_dev, b->dst_dev, d_Q, R, H, (uint32_t)g->n};
+    if (parts) {
+        Carve c(ws.ht.ptr);
+        RelParts t{};
+        carve_parts(c, t);
+        e = rel_build_parts(t, maxb, q, P, d_words, d_part, d_sc, d_bad, b, out, s);
+        if (e == hipSuccess) e = hipMemcpyAsync(hres, d_sc + 1, 16, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return status_of(e);
+        if (!(hres[1] & 2)) {
+            if (hres[1] != 0) return GRASS_EINVAL;
+            out->nodes = hres[0];
+            return out->nodes > out->node_capacity ? GRASS_ECAPACITY : GRASS_OK;
+        }
+        // a bucket's keys did not fit its table: the other way
+        if (ws.ht.reserve(slots * (wide ? 16 : 8)) != hipSuccess) return GRASS_ENOMEM;
+    }
     if (wide) {
         RelTab16 t{(unsigned long long*)ws.ht.ptr, slots - 1, 64 - lg};
         e = rel_build(t, q, P, d_len, d_words, d_part, d_sc, d_bad, b, out, s);
