@@ -1004,7 +1004,7 @@ static int mdrw_run(grass_graph* g, MdrwState& st, hipStream_t s, bool replay) {
     Carve c2(st.tmp2.p);
     uint64_t* d_coff = c2.take<uint64_t>(NV + 1);
     uint64_t* d_part2 = c2.take<uint64_t>(nbV + 2);
-    e = exclusive_scan(ChunkGen{o_verts, dg.deg}, Count{NV, nullptr}, NV, d_coff, d_part2, d_part2 + nbV + 1, s);
+    e = exclusive_scan<1, 1>(ChunkGen{o_verts, dg.deg}, Count{NV, nullptr}, NV, d_coff, d_part2, d_part2 + nbV + 1, s);
     if (e != hipSuccess) return status_of(e);
     if (!replay) {
         int rc = sync_read(s, &st.NC, d_coff + NV, 8);
@@ -1071,7 +1071,7 @@ static int mdrw_run(grass_graph* g, MdrwState& st, hipStream_t s, bool replay) {
                            (const uint32_t*)d_dmap, d_rows);
         e = exclusive_scan(PopGen{d_rows, W}, Count{0, d_nd}, n, d_pbase, d_partN, d_partN + nbN + 1, s);
         if (e == hipSuccess)
-            e = exclusive_scan(UChunkGen{d_dvert, dg.deg}, Count{0, d_nd}, n, d_uoff, d_partN, d_nu, s);
+            e = exclusive_scan<1, 1>(UChunkGen{d_dvert, dg.deg}, Count{0, d_nd}, n, d_uoff, d_partN, d_nu, s);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(mdrw_xpair_kernel, dim3(sgrid), dim3(256), 0, s, verts, voff, i0, i1, W,
                            (const uint32_t*)d_dmap, (const unsigned long long*)d_rows, (const uint64_t*)d_pbase,

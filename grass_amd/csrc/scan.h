@@ -161,12 +161,13 @@ __global__ __launch_bounds__(kScanBlock) void scan_write_kernel(Gen gen, Count c
 
 inline uint64_t scan_blocks(uint64_t n_max) { return n_max ? (n_max + kScanTile - 1) / kScanTile : 1; }
 
-// Scratch: partials[scan_blocks(n_max)] and total[1].
-template <int STRIDE = 1, class Gen>
+// Scratch: partials[scan_blocks(n_max)] and total[1].  DIRECT: the most tiles for one launch; 1 for a generator
+// that gathers (13 k values by two dependent random loads each: 39 us in one launch, 20 in two).
+template <int STRIDE = 1, uint64_t DIRECT = kScanDirectMax, class Gen>
 hipError_t exclusive_scan(Gen gen, Count cnt, uint64_t n_max, uint64_t* out, uint64_t* partials,
                           uint64_t* total, hipStream_t stream) {
     const uint64_t nb = scan_blocks(n_max);
-    if (nb <= kScanDirectMax) {
+    if (nb <= DIRECT) {
         hipLaunchKernelGGL((scan_write_kernel<Gen, kScanDirect, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
                            gen, cnt, (const uint64_t*)nullptr, total, out);
         return hipGetLastError();
