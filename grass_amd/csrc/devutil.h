@@ -206,6 +206,40 @@ __device__ __forceinline__ void put_field(uint32_t* B, uint64_t w0, uint64_t at,
     }
 }
 
+// 64 x 64 bits over the wave: lane i holds row i; the result's lane j holds column j (bit i = bit j of lane
+// i's row).  Six exchanges with the lane 32, 16, .. 1 away, each keeping half of the own bits: swaps
+// of lane halves and rows, byte selects, then rotated bits, 30 instructions in all.
+struct BitTranspose {
+    uint32_t p16, p8, r4, r2, r1, k4, k2, k1;  // the lane's byte selectors, rotations and kept bits
+    __device__ __forceinline__ BitTranspose() {
+        const uint32_t lane = lane_id();
+        p16 = lane & 16 ? 0x07060302u : 0x05040100u;  // high (low) halves of the even row's word, then of the odd's
+        p8 = lane & 8 ? 0x03070105u : 0x06020400u;    // bytes of {own, other}
+        r4 = lane & 4 ? 4u : 28u;
+        r2 = lane & 2 ? 2u : 30u;
+        r1 = lane & 1 ? 1u : 31u;
+        k4 = lane & 4 ? 0xF0F0F0F0u : 0x0F0F0F0Fu;
+        k2 = lane & 2 ? 0xCCCCCCCCu : 0x33333333u;
+        k1 = lane & 1 ? 0xAAAAAAAAu : 0x55555555u;
+    }
+    __device__ __forceinline__ uint32_t half(uint32_t x) const {
+        const auto s = __builtin_amdgcn_permlane16_swap(x, x, false, false);  // {even row's word, odd row's}
+        x = __builtin_amdgcn_perm(s[1], s[0], p16);
+        uint32_t y = dpp_move<0x128>(x);  // lane ^ 8
+        x = __builtin_amdgcn_perm(y, x, p8);
+        y = dpp_move<0x141>(dpp_move<0x1B>(x));  // lane ^ 4: ^ 3, ^ 7
+        x = (x & k4) | (__builtin_amdgcn_alignbit(y, y, r4) & ~k4);
+        y = dpp_move<0x4E>(x);
+        x = (x & k2) | (__builtin_amdgcn_alignbit(y, y, r2) & ~k2);
+        y = dpp_move<0xB1>(x);
+        return (x & k1) | (__builtin_amdgcn_alignbit(y, y, r1) & ~k1);
+    }
+    __device__ __forceinline__ unsigned long long operator()(unsigned long long m) const {
+        const auto s = __builtin_amdgcn_permlane32_swap((uint32_t)m, (uint32_t)(m >> 32), false, false);
+        return ((unsigned long long)half(s[1]) << 32) | half(s[0]);
+    }
+};
+
 // p[0..count) = value.  Used instead of hipMemsetAsync for anything a caller might capture in a
 // HIP graph.
 template <typename T>

@@ -458,6 +458,8 @@ constexpr uint32_t kSliceWords = kSlice / 64;
 constexpr int kIndBlock = 256;
 constexpr int kIndWaves = kIndBlock / kWave;
 constexpr uint32_t kRowPitch = kSliceWords + 1;  // u64 words per staged row in LDS (odd: fewer bank conflicts)
+constexpr uint32_t kStageHits = 512;  // hits of a window gathered in LDS
+constexpr uint32_t kFewInstances = 16;  // 6: 2.20 ms, and 70 us where s16 takes 60; every window: 2.32
 
 // Instance of pair p: the largest i in [i0, i1) with voff[i] <= p.
 __device__ __forceinline__ uint32_t inst_of(const uint64_t* __restrict__ voff, uint32_t i0, uint32_t i1,
@@ -571,17 +573,15 @@ __global__ __launch_bounds__(256) void mdrw_xpair_kernel(const uint32_t* __restr
     }
 }
 
-// chunk c of the slice's distinct vertices: ux[c] = dense id, uk[c] = chunk index in its list
+// chunk c of the slice's distinct vertices: {dense id, chunk index in its list, vertex}
 __global__ __launch_bounds__(256) void mdrw_uexpand_kernel(const uint64_t* __restrict__ uoff,
                                                            const uint64_t* __restrict__ nd,
-                                                           uint32_t* __restrict__ ux, uint32_t* __restrict__ uk) {
+                                                           const uint32_t* __restrict__ dvert,
+                                                           uint4* __restrict__ uchunk) {
     const uint64_t ND = *nd;
     for (uint64_t d = (uint64_t)blockIdx.x * 256 + threadIdx.x; d < ND; d += (uint64_t)gridDim.x * 256) {
         const uint64_t b = uoff[d], e = uoff[d + 1];
-        for (uint64_t c = b; c < e; ++c) {
-            ux[c] = (uint32_t)d;
-            uk[c] = (uint32_t)(c - b);
-        }
+        for (uint64_t c = b; c < e; ++c) uchunk[c] = make_uint4((uint32_t)d, (uint32_t)(c - b), dvert[d], 0u);
     }
 }
 
@@ -591,18 +591,23 @@ __global__ __launch_bounds__(256) void mdrw_uexpand_kernel(const uint64_t* __res
 // sources, x for the whole range of pair (i, x)).  Output slot of (instance i, x, chunk k) is
 // coff[pair (i, x)] + k in the instance-major chunk enumeration, so a scan of the counts gives
 // every (i, x, k) its position and the edges land ordered by instance, vertex and list position.
-// COUNT: each lane adds its own entry's matches to per-wave LDS counters (the order of the adds
-// does not matter).  WRITE: lane l keeps the next output slot of instance 64 w + l of each mask
-// word w in registers, and per matched instance one ballot ranks the wave's hits in list order.
+// The 64 words mask(x) & mask(y) of a window, transposed over the wave, give lane l the window's
+// entries of instance 64 w + l: COUNT adds up their numbers in registers.  WRITE: lane l keeps the
+// instance's next output slot, and a window goes instance by instance: one ballot and one masked store
+// each.  One mask word, more than kFewInstances instances and at most kStageHits hits: these are ranked
+// from the transposed word and gathered in LDS instead, so that each instance's run is stored by
+// neighbouring lanes (with more words the registers for it cost more than it gives).
+// Bound by instruction issue and by the chain of loads that starts a chunk, so a slice of one mask word
+// has its own instantiation (a third of the registers, rows kept in them) and the next chunk's start
+// is loaded ahead.  64 instances of 16384, R-MAT s22, 103 M entries, 262 M hits: count 1.61 ms (an LDS
+// atomic per hit, no loads ahead) -> 1.21, write 2.52 (every window instance by instance) -> 2.17.
 // MODE 0 counts; MODE 1 writes with 32-bit output slots (fewer than 2^32 induced edges), MODE 2
 // with 64-bit ones.
-template <int FMT, int MODE>
+template <int FMT, int MODE, uint32_t NW>
 __global__ __launch_bounds__(kIndBlock) void mdrw_induced_kernel(DevGraph g, const unsigned long long* __restrict__ rows,
                                                                  uint32_t W, const ulonglong2* __restrict__ dbits,
-                                                                 const uint32_t* __restrict__ dvert,
                                                                  const uint64_t* __restrict__ nchunks,
-                                                                 const uint32_t* __restrict__ ux,
-                                                                 const uint32_t* __restrict__ uk,
+                                                                 const uint4* __restrict__ uchunk,
                                                                  const uint64_t* __restrict__ pbase,
                                                                  const uint64_t* __restrict__ xpair,
                                                                  uint64_t* __restrict__ ccnt,
@@ -610,35 +615,65 @@ __global__ __launch_bounds__(kIndBlock) void mdrw_induced_kernel(DevGraph g, con
                                                                  uint32_t* __restrict__ idst) {
     constexpr bool WRITE = MODE != 0;
     using Slot = typename std::conditional<MODE == 2, uint64_t, uint32_t>::type;
-    __shared__ uint32_t counts[WRITE ? 1 : kIndWaves][kSlice];  // COUNT: per wave and instance
-    __shared__ unsigned long long staged[kIndWaves][kWave * kRowPitch];  // the window's rows
+    // the window's rows, or (one word a row) its gathered hits
+    constexpr bool GATHER = MODE == 1 && NW == 1;
+    __shared__ __align__(16) unsigned long long staged[kIndWaves][NW > 1 ? kWave * kRowPitch : GATHER ? kStageHits : 1];
+    __shared__ uint4 columns[GATHER ? kIndWaves : 1][kWave];  // WRITE: per instance {entries, first hit, slot}
     const int lane = lane_id();
     const unsigned long long below = (1ull << lane) - 1;
     const uint64_t NU = *nchunks;
     const uint64_t waves = (uint64_t)gridDim.x * kIndWaves;
-    uint32_t* cnt = counts[WRITE ? 0 : threadIdx.x / kWave];
-    unsigned long long* R = staged[threadIdx.x / kWave];
-    for (uint64_t c = (uint64_t)blockIdx.x * kIndWaves + threadIdx.x / kWave; c < NU; c += waves) {
-        const uint32_t dx = __builtin_amdgcn_readfirstlane(ux[c]);
-        const uint32_t kc = __builtin_amdgcn_readfirstlane(uk[c]);
-        const uint32_t x = __builtin_amdgcn_readfirstlane(dvert[dx]);
-        const uint64_t pb = pbase[dx];
-        unsigned long long mx[kSliceWords];
-        Slot acc[kSliceWords];  // WRITE, lane l: next output slot of instance 64 w + l
+    const uint32_t wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    unsigned long long* R = staged[wid];
+    uint4* cols = columns[GATHER ? wid : 0];
+    uint2* hits = (uint2*)R;  // {output slot, y}
+    const BitTranspose transpose;
+    // One word a row: a chunk's vertex, rows and header are loaded while the chunk before is decoded, and
+    // where they are a chunk earlier still.
+    struct Meta {
+        uint4 u;  // {dense id, chunk index, vertex}
+        uint64_t pb;
+        unsigned long long mx[NW];
+        uint4 hw;
+    };
+    auto load_meta = [&](const uint4 u) {
+        Meta t;
+        t.u = u;
+        t.pb = pbase[u.x];
+#pragma unroll
+        for (uint32_t w = 0; w < NW; ++w) t.mx[w] = NW == 1 || w < W ? rows[(uint64_t)u.x * (NW == 1 ? 1 : W) + w] : 0ull;
+        t.hw = load_hdr_words(g, u.z);
+        return t;
+    };
+    const uint64_t c0 = (uint64_t)blockIdx.x * kIndWaves + wid;
+    if (c0 >= NU) return;
+    Meta next;
+    uint4 after = make_uint4(0u, 0u, 0u, 0u);
+    if (NW == 1) {
+        next = load_meta(uchunk[c0]);
+        after = uchunk[min(c0 + waves, NU - 1)];
+    }
+    for (uint64_t c = c0; c < NU; c += waves) {
+        const Meta t = NW == 1 ? next : load_meta(uchunk[c]);
+        if (NW == 1) {
+            next = load_meta(after);
+            after = uchunk[min(c + 2 * waves, NU - 1)];
+        }
+        const uint32_t kc = t.u.y, x = t.u.z;
+        const uint64_t pb = t.pb;
+        unsigned long long mx[NW];
+        Slot acc[NW];  // lane l: hits so far (WRITE: next output slot) of instance 64 w + l
         uint32_t rbase = 0;
 #pragma unroll
-        for (uint32_t w = 0; w < kSliceWords; ++w) {
-            const unsigned long long v = w < W ? rows[(uint64_t)dx * W + w] : 0ull;
-            mx[w] = readfirstlane_u64(v);
+        for (uint32_t w = 0; w < NW; ++w) {
+            mx[w] = readfirstlane_u64(t.mx[w]);
             acc[w] = 0;
             if (WRITE && ((mx[w] >> lane) & 1ull))
                 acc[w] = (Slot)cpos[xpair[pb + rbase + __popcll(mx[w] & below)] + kc];
-            if (!WRITE) cnt[w * 64 + lane] = 0;
             rbase += __popcll(mx[w]);
         }
-        if (!WRITE) wave_sync();
         Hdr h;
-        load_hdr<FMT>(g, x, h);
+        unpack_hdr<FMT>(t.hw, h);
         UDiv d1, d0;
         d1.init(h.q + 1);
         d0.init(h.q);
@@ -680,14 +715,14 @@ __global__ __launch_bounds__(kIndBlock) void mdrw_induced_kernel(DevGraph g, con
         // so a row is one memory access instead of one per mask word; the loads land in registers
         // (fetch_rows) and go to LDS in the per-lane row layout later (stage_rows).
         const uint32_t cpr = W >> 1, per = W >= 2 ? kWave / cpr : kWave;  // chunks per row, rows per round
-        ulonglong2 rv[kSliceWords / 2];
+        ulonglong2 rv[NW > 1 ? NW / 2 : 1];
         auto fetch_rows = [&](uint32_t dy) {
-            if (W == 1) {
+            if (NW == 1 || W == 1) {
                 rv[0].x = dy != kNoRow ? rows[dy] : 0ull;
                 return;
             }
 #pragma unroll
-            for (uint32_t r = 0; r < kSliceWords / 2; ++r) {
+            for (uint32_t r = 0; r < NW / 2; ++r) {
                 if (r >= cpr) break;
                 const uint32_t e = r * per + lane / cpr, q = lane % cpr;
                 const uint32_t de = __shfl(dy, (int)e, kWave);
@@ -696,12 +731,13 @@ __global__ __launch_bounds__(kIndBlock) void mdrw_induced_kernel(DevGraph g, con
             }
         };
         auto stage_rows = [&]() {
+            if (NW == 1) return;
             if (W == 1) {
                 R[lane * kRowPitch] = rv[0].x;
                 return;
             }
 #pragma unroll
-            for (uint32_t r = 0; r < kSliceWords / 2; ++r) {
+            for (uint32_t r = 0; r < NW / 2; ++r) {
                 if (r >= cpr) break;
                 const uint32_t e = r * per + lane / cpr, q = lane % cpr;
                 R[e * kRowPitch + 2 * q] = rv[r].x;
@@ -716,21 +752,49 @@ __global__ __launch_bounds__(kIndBlock) void mdrw_induced_kernel(DevGraph g, con
             const bool more = base + kWave < ke;  // uniform
             uint32_t yn = 0;
             if (more) decode_window(base + kWave, yn, dy);
-            wave_sync();
+            unsigned long long m1 = 0;
+            if (NW == 1) {  // the next window's rows can be on their way
+                m1 = mx[0] & rv[0].x;
+                if (more) fetch_rows(dy);
+            } else {
+                wave_sync();
+            }
 #pragma unroll
-            for (uint32_t w = 0; w < kSliceWords; ++w) {
+            for (uint32_t w = 0; w < NW; ++w) {
                 if (mx[w] == 0ull) continue;  // uniform
-                const unsigned long long m = mx[w] & R[lane * kRowPitch + w];
+                const unsigned long long m = NW == 1 ? m1 : mx[w] & R[lane * kRowPitch + w];
+                if (!__any(m != 0ull)) continue;
                 if (!WRITE) {
-                    for (unsigned long long b2 = m; b2; b2 &= b2 - 1)
-                        atomicAdd(&cnt[w * 64 + __builtin_ctzll(b2)], 1u);
+                    acc[w] += (Slot)__popcll(transpose(m));
                     continue;
+                }
+                const unsigned long long bits = wave_or_u64(m);
+                if (GATHER && __popcll(bits) > kFewInstances) {
+                    const unsigned long long t = transpose(m);
+                    const uint32_t c = (uint32_t)__popcll(t), inc = wave_inclusive_sum(c);
+                    const uint32_t H = lane_get(inc, kWave - 1);
+                    if (H <= kStageHits) {
+                        cols[lane] = make_uint4((uint32_t)t, (uint32_t)(t >> 32), inc - c, (uint32_t)acc[w]);
+                        wave_sync();
+                        for (unsigned long long b2 = m; b2; b2 &= b2 - 1) {
+                            const uint4 q = cols[__builtin_ctzll(b2)];
+                            const uint32_t k = lanes_below(((unsigned long long)q.y << 32) | q.x);
+                            hits[q.z + k] = make_uint2(q.w + k, y);
+                        }
+                        wave_sync();
+                        for (uint32_t i = lane; i < H; i += kWave) {
+                            const uint2 s = hits[i];
+                            idst[s.x] = s.y;
+                        }
+                        wave_sync();  // (the next word's hits)
+                        acc[w] += (Slot)c;
+                        continue;
+                    }
                 }
                 // Uniform loop over the instances with at least one hit in the window (a third of
                 // x's instances in the window have none), by 32-bit halves of the word: per
                 // instance one ballot, one masked store of its run (the sources are filled per pair
                 // by mdrw_src_kernel) and one writelane that moves its slot on.
-                const unsigned long long bits = wave_or_u64(m);
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
                     uint32_t hb = (uint32_t)(bits >> (32 * half));
@@ -747,23 +811,21 @@ __global__ __launch_bounds__(kIndBlock) void mdrw_induced_kernel(DevGraph g, con
                     }
                 }
             }
-            wave_sync();  // every lane is done with the rows: the next window's replace them
-            if (more) {
+            if (NW > 1) wave_sync();  // every lane is done with the rows: the next window's replace them
+            if (NW > 1 && more) {
                 fetch_rows(dy);
                 stage_rows();
             }
             y = yn;
         }
         if (!WRITE) {
-            wave_sync();
             rbase = 0;
 #pragma unroll
-            for (uint32_t w = 0; w < kSliceWords; ++w) {
+            for (uint32_t w = 0; w < NW; ++w) {
                 if ((mx[w] >> lane) & 1ull)
-                    ccnt[xpair[pb + rbase + __popcll(mx[w] & below)] + kc] = cnt[w * 64 + lane];
+                    ccnt[xpair[pb + rbase + __popcll(mx[w] & below)] + kc] = acc[w];
                 rbase += __popcll(mx[w]);
             }
-            wave_sync();  // the counters are cleared for the next chunk
         }
     }
 }
@@ -1022,7 +1084,8 @@ static int mdrw_run(grass_graph* g, MdrwState& st, hipStream_t s, bool replay) {
     unsigned long long* d_rows = nullptr;
     uint64_t *d_did = nullptr, *d_pbase = nullptr, *d_uoff = nullptr, *d_nu = nullptr, *d_partN = nullptr,
              *d_ccnt = nullptr, *d_cpos = nullptr, *d_part3 = nullptr;
-    uint32_t *d_dmap = nullptr, *d_dvert = nullptr, *d_ux = nullptr, *d_uk = nullptr;
+    uint32_t *d_dmap = nullptr, *d_dvert = nullptr;
+    uint4* d_uchunk = nullptr;
     uint64_t* d_xpair = nullptr;
     ulonglong2* d_dbits = nullptr;
     auto plan3 = [&](Carve& c) {
@@ -1036,8 +1099,7 @@ static int mdrw_run(grass_graph* g, MdrwState& st, hipStream_t s, bool replay) {
         d_dbits = c.take<ulonglong2>((n + kWave - 1) / kWave);
         d_dvert = c.take<uint32_t>(n);
         d_xpair = c.take<uint64_t>(NV);
-        d_ux = c.take<uint32_t>(NC);
-        d_uk = c.take<uint32_t>(NC);
+        d_uchunk = c.take<uint4>(NC);
         d_ccnt = c.take<uint64_t>(NC + 1);
         d_cpos = c.take<uint64_t>(NC + 1);
         d_part3 = c.take<uint64_t>(nbC + 2);
@@ -1077,22 +1139,30 @@ static int mdrw_run(grass_graph* g, MdrwState& st, hipStream_t s, bool replay) {
                            (const uint32_t*)d_dmap, (const unsigned long long*)d_rows, (const uint64_t*)d_pbase,
                            (const uint64_t*)d_coff, d_xpair);
         hipLaunchKernelGGL(mdrw_uexpand_kernel, dim3(sgrid), dim3(256), 0, s, (const uint64_t*)d_uoff, d_nd,
-                           d_ux, d_uk);
+                           (const uint32_t*)d_dvert, d_uchunk);
         return hipGetLastError();
     };
     // mode 0 counts, 1 writes with 32-bit output slots, 2 with 64-bit ones
     auto induced = [&](int mode, uint32_t* idst) {
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(sgrid), dim3(kIndBlock), 0, s, dg, (const unsigned long long*)d_rows, W,
-                               (const ulonglong2*)d_dbits, (const uint32_t*)d_dvert, (const uint64_t*)d_nu,
-                               (const uint32_t*)d_ux, (const uint32_t*)d_uk, (const uint64_t*)d_pbase,
+                               (const ulonglong2*)d_dbits, (const uint64_t*)d_nu, (const uint4*)d_uchunk, (const uint64_t*)d_pbase,
                                (const uint64_t*)d_xpair, d_ccnt, (const uint64_t*)d_cpos,
                                idst);
         };
-        if (le)
-            go(mode == 0 ? mdrw_induced_kernel<kLE, 0> : mode == 1 ? mdrw_induced_kernel<kLE, 1> : mdrw_induced_kernel<kLE, 2>);
-        else
-            go(mode == 0 ? mdrw_induced_kernel<kGT, 0> : mode == 1 ? mdrw_induced_kernel<kGT, 1> : mdrw_induced_kernel<kGT, 2>);
+        auto pick = [&](auto fmt, auto words) {
+            constexpr int F = decltype(fmt)::value;
+            constexpr uint32_t N = decltype(words)::value;
+            if (mode == 0) go(mdrw_induced_kernel<F, 0, N>);
+            else if (mode == 1) go(mdrw_induced_kernel<F, 1, N>);
+            else go(mdrw_induced_kernel<F, 2, N>);
+        };
+        using One = std::integral_constant<uint32_t, 1>;
+        using All = std::integral_constant<uint32_t, kSliceWords>;
+        using Le = std::integral_constant<int, kLE>;
+        using Gt = std::integral_constant<int, kGT>;
+        if (le) W == 1 ? pick(Le{}, One{}) : pick(Le{}, All{});
+        else W == 1 ? pick(Gt{}, One{}) : pick(Gt{}, All{});
         return hipGetLastError();
     };
     for (uint32_t i0 = 0; i0 < I; i0 += kSlice) {
