@@ -193,7 +193,8 @@ struct grass_graph {
     uint32_t* d_wstart[grass::kWaveStartSlots] = {};
     uint64_t* d_roff = nullptr;  // full decode by runs: runs before each vertex (n + 1)
     uint64_t dec_runs = 0;       // and their total (set at load)
-    grass::Scratch dec_part;     // full decode: the row-pointer scan's partials (under mu)
+    uint64_t* d_dpre = nullptr;  // full decode: entries before each tile of the row-pointer scan, and all
+    grass::Scratch dec_part;     // until that is there: the scan's partials (under mu)
     hipEvent_t dec_ev = nullptr;  // recorded after each full decode's scan
     hipStream_t stream = nullptr;
     std::mutex mu;

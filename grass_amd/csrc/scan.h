@@ -185,4 +185,21 @@ hipError_t exclusive_scan(Gen gen, Count cnt, uint64_t n_max, uint64_t* out, uin
     return hipGetLastError();
 }
 
+// The two halves of a scan whose tiles' prefixes are kept: made once (prefixes[scan_blocks(n)], and the
+// total after them), then any number of scans of the same values in one launch each.
+template <class Gen>
+hipError_t scan_prefixes(Gen gen, uint64_t n, uint64_t* prefixes, hipStream_t stream) {
+    const uint64_t nb = scan_blocks(n);
+    hipLaunchKernelGGL(scan_reduce_kernel<Gen>, dim3((unsigned)nb), dim3(kScanBlock), 0, stream, gen, Count{n, nullptr}, prefixes);
+    hipLaunchKernelGGL(scan_partials_kernel<uint64_t>, dim3(1), dim3(1024), 0, stream, prefixes, nb, prefixes + nb);
+    return hipGetLastError();
+}
+template <class Gen>
+hipError_t scan_from_prefixes(Gen gen, uint64_t n, const uint64_t* prefixes, uint64_t* out, hipStream_t stream) {
+    const uint64_t nb = scan_blocks(n);
+    hipLaunchKernelGGL((scan_write_kernel<Gen, kScanThree, 1>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream, gen,
+                       Count{n, nullptr}, prefixes, const_cast<uint64_t*>(prefixes) + nb, out);
+    return hipGetLastError();
+}
+
 }  // namespace grass
