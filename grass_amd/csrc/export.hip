@@ -17,7 +17,7 @@
 // the random atomics of the inserts, which the chip takes at 22 to 27 G/s whatever the table's size
 // (a load of a slot and a CAS on it: 25.7 G/s), so a position touches the table once: 16 x 8192 seeds
 // [25, 10] on R-MAT s24, 10.7 M positions, insert 435 us; a second pass that looked every key up again
-// took 196 us more.  A large one therefore makes step 2 by partition (rel_part_*): 241 us with all its
+// took 196 us more.  A large one therefore makes step 2 by partition (rel_part_*): 221 us with all its
 // passes.  The emit, by lookups of the sources and loads a word ahead, is 150 us (229 without either).
 #include <hip/hip_runtime.h>
 
@@ -484,7 +484,7 @@ hipError_t rel_build(const Tab& t, const RelSeq& q, uint64_t P, uint64_t* d_len,
 // (a request's keys of one hash range) are written next to each other as {vertex, position}, and one
 // workgroup deduplicates a bucket in LDS.  fpos[p] becomes the first position of p's key where that is
 // not p; the bucket's table goes to memory for the lookups of the edges' sources.  10.7 M positions, R-MAT
-// s24: prepare 12 us, count 30, scatter 69, dedup 110, words 15.
+// s24: prepare 13 us, count 30, scatter 68, dedup 90 (110 with its positions read and looked up twice), words 15.
 
 struct RelParts {
     const uint32_t* tile0;  // R + 1: first tile, first bucket of each request
@@ -614,41 +614,56 @@ __global__ __launch_bounds__(kPartBlock) void rel_part_kernel(RelSeq q, RelParts
     }
 }
 
-// One workgroup per bucket.  *bad |= 2: more distinct keys than slots.
+// Puts position w into the bucket's table: its slot, or kPartSlots when every slot holds another key.
+__device__ __forceinline__ uint32_t part_insert(unsigned long long* tab, unsigned long long w) {
+    uint32_t s = part_slot(part_hash((uint32_t)(w >> 32)));
+    for (uint32_t probes = 0; probes < kPartSlots; ++probes, s = (s + 1) & (kPartSlots - 1)) {
+        unsigned long long cur = *(volatile unsigned long long*)&tab[s];
+        if (cur == ~0ull) cur = atomicCAS(&tab[s], ~0ull, w);
+        if (cur == ~0ull) return s;
+        if (((cur ^ w) >> 32) == 0) {
+            if (cur > w) atomicMin(&tab[s], w);
+            return s;
+        }
+    }
+    return kPartSlots;
+}
+
+// One workgroup per bucket, whose positions (but for repeats past kPartHeld per thread) it holds in
+// registers: loaded together, and not looked up again.  *bad |= 2: more distinct keys than slots.
+constexpr int kPartHeld = 8;
 __global__ __launch_bounds__(kPartBlock) void rel_part_dedup_kernel(RelSeq q, RelParts t, uint32_t* bad) {
     __shared__ unsigned long long tab[kPartSlots];
     const uint32_t k = blockIdx.x;
     if (k >= t.bkt0[q.R]) return;
+    const uint32_t lo = (k ? t.bend[k - 1] : 0u) + threadIdx.x, hi = t.bend[k];
+    unsigned long long w[kPartHeld];
+    uint32_t s[kPartHeld];
+#pragma unroll
+    for (int j = 0; j < kPartHeld; ++j) w[j] = lo + j * kPartBlock < hi ? t.rec[lo + j * kPartBlock] : ~0ull;
     for (uint32_t i = threadIdx.x; i < kPartSlots; i += kPartBlock) tab[i] = ~0ull;
     __syncthreads();
-    const uint32_t lo = k ? t.bend[k - 1] : 0u, hi = t.bend[k];
     bool full = false;
-    for (uint32_t i = lo + threadIdx.x; i < hi; i += kPartBlock) {
-        const unsigned long long w = t.rec[i];
-        uint32_t s = part_slot(part_hash((uint32_t)(w >> 32))), probes = 0;
-        for (;; ++s) {
-            unsigned long long* slot = &tab[s & (kPartSlots - 1)];
-            unsigned long long cur = *(volatile unsigned long long*)slot;
-            if (cur == ~0ull) cur = atomicCAS(slot, ~0ull, w);
-            if (cur == ~0ull) break;
-            if (((cur ^ w) >> 32) == 0) {
-                if (cur > w) atomicMin(slot, w);
-                break;
-            }
-            if (++probes == kPartSlots) {
-                full = true;
-                break;
-            }
-        }
+#pragma unroll
+    for (int j = 0; j < kPartHeld; ++j) {
+        s[j] = w[j] != ~0ull ? part_insert(tab, w[j]) : 0u;
+        full = full || s[j] == kPartSlots;
+        s[j] &= kPartSlots - 1;
     }
+    for (uint32_t i = lo + kPartHeld * kPartBlock; i < hi; i += kPartBlock) full = part_insert(tab, t.rec[i]) == kPartSlots || full;
     if (full) atomicOr(bad, 2u);
     __syncthreads();
-    for (uint32_t i = lo + threadIdx.x; i < hi; i += kPartBlock) {
-        const unsigned long long w = t.rec[i];
-        uint32_t s = part_slot(part_hash((uint32_t)(w >> 32))), probes = 0;
-        unsigned long long cur = tab[s & (kPartSlots - 1)];
-        while (((cur ^ w) >> 32) && ++probes < kPartSlots) cur = tab[++s & (kPartSlots - 1)];
-        if (cur < w) t.fpos[(uint32_t)w] = (uint32_t)cur;
+#pragma unroll
+    for (int j = 0; j < kPartHeld; ++j) {
+        if (w[j] == ~0ull) continue;
+        const unsigned long long cur = tab[s[j]];
+        if (cur < w[j]) t.fpos[(uint32_t)w[j]] = (uint32_t)cur;
+    }
+    for (uint32_t i = lo + kPartHeld * kPartBlock; i < hi; i += kPartBlock) {
+        const unsigned long long x = t.rec[i];
+        const uint32_t sx = part_insert(tab, x);  // (already there)
+        const unsigned long long cur = tab[sx & (kPartSlots - 1)];
+        if (cur < x) t.fpos[(uint32_t)x] = (uint32_t)cur;
     }
     unsigned long long* out = t.tab + (uint64_t)k * kPartSlots;
     for (uint32_t i = threadIdx.x; i < kPartSlots; i += kPartBlock) out[i] = tab[i];
