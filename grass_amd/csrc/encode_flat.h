@@ -2,10 +2,10 @@
 // its header, then one per field in stream order (LE: rocks, then seas; GT: list order).  A wave
 // takes consecutive slots, 64 a pass, so lists of any length fill its lanes and the column ids are
 // read in order.  Rows have to be strictly ascending with ids below 2^31 (the plan finds out), which
-// keeps every value in 32 bits.  Bound by instruction issue (about 300 a pass).  Measured on R-MAT s22
+// keeps every value in 32 bits.  Bound by instruction issue (about 200 a pass).  Measured on R-MAT s22
 // (2.4 M rows, 128 M entries, GT): a wave per vertex planned in 1.63 ms, wrote the image in 3.65 and made
-// the resident stream of it in 3.2 more; by slots the plan takes 0.83 ms and the stream, straight from the
-// rows, 0.91.
+// the resident stream of it in 3.2 more; by slots the plan takes 0.71 ms and the stream, straight from the
+// rows, 0.81 (0.84 and 0.91 before passes inside one list kept its constants and skipped the placing).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -81,6 +81,34 @@ __device__ __forceinline__ void flat_pos(uint32_t k, uint32_t q, uint32_t R, uin
     c = lo ? b : b + R;
 }
 
+// A list's constants, uniform over the wave: kept while whole passes lie in one list.
+template <int FMT>
+struct FlatList {
+    uint32_t v = 0xFFFFFFFFu;  // whose they are
+    uint32_t C, q, R;
+    UDiv d1, d0;
+    __device__ __forceinline__ void of(uint32_t vertex, uint32_t d) {
+        if (vertex == v) return;
+        v = vertex;
+        flat_geometry<FMT>(d, C, q, R);
+        C = (uint32_t)__builtin_amdgcn_readfirstlane((int)C);
+        q = (uint32_t)__builtin_amdgcn_readfirstlane((int)q);
+        R = (uint32_t)__builtin_amdgcn_readfirstlane((int)R);
+        d1.init(q + 1);
+        d0.init(q);
+    }
+    __device__ __forceinline__ void pos(uint32_t k, uint32_t& c, uint32_t& i) const {  // flat_pos
+        const uint32_t big = R * (q + 1);
+        const bool lo = k < big;
+        UDiv u;
+        u.d = lo ? q + 1 : q;
+        u.m = lo ? d1.m : d0.m;
+        const uint32_t kk = lo ? k : k - big, b = u.div(kk);
+        i = kk - __umul24(b, u.d);
+        c = lo ? b : b + R;
+    }
+};
+
 // Residual of LE sea i of the chunk at list position s0 with L positions (le_residual for ascending rows).
 __device__ __forceinline__ int32_t flat_residual(uint32_t x, uint32_t rl, uint32_t rr, uint32_t i, uint32_t L) {
     return (int32_t)(x - (rl + i * udiv_chunk(rr - rl, L)));
@@ -135,6 +163,10 @@ struct SlotWalk {
         k = (int32_t)(e0 + lane - p) - 1;
         d = e - p - 1;
         head = p > e0 ? p - e0 : 0u;
+    }
+    // Whether slots base .. base + 63 are all fields of vertex cur.
+    __device__ __forceinline__ bool in_list(uint64_t base) const {
+        return base > sc && base + kWave <= readlane_u64(bj, 0);
     }
     // To the vertex of the slot after the last active lane's, which is at place jl: the next vertex when
     // that slot was its last (`end`), so that the 64 from `cur` always hold the next pass.
@@ -192,6 +224,17 @@ struct SegmentScan {
     }
 };
 
+// The OR of all lanes, in lane 63 (the other lanes hold parts of it).
+__device__ __forceinline__ uint32_t wave_or_last(uint32_t x) {
+    x |= dpp_move<0x111>(x);
+    x |= dpp_move<0x112>(x);
+    x |= dpp_move<0x114>(x);
+    x |= dpp_move<0x118>(x);
+    x |= dpp_move<0x142, 0xa>(x);
+    x |= dpp_move<0x143, 0xc>(x);
+    return x;
+}
+
 // A plan's totals.
 struct FlatStats {
     unsigned long long bits;     // of the .graph records
@@ -232,27 +275,42 @@ __global__ __launch_bounds__(kFlatBlock) void flat_plan_kernel(const uint64_t* _
         SlotWalk walk{rowptr, n};
         walk.seek(s0);
         const uint32_t before = walk.sc < s0 ? walk.cur : 0xFFFFFFFFu;  // a vertex begun by another chunk
+        FlatList<FMT> list;
         uint32_t ca = 0, cb = 0;  // the ORs so far of the pass's first vertex
         uint32_t px = s0 - walk.sc >= 2 ? col[s0 - walk.cur - 2] : 0u;  // the id before the pass's first
         for (uint64_t base = s0; base < s1; base += kWave) {
             const uint32_t last = (uint32_t)(s1 - base < (uint64_t)kWave ? s1 - base - 1 : kWave - 1);
-            uint32_t j, d, head;
+            uint32_t j, d, head, C, q, R, c, i;
             int32_t k;
-            walk.place(base, last, own, j, k, d, head);
+            const bool whole = last == kWave - 1 && walk.in_list(base);  // the pass is in one list
+            if (whole) {
+                j = head = 0;
+                k = (int32_t)(base - walk.sc) + (int32_t)lane - 1;
+                d = (uint32_t)(readlane_u64(walk.bj, 0) - walk.sc) - 1;
+                list.of(walk.cur, d);
+                C = list.C;
+                q = list.q;
+                R = list.R;
+                list.pos((uint32_t)k, c, i);
+            } else {
+                walk.place(base, last, own, j, k, d, head);
+                flat_geometry<FMT>(d, C, q, R);
+                flat_pos(k < 0 ? 0u : (uint32_t)k, q, R, c, i);
+            }
             const bool end = k + 1 == (int32_t)d;
             const bool ended = __builtin_amdgcn_readlane((int)end, (int)last);
             const uint32_t v = walk.cur + j;
-            walk.advance((uint32_t)__builtin_amdgcn_readlane((int)j, (int)last), ended);
-            if (base + kWave < s1) walk.request();
+            if (!whole || ended) {
+                walk.advance((uint32_t)__builtin_amdgcn_readlane((int)j, (int)last), ended);
+                if (base + kWave < s1) walk.request();
+            }
             const bool act = lane <= last, field = act && k >= 0;
             const uint64_t at = base + lane - v - 1;  // the entry (k >= 0)
             const uint32_t x = field ? col[at] : 0u;
             uint32_t prev = dpp_move<0x138>(x);
             if (lane == 0) prev = px;
             px = (uint32_t)__builtin_amdgcn_readlane((int)x, kWave - 1);
-            uint32_t C, q, R, c, i, a = 0, b = 0;
-            flat_geometry<FMT>(d, C, q, R);
-            flat_pos(k < 0 ? 0u : (uint32_t)k, q, R, c, i);
+            uint32_t a = 0, b = 0;
             const uint32_t diff = x < v ? v - x : x - v;
             if (field) {
                 general |= (x >> 31) || (k && x <= prev);
@@ -271,9 +329,14 @@ __global__ __launch_bounds__(kFlatBlock) void flat_plan_kernel(const uint64_t* _
                 }
                 if (x < v ? end : !k || prev < v) fps[v] = x < v ? (FMT == kLE ? C + 1 : C) : c + (i != 0);
             }
-            const SegmentScan seg(head);
-            a = seg.any(a) | (j ? 0u : ca);
-            b = seg.any(b) | (j ? 0u : cb);
+            if (whole) {  // lane 63 alone can end the list
+                a = wave_or_last(a) | ca;
+                b = wave_or_last(b) | cb;
+            } else {
+                const SegmentScan seg(head);
+                a = seg.any(a) | (j ? 0u : ca);
+                b = seg.any(b) | (j ? 0u : cb);
+            }
             if (act && end) {
                 if (v == before) {
                     atomicOr(&ors[v].x, a);
@@ -460,31 +523,47 @@ __global__ __launch_bounds__(kFlatBlock) void flat_write_kernel(const uint64_t* 
             }
         };
         request();
+        FlatList<FMT> list;
         uint32_t px = FMT == kGT && s0 - walk.sc >= 2 ? col[s0 - walk.cur - 2] : 0u;
         for (uint32_t t = 0; t < passes; ++t) {
             const uint64_t base = s0 + (uint64_t)t * kWave;
             if (base >= slots) break;
             const bool fin = t + 1 == passes || base + kWave >= slots;
             const uint32_t last = (uint32_t)(slots - base < (uint64_t)kWave ? slots - base - 1 : kWave - 1);
-            uint32_t j, d, head;
+            uint32_t j, d, head, C, q, R, wx, fp = 0;
             int32_t k;
-            walk.place(base, last, own, j, k, d, head);
+            uint64_t sv;
+            const bool whole = last == kWave - 1 && walk.in_list(base);  // the pass is in one list
+            if (whole) {
+                j = 0;
+                k = (int32_t)(base - walk.sc) + (int32_t)lane - 1;
+                d = (uint32_t)(readlane_u64(walk.bj, 0) - walk.sc) - 1;
+                list.of(walk.cur, d);
+                C = list.C;
+                q = list.q;
+                R = list.R;
+                wx = lane_get(wd.x, 0);
+                sv = readlane_u64(st, 0);
+            } else {
+                walk.place(base, last, own, j, k, d, head);
+                flat_geometry<FMT>(d, C, q, R);
+                wx = __shfl(wd.x, (int)j, kWave);
+                if (!STREAM) fp = __shfl(wd.y, (int)j, kWave);
+                sv = ((uint64_t)__shfl((uint32_t)(st >> 32), (int)j, kWave) << 32) | __shfl((uint32_t)st, (int)j, kWave);
+            }
             const uint32_t v = walk.cur + j;
-            const uint32_t wx = __shfl(wd.x, (int)j, kWave);
-            const uint32_t fp = STREAM ? 0u : __shfl(wd.y, (int)j, kWave);
-            const uint64_t sv = ((uint64_t)__shfl((uint32_t)(st >> 32), (int)j, kWave) << 32) | __shfl((uint32_t)st, (int)j, kWave);
-            walk.advance((uint32_t)__builtin_amdgcn_readlane((int)j, (int)last),
-                         __builtin_amdgcn_readlane((int)(k + 1 == (int32_t)d), (int)last));
-            if (!fin) {
-                walk.request();
-                request();
+            const bool ended = __builtin_amdgcn_readlane((int)(k + 1 == (int32_t)d), (int)last);
+            if (!whole || ended) {
+                walk.advance((uint32_t)__builtin_amdgcn_readlane((int)j, (int)last), ended);
+                if (!fin) {
+                    walk.request();
+                    request();
+                }
             }
             const bool act = lane <= last, field = act && k >= 0;
             const uint32_t f1 = wx & 0xFFu, f2 = (wx >> 8) & 0xFFu, hb = STREAM ? 0u : wx >> 16;
             const uint64_t pay = STREAM ? sv << 5 : sv + hb;
             const uint64_t row = base + lane - v - 1 - (int64_t)k;  // the list's first entry
-            uint32_t C, q, R;
-            flat_geometry<FMT>(d, C, q, R);
             uint64_t at = pay;
             uint32_t wdt = 0, val = 0;
             if (FMT == kGT) {
@@ -493,7 +572,8 @@ __global__ __launch_bounds__(kFlatBlock) void flat_write_kernel(const uint64_t* 
                 if (lane == 0) prev = px;
                 px = (uint32_t)__builtin_amdgcn_readlane((int)x, kWave - 1);
                 uint32_t b, i;
-                flat_pos(k < 0 ? 0u : (uint32_t)k, q, R, b, i);
+                if (whole) list.pos((uint32_t)k, b, i);
+                else flat_pos(k < 0 ? 0u : (uint32_t)k, q, R, b, i);
                 const uint32_t diff = x < v ? v - x : x - v, heads = b + (i != 0);
                 if (field) {
                     at = pay + __umul24(heads, f1) + (uint64_t)((uint32_t)k - heads) * f2;
