@@ -113,6 +113,27 @@ static __global__ __launch_bounds__(1024) void firsts_scan_kernel(FirstWord* wor
     segment_firsts(words, n, total, off, R, foff, count, threadIdx.x, 1024);
 }
 
+// The same as marks of the scan (its items are the words).
+struct SegmentMarks {
+    const FirstWord* words;
+    Count cnt;
+    const uint64_t* off;
+    uint64_t* foff;
+    uint64_t* total;
+    uint32_t count;  // R + 1
+    __device__ __forceinline__ uint64_t at(uint32_t r) const {
+        const uint64_t p = off[r];
+        return p < cnt.get() ? p / kWave : ~0ull;
+    }
+    __device__ __forceinline__ void put(uint32_t r, uint64_t before) const {
+        const uint64_t p = off[r];
+        foff[r] = before + (p < cnt.get() ? (uint64_t)__popcll(words[p / kWave].x & ((1ull << (p & 63)) - 1)) : 0);
+    }
+    __device__ __forceinline__ void end(uint64_t t) const {
+        if (total) *total = t;
+    }
+};
+
 static __global__ __launch_bounds__(256) void firsts_segments_kernel(const FirstWord* words, Count cnt,
                                                                      const uint64_t* __restrict__ off, uint32_t R,
                                                                      uint64_t* __restrict__ foff, uint64_t* count) {
@@ -220,7 +241,7 @@ __device__ __forceinline__ uint32_t one_wg_rank(OneWgFirsts& f, uint32_t n, cons
 inline uint64_t firsts_words(uint64_t n_max) { return (n_max + kWave - 1) / kWave + 1; }
 
 // Fills the words' counts for n positions and the ranks of the R segments that start at off[] (off[R]
-// = n): foff[0..R], *count = all firsts.  Scratch: partials[scan_blocks(words)] and total[1].
+// = n; a scan of several workgroups takes fewer than kScanMarksMax of them along): foff[0..R], *count = all firsts.  Scratch: partials[scan_blocks(words)] and total[1].
 inline hipError_t scan_firsts(FirstWord* words, Count n, uint64_t n_max, const uint64_t* off, uint32_t R,
                               uint64_t* foff, uint64_t* count, uint64_t* partials, uint64_t* total, hipStream_t s) {
     const uint64_t nw = firsts_words(n_max);
@@ -230,6 +251,9 @@ inline hipError_t scan_firsts(FirstWord* words, Count n, uint64_t n_max, const u
     }
     Count in_words = n;
     in_words.shift = 6;
+    if (R < kScanMarksMax)
+        return exclusive_scan<2>(FirstsGen{words}, in_words, nw, (uint64_t*)words + 1, partials, total, s,
+                                 SegmentMarks{words, n, off, foff, count, R + 1});
     hipError_t e = exclusive_scan<2>(FirstsGen{words}, in_words, nw, (uint64_t*)words + 1, partials, total, s);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(firsts_segments_kernel, dim3(std::min<uint32_t>(R / 256 + 1, 1024)), dim3(256), 0, s,

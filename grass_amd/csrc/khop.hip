@@ -226,6 +226,22 @@ __device__ __forceinline__ void hop_offsets(const uint64_t* __restrict__ foff, u
     }
 }
 
+// The same as marks of the draws' scan.
+struct OffsetMarks {
+    const uint64_t* foff;
+    uint64_t* eoff_r;
+    uint64_t* hb;
+    uint32_t h;
+    uint64_t* out_off;  // of hop h
+    uint32_t count;     // R + 1
+    __device__ __forceinline__ uint64_t at(uint32_t r) const { return foff[r]; }
+    __device__ __forceinline__ void put(uint32_t r, uint64_t e) const {
+        eoff_r[r] = e;
+        out_off[r] = hb[h] + e;
+    }
+    __device__ __forceinline__ void end(uint64_t total) const { hb[h + 1] = hb[h] + total; }
+};
+
 __global__ void hop_offsets_kernel(const uint64_t* __restrict__ foff, uint32_t R, const uint64_t* eoff,
                                    uint64_t* __restrict__ eoff_r, uint64_t* hb, uint32_t h,
                                    uint64_t* __restrict__ out_off) {
@@ -943,22 +959,27 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     for (uint32_t h = 0; h < H; ++h) {
         const int cur = h & 1, nxt = cur ^ 1;
         const bool small_pass = h ? small_hops : small_seeds;  // the frontier came with its offsets
+        const uint64_t items = h ? Imax : S;
         if (small_pass) {
-        } else if (Imax <= kOneWgItems) {
+        } else if (items <= kOneWgItems) {
             hipLaunchKernelGGL(small_offsets_kernel, dim3(1), dim3(1024), 0, s, (const uint32_t*)d_fc[cur],
                                (const uint64_t*)d_icount[cur], d_eoff, d_etot, (const uint64_t*)d_foff[cur], R, d_eoff_r,
                                d_hb, h, out->offsets_dev);
+        } else if (R < kScanMarksMax) {
+            e = exclusive_scan(DrawsGen{d_fc[cur]}, Count{0, d_icount[cur]}, items, d_eoff, d_part, d_etot, s,
+                               OffsetMarks{d_foff[cur], d_eoff_r, d_hb, h, out->offsets_dev + (uint64_t)h * (R + 1), R + 1});
+            if (e != hipSuccess) return status_of(e);
         } else {
-            e = exclusive_scan(DrawsGen{d_fc[cur]}, Count{0, d_icount[cur]}, Imax, d_eoff, d_part, d_etot, s);
+            e = exclusive_scan(DrawsGen{d_fc[cur]}, Count{0, d_icount[cur]}, items, d_eoff, d_part, d_etot, s);
             if (e != hipSuccess) return status_of(e);
             hipLaunchKernelGGL(hop_offsets_kernel, dim3((R + 256) / 256), dim3(256), 0, s, d_foff[cur], R, d_eoff,
                                d_eoff_r, d_hb, h, out->offsets_dev);
         }
         if (g->fmt == kLE)
-            launch_sample<kLE>(g, lanes[h], fmax[h], layout, h ? Imax : S, s, d_fv[cur], d_fr[cur], d_fd[cur], d_icount[cur],
+            launch_sample<kLE>(g, lanes[h], fmax[h], layout, items, s, d_fv[cur], d_fr[cur], d_fd[cur], d_icount[cur],
                                d_req, h, seed, d_eoff, d_hb, out->src_dev, out->dst_dev, out->capacity, err);
         else
-            launch_sample<kGT>(g, lanes[h], fmax[h], layout, h ? Imax : S, s, d_fv[cur], d_fr[cur], d_fd[cur], d_icount[cur],
+            launch_sample<kGT>(g, lanes[h], fmax[h], layout, items, s, d_fv[cur], d_fr[cur], d_fd[cur], d_icount[cur],
                                d_req, h, seed, d_eoff, d_hb, out->src_dev, out->dst_dev, out->capacity, err);
         if (h + 1 == H) break;
         const EdgeIn in{out->dst_dev, d_hb + h, out->capacity};

@@ -13,6 +13,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "devutil.h"
 
 namespace grass {
@@ -95,12 +97,29 @@ __device__ __forceinline__ uint64_t wave_inclusive_sum_u64(uint64_t x) {
 // those before it, and the tile holding item n - 1 also writes *total; kScanDirect: the same from the
 // values themselves, partials[] unread; kScanThree: partials[] are
 // the tiles' exclusive prefixes and *total was written with them.  Outputs lie STRIDE words apart.
-template <class Gen, ScanMode MODE, int STRIDE>
+//
+// `marks` may name items whose prefixes are wanted by themselves (the ends of requests): once a tile's
+// prefixes are written, its workgroup looks the marks that lie in it up, in place of a launch after
+// the scan.  marks.at(r) is mark r's item, below n or (at the end) at least n; marks.put(r, prefix) takes
+// it; marks.end(total) is called once, by a thread of the last tile.
+struct NoMarks {
+    static constexpr uint32_t count = 0;
+    __device__ __forceinline__ uint64_t at(uint32_t) const { return 0; }
+    __device__ __forceinline__ void put(uint32_t, uint64_t) const {}
+    __device__ __forceinline__ void end(uint64_t) const {}
+};
+// Marks up to which the scan takes them: every tile reads all of them, so a thousand (four loads a thread,
+// cached) cost less than a launch (4.7 us) and many thousands would not.  16 x 8192 seeds, two hops
+// and blocks: 898 -> 887 us; 33 x 700 seeds, three hops: 975 -> 956.
+constexpr uint32_t kScanMarksMax = 1024;
+
+template <class Gen, ScanMode MODE, int STRIDE, class Marks>
 __global__ __launch_bounds__(kScanBlock) void scan_write_kernel(Gen gen, Count cnt,
                                                                 const uint64_t* partials,
                                                                 uint64_t* total,
-                                                                uint64_t* out) {
+                                                                uint64_t* out, Marks marks) {
     constexpr bool FOLD = MODE != kScanThree;
+    constexpr bool MARKS = !std::is_same<Marks, NoMarks>::value;
     __shared__ uint64_t wsum[kScanBlock / kWave];
     __shared__ uint64_t fold_lds[kScanBlock / kWave];
     const uint64_t n = cnt.get();
@@ -109,9 +128,14 @@ __global__ __launch_bounds__(kScanBlock) void scan_write_kernel(Gen gen, Count c
         if (base == 0 && threadIdx.x == 0) {  // empty sequence
             out[0] = 0;
             if (FOLD && total) *total = 0;
+            if (MARKS) marks.end(0);
         }
+        if (MARKS && base == 0)
+            for (uint32_t r = threadIdx.x; r < marks.count; r += kScanBlock) marks.put(r, 0);
         return;
     }
+    uint64_t mark = 0;  // of the first round, asked for early
+    if (MARKS && threadIdx.x < marks.count) mark = marks.at(threadIdx.x);
     uint64_t start;
     if (FOLD) {
         uint64_t p = 0;
@@ -153,8 +177,19 @@ __global__ __launch_bounds__(kScanBlock) void scan_write_kernel(Gen gen, Count c
             for (int w = 0; w < kScanBlock / kWave; ++w) t += wsum[w];
             out[n * STRIDE] = t;
             if (total) *total = t;
+            if (MARKS) marks.end(t);
         } else {
             out[n * STRIDE] = *total;
+            if (MARKS) marks.end(*total);
+        }
+    }
+    if (MARKS) {
+        __syncthreads();  // the prefixes are read across the workgroup
+        const uint64_t next = base + kScanTile;
+        for (uint32_t r = threadIdx.x; r < marks.count; r += kScanBlock) {
+            if (r >= (uint32_t)kScanBlock) mark = marks.at(r);
+            if (mark >= base && mark < next && mark < n) marks.put(r, out[mark * STRIDE]);
+            else if (mark >= n && next >= n) marks.put(r, out[n * STRIDE]);
         }
     }
 }
@@ -163,24 +198,24 @@ inline uint64_t scan_blocks(uint64_t n_max) { return n_max ? (n_max + kScanTile 
 
 // Scratch: partials[scan_blocks(n_max)] and total[1].  DIRECT: the most tiles for one launch; 1 for a generator
 // that gathers (13 k values by two dependent random loads each: 39 us in one launch, 20 in two).
-template <int STRIDE = 1, uint64_t DIRECT = kScanDirectMax, class Gen>
+template <int STRIDE = 1, uint64_t DIRECT = kScanDirectMax, class Gen, class Marks = NoMarks>
 hipError_t exclusive_scan(Gen gen, Count cnt, uint64_t n_max, uint64_t* out, uint64_t* partials,
-                          uint64_t* total, hipStream_t stream) {
+                          uint64_t* total, hipStream_t stream, Marks marks = Marks()) {
     const uint64_t nb = scan_blocks(n_max);
     if (nb <= DIRECT) {
-        hipLaunchKernelGGL((scan_write_kernel<Gen, kScanDirect, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
-                           gen, cnt, (const uint64_t*)nullptr, total, out);
+        hipLaunchKernelGGL((scan_write_kernel<Gen, kScanDirect, STRIDE, Marks>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
+                           gen, cnt, (const uint64_t*)nullptr, total, out, marks);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(scan_reduce_kernel<Gen>, dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
                        gen, cnt, partials);
     if (nb <= kScanFoldMax) {
-        hipLaunchKernelGGL((scan_write_kernel<Gen, kScanFold, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
-                           gen, cnt, (const uint64_t*)partials, total, out);
+        hipLaunchKernelGGL((scan_write_kernel<Gen, kScanFold, STRIDE, Marks>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
+                           gen, cnt, (const uint64_t*)partials, total, out, marks);
     } else {
         hipLaunchKernelGGL(scan_partials_kernel<uint64_t>, dim3(1), dim3(1024), 0, stream, partials, nb, total);
-        hipLaunchKernelGGL((scan_write_kernel<Gen, kScanThree, STRIDE>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
-                           gen, cnt, (const uint64_t*)partials, total, out);
+        hipLaunchKernelGGL((scan_write_kernel<Gen, kScanThree, STRIDE, Marks>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream,
+                           gen, cnt, (const uint64_t*)partials, total, out, marks);
     }
     return hipGetLastError();
 }
@@ -197,8 +232,8 @@ hipError_t scan_prefixes(Gen gen, uint64_t n, uint64_t* prefixes, hipStream_t st
 template <class Gen>
 hipError_t scan_from_prefixes(Gen gen, uint64_t n, const uint64_t* prefixes, uint64_t* out, hipStream_t stream) {
     const uint64_t nb = scan_blocks(n);
-    hipLaunchKernelGGL((scan_write_kernel<Gen, kScanThree, 1>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream, gen,
-                       Count{n, nullptr}, prefixes, const_cast<uint64_t*>(prefixes) + nb, out);
+    hipLaunchKernelGGL((scan_write_kernel<Gen, kScanThree, 1, NoMarks>), dim3((unsigned)nb), dim3(kScanBlock), 0, stream, gen,
+                       Count{n, nullptr}, prefixes, const_cast<uint64_t*>(prefixes) + nb, out, NoMarks());
     return hipGetLastError();
 }
 
