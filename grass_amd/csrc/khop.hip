@@ -615,7 +615,8 @@ __global__ __launch_bounds__(kKhBlock) void sample_packed_kernel(DevGraph g, con
 #undef GRASS_SAMPLE_ARGS
 
 int khop_bound(const grass_graph* g, const grass_khop_request* reqs, uint32_t count,
-               uint64_t* edges, uint64_t* items, uint64_t* dedup, uint32_t* max_hops) {
+               uint64_t* edges, uint64_t* items, uint64_t* dedup, uint32_t* max_hops, uint64_t* hop_items,
+               uint64_t* hop_edges) {
     uint64_t E = 0, I = 0, D = 0;
     uint32_t H = 0;
     std::vector<uint64_t> Ih(GRASS_KHOP_MAX_HOPS, 0), Eh(GRASS_KHOP_MAX_HOPS, 0);
@@ -645,6 +646,8 @@ int khop_bound(const grass_graph* g, const grass_khop_request* reqs, uint32_t co
         E += Eh[h];
         I = std::max(I, Ih[h]);
         if (h + 1 < H) D = std::max(D, Eh[h]);
+        if (hop_items) hop_items[h] = Ih[h];
+        if (hop_edges) hop_edges[h] = Eh[h];
     }
     I = std::max(I, S);
     if (edges) *edges = E;
@@ -704,10 +707,14 @@ static uint32_t bit_width(uint64_t x) {
     return k;
 }
 
-// Slots of the packed dedup table for `entries` positions (load <= 2/3).
+// Slots of the packed dedup table for `entries` positions: load <= 2/3, and <= 1/4 as long as that takes
+// no more than kSparseSlots (16 MB), since a pass of few entries lasts as long as its longest chain of
+// probes: 131 k entries in 2^18 slots 24 us, in 2^19 14.5, in 2^20 13; 231 k in 2^19 30, in 2^20 17.  (At
+// 1/8 the clear costs a small batch that runs beside walks more than the probes: 219 us, 225.)
+constexpr uint64_t kSparseSlots = 1u << 21;
 static uint64_t pack_slots(uint64_t entries) {
     uint64_t slots = 1024;
-    while (slots < entries + entries / 2 + 2) slots <<= 1;
+    while (slots < entries + entries / 2 + 2 || (slots < kSparseSlots && slots < 4 * entries)) slots <<= 1;
     return slots;
 }
 
@@ -726,12 +733,20 @@ static bool kh_packed_table(const grass_graph* g, uint32_t R, uint64_t S, uint64
 constexpr uint64_t kTablesAtOnce = 64ull << 20;
 struct Tables {
     bool at_once;
-    uint64_t slots;  // of all tables, or of the shared one
+    uint64_t slots;                         // of all tables, or of the shared one
+    uint64_t first[GRASS_KHOP_MAX_HOPS];  // where a pass's table begins
 };
-static Tables plan_tables(uint64_t S, uint64_t Dmax, uint32_t H) {
-    const uint64_t all = pack_slots(S) + (H - 1) * pack_slots(Dmax);
-    if (all * 8 <= kTablesAtOnce) return Tables{true, all};
-    return Tables{false, pack_slots(std::max(S, Dmax))};
+// n[pass]: the most entries of a pass (0: the seeds, h + 1: hop h's destinations).
+static Tables plan_tables(const uint64_t* n, uint32_t H) {
+    Tables t{true, 0, {}};
+    uint64_t largest = 0;
+    for (uint32_t p = 0; p < H; ++p) {
+        t.first[p] = t.slots;
+        t.slots += pack_slots(n[p]);
+        largest = std::max(largest, pack_slots(n[p]));
+    }
+    if (t.slots * 8 <= kTablesAtOnce) return t;
+    return Tables{false, largest, {}};
 }
 static uint64_t kh_words(uint64_t S, uint64_t Dmax, uint32_t H) { return firsts_words(S) + (H - 1) * firsts_words(Dmax); }
 
@@ -807,7 +822,11 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     if (R > (1u << 17)) return GRASS_EINVAL;
     uint64_t Ebound, Ibound, Dbound;
     uint32_t H;
-    int rc = khop_bound(g, reqs, R, &Ebound, &Ibound, &Dbound, &H);
+    // The most items of a hop's frontier, and the most entries of a pass.  Each hop's own, for its table,
+    // words and scans: three hops [10, 10, 5] of 23 k seeds deduplicate 0.2 M, then 2.3 M destinations
+    // (929 -> 910 us with blocks; by the largest hop's, no table fitted beside another).
+    uint64_t hop_items[GRASS_KHOP_MAX_HOPS], entries[GRASS_KHOP_MAX_HOPS + 1];
+    int rc = khop_bound(g, reqs, R, &Ebound, &Ibound, &Dbound, &H, hop_items, entries + 1);
     if (rc) return rc;
     out->max_hops = H;
     if (H == 0) return GRASS_OK;
@@ -829,7 +848,7 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
         hreq[r] = q;
         sbeg[r + 1] = sbeg[r] + reqs[r].num_seeds;
     }
-    const uint64_t S = sbeg[R];
+    const uint64_t S = entries[0] = sbeg[R];
     const uint64_t Imax = std::max<uint64_t>(Ibound, 1), Dmax = std::max<uint64_t>(Dbound, 1);
     const uint64_t nbI = scan_blocks(Imax), nbD = scan_blocks(firsts_words(std::max(S, Dmax)));
     hipError_t e = ws.scratch.reserve(kh_scratch_need(R, S, Imax, Dmax, H));
@@ -844,7 +863,11 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     uint32_t* d_fd[2] = {cv.take<uint32_t>(Imax), cv.take<uint32_t>(Imax)};  // frontier degrees
     uint32_t* d_fc[2] = {cv.take<uint32_t>(Imax), cv.take<uint32_t>(Imax)};  // and draws
     uint64_t* d_eoff = cv.take<uint64_t>(Imax + 1);
-    const uint64_t nwords = kh_words(S, Dmax, H);
+    uint64_t nwords = 0, words_at[GRASS_KHOP_MAX_HOPS];  // of each pass; at most kh_words(S, Dmax, H) in all
+    for (uint32_t p = 0; p < H; ++p) {
+        words_at[p] = nwords;
+        nwords += firsts_words(entries[p]);
+    }
     FirstWord* d_words = cv.take<FirstWord>(nwords);
     uint64_t* d_part = cv.take<uint64_t>(std::max(nbI, nbD));
     uint64_t* d_sc = cv.take<uint64_t>(64);  // [0..1] item counts, [2] edges total, [3] firsts total,
@@ -859,7 +882,7 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     const uint32_t vb = std::max<uint32_t>(bit_width(g->n ? g->n - 1 : 0), 1u);
     const uint32_t pb = std::max<uint32_t>(bit_width(std::max(S, Dmax)), 1u);  // positions < 2^pb - 1
     const bool packed = kh_packed_table(g, R, S, Dmax);
-    const Tables tables = plan_tables(S, Dmax, H);
+    const Tables tables = plan_tables(entries, H);
     HashTab ht{};
     if (packed) {
         if (ws.ht.reserve(tables.slots * 8) != hipSuccess) return GRASS_ENOMEM;
@@ -871,16 +894,14 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     uint32_t* err = err_word(g, ws);
     // Inserts pass `pass`'s entries (0: the seeds, h + 1: hop h's destinations): packed table of the
     // pass or the shared one, or the next generation of the 16-byte one.
-    auto words_of = [&](uint32_t pass) { return pass ? d_words + firsts_words(S) + (pass - 1) * firsts_words(Dmax) : d_words; };
+    auto words_of = [&](uint32_t pass) { return d_words + words_at[pass]; };
     auto insert = [&](auto in, Count E, const uint64_t* off_r, uint32_t pass) {
-        const uint64_t entries = pass ? Dmax : S;
-        const unsigned grid = (unsigned)std::min<uint64_t>((entries + kKhBlock - 1) / kKhBlock, 2048);
+        const uint64_t most = std::max<uint64_t>(entries[pass], 1);
+        const unsigned grid = (unsigned)std::min<uint64_t>((most + kKhBlock - 1) / kKhBlock, 2048);
         if (packed) {
-            const uint64_t slots = pack_slots(entries);
-            unsigned long long* p = (unsigned long long*)ws.ht.ptr;
-            if (tables.at_once) {
-                if (pass) p += pack_slots(S) + (pass - 1) * slots;
-            } else {
+            const uint64_t slots = pack_slots(entries[pass]);
+            unsigned long long* p = (unsigned long long*)ws.ht.ptr + tables.first[pass];
+            if (!tables.at_once) {
                 hipLaunchKernelGGL(fill_kernel<unsigned long long>, dim3((unsigned)std::min<uint64_t>((slots + 255) / 256, 4096)),
                                    dim3(256), 0, s, p, slots, ~0ull);
             }
@@ -895,10 +916,10 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     };
     // The pass's first appearances, numbered and written as the frontier of hop h into buffer k.
     auto next_frontier = [&](auto in, Count E, const uint64_t* off_r, uint32_t pass, uint32_t h, int k) -> hipError_t {
-        const uint64_t entries = pass ? Dmax : S;
-        hipError_t e = scan_firsts(words_of(pass), E, entries, off_r, R, d_foff[k], d_icount[k], d_part, d_ftot, s);
+        const uint64_t most = entries[pass];
+        hipError_t e = scan_firsts(words_of(pass), E, most, off_r, R, d_foff[k], d_icount[k], d_part, d_ftot, s);
         if (e != hipSuccess) return e;
-        const unsigned grid = (unsigned)std::min<uint64_t>(std::max<uint64_t>((entries + kKhBlock - 1) / kKhBlock, 1), 4096);
+        const unsigned grid = (unsigned)std::min<uint64_t>(std::max<uint64_t>((most + kKhBlock - 1) / kKhBlock, 1), 4096);
         hipLaunchKernelGGL((compact_kernel<decltype(in)>), dim3(grid), dim3(kKhBlock), 0, s, in, E, off_r, R,
                            (const FirstWord*)words_of(pass), (const uint32_t*)g->d_deg, (const KhReq*)d_req, h, d_fv[k],
                            d_fr[k], d_fd[k], d_fc[k]);
@@ -967,7 +988,7 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     for (uint32_t h = 0; h < H; ++h) {
         const int cur = h & 1, nxt = cur ^ 1;
         const bool small_pass = h ? small_hops : small_seeds;  // the frontier came with its offsets
-        const uint64_t items = h ? Imax : S;
+        const uint64_t items = std::max<uint64_t>(hop_items[h], 1);
         if (small_pass) {
         } else if (items <= kOneWgItems) {
             hipLaunchKernelGGL(small_offsets_kernel, dim3(1), dim3(1024), 0, s, (const uint32_t*)d_fc[cur],

@@ -311,7 +311,8 @@ int random_walk_batch_noalloc(grass_graph* g, const grass_rw_request* reqs, uint
 
 // khop.hip
 int khop_bound(const grass_graph* g, const grass_khop_request* reqs, uint32_t count,
-               uint64_t* edges, uint64_t* items, uint64_t* dedup, uint32_t* max_hops);
+               uint64_t* edges, uint64_t* items, uint64_t* dedup, uint32_t* max_hops,
+               uint64_t* hop_items = nullptr, uint64_t* hop_edges = nullptr);
 int khop_batch(grass_graph* g, const grass_khop_request* reqs, uint32_t count, uint64_t seed,
                grass_khop_output* out, hipStream_t stream);
 // As rw_batch_enqueue; the batch's edge total reaches *ws.result_slot() (pinned host memory)
