@@ -27,6 +27,14 @@ namespace {
 
 using Clock = std::chrono::steady_clock;
 
+// A failed allocation reaches its caller by the return value alone: HIP keeps it as the thread's last
+// error through later successful calls, where the launch checks of a caller that goes on without the
+// memory (or got it at the second attempt) would find it.
+hipError_t quiet(hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 constexpr size_t kDeviceMax = 16ull << 30;
 constexpr size_t kPinnedMax = 256ull << 20;
 constexpr int kKeepSeconds = 10;
@@ -65,11 +73,10 @@ class BlockCache {
         if (*p) return hipSuccess;
         const size_t unit = need >= (8u << 20) ? (2u << 20) : 4096;
         *got = (need + unit - 1) / unit * unit;
-        hipError_t e = allocate(p, *got);
+        hipError_t e = quiet(allocate(p, *got));
         if (e != hipSuccess) {
-            (void)hipGetLastError();
             clear();
-            e = allocate(p, *got);
+            e = quiet(allocate(p, *got));
         }
         return e;
     }
@@ -182,13 +189,12 @@ void PinnedWork::reset() {
 }
 
 hipError_t device_malloc(void** p, size_t bytes) {
-    hipError_t e = hipMalloc(p, bytes);
+    hipError_t e = quiet(hipMalloc(p, bytes));
     if (e == hipSuccess) return e;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return e;
-    (void)hipGetLastError();
     if (BlockCache* c = device_cache(dev)) c->clear();
-    return hipMalloc(p, bytes);
+    return quiet(hipMalloc(p, bytes));
 }
 
 }  // namespace grass

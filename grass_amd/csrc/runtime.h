@@ -12,7 +12,8 @@
 
 namespace grass {
 
-// hipMalloc that frees the idle working memory kept between calls (pool.cpp) before it fails.
+// hipMalloc that frees the idle working memory kept between calls (pool.cpp) before it fails.  A
+// failure is in the return value only, not in the thread's last error.
 hipError_t device_malloc(void** p, size_t bytes);
 
 // Device scratch that grows on demand and is reused across calls (no per-call hipMalloc in
