@@ -761,7 +761,9 @@ static size_t kh_scratch_need(uint64_t R, uint64_t S, uint64_t Imax, uint64_t Dm
 static hipError_t ensure_table(Workspace& ws, uint64_t entries, HashTab& t) {
     uint64_t slots = 1024;
     while (slots < 2 * entries + 2) slots <<= 1;
-    if (slots > ws.ht_slots) {
+    // (the memory may have been given back since, or hold less: other tables use it too)
+    if (slots > ws.ht_slots || ws.ht_slots * 16 > ws.ht.bytes) {
+        ws.ht_slots = 0;
         hipError_t e = ws.ht.reserve(slots * 16);
         if (e != hipSuccess) return e;
         ws.ht_slots = slots;

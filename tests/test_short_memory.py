@@ -32,5 +32,45 @@ def test_blocks_on_memory_others_left(fake, ga):
     assert "rel_part_dedup_kernel" in names and "rel_insert" not in names
 
 
+def _table_fits(fake, ga, g):
+    """A batch on the 16-byte table clears no more than the table's memory."""
+    os.environ["GRASS_KHOP_SLOT"] = "16"
+    fk.launches(fake)
+    rc = fk.khop(ga, g, [5000], (10, 10))
+    assert rc == ga.OK, ga.strerror(rc)
+    clears = [a for k, _, a in fk.launches(fake) if "ht_clear_kernel" in k]
+    assert clears  # (new memory holds anything)
+    for slot, mask, _ in clears:
+        assert fake.fake_room(slot) >= (mask + 1) * 16
+    del os.environ["GRASS_KHOP_SLOT"]
+
+
+@fk.on_fake
+def test_khop_table_after_failed_blocks(fake, ga):
+    """The 16-byte table's size is not remembered past its memory: blocks that failed gave that back, and
+    smaller ones took less in its place."""
+    g = fk.graph(ga, 1 << 12)
+    os.environ["GRASS_KHOP_SLOT"] = "16"
+    assert fk.khop(ga, g, [500_000], (10, 10)) == ga.OK
+    del os.environ["GRASS_KHOP_SLOT"]
+    fake.fake_limit(P)
+    assert fk.blocks(ga, g, [4 * P], 50) == ga.ENOMEM
+    fk.unlimited(fake)
+    assert fk.blocks(ga, g, [20_000], 50) == ga.OK
+    _table_fits(fake, ga, g)
+
+
+@fk.on_fake
+def test_khop_table_after_a_failed_one(fake, ga):
+    """Nor past a larger table that could not be had (but the batch's other memory, 215 MB, could)."""
+    g = fk.graph(ga, 1 << 12)
+    os.environ["GRASS_KHOP_SLOT"] = "16"
+    assert fk.khop(ga, g, [500_000], (10, 10)) == ga.OK
+    fake.fake_limit(250 << 20)
+    assert fk.khop(ga, g, [4 * P], (10, 10)) == ga.ENOMEM
+    fk.unlimited(fake)
+    _table_fits(fake, ga, g)
+
+
 if __name__ == "__main__":
     fk.main(globals())
