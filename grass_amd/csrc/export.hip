@@ -630,9 +630,9 @@ __device__ __forceinline__ uint32_t part_insert(unsigned long long* tab, unsigne
 }
 
 // One workgroup per bucket, whose positions (but for repeats past kPartHeld per thread) it holds in
-// registers: loaded together, and not looked up again.  *bad |= 2: more distinct keys than slots.
+// registers: loaded together, and not looked up again.  *invalid |= 2: more distinct keys than slots.
 constexpr int kPartHeld = 8;
-__global__ __launch_bounds__(kPartBlock) void rel_part_dedup_kernel(RelSeq q, RelParts t, uint32_t* bad) {
+__global__ __launch_bounds__(kPartBlock) void rel_part_dedup_kernel(RelSeq q, RelParts t, uint32_t* invalid) {
     __shared__ unsigned long long tab[kPartSlots];
     const uint32_t k = blockIdx.x;
     if (k >= t.bkt0[q.R]) return;
@@ -651,7 +651,7 @@ __global__ __launch_bounds__(kPartBlock) void rel_part_dedup_kernel(RelSeq q, Re
         s[j] &= kPartSlots - 1;
     }
     for (uint32_t i = lo + kPartHeld * kPartBlock; i < hi; i += kPartBlock) full = part_insert(tab, t.rec[i]) == kPartSlots || full;
-    if (full) atomicOr(bad, 2u);
+    if (full) atomicOr(invalid, 2u);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kPartHeld; ++j) {
@@ -688,7 +688,7 @@ hipError_t rel_build_parts(const RelParts& t, uint32_t maxb, const RelSeq& q, ui
     hipLaunchKernelGGL(rel_part_kernel<false>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad);
     hipLaunchKernelGGL(scan_partials_kernel<uint32_t>, dim3(1), dim3(1024), 0, s, t.bend, (uint64_t)maxb, (uint32_t*)nullptr);
     hipLaunchKernelGGL(rel_part_kernel<true>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad);
-    hipLaunchKernelGGL(rel_part_dedup_kernel, dim3(maxb), dim3(kPartBlock), 0, s, q, t, d_bad);
+    hipLaunchKernelGGL(rel_part_dedup_kernel, dim3(maxb), dim3(kPartBlock), 0, s, q, t, d_bad + 1);
     const unsigned gP = (unsigned)std::min<uint64_t>((P + kExBlock - 1) / kExBlock + 1, kExGrid);
     hipLaunchKernelGGL(rel_part_words_kernel, dim3(gP), dim3(kExBlock), 0, s, (const uint32_t*)t.fpos, P, d_words);
     return rel_number(t, q, P, d_words, d_part, d_sc, d_bad, out, s);
@@ -864,12 +864,12 @@ int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, cons
         if (e == hipSuccess) e = hipMemcpyAsync(hres, d_sc + 1, 16, hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (e != hipSuccess) return status_of(e);
-        if (!(hres[1] & 2)) {
+        if (!(hres[1] >> 32 & 2)) {
             if (hres[1] != 0) return GRASS_EINVAL;
             out->nodes = hres[0];
             return out->nodes > out->node_capacity ? GRASS_ECAPACITY : GRASS_OK;
         }
-        // a bucket's keys did not fit its table: the other way
+        // a bucket's keys did not fit its table (nothing was emitted): the other way
         if (ws.ht.reserve(slots * (wide ? 16 : 8)) != hipSuccess) return GRASS_ENOMEM;
     }
     if (wide) {

@@ -1,0 +1,44 @@
+"""Blocks that go by partition and cannot stay there: what the failed attempt leaves behind."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from test_gpu_block_parts import N, _hash, graph  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def _build(g, seeds):
+    """Blocks of one request of one hop, one neighbour each, into nodes filled with ~0: (status, nodes, count)."""
+    import torch
+
+    import grass_amd
+    dev = "cuda:0"
+    arr, keep = g.khop_request_array([seeds], [[1]], None)
+    src, dst = (torch.empty(len(seeds), dtype=torch.int32, device=dev) for _ in range(2))
+    off = torch.zeros(2, dtype=torch.int64, device=dev)
+    out = grass_amd.KhopOutput(src.data_ptr(), dst.data_ptr(), len(seeds), off.data_ptr(), 0, 0)
+    assert grass_amd.lib().grass_khop_batch(g._h, arr, 1, 3, C.byref(out), None) == 0
+    P = len(seeds) + out.total
+    assert P >= 1 << 20
+    nodes = torch.full((P,), -1, dtype=torch.int32, device=dev)
+    node_off = torch.zeros(2, dtype=torch.int64, device=dev)
+    lsrc, ldst = (torch.empty(len(seeds), dtype=torch.int32, device=dev) for _ in range(2))
+    b = grass_amd.KhopBlocks(nodes.data_ptr(), P, node_off.data_ptr(), lsrc.data_ptr(), ldst.data_ptr(), 0)
+    rc = grass_amd.lib().grass_khop_blocks_build(g._h, arr, 1, C.byref(out), C.byref(b), None)
+    seq = np.concatenate([seeds, dst[:out.total].cpu().numpy().view(np.uint32)])
+    _, first = np.unique(seq, return_index=True)
+    return rc, nodes.cpu().numpy().view(np.uint32), b.nodes, seq[np.sort(first)]
+
+
+def test_nodes_past_the_count(graph):  # noqa: F811
+    """More distinct vertices in a bucket than its table takes: nothing is written past the nodes."""
+    v = np.arange(N, dtype=np.uint32)
+    few = v[_hash(v) * 422 >> 32 == 7]
+    seeds = few[np.random.default_rng(3).integers(0, len(few), size=422 * 2560 - len(few))]
+    seeds[:len(few)] = few
+    rc, nodes, count, expected = _build(graph, seeds)
+    assert rc == 0 and count == len(expected)
+    np.testing.assert_array_equal(nodes[:count], expected)
+    assert (nodes[count:] == 0xFFFFFFFF).all()
