@@ -545,15 +545,25 @@ __global__ __launch_bounds__(1024) void rel_part_prepare_kernel(RelParts t, uint
 constexpr uint64_t kPartMin = 1ull << 20;
 constexpr int kPartBlock = 512;
 constexpr int kPartPer = kPartTile / kPartBlock;
+constexpr int kPartHeld = 8;  // a bucket's positions that a thread of its workgroup holds
+constexpr uint32_t kPartHeldAll = kPartHeld * kPartBlock;
+// The positions of a vertex that many repeat are one workgroup's work, 1.4 ns each past kPartHeldAll (2.4
+// before they went by kPartHeld loads), where the table's inserts of a repeat are a read.  A bucket of more
+// than kPartMost, unless others are as large, therefore sends the batch back to the table; the counts tell, and
+// the batch has lost 0.1 ms.  A cycle of 2.4 M vertices, us by table / by partition without this / with it: one
+// request of 12.3 M positions, one vertex 1 % of the seeds 661 / 853 / 767, 3 % 739 / 1326 / 870, 10 % 929 /
+// 2910 / 1015, 50 % 2063 / 12180 / 2023; four requests of 0.7 M, 50 % each, 961 / 610 / 475.
+constexpr uint32_t kPartMost = 1u << 17;
 
 // One workgroup per tile: counts its buckets' positions (SCATTER: takes room for them in each bucket,
 // and writes them there).
 template <bool SCATTER>
-__global__ __launch_bounds__(kPartBlock) void rel_part_kernel(RelSeq q, RelParts t, uint32_t* err) {
+__global__ __launch_bounds__(kPartBlock) void rel_part_kernel(RelSeq q, RelParts t, uint32_t* err,
+                                                              const uint32_t* __restrict__ invalid) {
     __shared__ uint32_t hist[kPartBuckets];
     __shared__ uint64_t beg[GRASS_KHOP_MAX_HOPS + 1];
     __shared__ const uint32_t* arr[GRASS_KHOP_MAX_HOPS + 1];
-    if (blockIdx.x >= t.tile0[q.R]) return;
+    if (blockIdx.x >= t.tile0[q.R] || (SCATTER && *invalid)) return;
     uint32_t r = 0;
     for (uint32_t hi = q.R - 1; r < hi;) {  // the last request whose first tile is not after this one
         const uint32_t mid = r + (hi - r + 1) / 2;
@@ -629,41 +639,85 @@ __device__ __forceinline__ uint32_t part_insert(unsigned long long* tab, unsigne
     return kPartSlots;
 }
 
-// One workgroup per bucket, whose positions (but for repeats past kPartHeld per thread) it holds in
-// registers: loaded together, and not looked up again.  *invalid |= 2: more distinct keys than slots.
-constexpr int kPartHeld = 8;
+// The buckets' counts become their starts (one workgroup).  *invalid |= 2: few buckets hold so many
+// positions that the workgroups of these would be the time (kPartMost).
+__global__ __launch_bounds__(1024) void rel_part_starts_kernel(uint32_t* bend, uint32_t nb, uint32_t* invalid) {
+    __shared__ uint32_t lds[1024 / kWave];
+    __shared__ uint64_t lds64[1024 / kWave];
+    const uint32_t per = (nb + 1023) / 1024, lo = threadIdx.x * per, hi = min(lo + per, nb);
+    uint32_t s = 0, largest = 0, total;
+    uint64_t past = 0;  // positions that are not held
+    for (uint32_t i = lo; i < hi; ++i) {
+        const uint32_t c = bend[i];
+        s += c;
+        largest = max(largest, c);
+        past += c > kPartHeldAll ? c - kPartHeldAll : 0u;
+    }
+    largest = block_max<uint32_t, 1024>(largest, lds);
+    past = block_sum<uint64_t, 1024>(past, lds64);
+    if (threadIdx.x == 0 && largest > kPartMost && 3ull * largest > past) atomicOr(invalid, 2u);
+    uint32_t pre = block_exclusive_sum<uint32_t, 1024>(s, total, lds);
+    for (uint32_t i = lo; i < hi; ++i) {
+        const uint32_t c = bend[i];
+        bend[i] = pre;
+        pre += c;
+    }
+}
+
+// One workgroup per bucket, whose positions (but for those past kPartHeld per thread, mostly repeats) it
+// holds in registers: loaded together, and not looked up again.  The others go through twice, kPartHeld
+// loads at a time.  *invalid |= 2: more distinct keys than slots.
 __global__ __launch_bounds__(kPartBlock) void rel_part_dedup_kernel(RelSeq q, RelParts t, uint32_t* invalid) {
     __shared__ unsigned long long tab[kPartSlots];
+    __shared__ uint32_t stop;  // (other workgroups may be setting it)
     const uint32_t k = blockIdx.x;
     if (k >= t.bkt0[q.R]) return;
+    if (threadIdx.x == 0) stop = *(volatile uint32_t*)invalid;
     const uint32_t lo = (k ? t.bend[k - 1] : 0u) + threadIdx.x, hi = t.bend[k];
     unsigned long long w[kPartHeld];
     uint32_t s[kPartHeld];
+    auto load = [&](uint32_t at) {
 #pragma unroll
-    for (int j = 0; j < kPartHeld; ++j) w[j] = lo + j * kPartBlock < hi ? t.rec[lo + j * kPartBlock] : ~0ull;
+        for (int j = 0; j < kPartHeld; ++j) w[j] = at + j * kPartBlock < hi ? t.rec[at + j * kPartBlock] : ~0ull;
+    };
+    auto insert = [&]() {
+        bool full = false;
+#pragma unroll
+        for (int j = 0; j < kPartHeld; ++j) {
+            s[j] = w[j] != ~0ull ? part_insert(tab, w[j]) : 0u;
+            full = full || s[j] == kPartSlots;
+            s[j] &= kPartSlots - 1;
+        }
+        return full;
+    };
+    auto put = [&]() {
+#pragma unroll
+        for (int j = 0; j < kPartHeld; ++j) {
+            if (w[j] == ~0ull) continue;
+            const unsigned long long cur = tab[s[j]];
+            if (cur < w[j]) t.fpos[(uint32_t)w[j]] = (uint32_t)cur;
+        }
+    };
+    load(lo);
     for (uint32_t i = threadIdx.x; i < kPartSlots; i += kPartBlock) tab[i] = ~0ull;
     __syncthreads();
+    if (stop) return;
     bool full = false;
-#pragma unroll
-    for (int j = 0; j < kPartHeld; ++j) {
-        s[j] = w[j] != ~0ull ? part_insert(tab, w[j]) : 0u;
-        full = full || s[j] == kPartSlots;
-        s[j] &= kPartSlots - 1;
+    if (lo + kPartHeldAll < hi) {
+        for (uint32_t i = lo + kPartHeldAll; i < hi; i += kPartHeldAll) {
+            load(i);
+            full = insert() || full;
+        }
+        load(lo);
     }
-    for (uint32_t i = lo + kPartHeld * kPartBlock; i < hi; i += kPartBlock) full = part_insert(tab, t.rec[i]) == kPartSlots || full;
+    full = insert() || full;
     if (full) atomicOr(invalid, 2u);
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kPartHeld; ++j) {
-        if (w[j] == ~0ull) continue;
-        const unsigned long long cur = tab[s[j]];
-        if (cur < w[j]) t.fpos[(uint32_t)w[j]] = (uint32_t)cur;
-    }
-    for (uint32_t i = lo + kPartHeld * kPartBlock; i < hi; i += kPartBlock) {
-        const unsigned long long x = t.rec[i];
-        const uint32_t sx = part_insert(tab, x);  // (already there)
-        const unsigned long long cur = tab[sx & (kPartSlots - 1)];
-        if (cur < x) t.fpos[(uint32_t)x] = (uint32_t)cur;
+    put();
+    for (uint32_t i = lo + kPartHeldAll; i < hi; i += kPartHeldAll) {
+        load(i);
+        insert();  // (already there)
+        put();
     }
     unsigned long long* out = t.tab + (uint64_t)k * kPartSlots;
     for (uint32_t i = threadIdx.x; i < kPartSlots; i += kPartBlock) out[i] = tab[i];
@@ -683,12 +737,13 @@ hipError_t rel_build_parts(const RelParts& t, uint32_t maxb, const RelSeq& q, ui
                            uint64_t* d_part, uint64_t* d_sc, uint32_t* d_bad, const grass_khop_output* b,
                            grass_khop_blocks* out, hipStream_t s) {
     const unsigned tiles = (unsigned)(P / kPartTile + q.R);
+    uint32_t* d_invalid = d_bad + 1;
     hipLaunchKernelGGL(rel_part_prepare_kernel, dim3(1 + (unsigned)std::min<uint64_t>(P / 16384 + 1, 512)), dim3(1024), 0, s, t,
-                       maxb, q.off, q.req, q.R, q.H, b->total, P, const_cast<uint64_t*>(q.Q), d_bad, d_bad + 1);
-    hipLaunchKernelGGL(rel_part_kernel<false>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad);
-    hipLaunchKernelGGL(scan_partials_kernel<uint32_t>, dim3(1), dim3(1024), 0, s, t.bend, (uint64_t)maxb, (uint32_t*)nullptr);
-    hipLaunchKernelGGL(rel_part_kernel<true>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad);
-    hipLaunchKernelGGL(rel_part_dedup_kernel, dim3(maxb), dim3(kPartBlock), 0, s, q, t, d_bad + 1);
+                       maxb, q.off, q.req, q.R, q.H, b->total, P, const_cast<uint64_t*>(q.Q), d_bad, d_invalid);
+    hipLaunchKernelGGL(rel_part_kernel<false>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad, (const uint32_t*)d_invalid);
+    hipLaunchKernelGGL(rel_part_starts_kernel, dim3(1), dim3(1024), 0, s, t.bend, maxb, d_invalid);
+    hipLaunchKernelGGL(rel_part_kernel<true>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad, (const uint32_t*)d_invalid);
+    hipLaunchKernelGGL(rel_part_dedup_kernel, dim3(maxb), dim3(kPartBlock), 0, s, q, t, d_invalid);
     const unsigned gP = (unsigned)std::min<uint64_t>((P + kExBlock - 1) / kExBlock + 1, kExGrid);
     hipLaunchKernelGGL(rel_part_words_kernel, dim3(gP), dim3(kExBlock), 0, s, (const uint32_t*)t.fpos, P, d_words);
     return rel_number(t, q, P, d_words, d_part, d_sc, d_bad, out, s);
@@ -869,7 +924,7 @@ int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, cons
             out->nodes = hres[0];
             return out->nodes > out->node_capacity ? GRASS_ECAPACITY : GRASS_OK;
         }
-        // a bucket's keys did not fit its table (nothing was emitted): the other way
+        // a bucket's keys did not fit its table: the other way
         if (ws.ht.reserve(slots * (wide ? 16 : 8)) != hipSuccess) return GRASS_ENOMEM;
     }
     if (wide) {
