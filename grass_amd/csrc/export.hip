@@ -554,6 +554,10 @@ constexpr uint32_t kPartHeldAll = kPartHeld * kPartBlock;
 // request of 12.3 M positions, one vertex 1 % of the seeds 661 / 853 / 767, 3 % 739 / 1326 / 870, 10 % 929 /
 // 2910 / 1015, 50 % 2063 / 12180 / 2023; four requests of 0.7 M, 50 % each, 961 / 610 / 475.
 constexpr uint32_t kPartMost = 1u << 17;
+// Distinct vertices a request may have: the buckets' tables three quarters full.  By table / by partition,
+// us, one request, seven eighths of its positions distinct: 23 M positions 1489 / 1150, 25 M 1613 / 1306, 28 M 1793 /
+// 1604, 30 M 1909 / 2028; more than the tables hold, and most probes see every slot: 60 M 4255 / 157313.
+constexpr uint64_t kPartDistinct = (uint64_t)kPartBuckets * (kPartSlots / 4 * 3);
 
 // One workgroup per tile: counts its buckets' positions (SCATTER: takes room for them in each bucket,
 // and writes them there).
@@ -820,6 +824,20 @@ __global__ __launch_bounds__(kOneWgThreads) void rel_small_kernel(RelSeq q, cons
     }
 }
 
+// Whether a request may have more than kPartDistinct distinct vertices.
+bool too_many_distinct(const grass_graph* g, const grass_khop_request* reqs, uint32_t R, uint64_t P) {
+    if (std::min<uint64_t>(P, g->n) <= kPartDistinct) return false;
+    for (uint32_t r = 0; r < R; ++r) {
+        uint64_t front = std::min<uint64_t>(reqs[r].num_seeds, g->n), all = front;
+        for (uint32_t h = 0; h < reqs[r].hops; ++h) {
+            front = std::min<uint64_t>(front * std::min<uint64_t>(reqs[r].fanout[h], g->max_degree), g->n);
+            all += front;
+        }
+        if (std::min<uint64_t>(all, P) > kPartDistinct) return true;
+    }
+    return false;
+}
+
 int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, const grass_khop_output* b,
                 grass_khop_blocks* out, hipStream_t s) {
     std::lock_guard<std::mutex> lock(g->mu);
@@ -866,7 +884,8 @@ int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, cons
         t.tab = c.take<unsigned long long>((uint64_t)maxb * kPartSlots);
         t.fpos = c.take<uint32_t>(P);
     };
-    bool parts = P >= kPartMin && P < 0xFFFFFFFFull && R && R <= kPrepRequests && P / R >= kPartTile && !force;
+    bool parts = P >= kPartMin && P < 0xFFFFFFFFull && R && R <= kPrepRequests && P / R >= kPartTile && !force &&
+                 !too_many_distinct(g, reqs, R, P);
     if (parts) {
         Carve size(nullptr);
         RelParts t{};
