@@ -275,6 +275,9 @@ int grass_sync(grass_graph* g, void* stream) {
     if (!g) return GRASS_EINVAL;
     DeviceGuard guard(g->device);
     hipStream_t s = pick(g, stream);
+    // (the copy below must not become a node of the caller's graph: its target is only this call's)
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return GRASS_EDEVICE;
     // The error word's copy is queued behind the work, so that the host waits once: 64 walks of 10 steps
     // and this call took 41 us with a copy started after the wait, 30 with it queued.
     PinnedWork word;
