@@ -135,7 +135,7 @@ int new_graph(int format, int device, grass_graph** out) {
     }
     int rc = GRASS_OK;
     if (hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess) rc = GRASS_EDEVICE;
-    if (!rc && hipMalloc(&g->d_err, 64) != hipSuccess) rc = GRASS_ENOMEM;
+    if (!rc && device_malloc((void**)&g->d_err, 64) != hipSuccess) rc = GRASS_ENOMEM;
     if (!rc && hipMemset(g->d_err, 0, 64) != hipSuccess) rc = GRASS_EDEVICE;
     if (rc) {
         free_graph(g);
@@ -247,7 +247,7 @@ int grass_device_alloc(grass_graph* g, uint64_t bytes, void** ptr_dev) {
     *ptr_dev = nullptr;
     DeviceGuard guard(g->device);
     if (!guard.ok) return GRASS_EDEVICE;
-    return hipMalloc(ptr_dev, bytes ? bytes : 1) == hipSuccess ? GRASS_OK : GRASS_ENOMEM;
+    return device_malloc(ptr_dev, bytes ? bytes : 1) == hipSuccess ? GRASS_OK : GRASS_ENOMEM;
 }
 
 int grass_device_free(grass_graph* g, void* ptr_dev) {

@@ -197,4 +197,11 @@ hipError_t device_malloc(void** p, size_t bytes) {
     return quiet(hipMalloc(p, bytes));
 }
 
+hipError_t pinned_malloc(void** p, size_t bytes) {
+    hipError_t e = quiet(hipHostMalloc(p, bytes, hipHostMallocDefault));
+    if (e == hipSuccess) return e;
+    if (BlockCache* c = pinned_cache()) c->clear();
+    return quiet(hipHostMalloc(p, bytes, hipHostMallocDefault));
+}
+
 }  // namespace grass

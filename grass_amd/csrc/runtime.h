@@ -15,6 +15,8 @@ namespace grass {
 // hipMalloc that frees the idle working memory kept between calls (pool.cpp) before it fails.  A
 // failure is in the return value only, not in the thread's last error.
 hipError_t device_malloc(void** p, size_t bytes);
+// The same of hipHostMalloc.
+hipError_t pinned_malloc(void** p, size_t bytes);
 
 // Device scratch that grows on demand and is reused across calls (no per-call hipMalloc in
 // steady state).  Guarded by the owning graph's mutex.
@@ -53,7 +55,7 @@ struct PinnedBuf {
             bytes = 0;
         }
         size_t cap = need + need / 2 + 4096;
-        hipError_t e = hipHostMalloc(&ptr, cap, hipHostMallocDefault);
+        hipError_t e = pinned_malloc(&ptr, cap);
         if (e == hipSuccess) bytes = cap;
         return e;
     }

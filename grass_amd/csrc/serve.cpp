@@ -41,7 +41,7 @@ class Arena {
   public:
     hipError_t init(size_t bytes) {
         bytes &= ~(size_t)255;
-        hipError_t e = hipMalloc(&base_, bytes);
+        hipError_t e = device_malloc(&base_, bytes);
         if (e != hipSuccess) return e;
         size_ = bytes;
         free_[0] = bytes;
@@ -602,8 +602,8 @@ int grass_session_create(grass_graph* g, const grass_session_config* cfg, grass_
             hipEventCreateWithFlags(&sl.ev_kh, hipEventDisableTiming) != hipSuccess)
             rc = GRASS_EDEVICE;
         // each slot's kernels record errors in words of their own, read back with the group
-        else if (hipMalloc((void**)&sl.ws_rw.err, 64) != hipSuccess ||
-                 hipMalloc((void**)&sl.ws_kh.err, 64) != hipSuccess || sl.errs.reserve(64) != hipSuccess)
+        else if (device_malloc((void**)&sl.ws_rw.err, 64) != hipSuccess ||
+                 device_malloc((void**)&sl.ws_kh.err, 64) != hipSuccess || sl.errs.reserve(64) != hipSuccess)
             rc = GRASS_ENOMEM;
         else if (hipMemset(sl.ws_rw.err, 0, 64) != hipSuccess || hipMemset(sl.ws_kh.err, 0, 64) != hipSuccess)
             rc = GRASS_EDEVICE;

@@ -129,7 +129,7 @@ int grass_autotune(grass_graph* g, uint32_t what, grass_tuning* chosen, grass_tu
         uint64_t words = 0;
         for (uint32_t i = 0; i < 128; ++i) words += 2048ull * (21 + (i * 37) % 61);
         DevMem out;
-        if (hipMalloc(&out.p, words * 4) != hipSuccess) rc = GRASS_ENOMEM;
+        if (device_malloc(&out.p, words * 4) != hipSuccess) rc = GRASS_ENOMEM;
         uint64_t off = 0;
         for (uint32_t i = 0; i < 128 && !rc; ++i) {
             const uint32_t L = 20 + (i * 37) % 61;
@@ -179,7 +179,7 @@ int grass_autotune(grass_graph* g, uint32_t what, grass_tuning* chosen, grass_tu
                 seeds[j] = (uint32_t)uniform(kTuneSeed, i, (uint32_t)(j - first[i]), kTagStart, 1, n);
         DevMem d_seeds, d_out;
         std::vector<grass_khop_request> reqs(R);
-        if (hipMalloc(&d_seeds.p, seeds.size() * 4) != hipSuccess ||
+        if (device_malloc(&d_seeds.p, seeds.size() * 4) != hipSuccess ||
             hipMemcpy(d_seeds.p, seeds.data(), seeds.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
             rc = GRASS_ENOMEM;
         for (uint32_t i = 0; i < R && !rc; ++i) {
@@ -194,7 +194,7 @@ int grass_autotune(grass_graph* g, uint32_t what, grass_tuning* chosen, grass_tu
         }
         uint64_t cap = 0;
         if (!rc) rc = khop_bound(g, reqs.data(), R, &cap, nullptr, nullptr, nullptr);
-        if (!rc && hipMalloc(&d_out.p, cap * 8 + 8ull * 2 * (R + 1)) != hipSuccess) rc = GRASS_ENOMEM;
+        if (!rc && device_malloc(&d_out.p, cap * 8 + 8ull * 2 * (R + 1)) != hipSuccess) rc = GRASS_ENOMEM;
         Pick pick;
         const uint32_t start = best.khop_lane_scale;
         for (uint32_t sc : {0u, 1u, 2u}) {
@@ -222,8 +222,8 @@ int grass_autotune(grass_graph* g, uint32_t what, grass_tuning* chosen, grass_tu
         (void)hipMemGetInfo(&fr, &tot);
         const uint64_t need = (g->n + 1) * 8 + g->m * 4;
         DevMem rp, col;
-        if (need < fr / 2 && hipMalloc(&rp.p, (g->n + 1) * 8) == hipSuccess &&
-            hipMalloc(&col.p, std::max<uint64_t>(g->m, 1) * 4) == hipSuccess) {
+        if (need < fr / 2 && device_malloc(&rp.p, (g->n + 1) * 8) == hipSuccess &&
+            device_malloc(&col.p, std::max<uint64_t>(g->m, 1) * 4) == hipSuccess) {
             Pick pick;
             const uint32_t start = best.decode_edges_per_wave;
             for (uint32_t e : {512u, 1024u, 2048u, 4096u, 8192u}) {

@@ -34,6 +34,7 @@ def main(module):
     sys.modules["torch"] = None  # its HIP runtime stays out
     fake = C.CDLL(os.environ[CHILD], mode=C.RTLD_GLOBAL)
     fake.fake_limit.argtypes = [C.c_size_t]
+    fake.fake_limit_of.argtypes = [C.c_int, C.c_size_t]
     fake.fake_used.restype = fake.fake_room.restype = fake.fake_copies_in_capture.restype = C.c_size_t
     fake.fake_room.argtypes = [C.c_size_t]
     fake.fake_launches.restype = C.c_char_p

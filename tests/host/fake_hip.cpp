@@ -16,7 +16,7 @@ namespace {
 
 std::recursive_mutex mu;
 std::map<uintptr_t, size_t> live[2];  // device, pinned
-size_t used[2], limit = ~(size_t)0;
+size_t used[2], limit[2] = {~(size_t)0, ~(size_t)0};
 hipError_t last = hipSuccess;
 bool capturing = false;
 size_t copies_in_capture = 0;
@@ -33,7 +33,7 @@ thread_local std::vector<Config> configs;
 hipError_t take(int kind, void** p, size_t bytes) {
     std::lock_guard<std::recursive_mutex> lock(mu);
     *p = nullptr;
-    if (kind == 0 && bytes > limit - used[0]) return last = hipErrorOutOfMemory;
+    if (bytes > limit[kind] - used[kind]) return last = hipErrorOutOfMemory;
     void* m = mmap(nullptr, bytes ? bytes : 1, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
     if (m == MAP_FAILED) return last = hipErrorOutOfMemory;
     live[kind][(uintptr_t)m] = bytes;
@@ -56,11 +56,12 @@ hipError_t give(int kind, void* p) {
 extern "C" {
 
 // ---- for the tests
-// Device memory: `free_bytes` more than is held now.
-void fake_limit(size_t free_bytes) {
+// Device (kind 0) or pinned (1) memory: `free_bytes` more than is held now.
+void fake_limit_of(int kind, size_t free_bytes) {
     std::lock_guard<std::recursive_mutex> lock(mu);
-    limit = free_bytes == ~(size_t)0 ? free_bytes : used[0] + free_bytes;
+    limit[kind] = free_bytes == ~(size_t)0 ? free_bytes : used[kind] + free_bytes;
 }
+void fake_limit(size_t free_bytes) { fake_limit_of(0, free_bytes); }
 size_t fake_used(int kind) {
     std::lock_guard<std::recursive_mutex> lock(mu);
     return used[kind];
@@ -155,7 +156,7 @@ hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 
-void** __hipRegisterFatBinary(const void*) { return (void**)&limit; }
+void** __hipRegisterFatBinary(const void*) { return (void**)limit; }
 void __hipUnregisterFatBinary(void**) {}
 void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*, dim3*, dim3*, int*) {
     names[f] = name;

@@ -20,5 +20,47 @@ def test_sync_of_a_capturing_stream(fake, ga):
     assert ga.lib().grass_sync(g, s) == ga.OK
 
 
+def _idle(fake, ga):
+    """A graph whose building left memory idle, and no other: (graph, bytes idle)."""
+    before = fk.used(fake)
+    g = fk.graph(ga, 1 << 20)
+    idle = fk.used(fake) - before - 20 * (1 << 20)  # (headers and degrees)
+    assert idle > 16 << 20
+    fake.fake_limit(0)
+    return g, idle
+
+
+@fk.on_fake
+def test_device_alloc_on_idle_memory(fake, ga):
+    g, idle = _idle(fake, ga)
+    p = C.c_void_p()
+    assert ga.lib().grass_device_alloc(g, idle // 2, C.byref(p)) == ga.OK
+
+
+@fk.on_fake
+def test_graph_on_idle_memory(fake, ga):
+    g, idle = _idle(fake, ga)
+    fk.graph(ga, 1 << 10)  # (its working memory does not fit any idle block)
+
+
+@fk.on_fake
+def test_session_on_idle_memory(fake, ga):
+    from grass_amd import serve
+    g, idle = _idle(fake, ga)
+    cfg = serve.Config(idle // 2, 4, 1, 1, 1024)
+    s = C.c_void_p()
+    assert serve.lib().grass_session_create(g, C.byref(cfg), C.byref(s)) == ga.OK
+    assert serve.lib().grass_session_destroy(s) == ga.OK
+
+
+@fk.on_fake
+def test_pinned_memory_that_fails(fake, ga):
+    """A failure is in the status alone."""
+    g = fk.graph(ga, 1 << 10)
+    fake.fake_limit_of(1, 0)
+    assert fk.khop(ga, g, [100] * 1000, (2, 2)) == ga.ENOMEM
+    assert fake.hipGetLastError() == 0
+
+
 if __name__ == "__main__":
     fk.main(globals())
