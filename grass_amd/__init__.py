@@ -143,6 +143,7 @@ def lib():
             "grass_open_device_images": (I32, [P, U64, P, U64, I32, I32, P]),
             "grass_compress_device_open": (I32, [P, P, U64, I32, I32, P, P]),
             "grass_close": (I32, [P]),
+            "grass_trim": (I32, [I32]),
             "grass_info": (I32, [P, P]),
             "grass_device_arrays": (I32, [P, P, P, P]),
             "grass_sync": (I32, [P, P]),
@@ -188,6 +189,11 @@ def strerror(status):
 def _check(rc, what):
     if rc != OK:
         raise GrassError(rc, what)
+
+
+def trim(device=0):
+    """Gives back the working memory that calls left idle (grass_trim)."""
+    _check(lib().grass_trim(device), "grass_trim")
 
 
 def _torch():

@@ -213,7 +213,19 @@ int grass_close(grass_graph* g) {
     if (!g) return GRASS_OK;
     DeviceGuard guard(g->device);
     if (g->stream) (void)hipStreamSynchronize(g->stream);
+    const int device = g->device;
     free_graph(g);
+    release_aged(device);
+    return GRASS_OK;
+}
+
+int grass_trim(int device) {
+    int ndev = 0;
+    if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return GRASS_EDEVICE;
+    if (device < 0 || device >= ndev) return GRASS_EINVAL;
+    DeviceGuard guard(device);
+    if (!guard.ok) return GRASS_EDEVICE;
+    release_idle(device);
     return GRASS_OK;
 }
 
@@ -285,6 +297,7 @@ int grass_sync(grass_graph* g, void* stream) {
     uint32_t* err = word.alloc(64) == hipSuccess ? (uint32_t*)word.p : pageable;
     const hipError_t e = hipMemcpyAsync(err, g->d_err, 8, hipMemcpyDeviceToHost, s);
     if (hipStreamSynchronize(s) != hipSuccess || e != hipSuccess) return GRASS_EDEVICE;
+    release_aged(g->device);
     if (err[0] == kErrNone) return GRASS_OK;
     const uint32_t kind = err[0];
     if (hipMemset(g->d_err, 0, 8) != hipSuccess) return GRASS_EDEVICE;
@@ -312,7 +325,9 @@ int grass_random_walk_batch(grass_graph* g, const grass_rw_request* reqs, uint32
     DeviceGuard guard(g->device);
     for (uint32_t i = 0; reqs && i < count; ++i)
         if (reqs[i].walkers && !reqs[i].out_dev) return GRASS_EINVAL;
-    return random_walk_batch(g, reqs, count, seed, pick(g, stream), nullptr);
+    const int rc = random_walk_batch(g, reqs, count, seed, pick(g, stream), nullptr);
+    release_aged(g->device);
+    return rc;
 }
 
 int grass_random_walk_batch_noalloc(grass_graph* g, const grass_rw_request* reqs, uint32_t count,
@@ -333,7 +348,9 @@ int grass_khop_batch(grass_graph* g, const grass_khop_request* reqs, uint32_t co
                      grass_khop_output* out, void* stream) {
     if (!g || (count && !reqs) || !out) return GRASS_EINVAL;
     DeviceGuard guard(g->device);
-    return khop_batch(g, reqs, count, seed, out, pick(g, stream));
+    const int rc = khop_batch(g, reqs, count, seed, out, pick(g, stream));
+    release_aged(g->device);
+    return rc;
 }
 
 int grass_random_walk_bytes(grass_graph* g, const uint32_t* starts_dev, uint64_t walkers,

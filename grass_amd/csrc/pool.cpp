@@ -11,11 +11,15 @@
 // What a block holds is never read by its next owner.  A block enters the cache idle: its owner has
 // waited for the stream it was used on (WorkMem does).  Bounded: at most kDeviceMax bytes idle per
 // GPU (and a sixteenth of its memory) and kPinnedMax of host memory, the longest idle freed first;
-// blocks idle for kKeepSeconds go at the next call that takes or returns one, and all of them when
-// an allocation fails.  Memory that callers own (graphs, results) does not come from here.
+// blocks idle for kKeepSeconds go at the next call that takes or returns one or waits for the device anyway
+// (a program that builds its graph and then samples makes only the latter), and all of them when an
+// allocation fails or the caller asks (grass_trim).  Closing a graph does not free them: the next one
+// is built with them (R-MAT s22 from an edge list: 9 ms, 25 without).  Memory that callers own (graphs,
+// results) does not come from here.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <mutex>
 #include <new>
@@ -103,6 +107,17 @@ class BlockCache {
         release(drop);
     }
 
+    // Frees what is idle for too long (a look at the clock where nothing is).
+    void age() {
+        if (!count_.load(std::memory_order_relaxed)) return;
+        Dropped drop;
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            expire(drop);
+        }
+        release(drop);
+    }
+
    private:
     static constexpr int kMaxBlocks = 64;
     struct Dropped {
@@ -124,17 +139,22 @@ class BlockCache {
         return pinned_ ? hipHostMalloc(p, bytes, hipHostMallocDefault) : hipMalloc(p, bytes);
     }
     void release(const Dropped& drop) {
+        if (!drop.n) return;
+        // (another thread may be capturing a graph, which these calls are no part of)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
         for (int i = 0; i < drop.n; ++i) {
             if (pinned_) (void)hipHostFree(drop.b[i].p);
             else (void)hipFree(drop.b[i].p);
         }
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
     }
 
     const bool pinned_;
     const size_t limit_;
     std::mutex mu_;
     Block idle_[kMaxBlocks];
-    int count_ = 0;
+    std::atomic<int> count_{0};
     size_t held_ = 0;
 };
 
@@ -186,6 +206,16 @@ hipError_t PinnedWork::alloc(size_t need) {
 void PinnedWork::reset() {
     if (p) pinned_cache()->give(p, bytes);
     p = nullptr;
+}
+
+void release_aged(int dev) {
+    if (BlockCache* c = device_cache(dev)) c->age();
+    if (BlockCache* c = pinned_cache()) c->age();
+}
+
+void release_idle(int dev) {
+    if (BlockCache* c = device_cache(dev)) c->clear();
+    if (BlockCache* c = pinned_cache()) c->clear();
 }
 
 hipError_t device_malloc(void** p, size_t bytes) {

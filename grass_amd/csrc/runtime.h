@@ -17,6 +17,10 @@ namespace grass {
 hipError_t device_malloc(void** p, size_t bytes);
 // The same of hipHostMalloc.
 hipError_t pinned_malloc(void** p, size_t bytes);
+// Frees the working memory that has been idle for too long, or all that is idle, of a device and of the
+// host.  Waits for the device if there is any.
+void release_aged(int dev);
+void release_idle(int dev);
 
 // Device scratch that grows on demand and is reused across calls (no per-call hipMalloc in
 // steady state).  Guarded by the owning graph's mutex.

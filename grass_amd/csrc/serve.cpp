@@ -591,6 +591,8 @@ int grass_session_create(grass_graph* g, const grass_session_config* cfg, grass_
         delete s;
         return GRASS_EDEVICE;
     }
+    // (serving calls take and return none of it, so nothing would give it back)
+    grass::release_idle(g->device);
     int rc = s->arena.init(s->cfg.memory_budget) == hipSuccess ? GRASS_OK : GRASS_ENOMEM;
     s->slots.resize(s->cfg.max_inflight);
     for (Slot& sl : s->slots) {

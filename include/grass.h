@@ -82,8 +82,16 @@ int grass_open_device_images(const void *graph_dev, uint64_t graph_bytes, const 
 int grass_compress_device_open(const uint64_t *rowptr_dev, const uint32_t *col_dev, uint64_t n,
                                int format, int device, void *stream, grass_graph **out);
 
-/* Frees every device and host resource of the graph.  NULL is accepted. */
+/* Frees every device and host resource of the graph.  NULL is accepted.  Working memory that building
+ * and MDRW calls left idle is kept for the next ones (grass_trim). */
 int grass_close(grass_graph *g);
+
+/* Frees the working memory that calls left idle on `device` and in pinned host memory (at most 16 GiB and
+ * a sixteenth of the device's, and 256 MB); waits for the device.  Without it, idle blocks go when they
+ * have been so for 10 s and a call takes or returns working memory, closes a graph or waits for the device
+ * (grass_sync, grass_random_walk_batch, grass_khop_batch), when a session is created, or when an
+ * allocation of the library fails: call it where another allocator of the process needs the memory. */
+int grass_trim(int device);
 
 int grass_info(const grass_graph *g, grass_graph_info *info);
 

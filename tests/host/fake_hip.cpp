@@ -6,7 +6,9 @@
 #include <hip/hip_runtime_api.h>
 #include <string.h>
 #include <sys/mman.h>
+#include <time.h>
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <string>
@@ -19,6 +21,7 @@ std::map<uintptr_t, size_t> live[2];  // device, pinned
 size_t used[2], limit[2] = {~(size_t)0, ~(size_t)0};
 hipError_t last = hipSuccess;
 bool capturing = false;
+std::atomic<int64_t> ahead{0};
 size_t copies_in_capture = 0;
 std::map<const void*, std::string> names;
 std::vector<std::string> launches;
@@ -73,6 +76,13 @@ size_t fake_room(uintptr_t p) {
     if (it == live[0].begin()) return 0;
     --it;
     return p < it->first + it->second ? it->first + it->second - p : 0;
+}
+// std::chrono::steady_clock, so many seconds ahead.
+void fake_later(int seconds) { ahead += (int64_t)seconds * 1000000000; }
+int64_t _ZNSt6chrono3_V212steady_clock3nowEv() {
+    struct timespec t;
+    clock_gettime(CLOCK_MONOTONIC, &t);
+    return t.tv_sec * (int64_t)1000000000 + t.tv_nsec + ahead;
 }
 void fake_capturing(int on) { capturing = on; }
 size_t fake_copies_in_capture() { return copies_in_capture; }

@@ -62,5 +62,42 @@ def test_pinned_memory_that_fails(fake, ga):
     assert fake.hipGetLastError() == 0
 
 
+def _left(fake, ga):
+    """A graph on 4096 vertices, with the working memory of a larger one, closed, idle: (graph, bytes idle)."""
+    g = fk.graph(ga, 1 << 12)
+    ga.lib().grass_trim(0)
+    before = fk.used(fake)
+    big = fk.graph(ga, 1 << 20)
+    assert ga.lib().grass_close(big) == ga.OK
+    idle = fk.used(fake) - before
+    assert idle > 16 << 20  # (kept for the next graph)
+    return g, idle
+
+
+@fk.on_fake
+def test_trim(fake, ga):
+    g, idle = _left(fake, ga)
+    before = fk.used(fake)
+    assert ga.lib().grass_trim(0) == ga.OK
+    assert fk.used(fake) == before - idle and fake.fake_used(1) == 0
+    assert ga.lib().grass_trim(-1) == ga.EINVAL and ga.lib().grass_trim(1) == ga.EINVAL
+
+
+@fk.on_fake
+def test_idle_memory_goes(fake, ga):
+    """Blocks idle for 10 s go with the calls of a program that only samples."""
+    def walks(g):
+        r = ga.RwRequest(64, 4, 0, None, 64)
+        return ga.lib().grass_random_walk_batch(g, C.byref(r), 1, 1, None)
+    for call in (lambda g: ga.lib().grass_sync(g, C.c_void_p(4096)), lambda g: fk.khop(ga, g, [100], (2, 2)), walks):
+        g, idle = _left(fake, ga)
+        assert call(g) == ga.OK
+        before = fk.used(fake)
+        assert call(g) == ga.OK and fk.used(fake) == before
+        fake.fake_later(11)
+        assert call(g) == ga.OK
+        assert fk.used(fake) == before - idle
+
+
 if __name__ == "__main__":
     fk.main(globals())
