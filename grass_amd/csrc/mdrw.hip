@@ -711,13 +711,13 @@ __global__ __launch_bounds__(kIndBlock) void mdrw_induced_kernel(DevGraph g, con
                 if (bw.x & bit) dy = (uint32_t)bw.y + (uint32_t)__popcll(bw.x & (bit - 1));
             }
         };
-        // The 64 rows of a window.  With W >= 2 the W / 2 lanes of a row each load 16 bytes of it,
-        // so a row is one memory access instead of one per mask word; the loads land in registers
-        // (fetch_rows) and go to LDS in the per-lane row layout later (stage_rows).
-        const uint32_t cpr = W >> 1, per = W >= 2 ? kWave / cpr : kWave;  // chunks per row, rows per round
+        // The 64 rows of a window.  With more than one word a row (W >= 2, NW > 1) the W / 2 lanes of a row
+        // each load 16 bytes of it, so a row is one memory access instead of one per mask word; the loads
+        // land in registers (fetch_rows) and go to LDS in the per-lane row layout later (stage_rows).
+        const uint32_t cpr = W >> 1, per = NW > 1 ? kWave / cpr : kWave;  // chunks per row, rows per round
         ulonglong2 rv[NW > 1 ? NW / 2 : 1];
         auto fetch_rows = [&](uint32_t dy) {
-            if (NW == 1 || W == 1) {
+            if (NW == 1) {
                 rv[0].x = dy != kNoRow ? rows[dy] : 0ull;
                 return;
             }
@@ -732,10 +732,6 @@ __global__ __launch_bounds__(kIndBlock) void mdrw_induced_kernel(DevGraph g, con
         };
         auto stage_rows = [&]() {
             if (NW == 1) return;
-            if (W == 1) {
-                R[lane * kRowPitch] = rv[0].x;
-                return;
-            }
 #pragma unroll
             for (uint32_t r = 0; r < NW / 2; ++r) {
                 if (r >= cpr) break;
