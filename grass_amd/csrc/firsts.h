@@ -152,7 +152,7 @@ constexpr uint32_t kOneWgPosBits = 13;
 constexpr uint32_t kOneWgWords = kOneWgEntries / kWave;
 
 // Slots for n entries (load <= 2/3), a power of two.
-__host__ __device__ inline uint32_t one_wg_slots(uint32_t n) {
+__host__ __device__ constexpr uint32_t one_wg_slots(uint32_t n) {
     uint32_t slots = 1024;
     while (slots < n + n / 2 + 2) slots <<= 1;
     return slots;

@@ -381,7 +381,8 @@ __global__ __launch_bounds__(kOneWgThreads) void small_front_kernel(In in, Count
 }
 
 // LDS of small_front_kernel for at most n entries.
-static size_t small_front_lds(uint32_t n) { return (size_t)one_wg_slots(n) * 8; }
+static constexpr size_t small_front_lds(uint32_t n) { return (size_t)one_wg_slots(n) * 8; }
+static_assert(small_front_lds(kSmallFront) <= 65536, "a launch of more asks for it first");
 
 // Start of a batch: zeroed scalars, all-one first words, empty table slots.
 __global__ __launch_bounds__(256) void khop_init_kernel(uint64_t* sc, uint32_t nsc, FirstWord* words, uint64_t nwords,
@@ -936,10 +937,6 @@ int khop_enqueue(grass_graph* g, const grass_khop_request* reqs, uint32_t R, uin
     auto small_front = [&](auto in, Count E, const uint64_t* off_r, uint32_t pass, uint32_t h, int k) {
         using In = decltype(in);
         const size_t lds = small_front_lds((uint32_t)(pass ? Dmax : S));
-        if (lds > 65536) {
-            (void)hipFuncSetAttribute((const void*)small_front_kernel<In>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            (void)hipGetLastError();
-        }
         const FrontOut o{d_fv[k], d_fr[k], d_fd[k], d_fc[k], d_eoff, d_etot, d_foff[k], d_icount[k], d_eoff_r, d_hb,
                          out->offsets_dev, h + 1 == H ? ws.result_slot() : nullptr};
         const uint64_t desc_words = (R * sizeof(KhReq) + (R + 1) * 8) / 8;
