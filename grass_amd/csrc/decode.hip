@@ -239,7 +239,7 @@ __device__ __forceinline__ void decode_range(const DevGraph& g, const Src& src, 
 // counts (no row pointers), and the next pass's run ends and headers are requested before the
 // current pass decodes.  Measured on R-MAT, GT s24 (521 M entries) 1.05 -> 0.94 ms, 3.7 TB/s of the
 // 3.5 GB it needs (a copy reaches 4.85); LE s22 (128 M) 0.62 ms with a lane per position, 0.38 by
-// runs, 0.32 with the above.  Loading each lane's header by itself instead of 64 headers and a
+// runs, 0.30 with the above.  Loading each lane's header by itself instead of 64 headers and a
 // shuffle: GT 1.06 ms.
 
 struct RunGen {  // runs of vertex i, from its header

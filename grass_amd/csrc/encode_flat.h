@@ -2,7 +2,7 @@
 // its header, then one per field in stream order (LE: rocks, then seas; GT: list order).  A wave
 // takes consecutive slots, 64 a pass, so lists of any length fill its lanes and the column ids are
 // read in order.  Rows have to be strictly ascending with ids below 2^31 (the plan finds out), which
-// keeps every value in 32 bits.  Bound by instruction issue (about 200 a pass).  Measured on R-MAT s22
+// keeps every value in 32 bits.  Bound by instruction issue (250 to 300 a pass).  Measured on R-MAT s22
 // (2.4 M rows, 128 M entries, GT): a wave per vertex planned in 1.63 ms, wrote the image in 3.65 and made
 // the resident stream of it in 3.2 more; by slots the plan takes 0.71 ms and the stream, straight from the
 // rows, 0.81 (0.84 and 0.91 before passes inside one list kept its constants and skipped the placing).

@@ -10,12 +10,14 @@
 //                 neighbour positions, drawn by Floyd's algorithm with draw k taken from
 //                 Philox(seed, {instance, f, h, k}); edges (f, N_f[pos]) in ascending pos;
 //   frontier h+1 = destinations of hop h, duplicates dropped (first appearance kept).
-// Per hop: one fused count+scan (exclusive scan over items of min(fanout, deg)), a sampling
-// kernel (the c draws of a frontier vertex are made in parallel by c lanes -- in groups of a
+// Per hop: a scan of the frontier's draws min(fanout, deg), which also yields the requests' offsets; a
+// sampling kernel (the c draws of a frontier vertex are made in parallel by c lanes -- in groups of a
 // fixed width, or packed side by side when the hop's vertices often have fewer neighbours than
 // the fanout; Floyd's "taken?" test is resolved in draw order with wave shuffles; ranks give the
-// sorted order), and a dedup of (request, vertex) keys in a hash table where the smallest edge
-// position wins, followed by a flag scan and a compaction into the next frontier.
+// sorted order); and a dedup of (request, vertex) keys in a hash table where the smallest edge
+// position wins, which marks the first appearances as it inserts (firsts.h), followed by a scan of the
+// marks' words and a compaction into the next frontier, with its degrees and draws.  A pass of few
+// entries is one launch of one workgroup, its table in LDS (small_front_kernel).
 // Output is hop-major: edges of (hop h, request r) are [off[h][r], off[h][r+1]).
 #include <hip/hip_runtime.h>
 

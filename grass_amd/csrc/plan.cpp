@@ -2,12 +2,13 @@
 // and replayed as one submission.
 //
 // A steady-state sampling loop (the same request shapes every step, new seed vertices written
-// into the same device buffers) pays the ~30 kernel launches of a 2-hop pipeline plus the walk
+// into the same device buffers) pays the launches of a 2-hop pipeline (16, a small one four) plus the walk
 // launch every step.  A plan runs the batch once eagerly (which sizes every workspace, so that
 // nothing allocates while capturing), then captures it with the walks and the k-hop pipeline on
 // two branches forked from the launch stream and joined back into it, and instantiates the graph.
-// Each replay starts with a clear of the k-hop dedup tables (the captured pipeline uses the 16-byte
-// table's first generations), so replays are independent of each other and of any eager call.
+// Each replay clears the k-hop dedup tables it uses (the packed ones at its start or before a pass that
+// shares one, the 16-byte one at its start, whose first generations the pipeline takes; passes in LDS need
+// none), so replays are independent of each other and of any eager call.
 #include <hip/hip_runtime.h>
 #include <string.h>
 
