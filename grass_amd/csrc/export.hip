@@ -562,12 +562,11 @@ constexpr uint64_t kPartDistinct = (uint64_t)kPartBuckets * (kPartSlots / 4 * 3)
 // One workgroup per tile: counts its buckets' positions (SCATTER: takes room for them in each bucket,
 // and writes them there).
 template <bool SCATTER>
-__global__ __launch_bounds__(kPartBlock) void rel_part_kernel(RelSeq q, RelParts t, uint32_t* err,
-                                                              const uint32_t* __restrict__ invalid) {
+__global__ __launch_bounds__(kPartBlock) void rel_part_kernel(RelSeq q, RelParts t, uint32_t* err) {
     __shared__ uint32_t hist[kPartBuckets];
     __shared__ uint64_t beg[GRASS_KHOP_MAX_HOPS + 1];
     __shared__ const uint32_t* arr[GRASS_KHOP_MAX_HOPS + 1];
-    if (blockIdx.x >= t.tile0[q.R] || (SCATTER && *invalid)) return;
+    if (blockIdx.x >= t.tile0[q.R]) return;
     uint32_t r = 0;
     for (uint32_t hi = q.R - 1; r < hi;) {  // the last request whose first tile is not after this one
         const uint32_t mid = r + (hi - r + 1) / 2;
@@ -644,27 +643,44 @@ __device__ __forceinline__ uint32_t part_insert(unsigned long long* tab, unsigne
 }
 
 // The buckets' counts become their starts (one workgroup).  *invalid |= 2: few buckets hold so many
-// positions that the workgroups of these would be the time (kPartMost).
-__global__ __launch_bounds__(1024) void rel_part_starts_kernel(uint32_t* bend, uint32_t nb, uint32_t* invalid) {
-    __shared__ uint32_t lds[1024 / kWave];
-    __shared__ uint64_t lds64[1024 / kWave];
-    const uint32_t per = (nb + 1023) / 1024, lo = threadIdx.x * per, hi = min(lo + per, nb);
-    uint32_t s = 0, largest = 0, total;
-    uint64_t past = 0;  // positions that are not held
+// positions that the workgroups of these would be the time (kPartMost); no tile and no bucket is left then.
+__global__ __launch_bounds__(1024) void rel_part_starts_kernel(uint32_t* bend, uint32_t nb, uint32_t* tiles,
+                                                               uint32_t* buckets, uint32_t* invalid) {
+    constexpr uint32_t kWaves = 1024 / kWave;
+    __shared__ uint32_t sums[kWaves], most[kWaves], past[kWaves];
+    const uint32_t per = (nb + 1023) / 1024, lo = threadIdx.x * per, hi = min(lo + per, nb), wid = threadIdx.x / kWave;
+    uint32_t sum = 0, m = 0, p = 0;  // the counts, the largest, and the positions that are not held
     for (uint32_t i = lo; i < hi; ++i) {
         const uint32_t c = bend[i];
-        s += c;
-        largest = max(largest, c);
-        past += c > kPartHeldAll ? c - kPartHeldAll : 0u;
+        sum += c;
+        m = max(m, c);
+        p += c > kPartHeldAll ? c - kPartHeldAll : 0u;
     }
-    largest = block_max<uint32_t, 1024>(largest, lds);
-    past = block_sum<uint64_t, 1024>(past, lds64);
-    if (threadIdx.x == 0 && largest > kPartMost && 3ull * largest > past) atomicOr(invalid, 2u);
-    uint32_t pre = block_exclusive_sum<uint32_t, 1024>(s, total, lds);
+    const uint32_t inc = wave_inclusive_sum(sum);
+    m = wave_max(m);
+    p = wave_sum(p);
+    if (lane_id() == kWave - 1) {
+        sums[wid] = inc;
+        most[wid] = m;
+        past[wid] = p;
+    }
+    __syncthreads();
+    uint32_t pre = inc - sum;
+    for (uint32_t w = 0; w < wid; ++w) pre += sums[w];
     for (uint32_t i = lo; i < hi; ++i) {
         const uint32_t c = bend[i];
         bend[i] = pre;
         pre += c;
+    }
+    if (threadIdx.x == 0) {
+        for (uint32_t w = 1; w < kWaves; ++w) {
+            m = max(m, most[w]);
+            p += past[w];
+        }
+        if (m > kPartMost && 3ull * m > p) {
+            *invalid |= 2u;
+            *tiles = *buckets = 0;
+        }
     }
 }
 
@@ -673,10 +689,8 @@ __global__ __launch_bounds__(1024) void rel_part_starts_kernel(uint32_t* bend, u
 // loads at a time.  *invalid |= 2: more distinct keys than slots.
 __global__ __launch_bounds__(kPartBlock) void rel_part_dedup_kernel(RelSeq q, RelParts t, uint32_t* invalid) {
     __shared__ unsigned long long tab[kPartSlots];
-    __shared__ uint32_t stop;  // (other workgroups may be setting it)
     const uint32_t k = blockIdx.x;
     if (k >= t.bkt0[q.R]) return;
-    if (threadIdx.x == 0) stop = *(volatile uint32_t*)invalid;
     const uint32_t lo = (k ? t.bend[k - 1] : 0u) + threadIdx.x, hi = t.bend[k];
     unsigned long long w[kPartHeld];
     uint32_t s[kPartHeld];
@@ -705,7 +719,6 @@ __global__ __launch_bounds__(kPartBlock) void rel_part_dedup_kernel(RelSeq q, Re
     load(lo);
     for (uint32_t i = threadIdx.x; i < kPartSlots; i += kPartBlock) tab[i] = ~0ull;
     __syncthreads();
-    if (stop) return;
     bool full = false;
     if (lo + kPartHeldAll < hi) {
         for (uint32_t i = lo + kPartHeldAll; i < hi; i += kPartHeldAll) {
@@ -744,9 +757,10 @@ hipError_t rel_build_parts(const RelParts& t, uint32_t maxb, const RelSeq& q, ui
     uint32_t* d_invalid = d_bad + 1;
     hipLaunchKernelGGL(rel_part_prepare_kernel, dim3(1 + (unsigned)std::min<uint64_t>(P / 16384 + 1, 512)), dim3(1024), 0, s, t,
                        maxb, q.off, q.req, q.R, q.H, b->total, P, const_cast<uint64_t*>(q.Q), d_bad, d_invalid);
-    hipLaunchKernelGGL(rel_part_kernel<false>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad, (const uint32_t*)d_invalid);
-    hipLaunchKernelGGL(rel_part_starts_kernel, dim3(1), dim3(1024), 0, s, t.bend, maxb, d_invalid);
-    hipLaunchKernelGGL(rel_part_kernel<true>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad, (const uint32_t*)d_invalid);
+    hipLaunchKernelGGL(rel_part_kernel<false>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad);
+    hipLaunchKernelGGL(rel_part_starts_kernel, dim3(1), dim3(1024), 0, s, t.bend, maxb,
+                       const_cast<uint32_t*>(t.tile0) + q.R, const_cast<uint32_t*>(t.bkt0) + q.R, d_invalid);
+    hipLaunchKernelGGL(rel_part_kernel<true>, dim3(tiles), dim3(kPartBlock), 0, s, q, t, d_bad);
     hipLaunchKernelGGL(rel_part_dedup_kernel, dim3(maxb), dim3(kPartBlock), 0, s, q, t, d_invalid);
     const unsigned gP = (unsigned)std::min<uint64_t>((P + kExBlock - 1) / kExBlock + 1, kExGrid);
     hipLaunchKernelGGL(rel_part_words_kernel, dim3(gP), dim3(kExBlock), 0, s, (const uint32_t*)t.fpos, P, d_words);
