@@ -898,7 +898,8 @@ int khop_blocks(grass_graph* g, const grass_khop_request* reqs, uint32_t R, cons
         t.tab = c.take<unsigned long long>((uint64_t)maxb * kPartSlots);
         t.fpos = c.take<uint32_t>(P);
     };
-    bool parts = P >= kPartMin && P < 0xFFFFFFFFull && R && R <= kPrepRequests && P / R >= kPartTile && !force &&
+    // (a workgroup counts on in 32 bits past its bucket's last position)
+    bool parts = P >= kPartMin && P + kPartHeldAll <= 0xFFFFFFFFull && R && R <= kPrepRequests && P / R >= kPartTile && !force &&
                  !too_many_distinct(g, reqs, R, P);
     if (parts) {
         Carve size(nullptr);

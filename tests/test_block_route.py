@@ -37,5 +37,14 @@ def test_few_vertices(fake, ga):
     assert _parts(fake, ga, g, [DISTINCT * 3], 10, (1,))
 
 
+@fk.on_fake
+def test_positions_near_the_end_of_32_bits(fake, ga):
+    """A bucket's positions are counted by 4096 in 32 bits."""
+    g = fk.graph(ga, 1 << 12)
+    last = 2 ** 32 - 4096 - 1
+    assert _parts(fake, ga, g, [2 ** 31, last - 2 ** 31 - 5], 5, (1,))
+    assert not _parts(fake, ga, g, [2 ** 31, last - 2 ** 31 - 4], 5, (1,))
+
+
 if __name__ == "__main__":
     fk.main(globals())
